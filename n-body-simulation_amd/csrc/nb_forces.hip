@@ -8,7 +8,7 @@
 //                  same push order, same opening test)
 // FP32 kernels do the pair arithmetic in FP32 (fmaf, v_rsq_f32) and fold the
 // FP32 partial of every tile into FP64 accumulators:
-//   k_direct_f32c  LDS-staged source tiles, two targets per lane, split j
+//   k_direct_f32c  sources staged in LDS per wave, two targets per lane, split j
 //   k_bh_group     one wavefront per group (an octree cell of <= 64 bodies);
 //                  a cell is opened if any body of the group needs it; lanes
 //                  test 8 sibling sets at a time and accepted cells/bodies are
@@ -136,34 +136,50 @@ __global__ void __launch_bounds__(kF64Threads) k_direct_targets_f64(
 }
 
 // ---------------------------------------------------------------------------
-// Split direct sums: FP32 pairs with FP64 tile accumulation (k_direct_f32c),
-// and FP64 pairs with a corrected v_rsq_f64 (k_direct_f64f).
+// Split direct sums: FP32 pairs with FP64 accumulation (k_direct_f32c), and
+// FP64 pairs with a corrected v_rsq_f64 (k_direct_f64f).
 //
-// grid.x: tiles of kSplitTargets targets (kSplitPerLane per lane); grid.y:
-// source splits, each a contiguous source range.  Sources are staged in LDS
-// kSplitTile at a time, converted from the FP64 state arrays on the way (no
-// separate packing pass).  With one split a block writes its targets' sums;
-// with more, each block stores its partial sums and k_split_reduce adds them
-// in split order 0, 1, ..., so results do not depend on block timing.  (The
-// partials can also be added by the last block of each tile to arrive, but
-// the device-scope fence each block then needs writes back the L2: the
-// 16,384-body FP32 sum took 232 us that way against 98 us.)
-constexpr int kSplitThreads = 256;
-constexpr int kSplitPerLane = 2;  // targets per lane (each LDS read feeds 2 pairs)
-constexpr uint32_t kSplitTargets = kSplitThreads * kSplitPerLane;
-constexpr int kSplitTile = 256;   // sources per LDS stage
-constexpr uint32_t kSplitBlocks = 2048;  // blocks a launch aims for (2 per SIMD)
-// sources per interleaved FP64 step (x kSplitPerLane targets): 124 VGPRs, four
-// waves per SIMD; 2 (72 VGPRs, seven waves) and 8 (240) measured within 2 %,
-// five waves forced (spilling) 15 % slower
-constexpr int kF64fSources = 4;
-static_assert(kSplitTile % kF64fSources == 0, "whole steps per stage");
+// grid.x: tiles of 64 targets per lane's target (the same for all waves of a
+// block); grid.y: source splits, each a contiguous source range.  A block's
+// waves share the range: each stages kSplitTile sources of its own at a time in
+// LDS, converted from the FP64 state arrays on the way, with the next stage's
+// loads in flight, and no barrier until the waves' sums are added at the end.
+// With one split a block writes its targets' sums; with more it stores partial
+// sums and k_split_reduce adds them in split order 0, 1, ..., so results do not
+// depend on block timing.
+constexpr int kSplitWaves = 4;
+constexpr int kSplitThreads = 64 * kSplitWaves;
+constexpr uint32_t kSplitTile = 64;  // sources per stage of one wave
+constexpr int kF32cRun = 4;          // stages per FP32 sum
+constexpr int kF64fPerLane = 2;      // targets per lane: each LDS read feeds two pairs
+// Partial sums of a launch, at most (3 * 8 bytes each: 24 MiB).  A SIMD serves
+// its oldest waves first, so the waves resident at the end finish one after the
+// other with ever fewer to overlap: more blocks than fit at once (8 per CU)
+// keep it filled.
+constexpr uint32_t kSplitPartials = 1u << 20;
+// Pairs per interleaved step: FP32 four in 53 VGPRs, eight waves per SIMD (eight
+// pairs: 70 VGPRs and within 2 %); FP64 eight in 124 VGPRs, four waves (four
+// pairs within 1 %).
+constexpr int kF32cPairs = 4;
+constexpr int kF64fPairs = 8;
+
+// v_rsq_f32 with an s_nop on each side.  With two or more waves on a SIMD, two
+// waves' FP32 instructions issue at once (2.4 cycles at 2.4 GHz per wave
+// instruction instead of 4.2), but a v_rsq_f32 next to other vector
+// instructions ends that for the instructions around it as well: one pair (12
+// instructions and the v_rsq_f32) takes 53-57 cycles per 64 pairs, and 36-38
+// with the two wait states.  The same instruction, so the same bits.
+__device__ __forceinline__ float rsq_f32(float v) {
+    float y;
+    asm("s_nop 0\n\tv_rsq_f32 %0, %1\n\ts_nop 0" : "=v"(y) : "v"(v));
+    return y;
+}
 
 __device__ inline void pair_f32(const float4 s, float px, float py, float pz, float eps2,
                                 float &fx, float &fy, float &fz) {
     const float dx = s.x - px, dy = s.y - py, dz = s.z - pz;
     const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-    const float inv = __builtin_amdgcn_rsqf(r2);
+    const float inv = rsq_f32(r2);
     const float f = (s.w * inv) * (inv * inv);
     fx = fmaf(f, dx, fx);
     fy = fmaf(f, dy, fy);
@@ -184,47 +200,51 @@ __device__ inline double rsqrt_f64(double v) {
     return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
-__device__ inline void pair_f64f(const double4 s, double px, double py, double pz, double eps2,
-                                 double &fx, double &fy, double &fz) {
-    const double dx = s.x - px, dy = s.y - py, dz = s.z - pz;
-    const double r2 = fma(dx, dx, fma(dy, dy, fma(dz, dz, eps2)));
-    const double inv = rsqrt_f64(r2);
-    const double f = (s.w * inv) * (inv * inv);
-    fx = fma(f, dx, fx);
-    fy = fma(f, dy, fy);
-    fz = fma(f, dz, fz);
+// w v^(-3/2) from the same estimate: with y2 = y^2 and e = 1 - v y2,
+// v^(-3/2) = y^3 (1 - e)^(-3/2) = y^3 (1 + 3e/2 + 15e^2/8 + ...), truncation
+// near 35e^3/16 ~ 1e-23.  The rounding of y2 enters the factor y2 and, with
+// weight -3/2, e, so half of it remains.  Seven operations after the estimate.
+__device__ inline double rsqrt3_f64(double w, double v) {
+    const double y = __builtin_amdgcn_rsq(v);
+    const double y2 = y * y;
+    const double e = fma(-v, y2, 1.0);
+    const double t = (w * y) * y2;
+    return fma(t * e, fma(e, 1.875, 1.5), t);
 }
 
-__device__ inline uint32_t split_target(uint32_t q) {
-    return blockIdx.x * kSplitTargets + q * kSplitThreads + threadIdx.x;
-}
-
-// End of a split direct sum for this lane's targets: with one split the
-// block writes scale * sums; with more it stores its partial sums at
+// The end of a split direct sum: adds the waves' sums in wave order; with one
+// split the block writes scale * sums, with more it stores its partial sums at
 // partial[split][3][n] for k_split_reduce.
-__device__ inline void split_finish(uint32_t n, double scale, const double (&sx)[kSplitPerLane],
-                                    const double (&sy)[kSplitPerLane],
-                                    const double (&sz)[kSplitPerLane], double *partial,
-                                    double *out_x, double *out_y, double *out_z) {
-    const bool direct = gridDim.y == 1;
-    const uint64_t base = (uint64_t)blockIdx.y * 3ull * n;
+template <int PL>
+__device__ __forceinline__ void split_finish(uint32_t n, double scale, const double (&sx)[PL],
+                                             const double (&sy)[PL], const double (&sz)[PL],
+                                             double *comb, double *partial, double *out_x,
+                                             double *out_y, double *out_z) {
+    constexpr uint32_t kTargets = 64 * PL;
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    __syncthreads();  // comb lies over the waves' stages
 #pragma unroll
-    for (int q = 0; q < kSplitPerLane; ++q) {
-        const uint32_t i = split_target(q);
+    for (int q = 0; q < PL; ++q) {
+        double *c = comb + (w * 3) * kTargets + q * 64 + lane;
+        c[0] = sx[q];
+        c[kTargets] = sy[q];
+        c[2 * kTargets] = sz[q];
+    }
+    __syncthreads();
+    for (uint32_t k = threadIdx.x; k < 3 * kTargets; k += kSplitThreads) {
+        const uint32_t d = k / kTargets, t = k % kTargets;
+        double v = comb[k];
+#pragma unroll
+        for (int o = 1; o < kSplitWaves; ++o) v += comb[(o * 3) * kTargets + k];
+        const uint64_t i = (uint64_t)blockIdx.x * kTargets + t;
         if (i >= n) continue;
-        if (direct) {
-            out_x[i] = sx[q] * scale;
-            out_y[i] = sy[q] * scale;
-            out_z[i] = sz[q] * scale;
-        } else {
-            partial[base + i] = sx[q];
-            partial[base + n + i] = sy[q];
-            partial[base + 2ull * n + i] = sz[q];
-        }
+        if (gridDim.y == 1) (d == 0 ? out_x : (d == 1 ? out_y : out_z))[i] = v * scale;
+        else partial[((uint64_t)blockIdx.y * 3ull + d) * n + i] = v;
     }
 }
 
-// out = scale * (sum over splits 0, 1, ... in that order) of the partial sums.
+// out = scale * (sum over splits 0, 1, ... in that order) of the partial
+// sums; blockIdx.y is the component.
 __global__ void __launch_bounds__(kSplitThreads) k_split_reduce(uint32_t n, uint32_t splits,
                                                                 double scale,
                                                                 const double *__restrict__ partial,
@@ -232,105 +252,169 @@ __global__ void __launch_bounds__(kSplitThreads) k_split_reduce(uint32_t n, uint
                                                                 double *out_z) {
     const uint32_t i = blockIdx.x * kSplitThreads + threadIdx.x;
     if (i >= n) return;
-    double ox = 0, oy = 0, oz = 0;
-    // eight splits' loads in flight before their (ordered) additions: one
-    // wave per CU at 16,384 bodies, so the loads' latency is not hidden by
-    // other waves (18.8 us with one split at a time)
+    const double *__restrict__ p = partial + (uint64_t)blockIdx.y * n + i;
+    const uint64_t stride = 3ull * n;
+    double o = 0;
+    // eight splits' loads in flight before their (ordered) additions
     constexpr uint32_t kAhead = 8;
     uint32_t sp = 0;
     for (; sp + kAhead <= splits; sp += kAhead) {
-        double vx[kAhead], vy[kAhead], vz[kAhead];
+        double v[kAhead];
 #pragma unroll
-        for (uint32_t u = 0; u < kAhead; ++u) {
-            const uint64_t b = (uint64_t)(sp + u) * 3ull * n;
-            vx[u] = partial[b + i];
-            vy[u] = partial[b + n + i];
-            vz[u] = partial[b + 2ull * n + i];
-        }
+        for (uint32_t u = 0; u < kAhead; ++u) v[u] = p[(sp + u) * stride];
 #pragma unroll
-        for (uint32_t u = 0; u < kAhead; ++u) {
-            ox += vx[u];
-            oy += vy[u];
-            oz += vz[u];
-        }
+        for (uint32_t u = 0; u < kAhead; ++u) o += v[u];
     }
-    for (; sp < splits; ++sp) {
-        const uint64_t b = (uint64_t)sp * 3ull * n;
-        ox += partial[b + i];
-        oy += partial[b + n + i];
-        oz += partial[b + 2ull * n + i];
-    }
-    out_x[i] = ox * scale;
-    out_y[i] = oy * scale;
-    out_z[i] = oz * scale;
+    for (; sp < splits; ++sp) o += p[sp * stride];
+    (blockIdx.y == 0 ? out_x : (blockIdx.y == 1 ? out_y : out_z))[i] = o * scale;
 }
 
-// FP32 pairs on absolute FP32 positions with G*m as the source weight; each
-// stage's FP32 sums are folded into FP64.
-__global__ void __launch_bounds__(kSplitThreads) k_direct_f32c(
-    uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
-    const double *__restrict__ z, const double *__restrict__ m, double G, float eps2,
-    uint32_t chunk, double *partial, double *ax_out, double *ay_out, double *az_out) {
-    __shared__ float4 tile[kSplitTile];
-    float px[kSplitPerLane], py[kSplitPerLane], pz[kSplitPerLane];
-    double ax[kSplitPerLane], ay[kSplitPerLane], az[kSplitPerLane];
+// One wave's walk over its share of the block's sources [j0, j1): runs of kRun
+// stages of kSplitTile sources, the first at j0 + w kRun kSplitTile and
+// kSplitWaves runs apart.  use(cnt) gets a stage of cnt sources, padded to
+// kSplitTile with sources of zero mass; end_run() follows a run's last stage;
+// pack converts one source.
+template <int kRun, typename T4, typename Pack, typename Use, typename EndRun>
+__device__ __forceinline__ void split_stages(uint32_t j0, uint32_t j1,
+                                             const double *__restrict__ x,
+                                             const double *__restrict__ y,
+                                             const double *__restrict__ z,
+                                             const double *__restrict__ m, T4 *stage, T4 pad,
+                                             Pack pack, Use use, EndRun end_run) {
+    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    constexpr uint32_t run = kRun * kSplitTile;
+    double sx = 0, sy = 0, sz = 0, sm = 0;
+    auto load = [&](uint32_t j) {
+        if (j < j1) {
+            sx = x[j];
+            sy = y[j];
+            sz = z[j];
+            sm = m[j];
+        }
+    };
+    uint32_t k = j0 + w * run, end = k + run;
+    load(k + lane);
+    while (k < j1) {
+        const T4 p = pack(sx, sy, sz, sm);
+        stage[lane] = k + lane < j1 ? p : pad;
+        const uint32_t cnt = min(kSplitTile, j1 - k);
+        k += kSplitTile;
+        const bool last = k == end || k >= j1;
+        if (k == end) {
+            k += (kSplitWaves - 1) * run;
+            end = k + run;
+        }
+        load(k + lane);  // the next stage's, while this one is used
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        use(cnt);
+        if (last) end_run();
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+// FP32 pairs on absolute FP32 positions with G*m as the source weight; the
+// FP32 sums of every 256 sources (kF32cRun stages, from a multiple of 256) are
+// folded into FP64.  Bound by vector issue: 50,021 bodies in 0.703 ms (0.773
+// with 256-source stages shared by a block and no wait states around the
+// v_rsq_f32), 43 cycles at 2.4 GHz per 64 pairs, where a loop of such pairs alone takes 36-38.
+// PL: targets per lane, 1 for small sums (twice the waves).
+template <int PL>
+__global__ void __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(8)))
+k_direct_f32c(uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
+              const double *__restrict__ z, const double *__restrict__ m, double G, float eps2,
+              uint32_t chunk, double *partial, double *ax_out, double *ay_out, double *az_out) {
+    __shared__ double comb[kSplitWaves * 3 * 64 * PL];
+    static_assert(sizeof(float4) * kSplitTile * kSplitWaves <= sizeof(comb), "stages fit");
+    const uint32_t lane = threadIdx.x & 63u;
+    float4 *stage = reinterpret_cast<float4 *>(comb) + (threadIdx.x >> 6) * kSplitTile;
+    asm("" : "+v"(eps2));  // a scalar operand would end the double issue
+    float px[PL], py[PL], pz[PL], fx[PL], fy[PL], fz[PL];
+    double ax[PL], ay[PL], az[PL];
 #pragma unroll
-    for (int q = 0; q < kSplitPerLane; ++q) {
-        const uint32_t i = split_target(q);
+    for (int q = 0; q < PL; ++q) {
+        const uint32_t i = blockIdx.x * 64 * PL + q * 64 + lane;
         const uint32_t ii = i < n ? i : n - 1;
         px[q] = (float)x[ii];
         py[q] = (float)y[ii];
         pz[q] = (float)z[ii];
         ax[q] = ay[q] = az[q] = 0.0;
+        fx[q] = fy[q] = fz[q] = 0.f;
     }
     const uint32_t j0 = blockIdx.y * chunk;
     const uint32_t j1 = min(n, j0 + chunk);
-    for (uint32_t k = j0; k < j1; k += kSplitTile) {
-        const uint32_t j = k + threadIdx.x;
-        if (j < j1)
-            tile[threadIdx.x] =
-                make_float4((float)x[j], (float)y[j], (float)z[j], (float)(G * m[j]));
-        __syncthreads();
-        float fx[kSplitPerLane], fy[kSplitPerLane], fz[kSplitPerLane];
+    split_stages<kF32cRun, float4>(
+        j0, j1, x, y, z, m, stage, make_float4(1e30f, 0.f, 0.f, 0.f),
+        [&](double sx, double sy, double sz, double sm) {
+            return make_float4((float)sx, (float)sy, (float)sz, (float)(G * sm));
+        },
+        [&](uint32_t cnt) {
+            // kF32cPairs pairs at a time, stage by stage across the pairs, so
+            // that neighbouring instructions are independent; the same
+            // operations per pair as pair_f32
+            constexpr int kSources = kF32cPairs / PL;
+            static_assert(kSplitTile % kSources == 0, "whole steps per stage");
+            for (uint32_t jj = 0; jj < cnt; jj += kSources) {
+                float dx[kF32cPairs], dy[kF32cPairs], dz[kF32cPairs], inv[kF32cPairs],
+                    wt[kF32cPairs];
 #pragma unroll
-        for (int q = 0; q < kSplitPerLane; ++q) fx[q] = fy[q] = fz[q] = 0.f;
-        auto pairs = [&](int jj) {
-            const float4 sj = tile[jj];
+                for (int u = 0; u < kSources; ++u) {
+                    const float4 sj = stage[jj + u];
 #pragma unroll
-            for (int q = 0; q < kSplitPerLane; ++q)
-                pair_f32(sj, px[q], py[q], pz[q], eps2, fx[q], fy[q], fz[q]);
-        };
-        const uint32_t cnt = min((uint32_t)kSplitTile, j1 - k);  // uniform
-        if (cnt == (uint32_t)kSplitTile) {
-#pragma unroll 8
-            for (int jj = 0; jj < kSplitTile; ++jj) pairs(jj);
-        } else {
-            for (uint32_t jj = 0; jj < cnt; ++jj) pairs((int)jj);
-        }
+                    for (int q = 0; q < PL; ++q) {
+                        const int p = u * PL + q;
+                        dx[p] = sj.x - px[q];
+                        dy[p] = sj.y - py[q];
+                        dz[p] = sj.z - pz[q];
+                        wt[p] = sj.w;
+                        inv[p] = fmaf(dx[p], dx[p], fmaf(dy[p], dy[p], fmaf(dz[p], dz[p], eps2)));
+                    }
+                }
 #pragma unroll
-        for (int q = 0; q < kSplitPerLane; ++q) {
-            ax[q] += (double)fx[q];
-            ay[q] += (double)fy[q];
-            az[q] += (double)fz[q];
-        }
-        __syncthreads();
-    }
-    split_finish(n, 1.0, ax, ay, az, partial, ax_out, ay_out, az_out);
+                for (int p = 0; p < kF32cPairs; ++p) inv[p] = rsq_f32(inv[p]);
+#pragma unroll
+                for (int u = 0; u < kSources; ++u)
+#pragma unroll
+                    for (int q = 0; q < PL; ++q) {
+                        const int p = u * PL + q;
+                        const float f = (wt[p] * inv[p]) * (inv[p] * inv[p]);
+                        fx[q] = fmaf(f, dx[p], fx[q]);
+                        fy[q] = fmaf(f, dy[p], fy[q]);
+                        fz[q] = fmaf(f, dz[p], fz[q]);
+                    }
+            }
+        },
+        [&] {
+#pragma unroll
+            for (int q = 0; q < PL; ++q) {
+                ax[q] += (double)fx[q];
+                ay[q] += (double)fy[q];
+                az[q] += (double)fz[q];
+                fx[q] = fy[q] = fz[q] = 0.f;
+            }
+        });
+    split_finish<PL>(n, 1.0, ax, ay, az, comb, partial, ax_out, ay_out, az_out);
 }
 
-// FP64 pairs (the reference's formula, NaiveAlgorithm.cpp:318-351, with the
-// inverse square root from rsqrt_f64 and fused multiply-adds); G is applied
-// to the sum, as in the reference (:348-351).
+// FP64 pairs (the reference's formula, NaiveAlgorithm.cpp:318-351, with
+// m r^-3 from rsqrt3_f64 and fused multiply-adds); G is applied to the sum, as
+// in the reference (:348-351).  Bound by vector issue: 16 full-rate FP64
+// instructions and the quarter-rate estimate, 80 cycles per 64 pairs; 16,384
+// bodies in 0.169-0.173 ms (0.172-0.176 before), 3001 in 0.019 ms (0.052).
 __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
     uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, double G, double eps2,
     uint32_t chunk, double *partial, double *ax_out, double *ay_out, double *az_out) {
-    __shared__ double4 tile[kSplitTile];
-    double px[kSplitPerLane], py[kSplitPerLane], pz[kSplitPerLane];
-    double ax[kSplitPerLane], ay[kSplitPerLane], az[kSplitPerLane];
+    __shared__ double comb[kSplitWaves * 3 * 64 * kF64fPerLane];
+    static_assert(sizeof(double4) * kSplitTile * kSplitWaves <= sizeof(comb), "stages fit");
+    const uint32_t lane = threadIdx.x & 63u;
+    double4 *stage = reinterpret_cast<double4 *>(comb) + (threadIdx.x >> 6) * kSplitTile;
+    double px[kF64fPerLane], py[kF64fPerLane], pz[kF64fPerLane];
+    double ax[kF64fPerLane], ay[kF64fPerLane], az[kF64fPerLane];
 #pragma unroll
-    for (int q = 0; q < kSplitPerLane; ++q) {
-        const uint32_t i = split_target(q);
+    for (int q = 0; q < kF64fPerLane; ++q) {
+        const uint32_t i = blockIdx.x * 64 * kF64fPerLane + q * 64 + lane;
         const uint32_t ii = i < n ? i : n - 1;
         px[q] = x[ii];
         py[q] = y[ii];
@@ -339,60 +423,45 @@ __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
     }
     const uint32_t j0 = blockIdx.y * chunk;
     const uint32_t j1 = min(n, j0 + chunk);
-    for (uint32_t k = j0; k < j1; k += kSplitTile) {
-        const uint32_t j = k + threadIdx.x;
-        if (j < j1) tile[threadIdx.x] = make_double4(x[j], y[j], z[j], m[j]);
-        __syncthreads();
-        auto pairs = [&](int jj) {
-            const double4 sj = tile[jj];
+    split_stages<1, double4>(
+        j0, j1, x, y, z, m, stage, make_double4(0x1.3p+400, 0.0, 0.0, 0.0),
+        [&](double sx, double sy, double sz, double sm) { return make_double4(sx, sy, sz, sm); },
+        [&](uint32_t cnt) {
+            // stage by stage across the pairs: the compiler otherwise runs each
+            // pair's chain (the estimate, its correction, the force) to the end
+            // before the next pair starts
+            constexpr int kSources = kF64fPairs / kF64fPerLane;
+            static_assert(kSplitTile % kSources == 0, "whole steps per stage");
+            for (uint32_t jj = 0; jj < cnt; jj += kSources) {
+                double dx[kF64fPairs], dy[kF64fPairs], dz[kF64fPairs], r2[kF64fPairs], f[kF64fPairs];
 #pragma unroll
-            for (int q = 0; q < kSplitPerLane; ++q)
-                pair_f64f(sj, px[q], py[q], pz[q], eps2, ax[q], ay[q], az[q]);
-        };
-        // kF64fSources sources x kSplitPerLane targets, stage by stage across the
-        // pairs: the compiler otherwise runs each pair's chain (the estimate,
-        // its five-step correction, the force) to the end before the next
-        // pair starts.  The same operations per pair as pair_f64f, and each
-        // target's sum still runs over the sources in order: bit-identical.
-        auto pairs_s = [&](int jj) {
-            constexpr int P = kF64fSources * kSplitPerLane;
-            double dx[P], dy[P], dz[P], r2[P], yv[P], w[P];
+                for (int u = 0; u < kSources; ++u) {
+                    const double4 sj = stage[jj + u];
 #pragma unroll
-            for (int u = 0; u < kF64fSources; ++u) {
-                const double4 sj = tile[jj + u];
-#pragma unroll
-                for (int q = 0; q < kSplitPerLane; ++q) {
-                    const int p = u * kSplitPerLane + q;
-                    dx[p] = sj.x - px[q];
-                    dy[p] = sj.y - py[q];
-                    dz[p] = sj.z - pz[q];
-                    w[p] = sj.w;
-                    r2[p] = fma(dx[p], dx[p], fma(dy[p], dy[p], fma(dz[p], dz[p], eps2)));
+                    for (int q = 0; q < kF64fPerLane; ++q) {
+                        const int p = u * kF64fPerLane + q;
+                        dx[p] = sj.x - px[q];
+                        dy[p] = sj.y - py[q];
+                        dz[p] = sj.z - pz[q];
+                        f[p] = sj.w;
+                        r2[p] = fma(dx[p], dx[p], fma(dy[p], dy[p], fma(dz[p], dz[p], eps2)));
+                    }
                 }
+#pragma unroll
+                for (int p = 0; p < kF64fPairs; ++p) f[p] = rsqrt3_f64(f[p], r2[p]);
+#pragma unroll
+                for (int u = 0; u < kSources; ++u)
+#pragma unroll
+                    for (int q = 0; q < kF64fPerLane; ++q) {
+                        const int p = u * kF64fPerLane + q;
+                        ax[q] = fma(f[p], dx[p], ax[q]);
+                        ay[q] = fma(f[p], dy[p], ay[q]);
+                        az[q] = fma(f[p], dz[p], az[q]);
+                    }
             }
-#pragma unroll
-            for (int p = 0; p < P; ++p) yv[p] = rsqrt_f64(r2[p]);
-#pragma unroll
-            for (int u = 0; u < kF64fSources; ++u)
-#pragma unroll
-                for (int q = 0; q < kSplitPerLane; ++q) {
-                    const int p = u * kSplitPerLane + q;
-                    const double f = (w[p] * yv[p]) * (yv[p] * yv[p]);
-                    ax[q] = fma(f, dx[p], ax[q]);
-                    ay[q] = fma(f, dy[p], ay[q]);
-                    az[q] = fma(f, dz[p], az[q]);
-                }
-        };
-        // the split's last stage may be partial: only its staged sources
-        const uint32_t cnt = min((uint32_t)kSplitTile, j1 - k);  // uniform
-        if (cnt == (uint32_t)kSplitTile) {
-            for (int jj = 0; jj < kSplitTile; jj += kF64fSources) pairs_s(jj);
-        } else {
-            for (uint32_t jj = 0; jj < cnt; ++jj) pairs((int)jj);
-        }
-        __syncthreads();
-    }
-    split_finish(n, G, ax, ay, az, partial, ax_out, ay_out, az_out);
+        },
+        [] {});
+    split_finish<kF64fPerLane>(n, G, ax, ay, az, comb, partial, ax_out, ay_out, az_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -1654,19 +1723,37 @@ void launch_direct_targets_f64(uint32_t n, const double *x, const double *y, con
                        dim3(kF64Threads), 0, s, n, x, y, z, m, G, eps2, nt, targets, ax, ay, az);
 }
 
-// About kSplitBlocks blocks per launch; rounding the split count down keeps
-// the partial sums at most 3 * 8 * kSplitBlocks * kSplitTargets bytes (24 MiB)
-// for every n.
-uint32_t direct_split_count(uint32_t n) {
-    const uint32_t tiles = ceil_div(n, kSplitTargets);
-    const uint32_t splits = kSplitBlocks / tiles;
-    const uint32_t max_splits = std::max<uint32_t>(1, n / kSplitTile);
-    return std::max<uint32_t>(1, std::min(splits, max_splits));
+namespace {
+// How a split direct sum of n bodies is cut.
+struct SplitPlan {
+    uint32_t per_lane;  // targets per lane
+    uint32_t tiles;     // blocks of 64 per_lane targets
+    uint32_t splits;    // source ranges
+    uint32_t chunk;     // sources per range
+};
+// Small sums are cut as finely as the kernels allow (one run or stage per wave
+// and, FP32, one target per lane), to have as many waves as they can: FP32
+// 0.0147 ms for 1024 bodies, 0.0177 for 3001 and 0.0545 for 12,001 (two targets
+// per lane 0.024, 0.027 and 0.059; blocks of 512 targets and 256 sources 0.027,
+// 0.050 and 0.081); at 16,384 both take 0.086, beyond, two targets per lane are
+// faster (50,021: 0.703 against 0.725).
+SplitPlan split_plan(bool fp64, uint32_t n) {
+    SplitPlan p;
+    p.per_lane = fp64 ? (uint32_t)kF64fPerLane : (n < 16384 ? 1u : 2u);
+    p.tiles = ceil_div(n, 64 * p.per_lane);
+    const uint32_t step = kSplitTile * kSplitWaves * (fp64 ? 1u : (uint32_t)kF32cRun);
+    const uint32_t least = fp64 && n >= 8192 ? 2 * step : step;
+    const uint32_t most = kSplitPartials / (p.tiles * 64 * p.per_lane);
+    p.splits = std::max<uint32_t>(1, std::min(most, ceil_div(n, least)));
+    p.chunk = ceil_div(ceil_div(n, p.splits), step) * step;
+    p.splits = ceil_div(n, p.chunk);
+    return p;
 }
+}  // namespace
 
 // scratch: the partial sums [split][3][n] doubles (none with one split)
 uint64_t direct_split_scratch_bytes(uint32_t n) {
-    const uint32_t splits = direct_split_count(n);
+    const uint32_t splits = std::max(split_plan(false, n).splits, split_plan(true, n).splits);
     return splits > 1 ? 3ull * n * splits * sizeof(double) : 0;
 }
 
@@ -1674,19 +1761,20 @@ void launch_direct_split(bool fp64, uint32_t n, const double *x, const double *y
                          const double *z, const double *m, double G, double eps2, double *ax,
                          double *ay, double *az, double *partial, hipStream_t s) {
     if (n == 0) return;
-    const uint32_t splits = direct_split_count(n);
-    const uint32_t tiles = ceil_div(n, kSplitTargets);
-    const uint32_t chunk = ceil_div(ceil_div(n, splits), kSplitTile) * kSplitTile;
-    const dim3 grid(tiles, splits);
+    const SplitPlan p = split_plan(fp64, n);
+    const dim3 grid(p.tiles, p.splits), block(kSplitThreads);
     if (fp64)
-        hipLaunchKernelGGL(k_direct_f64f, grid, dim3(kSplitThreads), 0, s, n, x, y, z, m, G, eps2,
-                           chunk, partial, ax, ay, az);
+        hipLaunchKernelGGL(k_direct_f64f, grid, block, 0, s, n, x, y, z, m, G, eps2, p.chunk,
+                           partial, ax, ay, az);
+    else if (p.per_lane == 1)
+        hipLaunchKernelGGL(k_direct_f32c<1>, grid, block, 0, s, n, x, y, z, m, G, (float)eps2,
+                           p.chunk, partial, ax, ay, az);
     else
-        hipLaunchKernelGGL(k_direct_f32c, grid, dim3(kSplitThreads), 0, s, n, x, y, z, m, G,
-                           (float)eps2, chunk, partial, ax, ay, az);
-    if (splits > 1)
-        hipLaunchKernelGGL(k_split_reduce, dim3(ceil_div(n, kSplitThreads)), dim3(kSplitThreads),
-                           0, s, n, splits, fp64 ? G : 1.0, (const double *)partial, ax, ay, az);
+        hipLaunchKernelGGL(k_direct_f32c<2>, grid, block, 0, s, n, x, y, z, m, G, (float)eps2,
+                           p.chunk, partial, ax, ay, az);
+    if (p.splits > 1)
+        hipLaunchKernelGGL(k_split_reduce, dim3(ceil_div(n, kSplitThreads), 3), block, 0, s, n,
+                           p.splits, fp64 ? G : 1.0, (const double *)partial, ax, ay, az);
 }
 
 void launch_bh_exact(const TreeBufs &t, const double *x, const double *y, const double *z,

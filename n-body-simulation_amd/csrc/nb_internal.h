@@ -292,7 +292,6 @@ void launch_direct_targets_f64(uint32_t n, const double *x, const double *y, con
 void launch_direct_split(bool fp64, uint32_t n, const double *x, const double *y,
                          const double *z, const double *m, double G, double eps2, double *ax,
                          double *ay, double *az, double *partial, hipStream_t s);
-uint32_t direct_split_count(uint32_t n);
 uint64_t direct_split_scratch_bytes(uint32_t n);
 void launch_bh_exact(const TreeBufs &t, const double *x, const double *y, const double *z,
                      double G, double eps2, double theta, int sort_bodies, uint32_t *stack,

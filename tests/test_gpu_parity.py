@@ -133,6 +133,27 @@ def test_direct_f64_fast_tolerance(gpu, oracle, kind, n):
         assert mf <= max(2 * mr, 1e-15), (mf, mr)
 
 
+@pytest.mark.parametrize("n", [3, 63, 64, 65, 128, 129, 256, 257, 1024, 1025, 8191, 16383, 16385])
+def test_direct_split_edges(gpu, oracle, n):
+    # The split sums at the edges of a block's targets (64, 128), a wave's stage
+    # (64) and run (256), a block's sources (256, 1024) and the changes of the
+    # split rules (8192, 16,384).
+    # FP64: 1e-12 S_i as above.  FP32, with positions that are FP32 numbers: a
+    # term's relative error is at most about 20 roundings (r^2 5, raised to
+    # -3/2, v_rsq_f32 1 ulp three times, the products) and a run adds 256 terms
+    # before it is folded into FP64: 276 roundings, bound 512 * 2^-24 S_i.
+    d = uniform_cube(n, 100 + n)
+    for k in "xyz":
+        d[k] = d[k].astype(np.float32).astype(np.float64)
+    rx, ry, rz = oracle.naive_accel(d["x"], d["y"], d["z"], d["m"])
+    S = term_sum(d, oracle.G_ref(), oracle.eps2_ref())
+    for precision, bound in ((gpu.PREC_FP64_FAST, 1e-12), (gpu.PREC_FP32C, 512 * 2.0 ** -24)):
+        with ctx_for(gpu, d, precision=precision) as c:
+            ax, ay, az = c.forces_direct()
+        diff = np.sqrt((ax - rx) ** 2 + (ay - ry) ** 2 + (az - rz) ** 2)
+        assert np.all(diff <= bound * S), (precision, (diff / S).max())
+
+
 # ratio: the bound on quadrupole error / monopole error.  The star + disk sits
 # at the FP32 rounding floor (~9e-8, the star's force dominates), where cell
 # expansions change nothing: there the quadrupole must only not be worse.
