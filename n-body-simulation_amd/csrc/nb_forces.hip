@@ -24,115 +24,152 @@ namespace {
 __device__ inline void raise_flag(TreeHdr *h, uint32_t f) { atomicOr(&h->status, f); }
 
 constexpr uint32_t kXcds = 8;  // XCDs of an MI355X; workgroups are dealt round-robin
+constexpr uint32_t kCus = 256;  // CUs of an MI355X
 
 // ---------------------------------------------------------------------------
 // FP64 direct sum, reference order.  The sum over j = 0..n-1 of a target must
 // run in that order to be bit-exact, but only its three additions per pair
 // are sequential; the pair terms m_j (r_ij den_ij), with their IEEE division
-// and square root, are not.  A workgroup owns 64 targets (one per lane).
-// Sources are staged in LDS kF64Stage at a time; for each chunk of kF64Chunk
-// sources all sixteen waves compute the terms into one of two LDS tiles while
-// waves 0, 1 and 2 add the x, y and z components of the previous tile in
-// source order, eight terms' reads in flight ahead of their additions.
-// (16,384 bodies: 1.26 ms with 8 waves and one read per addition by wave 0,
-// 1.09 ms with 16 waves, 0.75 ms with the reads ahead, 0.72 ms with
-// 48-source chunks instead of 32, 0.66 ms with inv_sqrt_ieee, 0.58 ms with
-// the three components added by three waves instead of one.)
-constexpr int kDirectF64Tile = 64;                  // targets per workgroup
-constexpr int kF64Threads = 1024;                   // 16 waves computing pair terms
-constexpr int kF64Chunk = 48;                       // sources per term tile
-constexpr int kF64PerWave = kF64Chunk / (kF64Threads / 64);
-constexpr int kF64Stage = 240;                      // sources per LDS stage
-static_assert(kF64Stage % kF64Chunk == 0, "whole chunks per stage");
-static_assert(kF64Threads >= 3 * 64 && kF64Chunk % (kF64Threads / 64) == 0,
-              "three adder waves; whole terms per wave");
+// and square root, are not.  A workgroup of sixteen waves owns T targets; for
+// each chunk of sources its waves compute the terms into one of two LDS tiles
+// while the first 3 T threads (component d of target t in thread d T + t) add
+// the previous tile in source order.
+//  - T = 64: a wave computes the terms of one source at a time, which it reads
+//    through the scalar cache (staging the sources in LDS loads it with two
+//    more reads per term than the five that the terms need).
+//  - T = 16, where 64 targets per workgroup leave CUs idle: four sources at a
+//    time; wave 0 only adds, since the chain of additions bounds a workgroup.
+// The additions stand before the terms in a chunk, ahead of the other waves on
+// their SIMDs (s_setprio); a wave's terms are interleaved, with one test for
+// all that the IEEE sequences need no range handling.  16,384 bodies: 0.52 ms
+// with the additions last, sources staged in LDS and one term at a time; 0.45
+// now, 262 cycles at 2.4 GHz per 64 pairs where the 32 FP64 operations, two
+// quarter-rate estimates and three additions of a pair issue in about 208.
+// 700 bodies 0.026 -> 0.011, 5001 0.162 -> 0.086, 8192 0.262 -> 0.139, 20,001
+// 1.26 -> 0.79 ms.  T = 32 (two sources at a time) was slower than the better
+// of the two at every size.
+constexpr int kF64Waves = 16;
+constexpr int kF64Threads = 64 * kF64Waves;
+template <int T>
+struct DirectF64 {
+    static constexpr int kSub = 64 / T;             // sources per wave and step
+    static constexpr int kPer = T == 64 ? 3 : 1;    // steps per chunk: its terms interleave
+    static constexpr int kFirst = T == 64 ? 0 : 1;  // first wave that computes terms
+    static constexpr int kChunk = (kF64Waves - kFirst) * kSub * kPer;  // sources per tile
+    static constexpr int kTile = kChunk * T + (T < 64 ? T : 0);        // rows in other banks
+    static constexpr uint32_t kAdders = (3 * T + 63) / 64;  // waves
+};
+constexpr int kF64Ahead = 8;  // an adder's LDS reads in flight ahead of its ordered additions
 
-// Returns, in waves 0, 1 and 2, component 0, 1 or 2 (x, y, z) of the sum
-// over j in order of m_j (r_ij den_ij) for the lane's target at (px, py, pz):
-// the three sums are independent, so three waves on three SIMDs add them.
-__device__ inline double direct_f64_body(uint32_t n, const double *__restrict__ x,
-                                         const double *__restrict__ y,
-                                         const double *__restrict__ z,
-                                         const double *__restrict__ m, double eps2, double px,
-                                         double py, double pz) {
-    __shared__ double4 src[kF64Stage];
-    __shared__ double tx[2][kF64Chunk][kDirectF64Tile], ty[2][kF64Chunk][kDirectF64Tile],
-        tz[2][kF64Chunk][kDirectF64Tile];
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
-    double (*const own)[kF64Chunk][kDirectF64Tile] = w == 0 ? tx : (w == 1 ? ty : tz);
+// Returns, in thread d T + t (d < 3), component d of the sum over j in order
+// of m_j (r_ij den_ij) for target t, whose position (px, py, pz) every thread
+// with threadIdx.x % T == t passes.
+template <int T>
+__device__ __forceinline__ double direct_f64_body(uint32_t n, const double *__restrict__ x,
+                                                  const double *__restrict__ y,
+                                                  const double *__restrict__ z,
+                                                  const double *__restrict__ m, double eps2,
+                                                  double px, double py, double pz) {
+    using K = DirectF64<T>;
+    constexpr int P = K::kPer, C = K::kChunk;
+    __shared__ double term[2][3][K::kTile];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t t = lane % T, sub = lane / T;
+    const bool adds = w < K::kAdders, computes = w >= (uint32_t)K::kFirst;
+    const uint32_t comp = T == 64 ? min(w, 2u) : min(sub, 2u);
     double acc = 0;
-    uint32_t pending = 0;  // sources in the tile waves 0-2 still have to add
+    uint32_t pending = 0;  // sources in the tile the adders still have to add
     int buf = 0;
-    // waves 0-2: add their component of tile `b` (cnt sources) in source order
     auto add_tile = [&](int b, uint32_t cnt) {
-        uint32_t jj = 0;
-        // eight terms' LDS reads in flight before their (ordered) additions
-        for (; jj + 8 <= cnt; jj += 8) {
-            double v[8];
+        const double *own = &term[b][comp][t];
+        if (cnt == (uint32_t)C) {
+            double v[2][kF64Ahead];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = own[b][jj + u][lane];
+            for (int u = 0; u < kF64Ahead; ++u) v[0][u] = own[u * T];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) acc += v[u];
-        }
-        for (; jj < cnt; ++jj) acc += own[b][jj][lane];
-    };
-    for (uint32_t k0 = 0; k0 < n; k0 += kF64Stage) {
-        const uint32_t staged = min((uint32_t)kF64Stage, n - k0);
-        __syncthreads();  // the previous stage's terms are computed
-        for (uint32_t j = threadIdx.x; j < staged; j += kF64Threads)
-            src[j] = make_double4(x[k0 + j], y[k0 + j], z[k0 + j], m[k0 + j]);
-        __syncthreads();
-        for (uint32_t c = 0; c < staged; c += kF64Chunk) {
-            const uint32_t cnt = min((uint32_t)kF64Chunk, staged - c);
+            for (int jj = 0; jj < C; jj += kF64Ahead) {
+                const int c = (jj / kF64Ahead) & 1;
 #pragma unroll
-            for (int u = 0; u < kF64PerWave; ++u) {
-                const uint32_t jj = w * kF64PerWave + u;  // the same for the whole wave
-                if (jj < cnt) {
-                    const double4 sj = src[c + jj];
-                    const double r_x = sj.x - px;
-                    const double r_y = sj.y - py;
-                    const double r_z = sj.z - pz;
-                    double denominator = (r_x * r_x) + (r_y * r_y) + (r_z * r_z) + eps2;
-                    denominator = denominator * denominator * denominator;
-                    denominator = inv_sqrt_ieee(denominator);
-                    tx[buf][jj][lane] = sj.w * (r_x * denominator);
-                    ty[buf][jj][lane] = sj.w * (r_y * denominator);
-                    tz[buf][jj][lane] = sj.w * (r_z * denominator);
-                }
+                for (int u = 0; u < kF64Ahead; ++u)
+                    if (jj + kF64Ahead + u < C) v[c ^ 1][u] = own[(jj + kF64Ahead + u) * T];
+#pragma unroll
+                for (int u = 0; u < kF64Ahead; ++u)
+                    if (jj + u < C) acc += v[c][u];
             }
-            // waves 0-2 add the previous tile (written before the last barrier)
-            if (w < 3 && pending) add_tile(buf ^ 1, pending);
-            __syncthreads();
-            pending = cnt;
-            buf ^= 1;
+        } else {
+            for (uint32_t jj = 0; jj < cnt; ++jj) acc += own[jj * T];
         }
+    };
+    // a computing wave's sources of a chunk: (w - kFirst) kPer kSub + u kSub + sub
+    const uint32_t own0 = (w - (uint32_t)K::kFirst) * (P * K::kSub) + sub;
+    double sx[P], sy[P], sz[P], sm[P];
+    auto load = [&](uint32_t c) {
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const uint32_t j = min(c + own0 + u * K::kSub, n - 1);
+            sx[u] = x[j];
+            sy[u] = y[j];
+            sz[u] = z[j];
+            sm[u] = m[j];
+        }
+    };
+    if (computes) load(0);
+    for (uint32_t c = 0; c < n; c += C) {
+        // the adders first, ahead of the terms of the other waves on their SIMDs
+        if (adds && pending) {
+            __builtin_amdgcn_s_setprio(3);
+            add_tile(buf ^ 1, pending);
+            __builtin_amdgcn_s_setprio(0);
+        }
+        if (computes) {
+            double r_x[P], r_y[P], r_z[P], den[P], m_j[P];
+            bool in_range = true;
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                r_x[u] = sx[u] - px;
+                r_y[u] = sy[u] - py;
+                r_z[u] = sz[u] - pz;
+                m_j[u] = sm[u];
+                den[u] = (r_x[u] * r_x[u]) + (r_y[u] * r_y[u]) + (r_z[u] * r_z[u]) + eps2;
+                den[u] = den[u] * den[u] * den[u];
+                in_range = in_range && inv_sqrt_in_range(den[u]);
+            }
+            load(c + C);  // back before the barrier waits for it
+            if (in_range) {
+#pragma unroll
+                for (int u = 0; u < P; ++u) den[u] = inv_sqrt_core(den[u]);
+            } else {
+                for (int u = 0; u < P; ++u) den[u] = 1.0 / sqrt(den[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                const uint32_t k = (own0 + u * K::kSub) * T + t;
+                term[buf][0][k] = m_j[u] * (r_x[u] * den[u]);
+                term[buf][1][k] = m_j[u] * (r_y[u] * den[u]);
+                term[buf][2][k] = m_j[u] * (r_z[u] * den[u]);
+            }
+        }
+        __syncthreads();
+        pending = min((uint32_t)C, n - c);
+        buf ^= 1;
     }
-    if (w < 3 && pending) add_tile(buf ^ 1, pending);
+    if (adds && pending) add_tile(buf ^ 1, pending);
     return acc;
 }
 
+// ids: the targets' body indices, or null for targets 0 .. nt - 1
+template <int T>
 __global__ void __launch_bounds__(kF64Threads) k_direct_f64(
     uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, double G, double eps2,
-    double *ax, double *ay, double *az) {
-    const uint32_t i = blockIdx.x * kDirectF64Tile + (threadIdx.x & 63u);
-    const bool valid = i < n;
-    const uint32_t ii = valid ? i : 0;
-    const double acc = direct_f64_body(n, x, y, z, m, eps2, x[ii], y[ii], z[ii]);
-    const uint32_t w = threadIdx.x >> 6;
-    if (valid && w < 3) (w == 0 ? ax : (w == 1 ? ay : az))[i] = acc * G;
-}
-
-__global__ void __launch_bounds__(kF64Threads) k_direct_targets_f64(
-    uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
-    const double *__restrict__ z, const double *__restrict__ m, double G, double eps2,
-    uint32_t nt, const uint32_t *__restrict__ targets, double *ax, double *ay, double *az) {
-    const uint32_t t = blockIdx.x * kDirectF64Tile + (threadIdx.x & 63u);
-    const bool valid = t < nt;
-    const uint32_t i = valid ? targets[t] : 0;
-    const double acc = direct_f64_body(n, x, y, z, m, eps2, x[i], y[i], z[i]);
-    const uint32_t w = threadIdx.x >> 6;
-    if (valid && w < 3) (w == 0 ? ax : (w == 1 ? ay : az))[t] = acc * G;
+    uint32_t nt, const uint32_t *__restrict__ ids, double *ax, double *ay, double *az) {
+    const uint32_t k = blockIdx.x * T + threadIdx.x % T;
+    const bool valid = k < nt;
+    const uint32_t i = !valid ? 0u : (ids ? ids[k] : k);
+    const double acc = direct_f64_body<T>(n, x, y, z, m, eps2, x[i], y[i], z[i]);
+    const uint32_t d = threadIdx.x / T;
+    if (valid && d < 3) (d == 0 ? ax : (d == 1 ? ay : az))[k] = acc * G;
 }
 
 // ---------------------------------------------------------------------------
@@ -1707,20 +1744,30 @@ __global__ void __launch_bounds__(kGroup) k_ens_forces(EnsForceArgs a) {
 
 }  // namespace
 
-void launch_direct_f64(uint32_t n, const double *x, const double *y, const double *z,
-                       const double *m, double G, double eps2, double *ax, double *ay,
-                       double *az, hipStream_t s) {
-    hipLaunchKernelGGL(k_direct_f64, dim3(ceil_div(n, kDirectF64Tile)), dim3(kF64Threads), 0, s,
-                       n, x, y, z, m, G, eps2, ax, ay, az);
-}
-
 void launch_direct_targets_f64(uint32_t n, const double *x, const double *y, const double *z,
                                const double *m, double G, double eps2, uint32_t nt,
                                const uint32_t *targets, double *ax, double *ay, double *az,
                                hipStream_t s) {
     if (nt == 0) return;
-    hipLaunchKernelGGL(k_direct_targets_f64, dim3(ceil_div(nt, kDirectF64Tile)),
-                       dim3(kF64Threads), 0, s, n, x, y, z, m, G, eps2, nt, targets, ax, ay, az);
+    // A round of workgroups is one of 64 targets or two of 16 per CU (1024
+    // threads each), and a round of 16-target ones takes 0.6 of the other's time
+    // (0.139 ms for 8192 targets x sources against 0.223) and leaves a shorter
+    // remainder.
+    const uint32_t rounds = ceil_div(nt, 64 * kCus);
+    const bool small = 0.6 * std::max(1.0, nt / (2.0 * 16 * kCus)) < rounds;
+    const dim3 block(kF64Threads);
+    if (small)
+        hipLaunchKernelGGL(k_direct_f64<16>, dim3(ceil_div(nt, 16)), block, 0, s, n, x, y, z, m, G,
+                           eps2, nt, targets, ax, ay, az);
+    else
+        hipLaunchKernelGGL(k_direct_f64<64>, dim3(ceil_div(nt, 64)), block, 0, s, n, x, y, z, m, G,
+                           eps2, nt, targets, ax, ay, az);
+}
+
+void launch_direct_f64(uint32_t n, const double *x, const double *y, const double *z,
+                       const double *m, double G, double eps2, double *ax, double *ay,
+                       double *az, hipStream_t s) {
+    launch_direct_targets_f64(n, x, y, z, m, G, eps2, n, nullptr, ax, ay, az, s);
 }
 
 namespace {

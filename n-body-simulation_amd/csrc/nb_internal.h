@@ -395,9 +395,11 @@ __device__ inline double div_core(double a, double b) {  // |a|, |b| in [2^-300,
     return fma(e, y, q);
 }
 // 1.0 / sqrt(v), both operations correctly rounded (the reference's
-// inverse square root); the core for v in [2^-512, 2^512]
-__device__ inline double inv_sqrt_ieee(double v) {
-    if (!(v >= 0x1p-512 && v <= 0x1p512)) return 1.0 / sqrt(v);
+// inverse square root); the core for v in [2^-512, 2^512)
+__device__ inline bool inv_sqrt_in_range(double v) {  // on the sign and exponent: one compare
+    return (uint32_t)__double2hiint(v) - 0x1ff00000u < 0x40000000u;
+}
+__device__ inline double inv_sqrt_core(double v) {
     const double s = sqrt_core(v);
     double y = __builtin_amdgcn_rcp(s);
     double e = fma(-s, y, 1.0);
@@ -406,6 +408,9 @@ __device__ inline double inv_sqrt_ieee(double v) {
     y = fma(y, e, y);
     e = fma(-s, y, 1.0);  // the quotient 1.0 * y is y
     return fma(e, y, y);
+}
+__device__ inline double inv_sqrt_ieee(double v) {
+    return inv_sqrt_in_range(v) ? inv_sqrt_core(v) : 1.0 / sqrt(v);
 }
 // a / sqrt(v), both operations correctly rounded; the cores for v in
 // [2^-600, 2^600] and |a| in [2^-300, 2^300]

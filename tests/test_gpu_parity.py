@@ -133,6 +133,28 @@ def test_direct_f64_fast_tolerance(gpu, oracle, kind, n):
         assert mf <= max(2 * mr, 1e-15), (mf, mr)
 
 
+# Both kernels of the bit-exact sum (16 and 64 targets per workgroup, chosen by
+# the target count) at the edges of a workgroup's targets and of a chunk of
+# sources (60 and 48), and on both sides of the rule between them (13,653 and
+# 16,384 targets).  The second system has every other pair's term outside the
+# range of the short IEEE sequences.
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 48, 49, 59, 60, 61, 121, 13652, 13655, 16385])
+def test_direct_f64_kernels_bitexact(gpu, oracle, n):
+    for scale in (1.0, 2.0 ** 90):
+        if scale > 1 and n > 200:
+            continue
+        d = uniform_cube(n, 200 + n)
+        d["x"][::2] *= scale
+        with ctx_for(gpu, d) as c:
+            got = c.forces_direct()
+            t = np.arange(n - 1, -1, -1, dtype=np.uint32)[:300]
+            sel = c.forces_direct_targets(t)
+        ref = oracle.naive_accel(d["x"], d["y"], d["z"], d["m"])
+        for g, s_, r in zip(got, sel, ref):
+            np.testing.assert_array_equal(bits(g), bits(r))
+            np.testing.assert_array_equal(bits(s_), bits(r[t]))
+
+
 @pytest.mark.parametrize("n", [3, 63, 64, 65, 128, 129, 256, 257, 1024, 1025, 8191, 16383, 16385])
 def test_direct_split_edges(gpu, oracle, n):
     # The split sums at the edges of a block's targets (64, 128), a wave's stage
