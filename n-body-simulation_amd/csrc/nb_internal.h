@@ -412,14 +412,6 @@ __device__ inline double inv_sqrt_core(double v) {
 __device__ inline double inv_sqrt_ieee(double v) {
     return inv_sqrt_in_range(v) ? inv_sqrt_core(v) : 1.0 / sqrt(v);
 }
-// a / sqrt(v), both operations correctly rounded; the cores for v in
-// [2^-600, 2^600] and |a| in [2^-300, 2^300]
-__device__ inline double div_sqrt_ieee(double a, double v) {
-    const double fa = fabs(a);
-    if (!(v >= 0x1p-600 && v <= 0x1p600 && fa >= 0x1p-300 && fa <= 0x1p300)) return a / sqrt(v);
-    return div_core(a, sqrt_core(v));
-}
-
 inline uint32_t ceil_div(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
 // Host: canonical depth-first dump of an octree (children in digit order),

@@ -667,6 +667,22 @@ def test_energy_bitexact(gpu, oracle, kind, n):
         assert np.float64(e[k]).view(np.int64) == np.float64(r[k]).view(np.int64), k
 
 
+# The energy kernels at the edges of a workgroup's bodies (64) and of a chunk of
+# sources (48), with masses of which some take the plain operators (zero, and
+# below 2^-150 of the unit), and on both sides of the rule between the two
+# kernels (196,608 bodies; 768 and 769 blocks of rows, an odd round of them).
+@pytest.mark.parametrize("n", [1, 2, 47, 48, 49, 63, 64, 65, 96, 97, 129, 20011, 196607, 196869])
+def test_energy_edges_bitexact(gpu, oracle, n):
+    d = uniform_cube(n, 300 + n)
+    for k in range(3, n, 17):
+        d["m"][k] = 0.0 if k % 2 else 1e-60
+    with ctx_for(gpu, d) as c:
+        e = c.energy()
+    r = oracle.energy(d["x"], d["y"], d["z"], d["vx"], d["vy"], d["vz"], d["m"])
+    for k in ("kinetic", "potential", "total"):
+        assert np.float64(e[k]).view(np.int64) == np.float64(r[k]).view(np.int64), k
+
+
 # The FP64 kernels take 1/sqrt(v) and a/sqrt(v) through the IEEE sequences
 # without their range handling only for v (and a) inside fixed ranges
 # (den^3 in [2^-512, 2^512] for the forces, v in [2^-600, 2^600] and |a| in
