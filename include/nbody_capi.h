@@ -38,7 +38,7 @@ enum {
     NB_E_INVALID_ARG = 1,
     NB_E_HIP = 2,             /* a HIP runtime call failed */
     NB_E_NODE_OVERFLOW = 3,   /* octree needs more nodes than storage_size_param allows */
-    NB_E_STACK_OVERFLOW = 4,  /* per-body traversal stack exhausted */
+    NB_E_STACK_OVERFLOW = 4,  /* traversal stack exhausted, or a corrupt octree */
     NB_E_DEPTH = 5,           /* two bodies share all 42 octree digits (coincident bodies) */
     NB_E_ZERO_MASS = 6,       /* a non-empty cell has zero mass (reference: endless COM loop) */
     NB_E_NOT_BUILT = 7,       /* forces requested before an octree was built */
@@ -70,9 +70,14 @@ typedef struct nb_params {
     double eps2;          /* configuration::epsilon2, Configuration.cpp:6 */
     double theta;         /* configuration::barnes_hut_algorithm::theta, Configuration.cpp:10 */
     uint32_t precision;   /* NB_PREC_* for forces (integrator, AABB, COM are always FP64) */
-    uint32_t sort_bodies; /* configuration::barnes_hut_algorithm::sortBodies, Configuration.cpp:15 */
+    /* configuration::barnes_hut_algorithm::sortBodies, Configuration.cpp:15: in the
+     * reference the order in which bodies are walked, which changes no force; here
+     * they are walked in octree order in any case. */
+    uint32_t sort_bodies;
     uint32_t storage_size_param; /* main.cpp:122-127; node capacity = param * N (default 16) */
-    uint32_t stack_size_param;   /* main.cpp:129-134; traversal stack rule (default 16) */
+    /* main.cpp:129-134 (default 16).  The traversals here keep one stack entry per
+     * octree level and need no size rule. */
+    uint32_t stack_size_param;
     /* No counterpart in the reference (which uses monopole cells,
      * BarnesHutAlgorithm.cpp:361-367): nonzero adds each accepted cell's
      * traceless quadrupole moment to its monopole force in the NB_PREC_FP32C

@@ -30,8 +30,6 @@ struct nb_ctx {
     TreeBufs tree;
     bool tree_valid = false;
     TreeHdr *hdr_host = nullptr;  // pinned copy of tree.hdr
-    uint32_t *exact_stack = nullptr;
-    uint32_t exact_cap = 0;
     double *split_scratch = nullptr;  // partial sums of the split direct sums
     uint64_t split_scratch_bytes = 0;
     uint32_t *targets_dev = nullptr;
@@ -187,15 +185,6 @@ int finish(nb_ctx *c, bool read_tree_status) {
     return NB_OK;
 }
 
-uint32_t exact_stack_cap(const nb_ctx *c) {
-    // the reference's stackSize (Configuration.cpp:24-33), raised to the
-    // largest depth-first stack a depth-42 octree can need (1 + 7*42)
-    const uint32_t n = c->n;
-    const uint32_t lg = (uint32_t)std::ceil(std::log2((double)std::max<uint32_t>(n, 2)));
-    uint32_t ref = c->p.stack_size_param * lg + (n < 15000 ? 500u : 0u);
-    return std::max<uint32_t>(ref, 1 + 7 * nb::kMaxDepth + 8);
-}
-
 // Internal-cell capacity for storage_size_param * n nodes, in 64 bits; the
 // group traversal packs an internal-cell index into 26 bits.
 bool tree_capacity(uint32_t storage_size_param, uint32_t n, uint32_t *icap) {
@@ -212,7 +201,7 @@ void tree_free(nb_ctx *c, TreeBufs &t) {
                     t.lcp, t.chain, t.body_parent, t.int_depth, t.int_parent, t.int_node,
                     t.int_lvl, t.int_count, t.int_sums, t.int_local, t.int_first, t.groups,
                     t.group_size, t.group_slot, t.body4, t.gq, t.spanning, t.cross, t.ref,
-                    t.cm, t.edge, t.rec, t.radix_ctl, t.scan_part};
+                    t.cm, t.rec, t.radix_ctl, t.scan_part};
     for (void *b : bufs) dev_free(c, b);
     t = TreeBufs();
 }
@@ -271,7 +260,6 @@ int alloc_tree_into(nb_ctx *c, TreeBufs &t, uint32_t storage_size_param) {
     NB_TREE_ALLOC(t.cross, t.cross_cap);
     NB_TREE_ALLOC(t.ref, t.mcap);
     NB_TREE_ALLOC(t.cm, t.mcap);
-    NB_TREE_ALLOC(t.edge, t.mcap);
     NB_TREE_ALLOC(t.rec, t.mcap);
     const uint32_t ctl_words = nb::radix_ctl_words(n);
     NB_TREE_ALLOC(t.radix_ctl, ctl_words);
@@ -355,17 +343,8 @@ int bh_forces_enqueue(nb_ctx *c) {
     mark_begin(c, NB_PHASE_ACCEL);
     flush_marks(c);
     if (c->p.precision != NB_PREC_FP32C) {  // FP64 and FP64_FAST: the reference traversal
-        const uint32_t cap = exact_stack_cap(c);
-        if (!c->exact_stack || c->exact_cap != cap) {
-            dev_free(c, c->exact_stack);
-            c->exact_stack = nullptr;
-            int rc = dev_alloc(c, &c->exact_stack, (uint64_t)cap * c->n);
-            if (rc) return rc;
-            c->exact_cap = cap;
-        }
-        nb::launch_bh_exact(c->tree, c->x, c->y, c->z, c->p.G, c->p.eps2, c->p.theta,
-                            c->p.sort_bodies, c->exact_stack, c->exact_cap, c->ax, c->ay, c->az,
-                            c->inter, c->stream);
+        nb::launch_bh_exact(c->tree, c->x, c->y, c->z, c->p.G, c->p.eps2, c->p.theta, c->ax, c->ay,
+                            c->az, c->inter, c->stream);
     } else if (c->corr && c->quad_valid) {
         const nb::MlpWeights w = nb::mlp_weights(c->corr);
         const nb::CorrArgs ca{w.pack, w.master, c->mcell, c->corr_tau2};

@@ -4,8 +4,8 @@
 // (this file is compiled with -ffp-contract=off, and sycl::rsqrt is evaluated
 // as 1.0/sqrt(x), two correctly rounded IEEE operations):
 //   k_direct_f64   NaiveAlgorithm.cpp:299-352 (sum over j in index order)
-//   k_bh_exact     BarnesHutAlgorithm.cpp:319-393 (per-body stack traversal,
-//                  same push order, same opening test)
+//   k_bh_exact_*   BarnesHutAlgorithm.cpp:319-393 (per-body traversal, same
+//                  visit order, same opening test)
 // FP32 kernels do the pair arithmetic in FP32 (fmaf, v_rsq_f32) and fold the
 // FP32 partial of every tile into FP64 accumulators:
 //   k_direct_f32c  sources staged in LDS per wave, two targets per lane, split j
@@ -25,6 +25,13 @@ __device__ inline void raise_flag(TreeHdr *h, uint32_t f) { atomicOr(&h->status,
 
 constexpr uint32_t kXcds = 8;  // XCDs of an MI355X; workgroups are dealt round-robin
 constexpr uint32_t kCus = 256;  // CUs of an MI355X
+
+// A value every lane of the wave holds alike, made visibly uniform (SGPR).
+// The walks below are wave-collective (ballots, shuffles, one LDS list per
+// wave): every branch that steers them must be uniform to the compiler, or
+// control-flow structurisation may let parts of the wave run different
+// iterations with partial exec masks.
+__device__ inline uint32_t wave_uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // ---------------------------------------------------------------------------
 // FP64 direct sum, reference order.  The sum over j = 0..n-1 of a target must
@@ -223,24 +230,15 @@ __device__ inline void pair_f32(const float4 s, float px, float py, float pz, fl
     fz = fmaf(f, dz, fz);
 }
 
-// v^(-1/2) in FP64 from the hardware estimate y = v_rsq_f64(v), whose
-// relative error is near 1e-8 (single-precision accuracy): with
-// e = 1 - v y^2 (one fused multiply-add, so e is exact to the last bits),
-// v^(-1/2) = y (1 - e)^(-1/2) = y (1 + e/2 + 3e^2/8 + 5e^3/16 + ...).  The
+// w v^(-3/2) in FP64 from the hardware estimate y = v_rsq_f64(v), whose
+// relative error is near 1e-8 (single-precision accuracy): with y2 = y^2 and
+// e = 1 - v y2 (one fused multiply-add, so e is exact to the last bits),
+// v^(-3/2) = y^3 (1 - e)^(-3/2) = y^3 (1 + 3e/2 + 15e^2/8 + ...).  The
 // correction to second order in e leaves a truncation error near
-// 5e^3/16 ~ 1e-22, below FP64 rounding; five operations (a Newton step,
-// first order in e, would leave ~1e-14).  Checked against long-double
-// closed forms in the GPU tests.
-__device__ inline double rsqrt_f64(double v) {
-    const double y = __builtin_amdgcn_rsq(v);
-    const double e = fma(-(v * y), y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
-// w v^(-3/2) from the same estimate: with y2 = y^2 and e = 1 - v y2,
-// v^(-3/2) = y^3 (1 - e)^(-3/2) = y^3 (1 + 3e/2 + 15e^2/8 + ...), truncation
-// near 35e^3/16 ~ 1e-23.  The rounding of y2 enters the factor y2 and, with
+// 35e^3/16 ~ 1e-23, below FP64 rounding (a Newton step, first order in e,
+// would leave ~1e-14).  The rounding of y2 enters the factor y2 and, with
 // weight -3/2, e, so half of it remains.  Seven operations after the estimate.
+// Checked against long-double closed forms in the GPU tests.
 __device__ inline double rsqrt3_f64(double w, double v) {
     const double y = __builtin_amdgcn_rsq(v);
     const double y2 = y * y;
@@ -502,139 +500,387 @@ __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
 }
 
 // ---------------------------------------------------------------------------
-// Reference-semantics Barnes-Hut traversal (FP64).  Per body a depth-first
-// walk with its own stack (the older part in global memory, interleaved
-// across bodies so that lanes at the same stack depth touch adjacent words);
-// children are pushed in digit order 5,7,4,6,1,3,0,2 as in
-// BarnesHutAlgorithm.cpp:370-385, and the last pushed is visited at once.
-// The stack is kept as batches, one per opened cell (below).  The visit
-// order, and so every sum, is the reference's.  1M-body disk at theta 0.5:
-// 27.8 ms with one stack entry per child in memory; 16.9 ms with the top six
-// batches as seven registers each; 15.2 ms with four such batches, the
-// opening test decided from an estimate and a node's three loads issued
-// together; with a batch as one word, 14.4, 13.3, 12.5, 12.5 and 12.7 ms
-// with 2, 4, 8, 12 and 16 batches in registers.  Loading the record of the
-// stack top one visit ahead was slower: 13.8 ms (85 VGPRs, five waves).
-// Workgroups dealt to the XCDs in contiguous runs of bodies: 10.7 ms.
-constexpr int kExactThreads = 256;
+// Reference-semantics Barnes-Hut traversal (FP64).  The reference walks the tree
+// per body with a stack: children are pushed in digit order 5,7,4,6,1,3,0,2
+// (BarnesHutAlgorithm.cpp:370-385) and popped from the end, a depth-first
+// pre-order with the siblings in the order 2,0,3,1,6,4,7,5.
+// Two kernels walk it in that order, one for small systems and one for large
+// ones (launch_bh_exact chooses).  A stack per lane, one body per lane, loaded
+// each node's record from 64 places and ran the branch of the term for the few
+// lanes that needed it: 1M-body disk at theta 0.5 10.4 ms, now 6.0 (waves); 1024
+// bodies 0.52 ms, now 0.107; 30,001 (Plummer, theta 1.05) 0.47, now 0.174
+// (teams).
+//
+// k_bh_exact_team: a team of eight lanes walks the tree for one body and opens a
+// cell in one step: lane p loads and tests the child at visit position p.
+// Accepted nodes go to the team's list in LDS in the reference's order (those
+// behind an opened sibling wait on a stack, as a mask of the cell's children),
+// and once a list is nearly full, the lanes compute the terms of eight list
+// entries at a time and three lanes add them, one component each, in list order:
+// the reference's sum, bit for bit.  A walk takes one round trip to memory per
+// opened cell; what bounds it is that latency and, with more bodies than fit at
+// once, the bookkeeping of a step.
+constexpr int kExactWaves = 4;  // waves per workgroup
+constexpr int kExactThreads = 64 * kExactWaves;
+constexpr uint32_t kTeams = 8;  // bodies per wave
+constexpr uint32_t kTeamList = 40;  // entries; flushed above kTeamList - 16: a step adds up to 16
+constexpr uint32_t kTeamStack = kMaxDepth + 2;  // one entry per level
 
-__global__ void __launch_bounds__(kExactThreads) k_bh_exact(
-    uint32_t n, const uint32_t *__restrict__ order, const double *__restrict__ x,
-    const double *__restrict__ y, const double *__restrict__ z, const double4 *__restrict__ cm,
-    const double *__restrict__ edge, const int32_t *__restrict__ ref, double G, double eps2,
-    double theta, uint32_t *stack, uint32_t cap, uint32_t icap, double *ax, double *ay,
-    double *az, uint32_t *inter, TreeHdr *h) {
-    // Workgroup b runs on XCD b mod 8: give each XCD a contiguous run of the
-    // octree order, so that its L2 holds the records of one region of the tree.
-    const uint32_t nblk = gridDim.x, xcd = blockIdx.x % kXcds;
-    const uint32_t per = nblk / kXcds, extra = nblk % kXcds;
-    const uint32_t lb = xcd * per + min(xcd, extra) + blockIdx.x / kXcds;
-    const uint32_t id = lb * kExactThreads + threadIdx.x;
-    if (id >= n) return;
-    const uint32_t i = order ? order[id] : id;
+struct TeamLds {
+    uint32_t cell[kTeamStack][kTeams];   // cell with children left
+    uint32_t ref[kTeamStack][kTeams];    // its next child to open
+    uint32_t masks[kTeamStack][kTeams];  // level << 16 | children to open << 8 | to add
+    uint32_t list[kTeams][kTeamList];    // node ids
+    double term[kTeams][3][8];
+};
+
+// the slot of a cell's child at visit position p
+__device__ inline uint32_t visit_digit(uint32_t p) { return (0x57461302u >> (4u * p)) & 7u; }
+
+// Workgroup b runs on XCD b mod 8: give each XCD a contiguous run of blocks, so
+// that its L2 holds the records of one region of the tree.
+__device__ inline uint32_t xcd_contiguous_block() {
+    const uint32_t xcd = blockIdx.x % kXcds, per = gridDim.x / kXcds, extra = gridDim.x % kXcds;
+    return xcd * per + min(xcd, extra) + blockIdx.x / kXcds;
+}
+
+// The reference's opening test edge * (1.0 / sqrt(d2)) < theta of a child of
+// level l (edge = root edge 2^-l).  It is decided from d2 against edge^2 /
+// theta^2 (1 +- 2^-29), within a few roundings of the exact bound, and only the
+// squared distances between those two pay the IEEE square root and division
+// (exact).  A theta or a root edge whose squares could leave the normal range
+// turns the bounds into NaN: then every test is the exact one.
+struct ExactTest {
+    double edge, theta, bound;
+    __device__ ExactTest(double root_edge, double theta_) : edge(root_edge), theta(theta_) {
+        const double e2 = edge * edge;
+        const bool squares = (theta == 0.0 || (theta >= 1e-100 && theta <= 1e100)) &&
+                             e2 >= 1e-60 && e2 <= 1e60;
+        bound = squares ? e2 / (theta * theta) : __builtin_nan("");
+    }
+    __device__ double far2(int level) const { return ldexp(bound * (1.0 + 0x1p-29), -2 * level); }
+    __device__ double near2(int level) const { return ldexp(bound * (1.0 - 0x1p-29), -2 * level); }
+    __device__ bool far(int level, double d2) const {
+        const double scaled = ldexp(d2, 2 * level);  // against the root's bounds
+        bool yes = scaled > bound * (1.0 + 0x1p-29);
+        if (!yes && !(scaled < bound * (1.0 - 0x1p-29))) yes = exact(level, d2);
+        return yes;
+    }
+    __device__ bool exact(int level, double d2) const {
+        const double d = 1.0 / sqrt(d2);
+        return ldexp(edge, -level) * d < theta;
+    }
+};
+
+// what one wave's lanes wrote to LDS is read by others of the same wave
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__global__ void __launch_bounds__(kExactThreads) __attribute__((amdgpu_waves_per_eu(5)))
+k_bh_exact_team(uint32_t n, const uint32_t *__restrict__ order, const double *__restrict__ x,
+           const double *__restrict__ y, const double *__restrict__ z,
+           const double4 *__restrict__ cm, const int32_t *__restrict__ ref, double G, double eps2,
+           double theta, uint32_t icap, double *ax, double *ay, double *az, uint32_t *inter,
+           TreeHdr *h) {
+    __shared__ TeamLds lds[kExactWaves];
+    const uint32_t lb = xcd_contiguous_block();
+    const uint32_t lane = threadIdx.x & 63u, p = lane & 7u, team = lane >> 3, base = lane & 56u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    TeamLds &L = lds[wave];
+    const uint64_t id = (uint64_t)(lb * kExactWaves + wave) * kTeams + team;
+    const bool valid = id < n;
+    const uint32_t i = order[valid ? id : n - 1];
     const int32_t self_ref = ref_of_body(i);
-    const double pos_x_i = x[i], pos_y_i = y[i], pos_z_i = z[i];
-    uint32_t *stk = stack + id;
-    const uint64_t stride = n;
-    double acc_x = 0, acc_y = 0, acc_z = 0;
-    uint32_t cnt = 0;
-    // The opening test edge * (1.0 / sqrt(d2)) < theta is decided from
-    // edge * rsqrt_f64(d2), within 1e-14 of it, wherever that estimate is
-    // farther than 2^-30 (relative) from theta; only the rest pay the IEEE
-    // square root and division.  The decisions, and so the visit order and
-    // every sum, are the reference's.
-    const double theta_lo = theta * (1.0 - 0x1p-30), theta_hi = theta * (1.0 + 0x1p-30);
-    // The stack holds batches: the unvisited children of one opened cell r,
-    // pushed in digit order 5,7,4,6,1,3,0 and popped from the end, as one
-    // word (r << 3) | count (cell indices stay below 2^26).  The top kBatches
-    // batches live in registers, bw[0] on top, with no empty batch above a
-    // full one; older batches go to the memory stack one word each.  Popping
-    // a child is a shift of a constant; a memory pop returns a whole batch.
-    constexpr int kBatches = 8;  // 66 VGPRs
-    constexpr uint32_t kPopDigit = 0x0316475u;  // nibble c-1: the child popped at count c
-    uint32_t bw[kBatches];
+    const double px = x[i], py = y[i], pz = z[i];
+    const uint32_t digit = visit_digit(p), below = (1u << p) - 1u;
+    const ExactTest test(h->edge, theta);
+    double acc = 0.0;           // lane p < 3: component p of the body's sum
+    uint32_t cnt = 0;           // accepted nodes
+    uint32_t ln = 0, sp = 0;    // list and stack sizes
+    uint32_t cell = 0;          // the cell to open, if there is one
+    uint32_t level = 0;         // its children's level (the root is level 0)
+    bool have = false;
+    uint32_t late = kTeamStack;  // stack entry whose next child to open is being loaded
+    int32_t late_ref = 0;
+    uint32_t budget = icap + 16;  // a correct octree is entered once per cell
+
+    // the terms of the lists' full batches of eight (all: of every entry)
+    auto flush = [&](bool all) {
+        const uint32_t nb = all ? (ln + 7) >> 3 : ln >> 3;
+        for (uint32_t b = 0; __ballot(b < nb); ++b) {
+            const uint32_t k = 8 * b + p;
+            const bool use = b < nb && k < ln;
+            double t_x = 0.0, t_y = 0.0, t_z = 0.0;
+            if (use) {
+                const double4 c = cm[L.list[team][k]];
+                const double d_x = c.x - px;
+                const double d_y = c.y - py;
+                const double d_z = c.z - pz;
+                double den = (d_x * d_x) + (d_y * d_y) + (d_z * d_z) + eps2;
+                den = den * den * den;
+                den = inv_sqrt_ieee(den);
+                t_x = c.w * (d_x * den);
+                t_y = c.w * (d_y * den);
+                t_z = c.w * (d_z * den);
+            }
+            L.term[team][0][p] = t_x;
+            L.term[team][1][p] = t_y;
+            L.term[team][2][p] = t_z;
+            wave_lds_sync();
+            if (p < 3) {
+                double v[8];
 #pragma unroll
-    for (int k = 0; k < kBatches; ++k) bw[k] = 0;
-    uint32_t mtop = 0;      // batches in memory
-    uint32_t mentries = 0;  // children they hold
-    uint32_t node = 0;  // the root first
-    uint64_t budget = 1ull + 8ull * (uint64_t)icap;
-    for (;;) {
-        if (budget-- == 0) {
-            raise_flag(h, kFlagStack);
-            break;
+                for (int u = 0; u < 8; ++u) v[u] = L.term[team][p][u];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) acc += v[u];
+            }
+            wave_lds_sync();
         }
-        const double4 c = cm[node];
-        const int32_t r = ref[node];
-        const double e = edge[node];  // every slot below mcap has one, read or not
-        // all three loads in flight together: left to itself the compiler
-        // issues the centre of mass and the edge only after the tests on the
-        // mass and the reference, a second memory round trip per visit
-        asm volatile("" ::"v"(c.x), "v"(c.y), "v"(c.z), "v"(c.w), "v"(r), "v"(e));
-        bool opened = false;
-        if (c.w != 0 && r != self_ref) {
-            const double d_x = c.x - pos_x_i;
-            const double d_y = c.y - pos_y_i;
-            const double d_z = c.z - pos_z_i;
-            bool accept = r < 0;
-            if (!accept) {
-                const double d2 = d_x * d_x + d_y * d_y + d_z * d_z;
-                const double est = e * rsqrt_f64(d2);
-                if (est < theta_lo) {
-                    accept = true;
-                } else if (!(est > theta_hi)) {  // near theta, or not finite
-                    const double d = 1.0 / sqrt(d2);
-                    const double currentTheta = e * d;
-                    accept = currentTheta < theta;
+        const uint32_t done = 8 * nb;
+        if (!all && done > 0 && p < ln - done) L.list[team][p] = L.list[team][done + p];
+        ln = all ? 0u : ln - done;
+        wave_lds_sync();
+    };
+
+    // this lane's byte of a ballot: its team's positions
+    auto team_bits = [&](uint64_t m) {
+        return (uint32_t)((lane < 32 ? (uint32_t)m : (uint32_t)(m >> 32)) >> (base & 31u)) & 0xffu;
+    };
+    {
+        const double4 c = cm[0];
+        const int32_t r = ref[0];
+        const double d_x = c.x - px, d_y = c.y - py, d_z = c.z - pz;
+        const double d2 = d_x * d_x + d_y * d_y + d_z * d_z;
+        const bool real = valid && r != kRefEmpty && c.w != 0;
+        const bool take = real && (r < 0 ? r != self_ref : test.far(0, d2));
+        if (take) {
+            if (p == 0) L.list[team][0] = 0;
+            cnt = ln = 1;
+        } else if (real && r >= 0) {
+            have = true;
+            cell = (uint32_t)r;
+            level = 1;
+        }
+    }
+    while (__ballot(have || sp > 0)) {
+        if (__ballot(ln > kTeamList - 16)) flush(false);
+        if (late < kTeamStack) {
+            if (p == 0) L.ref[late][team] = (uint32_t)late_ref;
+            late = kTeamStack;
+        }
+        wave_lds_sync();
+        // Without a cell to open: back to the deepest cell with children left,
+        // for its accepted children before its next one to open.  One entry per
+        // step: the teams' pops then run side by side with each other and with
+        // the openings below, instead of in a loop as long as the longest.
+        if (!have && sp > 0) {
+            const uint32_t pc = L.cell[sp - 1][team], m = L.masks[sp - 1][team];
+            uint32_t et = m & 0xffu, eo = (m >> 8) & 0xffu;
+            const uint32_t q = (uint32_t)__builtin_ctz(eo | 0x100u);
+            const uint32_t before = (1u << q) - 1u, above = ~(2u * before + 1u);
+            const uint32_t emit = et & before;
+            if (emit >> p & 1u)
+                L.list[team][ln + __popc(emit & below)] = (uint32_t)(8ull * pc + 1u + digit);
+            ln += __popc(emit);
+            et &= above;
+            eo &= above;
+            have = q < 8;
+            level = (m >> 16) + 1;
+            cell = L.ref[sp - 1][team];
+            if (et | eo) {
+                if (p == 0) L.masks[sp - 1][team] = (m & 0xffff0000u) | eo << 8 | et;
+                if (eo) {
+                    late = sp - 1;
+                    late_ref = ref[8ull * pc + 1u + visit_digit((uint32_t)__builtin_ctz(eo))];
                 }
-            }
-            if (accept) {
-                double denominator = (d_x * d_x) + (d_y * d_y) + (d_z * d_z) + eps2;
-                denominator = denominator * denominator * denominator;
-                denominator = inv_sqrt_ieee(denominator);
-                acc_x += c.w * (d_x * denominator);
-                acc_y += c.w * (d_y * denominator);
-                acc_z += c.w * (d_z * denominator);
-                ++cnt;
             } else {
-                uint32_t held = 0;
-#pragma unroll
-                for (int k = 0; k < kBatches; ++k) held += bw[k] & 7u;
-                if (mentries + held + 8 > cap) {
-                    raise_flag(h, kFlagStack);
-                    break;
-                }
-                if (bw[0]) {
-                    // the bottom batch goes to memory, the others down one
-                    if (bw[kBatches - 1]) {
-                        stk[(uint64_t)(mtop++) * stride] = bw[kBatches - 1];
-                        mentries += bw[kBatches - 1] & 7u;
-                    }
-#pragma unroll
-                    for (int k = kBatches - 1; k > 0; --k) bw[k] = bw[k - 1];
-                }
-                bw[0] = ((uint32_t)r << 3) | 7u;
-                node = 8u * (uint32_t)r + 3u;  // child 2, pushed last
-                opened = true;
+                --sp;
             }
         }
-        if (!opened) {
-            if (bw[0] == 0) {  // every register batch is empty
-                if (mtop == 0) break;
-                bw[0] = stk[(uint64_t)(--mtop) * stride];
-                mentries -= bw[0] & 7u;
-            }
-            const uint32_t c = bw[0] & 7u;
-            node = (bw[0] & ~7u) + 1u + ((kPopDigit >> (4u * (c - 1u))) & 7u);
-            if (c == 1) {  // batch 0 is done: the others up one
-#pragma unroll
-                for (int k = 0; k < kBatches - 1; ++k) bw[k] = bw[k + 1];
-                bw[kBatches - 1] = 0;
+        bool take = false, open = false;
+        int32_t r = 0;
+        uint32_t node = 0;
+        if (have) {
+            node = 8u * cell + 1u + digit;
+            const double4 c = cm[node];
+            r = ref[node];
+            const double d_x = c.x - px;
+            const double d_y = c.y - py;
+            const double d_z = c.z - pz;
+            const double d2 = d_x * d_x + d_y * d_y + d_z * d_z;
+            const bool real = r != kRefEmpty && c.w != 0;
+            if (r < 0) {
+                take = real && r != self_ref;
             } else {
-                bw[0] -= 1u;
+                take = test.far((int)level, d2);
+                open = real && !take;
+                take = real && take;
+            }
+        }
+        uint32_t mt = team_bits(__ballot(take)), mo = team_bits(__ballot(open));
+        cnt += __popc(mt);
+        // the accepted children before the first one to open
+        const uint32_t q = (uint32_t)__builtin_ctz(mo | 0x100u);
+        const uint32_t before = (1u << q) - 1u, above = ~(2u * before + 1u);
+        if (take && p < q) L.list[team][ln + __popc(mt & below)] = node;
+        ln += __popc(mt & before);
+        mt &= above;
+        mo &= above;
+        const uint32_t q2 = (uint32_t)__builtin_ctz(mo | 0x100u);
+        const uint32_t next = (uint32_t)__shfl(r, (int)(base + (q & 7u)), 64);
+        const uint32_t next2 = (uint32_t)__shfl(r, (int)(base + (q2 & 7u)), 64);
+        have = q < 8;
+        if (have) {
+            if (mt | mo) {
+                if (p == 0) {
+                    L.cell[sp][team] = cell;
+                    L.ref[sp][team] = next2;
+                    L.masks[sp][team] = level << 16 | mo << 8 | mt;
+                }
+                ++sp;
+            }
+            cell = next;
+            ++level;
+            if (level > kMaxDepth + 1 || budget-- == 0) {  // a corrupt octree
+                if (p == 0) raise_flag(h, kFlagStack);
+                have = false;
+                sp = 0;
+                late = kTeamStack;
             }
         }
     }
+    flush(true);
+    if (!valid) return;
+    if (p < 3) (p == 0 ? ax : (p == 1 ? ay : az))[i] = acc * G;
+    if (inter && p == 3) inter[i] = cnt;
+}
+
+// k_bh_exact_wave: a wave walks the tree once for 64 bodies in octree order.  It
+// visits, in the reference's pre-order, every node that any of them visits, and
+// each lane takes part in the subtrees of the cells that its own body opens, so a
+// body's accepted nodes come by in its own visit order.  The node at hand is the
+// same for the whole wave: its record is an LDS broadcast (through v_readlane or
+// the scalar cache: 7.2 and 8.2 ms on the 1M-body disk), empty slots cost a bit
+// of a mask.  Bound by FP64 issue: on that disk a wave visits 2826 nodes, of
+// which a body accepts 1130, at about 320 cycles each.
+constexpr uint32_t kFrames = 8;  // levels of a wave's path whose children are kept in LDS
+struct WaveLds {
+    double4 cm[kFrames][8];           // by visit position
+    int32_t ref[kFrames][8];
+    uint2 path[kTeamStack];           // per level with children left: cell, their positions
+};
+
+__global__ void __launch_bounds__(kExactThreads) __attribute__((amdgpu_waves_per_eu(8)))
+k_bh_exact_wave(uint32_t n, const uint32_t *__restrict__ order, const double *__restrict__ x,
+                const double *__restrict__ y, const double *__restrict__ z,
+                const double4 *__restrict__ cm, const int32_t *__restrict__ ref, double G,
+                double eps2, double theta, uint32_t icap, double *ax, double *ay, double *az,
+                uint32_t *inter, TreeHdr *h) {
+    __shared__ WaveLds lds[kExactWaves];
+    const uint32_t lb = xcd_contiguous_block();
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    WaveLds &L = lds[w];
+    const uint64_t first = (uint64_t)(lb * kExactWaves + w) * 64u;
+    if (first >= n) return;
+    const bool valid = first + lane < n;
+    const uint32_t i = order[valid ? first + lane : first];
+    const int32_t self_ref = ref_of_body(i);
+    const double px = x[i], py = y[i], pz = z[i];
+    double acc_x = 0, acc_y = 0, acc_z = 0;
+    uint32_t cnt = 0;
+    const ExactTest test(h->edge, theta);
+    // Levels: the root's slot is the only child of level 0, the children of the
+    // root cell are level 1, and so on.  A lane takes part in level l if its
+    // body opened the cell above (opened >= l; -1: no body).
+    int opened = valid ? 0 : -1;
+    uint64_t frames = 1;  // the levels whose children are in their frame (level mod kFrames)
+    uint64_t resume = 0;  // the levels with children left
+    const uint32_t digit = visit_digit(lane & 7u);
+    int level = 0;
+    uint32_t cell = 0;  // above the level
+    // the children of `cell` into the level's frame; returns the positions of
+    // those with a mass
+    auto load_frame = [&](bool root) {
+        const uint64_t node = root ? 0ull : 8ull * cell + 1u + digit;
+        const double4 c = cm[node];
+        const int32_t r = ref[node];
+        const uint32_t k = (uint32_t)level % kFrames;
+        wave_lds_sync();
+        if (lane < 8) {
+            L.cm[k][lane] = c;
+            L.ref[k][lane] = r;
+        }
+        wave_lds_sync();
+        frames &= ~(0x0101010101010101ull << k);
+        frames |= 1ull << level;
+        return (uint32_t)__ballot(r != kRefEmpty && c.w != 0) & (root ? 1u : 0xffu);
+    };
+    uint32_t left = load_frame(true);
+    uint32_t budget = icap + 16;  // a correct octree enters a cell once
+    for (;;) {
+        const bool here = opened >= level;
+        const double far2 = test.far2(level), near2 = test.near2(level);
+        const uint32_t k = (uint32_t)level % kFrames;
+        bool open = false;
+        int32_t r = 0;
+        while (left) {  // the level's children until one is opened
+            const uint32_t p = (uint32_t)__builtin_ctz(left);
+            left &= left - 1;
+            const double4 c = L.cm[k][p];
+            r = (int32_t)wave_uniform((uint32_t)L.ref[k][p]);
+            const double d_x = c.x - px;
+            const double d_y = c.y - py;
+            const double d_z = c.z - pz;
+            const double d2 = d_x * d_x + d_y * d_y + d_z * d_z;
+            bool take;
+            if (r < 0) {
+                take = here && r != self_ref;
+            } else {
+                bool far = d2 > far2;
+                if (here && !far && !(d2 < near2)) far = test.exact(level, d2);
+                open = here && !far;
+                take = here && far;
+            }
+            if (take) {
+                double den = d2 + eps2;
+                den = den * den * den;
+                den = inv_sqrt_ieee(den);
+                acc_x += c.w * (d_x * den);
+                acc_y += c.w * (d_y * den);
+                acc_z += c.w * (d_z * den);
+                ++cnt;
+            }
+            if (__ballot(open)) break;
+        }
+        if (__ballot(open)) {
+            if (left) {
+                L.path[level] = make_uint2(cell, left);
+                resume |= 1ull << level;
+            }
+            ++level;
+            if (budget-- == 0 || level > kMaxDepth + 1) {  // a corrupt octree
+                if (lane == 0) raise_flag(h, kFlagStack);
+                break;
+            }
+            if (open) opened = level;
+            cell = (uint32_t)r;
+            left = load_frame(false);
+        } else {
+            if (resume == 0) break;
+            level = 63 - __clzll((long long)resume);
+            resume &= ~(1ull << level);
+            wave_lds_sync();
+            const uint2 at = L.path[level];
+            cell = wave_uniform(at.x);
+            if (!(frames >> level & 1ull)) (void)load_frame(false);
+            left = wave_uniform(at.y);
+            opened = min(opened, level);
+        }
+    }
+    if (!valid) return;
     ax[i] = acc_x * G;
     ay[i] = acc_y * G;
     az[i] = acc_z * G;
@@ -692,13 +938,6 @@ __device__ inline uint32_t count_below(uint64_t mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                      __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
-
-// A value every lane of the wave holds alike, made visibly uniform (SGPR).
-// The walks below are wave-collective (ballots, shuffles, one LDS list per
-// wave): every branch that steers them must be uniform to the compiler, or
-// control-flow structurisation may let parts of the wave run different
-// iterations with partial exec masks.
-__device__ inline uint32_t wave_uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // lane 0's value of v, uniform
 __device__ inline uint32_t lane0_uniform(uint32_t v) { return wave_uniform(__shfl(v, 0, 64)); }
@@ -1825,13 +2064,37 @@ void launch_direct_split(bool fp64, uint32_t n, const double *x, const double *y
 }
 
 void launch_bh_exact(const TreeBufs &t, const double *x, const double *y, const double *z,
-                     double G, double eps2, double theta, int sort_bodies, uint32_t *stack,
-                     uint32_t stack_cap, double *ax, double *ay, double *az,
+                     double G, double eps2, double theta, double *ax, double *ay, double *az,
                      uint32_t *interactions, hipStream_t s) {
-    hipLaunchKernelGGL(k_bh_exact, dim3(ceil_div(t.n, kExactThreads)), dim3(kExactThreads), 0, s,
-                       t.n, sort_bodies ? (const uint32_t *)t.sidx : nullptr, x, y, z,
-                       (const double4 *)t.cm, (const double *)t.edge, (const int32_t *)t.ref, G,
-                       eps2, theta, stack, stack_cap, t.icap, ax, ay, az, interactions, t.hdr);
+    // Waves of 64 bodies from 100,000 bodies at theta 0.5 and below, up to
+    // 210,000 at theta 1.05 and above: they need fewer instructions per node but
+    // leave one wave per 64 bodies, whose visits follow one another, and short
+    // walks share less.  Traversal, ms (teams, waves, a stack per lane):
+    //   80,001 disk, 0.5      0.79   1.27   1.42
+    //   100,003 Plummer, 0.7  1.03   1.05   1.24
+    //   100,003 Plummer, 1.05 0.49   0.56   0.57
+    //   131,072 Plummer, 0.5  2.68   2.40   2.86
+    //   150,001 disk, 1.05    0.34   0.44   0.37
+    //   200,001 disk, 0.7     0.96   0.91   0.97
+    //   262,144 Plummer, 0.7  2.48   1.48   1.87
+    //   205,001 disk, 1.05    0.47   0.49   0.42
+    //   230,001 Plummer, 1.05 1.14   0.77   0.84
+    //   300,001 disk, 0.85    -      0.85   0.79
+    //   600,000 Plummer, 1.05 2.60   1.46   1.62
+    //   1,048,576 disk, 1.05  2.36   1.49   1.49
+    // (a stack per lane still did a little better on short walks of 0.2 to 0.5 M
+    // bodies of a disk, whose neighbours share little of them)
+    const double from = 100e3 + 200e3 * std::min(std::max(theta - 0.5, 0.0), 0.55);
+    if (t.n >= from)
+        hipLaunchKernelGGL(k_bh_exact_wave, dim3(ceil_div(t.n, 64 * kExactWaves)),
+                           dim3(kExactThreads), 0, s, t.n, (const uint32_t *)t.sidx, x, y, z,
+                           (const double4 *)t.cm, (const int32_t *)t.ref, G, eps2, theta, t.icap,
+                           ax, ay, az, interactions, t.hdr);
+    else
+        hipLaunchKernelGGL(k_bh_exact_team, dim3(ceil_div(t.n, kTeams * kExactWaves)),
+                           dim3(kExactThreads), 0, s, t.n, (const uint32_t *)t.sidx, x, y, z,
+                           (const double4 *)t.cm, (const int32_t *)t.ref, G, eps2, theta, t.icap,
+                           ax, ay, az, interactions, t.hdr);
 }
 
 void launch_bh_group(const TreeBufs &t, const double *x, const double *y, const double *z,

@@ -5,8 +5,8 @@
 //   octree    per sorted position:  skey (u64), sidx (u32), klo (u64), lcp (i32)
 //             per internal node k:  depth, parent, node id, child count,
 //                                   arrival counter, sums {x*m, y*m, z*m, m}, count
-//             per node id:          ref (i32), cm {com_x, com_y, com_z, m} (double4),
-//                                   edge (double), r_open^2 (float)
+//             per node id:          ref (i32), cm {com_x, com_y, com_z, m} (double4)
+//                                   or an FP32 record (NodeF32)
 // A node id is 0 for the root and 1 + 8*k + digit for the child with octant
 // digit `digit` of internal node k, so the 8 children of a cell are adjacent.
 #pragma once
@@ -163,7 +163,6 @@ struct TreeBufs {
     uint32_t spanning_cap = 0;
     int32_t *ref = nullptr;
     double4 *cm = nullptr;          // FP64 records (reference-semantics traversal)
-    double *edge = nullptr;
     NodeF32 *rec = nullptr;         // FP32 records (group traversal)
     // scan / sort scratch
     uint32_t *scan_part = nullptr;
@@ -262,7 +261,7 @@ void launch_key_sort(TreeBufs &t, hipStream_t s);
 void launch_topology(const TreeBufs &t, const double *x, const double *y, const double *z,
                      hipStream_t s);
 // Centre of mass with the node records and traversal groups.  f64: FP64
-// records (cm, edge) for the reference-semantics traversal; f32: packed FP32
+// records (cm) for the reference-semantics traversal; f32: packed FP32
 // records and traversal groups for the group traversal.
 void launch_com(const TreeBufs &t, double G, bool f64, bool f32, GroupRule rule, hipStream_t s);
 // hdr->max_depth of the last build (not maintained by the build itself)
@@ -294,8 +293,7 @@ void launch_direct_split(bool fp64, uint32_t n, const double *x, const double *y
                          double *ay, double *az, double *partial, hipStream_t s);
 uint64_t direct_split_scratch_bytes(uint32_t n);
 void launch_bh_exact(const TreeBufs &t, const double *x, const double *y, const double *z,
-                     double G, double eps2, double theta, int sort_bodies, uint32_t *stack,
-                     uint32_t stack_cap, double *ax, double *ay, double *az,
+                     double G, double eps2, double theta, double *ax, double *ay, double *az,
                      uint32_t *interactions, hipStream_t s);
 // gquad: G*Q records of the internal cells (two float4 each) for the
 // quadrupole walk, or null for monopole cells

@@ -32,8 +32,8 @@
 //     and invalidate the L2 of an XCD at every arrival); the few cells that
 //     cross block boundaries are finished level by level by one workgroup.
 //  8. Node records for traversal (COM = numerator / mass as the reference
-//     divides per visit, edge = rootEdge * 2^-depth; an FP32 hi/lo record for
-//     the group traversal).
+//     divides per visit; an FP32 hi/lo record for the group traversal).  A
+//     cell's edge is rootEdge * 2^-depth wherever it is needed.
 #include <algorithm>
 #include <cmath>
 
@@ -519,9 +519,8 @@ __device__ inline double4 body_term(const double4 p) {
 // record, and its group if the root holds at most rule.group_max bodies.
 struct RecOut {
     double G;
-    int f64, f32;  // FP64 records (cm, edge); FP32 records and traversal groups
+    int f64, f32;  // FP64 records (cm); FP32 records and traversal groups
     double4 *cm;
-    double *edge;
     NodeF32 *rec;
     uint32_t *group_size, *group_slot;
     GroupRule rule;  // group size and packing limit
@@ -534,12 +533,8 @@ __device__ inline double4 term_com(const double4 v) {
     return make_double4(v.x / v.w, v.y / v.w, v.z / v.w, v.w);
 }
 
-__device__ inline void put_record(const RecOut &o, uint64_t j, int32_t r, const double4 c,
-                                  double e) {
-    if (o.f64) {
-        o.cm[j] = c;
-        o.edge[j] = e;
-    }
+__device__ inline void put_record(const RecOut &o, uint64_t j, int32_t r, const double4 c) {
+    if (o.f64) o.cm[j] = c;
     if (o.f32) {
         NodeF32 q;
         q.x = (float)c.x;
@@ -596,21 +591,19 @@ __device__ inline void put_child_groups(const RecOut &o, uint32_t first, const u
 // position `first`), given their refs, terms and body counts; the root's own
 // record and group when pk is the root.
 __device__ inline void cell_outputs(const RecOut &o, uint32_t pk, uint32_t depth, uint32_t first,
-                                    double root_edge, const int32_t (&r)[8],
-                                    const double4 (&v)[8], const uint32_t (&c)[8],
+                                    const int32_t (&r)[8], const double4 (&v)[8], const uint32_t (&c)[8],
                                     const double4 s, uint32_t cnt) {
     const uint64_t base = 1ull + 8ull * pk;
-    const double ce = ldexp(root_edge, -(int)(depth + 1));
 #pragma unroll
     for (int d = 0; d < 8; ++d) {
         if (r[d] == kRefEmpty)
-            put_record(o, base + d, kRefEmpty, make_double4(0.0, 0.0, 0.0, 0.0), 0.0);
+            put_record(o, base + d, kRefEmpty, make_double4(0.0, 0.0, 0.0, 0.0));
         else
-            put_record(o, base + d, r[d], term_com(v[d]), r[d] >= 0 ? ce : 0.0);
+            put_record(o, base + d, r[d], term_com(v[d]));
     }
     if (cnt > o.rule.group_max) put_child_groups(o, first, c);
     if (depth == 0) {
-        put_record(o, 0, (int32_t)pk, term_com(s), root_edge);
+        put_record(o, 0, (int32_t)pk, term_com(s));
         if (cnt <= o.rule.group_max) put_group(o, first, cnt);
     }
 }
@@ -618,7 +611,7 @@ __device__ inline void cell_outputs(const RecOut &o, uint32_t pk, uint32_t depth
 // The global-memory path: the cell's 8 children summed in digit order from 0.0,
 // then the children's records and groups.
 __device__ inline void sum_children_out(uint32_t pk, uint32_t depth, uint32_t first,
-                                        double root_edge, const double4 *__restrict__ body4,
+                                        const double4 *__restrict__ body4,
                                         const int32_t *__restrict__ ref, InternalSums *sums,
                                         uint32_t *counts, TreeHdr *h, const RecOut &o) {
     const uint64_t base = 1ull + 8ull * pk;
@@ -646,7 +639,7 @@ __device__ inline void sum_children_out(uint32_t pk, uint32_t depth, uint32_t fi
     sums[pk] = q;
     counts[pk] = cnt;
     if (q.m == 0) raise_flag(h, kFlagZeroMass);
-    cell_outputs(o, pk, depth, first, root_edge, r, v, c, make_double4(q.x, q.y, q.z, q.m), cnt);
+    cell_outputs(o, pk, depth, first, r, v, c, make_double4(q.x, q.y, q.z, q.m), cnt);
 }
 
 // Centre of mass, level by level from the deepest cells up: a cell's sums
@@ -735,7 +728,6 @@ __device__ __forceinline__ void com_local_block(
     const uint32_t t = threadIdx.x;
     const uint32_t s = blk * kComBlock;
     const uint32_t e = min(n, s + kComBlock);
-    const double root_edge = h->edge;
     {
         // all index loads, then all body loads, in flight together
         uint32_t bi[kComBodiesPerThread];
@@ -764,7 +756,7 @@ __device__ __forceinline__ void com_local_block(
     if (n < 2) {  // a lone body is the root leaf: no internal cell
         __syncthreads();
         if (t == 0) {
-            put_record(o, 0, ref_of_body(i_s[0]), term_com(body_term(b_s[0])), 0.0);
+            put_record(o, 0, ref_of_body(i_s[0]), term_com(body_term(b_s[0])));
             put_group(o, 0, 1);
         }
         return;
@@ -777,7 +769,7 @@ __device__ __forceinline__ void com_local_block(
     if (nc > kComLdsCells) {  // the same for the whole workgroup
         com_levels(kb, ke, [&](uint32_t k) { return int_local[k] == 1; }, int_depth, lvl, cnt,
                    cur, [&](uint32_t k) {
-                       sum_children_out(k, int_depth[k], int_first[k], root_edge, body4, ref,
+                       sum_children_out(k, int_depth[k], int_first[k], body4, ref,
                                         sums, counts, h, o);
                    });
         return;
@@ -887,25 +879,23 @@ __device__ __forceinline__ void com_local_block(
         const uint16_t code = code_s[j];
         const uint32_t pc = n_s[c];
         if (code == kCodeEmpty) {
-            put_record(o, slot, kRefEmpty, make_double4(0.0, 0.0, 0.0, 0.0), 0.0);
+            put_record(o, slot, kRefEmpty, make_double4(0.0, 0.0, 0.0, 0.0));
         } else if (code < kComLdsCells) {
-            put_record(o, slot, (int32_t)(kb + code), term_com(c_s[code]),
-                       ldexp(root_edge, -(int)(dc + 1)));
+            put_record(o, slot, (int32_t)(kb + code), term_com(c_s[code]));
         } else if ((code & kCodeAt) && code < kCodeFar) {
             const uint32_t pos = code & ~kCodeAt;
-            put_record(o, slot, ref_of_body(i_s[pos]), term_com(body_term(b_s[pos])), 0.0);
+            put_record(o, slot, ref_of_body(i_s[pos]), term_com(body_term(b_s[pos])));
         } else {  // not for a local cell: the child from global memory
             const int32_t r = ref[slot];
             if (r >= 0) {
                 const InternalSums g = sums[r];
-                put_record(o, slot, r, term_com(make_double4(g.x, g.y, g.z, g.m)),
-                           ldexp(root_edge, -(int)(dc + 1)));
+                put_record(o, slot, r, term_com(make_double4(g.x, g.y, g.z, g.m)));
             } else {
-                put_record(o, slot, r, term_com(body_term(body4[body_of_ref(r)])), 0.0);
+                put_record(o, slot, r, term_com(body_term(body4[body_of_ref(r)])));
             }
         }
         if (dc == 0 && (j & 7u) == 0) {  // the root (the block holds every body)
-            put_record(o, 0, (int32_t)(kb + c), term_com(c_s[c]), root_edge);
+            put_record(o, 0, (int32_t)(kb + c), term_com(c_s[c]));
             if (pc <= o.rule.group_max) put_group(o, s + first_s[c], pc);
         }
     }
@@ -956,7 +946,6 @@ __device__ __forceinline__ void com_span_block(
     const uint32_t r0 = sb * rows;
     const uint32_t r1 = min(nblocks, r0 + rows);
     const uint64_t slot0 = (uint64_t)r0 * kMaxDepth, slot1 = (uint64_t)r1 * kMaxDepth;
-    const double root_edge = h->edge;
     if (t == 0) {
         ncell = 0;
         nx = 0;
@@ -1011,7 +1000,7 @@ __device__ __forceinline__ void com_span_block(
                 for (uint32_t i = t; i < ncross; i += kComThreads)
                     if ((cross[i] & 63u) == (uint32_t)d) {
                         const uint32_t k = cross[i] >> 6;
-                        sum_children_out(k, (uint32_t)d, int_first[k], root_edge, body4, ref,
+                        sum_children_out(k, (uint32_t)d, int_first[k], body4, ref,
                                          sums, counts, h, o);
                     }
             } else {
@@ -1019,7 +1008,7 @@ __device__ __forceinline__ void com_span_block(
                      j += (uint64_t)kComThreads * kMaxDepth) {
                     const uint32_t k = spanning[j];
                     if (k != kNoCell && int_local[k] == want)
-                        sum_children_out(k, (uint32_t)d, int_first[k], root_edge, body4, ref,
+                        sum_children_out(k, (uint32_t)d, int_first[k], body4, ref,
                                          sums, counts, h, o);
                 }
             }
@@ -1054,14 +1043,14 @@ __device__ __forceinline__ void com_span_block(
                 const InternalSums q = sums[r];
                 v = make_double4(q.x, q.y, q.z, q.m);
                 code = counts[r];
-                put_record(o, j, r, term_com(v), ldexp(root_edge, -(int)(ldep[id] + 1u)));
+                put_record(o, j, r, term_com(v));
             }
         } else if (r != kRefEmpty) {
             v = body_term(body4[body_of_ref(r)]);
             code = 1;
-            put_record(o, j, r, term_com(v), 0.0);
+            put_record(o, j, r, term_com(v));
         } else {
-            put_record(o, j, kRefEmpty, v, 0.0);
+            put_record(o, j, kRefEmpty, v);
         }
         cv[p] = v;
         cc[p] = code;
@@ -1122,9 +1111,9 @@ __device__ __forceinline__ void com_span_block(
         const uint32_t pc = sn[id];
         if (code != kChildEmpty && (code & kChildHere))
             put_record(o, 1ull + 8ull * list[id] + dd, (int32_t)list[code & ~kChildHere],
-                       term_com(sv[code & ~kChildHere]), ldexp(root_edge, -(int)(ldep[id] + 1u)));
+                       term_com(sv[code & ~kChildHere]));
         if (dd == 0 && ldep[id] == 0) {  // the root
-            put_record(o, 0, (int32_t)list[id], term_com(sv[id]), root_edge);
+            put_record(o, 0, (int32_t)list[id], term_com(sv[id]));
             if (pc <= o.rule.group_max) put_group(o, fst[id], pc);
         }
     }
@@ -1480,7 +1469,7 @@ __device__ inline ForestTree forest_tree(const EnsSystem *__restrict__ sys, uint
     f.S = sys[s];
     f.h = fb.hdr + s;
     const uint32_t fo = f.S.fb_off;
-    f.o = RecOut{G, 0, 1, nullptr, nullptr, fb.rec + f.S.node_off, fb.group_size + fo,
+    f.o = RecOut{G, 0, 1, nullptr, fb.rec + f.S.node_off, fb.group_size + fo,
                  fb.group_slot + fo, rule};
     return f;
 }
@@ -1666,9 +1655,8 @@ void launch_max_depth(const TreeBufs &t, hipStream_t s) {
 
 void launch_com(const TreeBufs &t, double G, bool f64, bool f32, GroupRule rule, hipStream_t s) {
     const uint32_t nblocks = ceil_div(t.n, kComBlock);
-    const RecOut o{G,          (int)f64,      (int)f32,      t.cm,
-                   t.edge,     t.rec,         t.group_size,  t.group_slot,
-                   rule};
+    const RecOut o{G,     (int)f64,     (int)f32,     t.cm,
+                   t.rec, t.group_size, t.group_slot, rule};
     hipLaunchKernelGGL(k_com_local, dim3(nblocks), dim3(kComLocalThreads), 0, s, t.n, t.icap, t.hdr,
                        (const double4 *)t.body4, (const uint32_t *)t.sidx, (const int32_t *)t.ref,
                        (const uint32_t *)t.chain, (const uint8_t *)t.int_depth,

@@ -401,6 +401,33 @@ def test_bh_exact_bitexact(gpu, oracle, kind, n, theta):
         np.testing.assert_array_equal(bits(a), bits(r))
 
 
+# The two kernels of the bit-exact traversal: teams of eight lanes at the edges
+# of a wave's bodies (8) and a workgroup's (32), waves of 64 bodies on both sides
+# of the rule between them (100,000 bodies at theta 0.5, 210,000 at 1.05), whole
+# waves and one body over.  theta 1e-150 and 1e150 leave the range in which the
+# opening test is decided from squares.
+@pytest.mark.parametrize("kind,n,theta", [("cube", 7, 0.5), ("cube", 8, 0.3), ("cube", 9, 0.0),
+                                          ("cube", 31, 0.7), ("plummer", 33, 0.7),
+                                          ("plummer", 65, 1e-150), ("plummer", 700, 1e150),
+                                          ("plummer", 99999, 0.5), ("plummer", 100001, 0.5),
+                                          ("cluster", 100032, 0.5), ("disk", 140033, 0.7),
+                                          ("plummer", 209999, 1.05), ("disk", 210049, 1.05),
+                                          ("plummer", 100001, 1e150)])
+def test_bh_exact_kernels_bitexact(gpu, oracle, kind, n, theta):
+    d = make(gpu, kind, n, seed=17)
+    t = oracle.Tree(n)
+    t.build(d["x"], d["y"], d["z"], d["m"])
+    rx, ry, rz, rint = t.bh_accel(theta)
+    for sort_bodies in (1, 0):
+        with ctx_for(gpu, d, theta=theta, sort_bodies=sort_bodies) as c:
+            c.bh_build()
+            ax, ay, az = c.bh_forces()
+            inter = c.interactions()
+        np.testing.assert_array_equal(inter, rint)
+        for a, r in ((ax, rx), (ay, ry), (az, rz)):
+            np.testing.assert_array_equal(bits(a), bits(r))
+
+
 def test_bh_exact_deep_runs(gpu, oracle):
     # pairs closer than edge/2^21: each pair hangs under ~25 single-child
     # cells, so the walk opens long chains whose pushed batches are all empty
