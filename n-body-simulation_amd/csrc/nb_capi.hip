@@ -11,6 +11,7 @@
 #include <string>
 #include <vector>
 
+#include "nb_hostcopy.h"
 #include "nb_mlp.h"
 
 using nb::TreeBufs;
@@ -21,11 +22,14 @@ struct nb_ctx {
     nb_params p{};
     int device = 0;
     hipStream_t stream = nullptr;
+    // one allocation, the arrays `stride` doubles apart in this order
+    size_t stride = 0;
     double *x = nullptr, *y = nullptr, *z = nullptr;
     double *vx = nullptr, *vy = nullptr, *vz = nullptr;
-    double *vhx = nullptr, *vhy = nullptr, *vhz = nullptr;
     double *ax = nullptr, *ay = nullptr, *az = nullptr;
+    double *vhx = nullptr, *vhy = nullptr, *vhz = nullptr;
     double *m = nullptr;
+    nb::HostCopier copier;
     uint32_t *inter = nullptr;
     TreeBufs tree;
     bool tree_valid = false;
@@ -43,7 +47,7 @@ struct nb_ctx {
     nb::MlpCell *mcell = nullptr;    // per internal cell
     float4 *gquad = nullptr;         // 2 per internal cell: G*Q for the quadrupole walk
     bool quad_valid = false;         // quadrupoles match the current octree
-    // asynchronous snapshots: device staging (9 n doubles), two pinned host
+    // asynchronous snapshots: device staging (9 stride doubles), two pinned host
     // slots used in turn, the DMA stream and the event that ends each DMA
     double *snap_dev = nullptr;
     double *snap_host[2] = {nullptr, nullptr};
@@ -383,6 +387,16 @@ int direct_enqueue(nb_ctx *c) {
     return NB_OK;
 }
 
+// the arrays with a destination, n doubles each, to the host
+int copy_out(nb_ctx *c, double *const *dst, const double *const *src, int count) {
+    nb::HostCopier::Array a[nb::HostCopier::kArrays];
+    int k = 0;
+    for (int i = 0; i < count; ++i)
+        if (dst[i]) a[k++] = {dst[i], src[i], (size_t)c->n};
+    NB_HIP(c, c->copier.copy(c->stream, a, k));
+    return NB_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -450,19 +464,20 @@ int nb_create(nb_ctx **out, uint32_t n, const nb_params *p) {
     };
     if (hipGetDevice(&c->device) != hipSuccess) return bail(NB_E_HIP);
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) return bail(NB_E_HIP);
-    double **state[] = {&c->x, &c->y, &c->z, &c->vx, &c->vy, &c->vz, &c->vhx,
-                        &c->vhy, &c->vhz, &c->ax, &c->ay, &c->az, &c->m};
-    for (double **s : state)
-        if ((rc = dev_alloc(c, s, n))) return bail(rc);
+    double **state[] = {&c->x, &c->y, &c->z, &c->vx, &c->vy, &c->vz, &c->ax,
+                        &c->ay, &c->az, &c->vhx, &c->vhy, &c->vhz, &c->m};
+    c->stride = ((size_t)n + 31) / 32 * 32;  // 256-byte lines
+    if ((rc = dev_alloc(c, &c->x, 13ull * c->stride))) return bail(rc);
+    for (int k = 1; k < 13; ++k) *state[k] = c->x + k * c->stride;
     if ((rc = dev_alloc(c, &c->inter, n))) return bail(rc);
     if (hipHostMalloc((void **)&c->hdr_host, sizeof(TreeHdr), hipHostMallocDefault) != hipSuccess)
         return bail(NB_E_HIP);
     std::memset(c->hdr_host, 0, sizeof(TreeHdr));
+    if (c->copier.reserve_small(6ull * n) != hipSuccess) return bail(NB_E_HIP);
     if ((rc = alloc_tree(c))) return bail(rc);
     if (p->quadrupole && (rc = ensure_quad_buffers(c))) return bail(rc);
-    for (double **s : state)
-        if (hipMemsetAsync(*s, 0, (size_t)n * sizeof(double), c->stream) != hipSuccess)
-            return bail(NB_E_HIP);
+    if (hipMemsetAsync(c->x, 0, 13 * c->stride * sizeof(double), c->stream) != hipSuccess)
+        return bail(NB_E_HIP);
     if (hipMemsetAsync(c->inter, 0, (size_t)n * sizeof(uint32_t), c->stream) != hipSuccess)
         return bail(NB_E_HIP);
     if (hipStreamSynchronize(c->stream) != hipSuccess) return bail(NB_E_HIP);
@@ -573,37 +588,29 @@ int nb_set_positions(nb_ctx *c, const double *x, const double *y, const double *
 int nb_get_state(nb_ctx *c, double *x, double *y, double *z, double *vx, double *vy,
                  double *vz) {
     if (!c) return NB_E_INVALID_ARG;
-    const size_t bytes = (size_t)c->n * sizeof(double);
     double *dst[] = {x, y, z, vx, vy, vz};
     const double *src[] = {c->x, c->y, c->z, c->vx, c->vy, c->vz};
-    for (int k = 0; k < 6; ++k)
-        if (dst[k]) NB_HIP(c, hipMemcpyAsync(dst[k], src[k], bytes, hipMemcpyDeviceToHost, c->stream));
-    NB_HIP(c, hipStreamSynchronize(c->stream));
-    return NB_OK;
+    return copy_out(c, dst, src, 6);
 }
 
 int nb_get_accel(nb_ctx *c, double *ax, double *ay, double *az) {
     if (!c) return NB_E_INVALID_ARG;
-    const size_t bytes = (size_t)c->n * sizeof(double);
     double *dst[] = {ax, ay, az};
     const double *src[] = {c->ax, c->ay, c->az};
-    for (int k = 0; k < 3; ++k)
-        if (dst[k]) NB_HIP(c, hipMemcpyAsync(dst[k], src[k], bytes, hipMemcpyDeviceToHost, c->stream));
-    NB_HIP(c, hipStreamSynchronize(c->stream));
-    return NB_OK;
+    return copy_out(c, dst, src, 3);
 }
 
 int nb_snapshot_begin(nb_ctx *c) {
     if (!c) return NB_E_INVALID_ARG;
-    const size_t n = c->n, bytes = n * sizeof(double);
+    const size_t bytes = 9 * c->stride * sizeof(double);  // x .. az lie in a row
     if (!c->snap_done) {
         // first use; a failure part-way leaves what was made for the next try
         if (!c->snap_dev) {
-            int rc = dev_alloc(c, &c->snap_dev, 9ull * n);
+            int rc = dev_alloc(c, &c->snap_dev, 9ull * c->stride);
             if (rc) return rc;
         }
         for (double *&h : c->snap_host)
-            if (!h) NB_HIP(c, hipHostMalloc((void **)&h, 9 * bytes, hipHostMallocDefault));
+            if (!h) NB_HIP(c, hipHostMalloc((void **)&h, bytes, hipHostMallocDefault));
         if (!c->copy_stream)
             NB_HIP(c, hipStreamCreateWithFlags(&c->copy_stream, hipStreamNonBlocking));
         if (!c->snap_staged)
@@ -613,14 +620,11 @@ int nb_snapshot_begin(nb_ctx *c) {
         // the staging buffer is reused: the previous DMA must have read it
         NB_HIP(c, hipStreamWaitEvent(c->stream, c->snap_done, 0));
     }
-    const double *src[9] = {c->x, c->y, c->z, c->vx, c->vy, c->vz, c->ax, c->ay, c->az};
-    for (int k = 0; k < 9; ++k)
-        NB_HIP(c, hipMemcpyAsync(c->snap_dev + k * n, src[k], bytes, hipMemcpyDeviceToDevice,
-                                 c->stream));
+    NB_HIP(c, hipMemcpyAsync(c->snap_dev, c->x, bytes, hipMemcpyDeviceToDevice, c->stream));
     NB_HIP(c, hipEventRecord(c->snap_staged, c->stream));
     NB_HIP(c, hipStreamWaitEvent(c->copy_stream, c->snap_staged, 0));
     c->snap_slot ^= 1;
-    NB_HIP(c, hipMemcpyAsync(c->snap_host[c->snap_slot], c->snap_dev, 9 * bytes,
+    NB_HIP(c, hipMemcpyAsync(c->snap_host[c->snap_slot], c->snap_dev, bytes,
                              hipMemcpyDeviceToHost, c->copy_stream));
     NB_HIP(c, hipEventRecord(c->snap_done, c->copy_stream));
     c->snap_begun = true;
@@ -631,7 +635,7 @@ int nb_snapshot_wait(nb_ctx *c, const double **arrays) {
     if (!c || !arrays) return NB_E_INVALID_ARG;
     if (!c->snap_begun) return fail(c, NB_E_INVALID_ARG, "nb_snapshot_wait: no snapshot begun");
     NB_HIP(c, hipStreamSynchronize(c->copy_stream));
-    for (int k = 0; k < 9; ++k) arrays[k] = c->snap_host[c->snap_slot] + (size_t)k * c->n;
+    for (int k = 0; k < 9; ++k) arrays[k] = c->snap_host[c->snap_slot] + (size_t)k * c->stride;
     return NB_OK;
 }
 

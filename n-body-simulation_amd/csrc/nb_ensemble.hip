@@ -20,6 +20,7 @@
 #include <string>
 #include <vector>
 
+#include "nb_hostcopy.h"
 #include "nb_internal.h"
 
 using nb::EnsSystem;
@@ -53,6 +54,7 @@ struct nb_ensemble {
     std::vector<std::pair<int, size_t>> marks;
     double phase[kEnsPhases] = {0};
     std::vector<void *> allocations;
+    nb::HostCopier copier;
     std::string err;
 };
 
@@ -243,6 +245,16 @@ int reset_status(nb_ensemble *e) {
     return NB_OK;
 }
 
+// the arrays with a destination, one entry per body each, to the host
+int copy_out(nb_ensemble *e, double *const *dst, const double *const *src, int count) {
+    nb::HostCopier::Array a[nb::HostCopier::kArrays];
+    int k = 0;
+    for (int i = 0; i < count; ++i)
+        if (dst[i]) a[k++] = {dst[i], src[i], (size_t)e->nbody};
+    ENS_HIP(e, e->copier.copy(e->stream, a, k));
+    return NB_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -304,10 +316,12 @@ int nb_ensemble_create(nb_ensemble **out, uint32_t nsys, const uint32_t *sizes,
     if (io >= (1ull << 32) || fo >= (1ull << 30) || span >= (1ull << 32) || xo >= (1ull << 32))
         return bail(NB_E_INVALID_ARG);
     int rc;
-    double **st[] = {&e->x, &e->y, &e->z, &e->vx, &e->vy, &e->vz, &e->vhx,
-                     &e->vhy, &e->vhz, &e->ax, &e->ay, &e->az, &e->m};
-    for (double **a : st)
-        if ((rc = ealloc(e, a, total))) return bail(rc);
+    // one allocation, so that the arrays of a small ensemble leave in one DMA
+    double **st[] = {&e->x, &e->y, &e->z, &e->vx, &e->vy, &e->vz, &e->ax,
+                     &e->ay, &e->az, &e->vhx, &e->vhy, &e->vhz, &e->m};
+    const uint64_t stride = (total + 31) / 32 * 32;  // 256-byte lines
+    if ((rc = ealloc(e, &e->x, 13 * stride))) return bail(rc);
+    for (int k = 1; k < 13; ++k) *st[k] = e->x + k * stride;
     ForestBufs &f = e->fb;
     if ((rc = ealloc(e, &e->sys, nsys)) || (rc = ealloc(e, &e->dt_sys, nsys)) ||
         (rc = ealloc(e, &e->sys_of, total)) || (rc = ealloc(e, &f.hdr, nsys)) ||
@@ -333,6 +347,7 @@ int nb_ensemble_create(nb_ensemble **out, uint32_t nsys, const uint32_t *sizes,
         return bail(rc);
     f.slots = (uint32_t)fo;
     f.scan_cap = nb::scan_scratch_words((uint32_t)fo) + 1;
+    if (e->copier.reserve_small(6 * total) != hipSuccess) return bail(NB_E_HIP);
     if (hipHostMalloc((void **)&e->status_host, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
         return bail(NB_E_HIP);
     *e->status_host = 0;
@@ -407,24 +422,16 @@ int nb_ensemble_set_state(nb_ensemble *e, const double *x, const double *y, cons
 int nb_ensemble_get_state(nb_ensemble *e, double *x, double *y, double *z, double *vx, double *vy,
                           double *vz) {
     if (!e) return NB_E_INVALID_ARG;
-    const size_t bytes = e->nbody * sizeof(double);
     double *dst[] = {x, y, z, vx, vy, vz};
     const double *src[] = {e->x, e->y, e->z, e->vx, e->vy, e->vz};
-    for (int k = 0; k < 6; ++k)
-        if (dst[k]) ENS_HIP(e, hipMemcpyAsync(dst[k], src[k], bytes, hipMemcpyDeviceToHost, e->stream));
-    ENS_HIP(e, hipStreamSynchronize(e->stream));
-    return NB_OK;
+    return copy_out(e, dst, src, 6);
 }
 
 int nb_ensemble_get_accel(nb_ensemble *e, double *ax, double *ay, double *az) {
     if (!e) return NB_E_INVALID_ARG;
-    const size_t bytes = e->nbody * sizeof(double);
     double *dst[] = {ax, ay, az};
     const double *src[] = {e->ax, e->ay, e->az};
-    for (int k = 0; k < 3; ++k)
-        if (dst[k]) ENS_HIP(e, hipMemcpyAsync(dst[k], src[k], bytes, hipMemcpyDeviceToHost, e->stream));
-    ENS_HIP(e, hipStreamSynchronize(e->stream));
-    return NB_OK;
+    return copy_out(e, dst, src, 3);
 }
 
 int nb_ensemble_forces(nb_ensemble *e) {

@@ -1,0 +1,190 @@
+// nb_hostcopy.h -- device arrays into a caller's pageable host memory.
+//
+// hipMemcpyAsync into pageable memory takes about 17 us per call and runs at
+// 8 GB/s, bound by one thread that faults in and fills the caller's pages.  Here
+// the arrays go through pinned memory owned by the context or ensemble:
+//  - small copies (up to kSmall) by one kernel that stores them there, one wait,
+//    and a memcpy per array;
+//  - large ones (from kLarge) are cut into chunks that pass through a ring of
+//    pinned slots by DMA (56 GB/s), and several threads fill the caller's pages
+//    while later chunks are on their way.
+// In between, the runtime's copies into pageable memory are as fast (23,000
+// bodies 0.11 ms, 100,003 0.76; through the ring 0.57 and 0.65).
+// Six arrays of 1024 bodies: 25 us instead of 105; of 1,048,576 bodies (50 MB)
+// 2.5 ms instead of 6.4; of 4,194,304 7.9 ms instead of 21.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <atomic>
+#include <cstdint>
+#include <cstring>
+#include <thread>
+#include <vector>
+
+#include "nb_internal.h"
+
+namespace nb {
+
+class HostCopier {
+  public:
+    struct Array {
+        double *dst;
+        const double *src;  // device
+        size_t n;
+    };
+    static constexpr int kArrays = 6;
+
+    // Pinned memory for small copies of `doubles` in all, made with its owner: a
+    // first copy would pay for the allocation and for a fault per page (1.6 us).
+    hipError_t reserve_small(size_t doubles) {
+        const size_t bytes = doubles * sizeof(double);
+        if (bytes > kSmall) return hipSuccess;
+        const hipError_t e = reserve(bytes);
+        for (size_t o = 0; e == hipSuccess && o < bytes; o += 4096) ring_[o] = 0;
+        return e;
+    }
+
+    ~HostCopier() {
+        for (hipEvent_t e : events_) (void)hipEventDestroy(e);
+        if (ring_) (void)hipHostFree(ring_);
+    }
+
+    // Copies the arrays behind the work already issued on `stream`; returns when
+    // they have arrived.
+    hipError_t copy(hipStream_t stream, const Array *a, int count) {
+        size_t total = 0;
+        for (int k = 0; k < count; ++k) total += a[k].n * sizeof(double);
+        if (total == 0) return hipStreamSynchronize(stream);
+        if (total <= kSmall) return small(stream, a, count, total);
+        if (total >= kLarge) return large(stream, a, count, total);
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < count && e == hipSuccess; ++k)
+            e = hipMemcpyAsync(a[k].dst, a[k].src, a[k].n * sizeof(double), hipMemcpyDeviceToHost,
+                               stream);
+        const hipError_t s = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : s;
+    }
+
+  private:
+    static constexpr size_t kSmall = size_t(1) << 20;
+    static constexpr size_t kLarge = size_t(6) << 20;
+    static constexpr size_t kChunk = size_t(1) << 20;
+    static constexpr uint32_t kSlots = 8;
+    static constexpr unsigned kThreads = 8;
+
+    uint8_t *ring_ = nullptr;
+    size_t ring_bytes_ = 0;
+    std::vector<hipEvent_t> events_;
+
+    hipError_t reserve(size_t bytes) {
+        if (ring_bytes_ >= bytes) return hipSuccess;
+        if (ring_) (void)hipHostFree(ring_);
+        ring_ = nullptr;
+        ring_bytes_ = 0;
+        const hipError_t e = hipHostMalloc((void **)&ring_, bytes, hipHostMallocDefault);
+        if (e != hipSuccess) {
+            ring_ = nullptr;
+            return e;
+        }
+        ring_bytes_ = bytes;
+        return hipSuccess;
+    }
+
+    hipError_t small(hipStream_t stream, const Array *a, int count, size_t total) {
+        hipError_t e = reserve(total);
+        if (e != hipSuccess) return e;
+        CopyOut arg{};
+        size_t at = 0;
+        for (int k = 0; k < count; ++k) {
+            arg.src[k] = a[k].src;
+            arg.dst[k] = (double *)ring_ + at;
+            arg.n[k] = a[k].n;
+            at += a[k].n;
+        }
+        launch_copy_out(arg, count, stream);
+        e = hipGetLastError();
+        const hipError_t s = hipStreamSynchronize(stream);
+        if (e != hipSuccess) return e;
+        if (s != hipSuccess) return s;
+        for (int k = 0; k < count; ++k)
+            std::memcpy(a[k].dst, arg.dst[k], a[k].n * sizeof(double));
+        return hipSuccess;
+    }
+
+    hipError_t large(hipStream_t stream, const Array *a, int count, size_t total) {
+        const size_t chunk = total < 16 * kChunk ? kChunk / 4 : kChunk;
+        hipError_t e = reserve(kSlots * chunk);
+        while (e == hipSuccess && events_.size() < kSlots) {
+            hipEvent_t ev;
+            e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+            if (e == hipSuccess) events_.push_back(ev);
+        }
+        if (e != hipSuccess) return e;
+        struct Chunk {
+            uint8_t *dst;
+            const uint8_t *src;
+            size_t bytes;
+        };
+        std::vector<Chunk> chunks;
+        for (int k = 0; k < count; ++k)
+            for (size_t o = 0, all = a[k].n * sizeof(double); o < all; o += chunk)
+                chunks.push_back({(uint8_t *)a[k].dst + o, (const uint8_t *)a[k].src + o,
+                                  std::min(chunk, all - o)});
+        const uint32_t n = (uint32_t)chunks.size();
+        // Chunk i goes through slot i mod kSlots.  This thread issues the DMAs and
+        // waits for them in order; arrived: chunks that lie in their slots;
+        // filled[s]: chunks that have left slot s.  With threads they fill the
+        // caller's pages (no HIP calls there), without this one does.
+        std::atomic<uint32_t> arrived{0}, next{0};
+        std::atomic<uint32_t> filled[kSlots];
+        for (auto &f : filled) f.store(0);
+        std::atomic<bool> failed{false};
+        auto fill = [&](uint32_t i) {
+            std::memcpy(chunks[i].dst, ring_ + (i % kSlots) * chunk, chunks[i].bytes);
+            filled[i % kSlots].store(i / kSlots + 1, std::memory_order_release);
+        };
+        auto worker = [&] {
+            for (;;) {
+                const uint32_t i = next.fetch_add(1);
+                if (i >= n) return;
+                while (arrived.load(std::memory_order_acquire) <= i) {
+                    if (failed.load()) return;
+                    std::this_thread::yield();
+                }
+                fill(i);
+            }
+        };
+        std::vector<std::thread> threads;
+        const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
+        try {
+            threads.reserve(kThreads);
+            for (unsigned t = 0; t < std::min(cores, total < 16 * kChunk ? 4u : kThreads); ++t)
+                threads.emplace_back(worker);
+        } catch (...) {  // fewer threads, or none
+        }
+        for (uint32_t issued = 0, got = 0; got < n && e == hipSuccess;) {
+            if (issued < n && issued - got < kSlots &&
+                filled[issued % kSlots].load(std::memory_order_acquire) >= issued / kSlots) {
+                e = hipMemcpyAsync(ring_ + (issued % kSlots) * chunk, chunks[issued].src,
+                                   chunks[issued].bytes, hipMemcpyDeviceToHost, stream);
+                if (e == hipSuccess) e = hipEventRecord(events_[issued % kSlots], stream);
+                ++issued;
+            } else if (got < issued) {
+                e = hipEventSynchronize(events_[got % kSlots]);
+                if (e != hipSuccess) break;
+                arrived.store(++got, std::memory_order_release);
+                if (threads.empty()) fill(got - 1);
+            } else {
+                std::this_thread::yield();  // every slot waits to be filled
+            }
+        }
+        if (e != hipSuccess) failed.store(true);
+        for (auto &t : threads) t.join();
+        const hipError_t s = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : s;
+    }
+};
+
+}  // namespace nb

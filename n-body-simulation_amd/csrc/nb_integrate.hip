@@ -9,6 +9,8 @@
 // with nobody reading v in between, k_kick_kick_drift does the kick of step k
 // and the kick-drift of step k+1 in one pass over 120 bytes, with the same
 // roundings in the same order.
+#include <algorithm>
+
 #include "nb_internal.h"
 
 namespace nb {
@@ -80,7 +82,25 @@ __global__ void __launch_bounds__(kThreads) k_kick_kick_drift(
     z[i] = z[i] + hz * delta_t;
 }
 
+// Arrays into host memory: blockIdx.y is the array.
+__global__ void __launch_bounds__(kThreads) k_copy_out(CopyOut c) {
+    const double *__restrict__ src = c.src[blockIdx.y];
+    double *__restrict__ dst = c.dst[blockIdx.y];
+    const size_t n = c.n[blockIdx.y];
+    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n;
+         i += (size_t)gridDim.x * kThreads)
+        dst[i] = src[i];
+}
+
 }  // namespace
+
+void launch_copy_out(const CopyOut &c, int count, hipStream_t s) {
+    size_t most = 0;
+    for (int k = 0; k < count; ++k) most = std::max(most, c.n[k]);
+    if (most == 0) return;
+    const uint32_t blocks = std::min<uint32_t>(64, ceil_div(most, kThreads));
+    hipLaunchKernelGGL(k_copy_out, dim3(blocks, count), dim3(kThreads), 0, s, c);
+}
 
 void launch_kick_kick_drift(uint32_t n, double dt, const double *ax, const double *ay,
                             const double *az, double *vhx, double *vhy, double *vhz, double *x,

@@ -564,6 +564,32 @@ def test_snapshot_async_matches_sync_reads(gpu, oracle, algo):
 
 
 # ---- error handling ----------------------------------------------------------------------------
+# State and accelerations read back at the edges of the copy paths (six arrays:
+# one kernel up to 1 MiB, the runtime's copies up to 6 MiB, then chunks of
+# 256 KiB, from 16 MiB on of 1 MiB; the last chunk of an array is short), twice,
+# and with some of the arrays only.
+@pytest.mark.parametrize("n", [1, 31, 33, 21845, 21846, 131071, 131073, 349525, 349527, 400001])
+def test_state_read_back(gpu, n):
+    rng = np.random.default_rng(n)
+    keys = ("x", "y", "z", "vx", "vy", "vz", "m")
+    d = {k: rng.normal(0, 1, n) for k in keys}
+    with gpu.Context(n) as c:
+        c.set_state(*[d[k] for k in keys])
+        for _ in range(2):
+            s = c.state()
+            for k in keys[:6]:
+                np.testing.assert_array_equal(s[k], d[k])
+        y, vz = np.empty(n), np.empty(n)
+        none = None
+        assert c.lib.nb_get_state(c.h, none, y.ctypes.data_as(gpu._dp), none, none, none,
+                                  vz.ctypes.data_as(gpu._dp)) == 0
+        np.testing.assert_array_equal(y, d["y"])
+        np.testing.assert_array_equal(vz, d["vz"])
+        assert c.lib.nb_get_state(c.h, none, none, none, none, none, none) == 0
+        c.kick_drift(0.0)
+        assert all(np.all(a == 0) for a in c.accel())
+
+
 def test_coincident_bodies_reported(gpu):
     d = uniform_cube(100, 2)
     d["x"][5], d["y"][5], d["z"][5] = d["x"][9], d["y"][9], d["z"][9]
