@@ -202,7 +202,7 @@ bool tree_capacity(uint32_t storage_size_param, uint32_t n, uint32_t *icap) {
 // Every device buffer of an octree (null pointers are skipped).
 void tree_free(nb_ctx *c, TreeBufs &t) {
     void *bufs[] = {t.hdr, t.aabb_part, t.skey, t.skey_alt, t.klo, t.sidx, t.sidx_alt,
-                    t.lcp, t.chain, t.body_parent, t.int_depth, t.int_parent, t.int_node,
+                    t.lcp, t.chain, t.body_node, t.int_depth, t.int_node,
                     t.int_lvl, t.int_count, t.int_sums, t.int_local, t.int_first, t.groups,
                     t.group_size, t.group_slot, t.body4, t.gq, t.spanning, t.cross, t.ref,
                     t.cm, t.rec, t.radix_ctl, t.scan_part};
@@ -241,9 +241,8 @@ int alloc_tree_into(nb_ctx *c, TreeBufs &t, uint32_t storage_size_param) {
     NB_TREE_ALLOC(t.sidx_alt, n);
     NB_TREE_ALLOC(t.lcp, n);
     NB_TREE_ALLOC(t.chain, n);
-    NB_TREE_ALLOC(t.body_parent, n);
+    NB_TREE_ALLOC(t.body_node, n);
     NB_TREE_ALLOC(t.int_depth, t.icap);
-    NB_TREE_ALLOC(t.int_parent, t.icap);
     NB_TREE_ALLOC(t.int_node, t.icap);
     NB_TREE_ALLOC(t.int_lvl, t.icap);
     NB_TREE_ALLOC(t.int_count, t.icap);

@@ -572,12 +572,6 @@ struct ExactTest {
     }
 };
 
-// what one wave's lanes wrote to LDS is read by others of the same wave
-__device__ inline void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 __global__ void __launch_bounds__(kExactThreads) __attribute__((amdgpu_waves_per_eu(5)))
 k_bh_exact_team(uint32_t n, const uint32_t *__restrict__ order, const double *__restrict__ x,
            const double *__restrict__ y, const double *__restrict__ z,

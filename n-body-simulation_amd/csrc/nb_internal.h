@@ -36,6 +36,7 @@ enum : uint32_t {
 // node reference encoding
 constexpr int32_t kRefEmpty = -1;  // empty leaf
 constexpr uint32_t kNoCell = 0xffffffffu;  // no internal cell (tables, parents)
+constexpr uint32_t kSpanCross = 0x80000000u;  // table flag: the cell also crosses a super-block end
 __host__ __device__ inline int32_t ref_of_body(uint32_t b) { return -2 - (int32_t)b; }
 __host__ __device__ inline uint32_t body_of_ref(int32_t r) { return (uint32_t)(-2 - r); }
 
@@ -132,6 +133,12 @@ constexpr uint32_t kComBlock = 1024;
 constexpr uint32_t kComSuperBlocks = 64;
 constexpr uint32_t kComSuper = kComBlock * kComSuperBlocks;
 
+// what one wave's lanes wrote to LDS is read by others of the same wave
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Device buffers of one octree.
 struct TreeBufs {
     uint32_t n = 0;
@@ -143,9 +150,9 @@ struct TreeBufs {
     uint32_t *sidx = nullptr, *sidx_alt = nullptr;
     int32_t *lcp = nullptr;       // n entries (pair i between sorted i and i+1)
     uint32_t *chain = nullptr;    // n entries: internal nodes owned by pair i, then offsets
-    uint32_t *body_parent = nullptr;  // n: internal index of each sorted body's parent
+    uint32_t *body_node = nullptr;  // n: node (child slot) of each sorted body's leaf
     uint8_t *int_depth = nullptr;
-    uint32_t *int_parent = nullptr, *int_node = nullptr, *int_count = nullptr;
+    uint32_t *int_node = nullptr, *int_count = nullptr;  // node of a cell, its bodies
     uint32_t *int_lvl = nullptr;    // centre of mass: depth buckets, or LDS ids of spanning cells
     InternalSums *int_sums = nullptr;
     uint8_t *int_local = nullptr;   // 1: bodies in one kComBlock block; 2: crosses a kComSuper
@@ -194,13 +201,13 @@ struct ForestBufs {
     TreeHdr *hdr;  // one per system
     // per body (offset body_off)
     uint64_t *skey, *skey_alt, *klo;
-    uint32_t *sidx, *sidx_alt, *chain, *body_parent, *group_size, *group_slot;
+    uint32_t *sidx, *sidx_alt, *chain, *body_node, *group_size, *group_slot;
     int32_t *lcp;
     uint2 *groups;
     double4 *body4;  // {x, y, z, m} in the system's input order
     // per internal cell (offset int_off)
     uint8_t *int_depth, *int_local;
-    uint32_t *int_parent, *int_node, *int_lvl, *int_count, *int_first;
+    uint32_t *int_node, *int_lvl, *int_count, *int_first;
     InternalSums *int_sums;
     // per node (offset node_off)
     int32_t *ref;

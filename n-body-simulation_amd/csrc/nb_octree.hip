@@ -381,18 +381,19 @@ __global__ void __launch_bounds__(kThreads) k_fill(TreeHdr *h, uint32_t icap, in
 // Internal cells owned by pair i and the leaf of sorted body i.  A cell is
 // "local" (int_local 1) when its bodies stay inside one com_block-body block
 // of the sorted order; the others go to the table
-// spanning[block * kMaxDepth + depth], with int_local 2 if they also cross a
-// boundary of the com_super-body super-blocks and 0 if not.
+// spanning[block * kMaxDepth + depth], with int_local 2 (and kSpanCross set in
+// the table) if they also cross a boundary of the com_super-body super-blocks
+// and 0 if not.
 // No atomics: every cell, node slot and table entry has exactly one writer.
 __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h, KeyView kv,
                                const uint32_t *__restrict__ sidx, const int32_t *__restrict__ lcp,
                                const uint32_t *__restrict__ off, int32_t *ref, uint8_t *int_depth,
-                               uint32_t *int_parent, uint32_t *int_node, uint32_t *body_parent,
+                               uint32_t *int_node, uint32_t *body_node,
                                uint8_t *int_local, uint32_t *spanning, uint32_t spanning_cap,
                                uint32_t *int_first, uint32_t com_block, uint32_t com_super) {
     if (n == 1) {  // the root is a leaf holding the only body (max_depth stays 0)
         ref[0] = ref_of_body(sidx[0]);
-        body_parent[0] = 0xffffffffu;
+        body_node[0] = 0;
         return;
     }
     const int cp = i > 0 ? lcp[i - 1] : -1;
@@ -419,17 +420,17 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
         } else {
             // the same test at the next super-block boundary
             const uint32_t next_super = (i / com_super + 1) * com_super;
-            int_local[k] = next_super < n && kv.same(next_super, i, l) ? 2 : 0;
+            const bool cross = next_super < n && kv.same(next_super, i, l);
+            int_local[k] = cross ? 2 : 0;
             // the block of body i owns at most one crossing cell per depth:
             // the depth-l cell holding the block's last and the next block's
             // first body
             const uint64_t slot = (uint64_t)(i / com_block) * kMaxDepth + (uint32_t)l;
-            if (slot < spanning_cap) spanning[slot] = k;
+            if (slot < spanning_cap) spanning[slot] = cross ? k | kSpanCross : k;
             else raise_flag(h, kFlagNodeOverflow);
         }
         if (l == 0) {
             int_node[k] = 0;
-            int_parent[k] = 0xffffffffu;
             ref[0] = (int32_t)k;
             continue;
         }
@@ -440,7 +441,6 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
         }
         const uint32_t node = 1u + 8u * pk + kv.digit(i, l - 1);
         int_node[k] = node;
-        int_parent[k] = pk;
         ref[node] = (int32_t)k;
     }
     // the body's leaf: one level below the deepest cell it shares with a neighbour
@@ -448,12 +448,12 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
     const uint32_t pk = owner_index(kv.cell_start(i, D), D);
     if (pk >= icap) {
         raise_flag(h, kFlagNodeOverflow);
-        body_parent[i] = 0xffffffffu;
+        body_node[i] = 0xffffffffu;
         return;
     }
     const uint32_t leaf = 1u + 8u * pk + kv.digit(i, D);
     ref[leaf] = ref_of_body(sidx[i]);
-    body_parent[i] = pk;
+    body_node[i] = leaf;
     // the deepest leaf, 1 + max lcp, is taken from the lcp array (max_depth_of)
 }
 
@@ -463,8 +463,8 @@ __global__ void __launch_bounds__(kThreads) k_link(uint32_t n, uint32_t icap, Tr
                                                    const int32_t *__restrict__ lcp,
                                                    const uint32_t *__restrict__ off,
                                                    int32_t *ref, uint8_t *int_depth,
-                                                   uint32_t *int_parent, uint32_t *int_node,
-                                                   uint32_t *body_parent, uint8_t *int_local,
+                                                   uint32_t *int_node, uint32_t *body_node,
+                                                   uint8_t *int_local,
                                                    uint32_t *spanning, uint32_t spanning_cap,
                                                    uint32_t *int_first) {
     // the block's keys and kLinkBack before them in LDS
@@ -479,7 +479,7 @@ __global__ void __launch_bounds__(kThreads) k_link(uint32_t n, uint32_t icap, Tr
     kv.w1 = w1;
     const uint32_t i = b0 + threadIdx.x;
     if (i >= n) return;
-    link_at(i, n, icap, h, kv, sidx, lcp, off, ref, int_depth, int_parent, int_node, body_parent,
+    link_at(i, n, icap, h, kv, sidx, lcp, off, ref, int_depth, int_node, body_node,
             int_local, spanning, spanning_cap, int_first, kComBlock, kComSuper);
 }
 
@@ -647,6 +647,31 @@ __device__ inline void sum_children_out(uint32_t pk, uint32_t depth, uint32_t fi
 // depth can be summed at once, with a barrier between depths.
 constexpr int kComThreads = 1024;
 
+// Counts per depth, cnt[0, kMaxDepth), to first places (cnt, and a copy in cur;
+// cnt[kMaxDepth] the total), by the first wave; bit d of *levels: depth d has
+// cells.
+static_assert(kMaxDepth < 64, "one lane per depth and the total");
+__device__ inline void depth_starts(uint32_t *cnt, uint32_t *cur, unsigned long long *levels) {
+    const uint32_t t = threadIdx.x;
+    if (t >= 64) return;
+    const uint32_t c = t < (uint32_t)kMaxDepth ? cnt[t] : 0u;
+    uint32_t inc = c;
+#pragma unroll
+    for (int w = 1; w < 64; w <<= 1) {
+        const uint32_t v = __shfl_up(inc, w, 64);
+        if (t >= (uint32_t)w) inc += v;
+    }
+    if (t <= (uint32_t)kMaxDepth) cnt[t] = inc - c;
+    if (t < (uint32_t)kMaxDepth) cur[t] = inc - c;
+    const unsigned long long lv = __ballot(c != 0);
+    if (t == 0) *levels = lv;
+}
+
+__device__ __forceinline__ unsigned long long uniform64(unsigned long long v) {
+    return (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v) |
+           (unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(v >> 32)) << 32;
+}
+
 // Cells [kb, ke) bucketed by depth into lvl[kb ..) (cells with keep(k) only),
 // then sum(k) for each, deepest depth first.  cnt/cur: kMaxDepth + 1 and
 // kMaxDepth LDS words.  Every thread of the workgroup calls it.
@@ -654,261 +679,331 @@ template <typename Keep, typename Sum>
 __device__ inline void com_levels(uint32_t kb, uint32_t ke, Keep keep,
                                   const uint8_t *__restrict__ int_depth, uint32_t *lvl,
                                   uint32_t *cnt, uint32_t *cur, Sum sum) {
+    __shared__ unsigned long long levels;
     const uint32_t t = threadIdx.x, nt = blockDim.x;
     for (uint32_t d = t; d <= (uint32_t)kMaxDepth; d += nt) cnt[d] = 0;
     __syncthreads();
     for (uint32_t k = kb + t; k < ke; k += nt)
         if (keep(k)) atomicAdd(&cnt[min((uint32_t)int_depth[k], (uint32_t)kMaxDepth - 1)], 1u);
     __syncthreads();
-    if (t == 0) {
-        uint32_t run = 0;
-        for (int d = 0; d < kMaxDepth; ++d) {
-            const uint32_t c = cnt[d];
-            cnt[d] = run;
-            cur[d] = run;
-            run += c;
-        }
-        cnt[kMaxDepth] = run;
-    }
+    depth_starts(cnt, cur, &levels);
     __syncthreads();
     for (uint32_t k = kb + t; k < ke; k += nt)
         if (keep(k))
             lvl[kb + atomicAdd(&cur[min((uint32_t)int_depth[k], (uint32_t)kMaxDepth - 1)], 1u)] = k;
     __syncthreads();
-    for (int d = kMaxDepth - 1; d >= 0; --d) {
+    for (unsigned long long lv = uniform64(levels); lv;) {
+        const int d = 63 - __clzll((long long)lv);
+        lv ^= 1ull << d;
         const uint32_t lb = cnt[d], le = cnt[d + 1];
-        if (lb == le) continue;  // the same for every thread: LDS, read after a barrier
         for (uint32_t j = lb + t; j < le; j += nt) sum(lvl[kb + j]);
         __syncthreads();
+    }
+}
+
+// The levels in LDS, deepest first: cell c of order[cnt[d], cnt[d + 1]) gets
+// term[kCell + c] = the sum of its eight children's terms, in digit order from
+// 0.0 as sum_children_out, and m[kCell + c] = their bodies; at[8 c + digit] is
+// the place of a child's term, which for an empty slot holds zeros.  Four lanes
+// share a cell, one per component.  kThreads_ threads take part: a whole
+// workgroup with a barrier between levels, or one wave, which needs none (its
+// LDS accesses complete in order).  The chain from level to level is one read,
+// the eight additions and one write: the next step's cell and places are read
+// ahead of it, and the level bounds sit in the lanes of a register.
+template <uint32_t kThreads_, uint32_t kCell>
+__device__ __forceinline__ void sum_levels(uint32_t t, const uint32_t *cnt,
+                                           unsigned long long lv, const uint16_t *order,
+                                           const uint16_t *at_s, double (*term)[4], uint32_t *m_s) {
+    constexpr uint32_t step = kThreads_ / 4;
+    const uint32_t comp = t & 3u;
+    const int starts = (int)cnt[min(t & 63u, (uint32_t)kMaxDepth)];
+    uint32_t base = 0, end = 0;  // the next step's cells [base, min(base + step, end)): uniform
+    bool fresh = false;          // the next step opens a level
+    uint32_t nc = 0;
+    uint4 nw = make_uint4(0, 0, 0, 0);
+    bool has = false;
+    auto next = [&]() {
+        base += step;
+        fresh = base >= end;
+        if (fresh) {
+            if (!lv) {
+                end = 0;
+                has = false;
+                return;
+            }
+            const int d = 63 - __clzll((long long)lv);
+            lv ^= 1ull << d;
+            base = (uint32_t)__builtin_amdgcn_readlane(starts, d);
+            end = (uint32_t)__builtin_amdgcn_readlane(starts, d + 1);
+        }
+        const uint32_t j = base + (t >> 2);
+        has = j < end;
+        if (has) {
+            nc = order[j];
+            nw = *reinterpret_cast<const uint4 *>(at_s + 8 * nc);
+        }
+    };
+    next();
+    while (end) {
+        const uint32_t c = nc;
+        const uint4 w = nw;
+        const bool mine = has;
+        next();
+        if (mine) {
+            const uint32_t at[8] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16,
+                                    w.z & 0xffffu, w.z >> 16, w.w & 0xffffu, w.w >> 16};
+            double v[8];
+            uint32_t m[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = term[at[k]][comp];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) m[k] = m_s[at[k]];
+            double sum = 0;
+            uint32_t count = 0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                sum += v[k];
+                count += m[k];
+            }
+            term[kCell + c][comp] = sum;
+            m_s[kCell + c] = count;  // the same from all four lanes
+        }
+        if (kThreads_ == 64)
+            wave_lds_sync();
+        else if (fresh)
+            __syncthreads();
     }
 }
 
 // Pass 1: one workgroup per kComBlock consecutive (sorted) bodies sums the
 // cells that lie inside its block.  Pair i owns cells [off[i], off[i+1]), so
 // the block's cells are one contiguous range [kb, ke).  Up to kComLdsCells
-// cells are summed entirely in LDS.  Staged once (all loads in flight
-// together): the block's bodies and their input indices in sorted order, and
-// per cell its depth, first position and a 16-bit code per child slot
-// (empty, body, or the child cell's place in the block).  The children of a
-// cell cover consecutive sorted ranges in digit order, so a body child is the
-// body at the running position: the cell's first position plus the counts of
-// its earlier children; the level pass stores that position in the body's
-// code.  The levels touch LDS only (a barrier also waits for global stores).
-// A last pass writes the sums, the node records of the cells' child slots and
-// the group marks, consecutive threads on consecutive slots.  A larger block
-// falls back to the same work in global memory.  The block also clears the
-// group marks of its positions before any is set.
+// cells are summed entirely in LDS.  Staged once, two round trips to memory
+// deep: the terms of the block's bodies and their input indices in sorted
+// order; per child slot the place of the child's term, which bodies and cells
+// write into the slot the topology pass gave them; and the cells bucketed by
+// depth.  The levels touch LDS only (a barrier also waits for global stores).
+// Then every body and every cell is divided once into its record centre, and a
+// last pass writes the node records of the cells' child slots, consecutive
+// threads on consecutive slots.  A larger block falls back to the same work in
+// global memory.  The block also clears the group marks of its positions
+// before any is set.
+//
+// What bounds it is the chain of levels (6 to 10 of them), each a barrier and
+// three LDS round trips, not bytes.  So a level touches only its own cells;
+// four lanes share a cell, one per component, and read all eight children
+// together: body terms, cell sums and a zero for empty slots share one LDS
+// table, so no child needs a branch.  An empty slot adds +0.0, which changes no
+// running sum that starts at +0.0.
+// (1024 bodies: 40 us with one lane per cell and a scan of all cells per level,
+// 13.5 now; 100,003: 43 and 17; 1,048,576, disk: 107 and 58.)
 constexpr uint32_t kComLdsCells = 576;   // about 490 per block; 537 the most seen (disk, Plummer)
 constexpr int kComLocalThreads = 512;
 constexpr int kComBodiesPerThread = kComBlock / kComLocalThreads;
-constexpr int kComRefsPerThread = 8 * kComLdsCells / kComLocalThreads;  // child slots
-static_assert(kComBlock % kComLocalThreads == 0 && (8 * kComLdsCells) % kComLocalThreads == 0,
-              "whole staging rounds");
-constexpr uint16_t kCodeEmpty = 0xffffu, kCodeBody = 0xfffeu, kCodeFar = 0xfffdu;
-constexpr uint16_t kCodeAt = 0x8000u;    // | sorted position - block start: a placed body
-static_assert(kComLdsCells < kCodeAt && kComBlock <= 0x7ffdu, "16-bit LDS codes");
+constexpr int kComCellsPerThread = (kComLdsCells + kComLocalThreads - 1) / kComLocalThreads;
+static_assert(kComBlock % kComLocalThreads == 0, "whole staging rounds");
+// The LDS table of terms: the block's bodies, its cells, one zero.
+constexpr uint32_t kTermCell = kComBlock, kTermZero = kTermCell + kComLdsCells;
+static_assert(kTermZero < 0xffffu, "16-bit places");
 // Block blk of one octree (the one-system kernel below, and the ensemble's,
 // which runs the blocks of every system in one launch).
 __device__ __forceinline__ void com_local_block(
     uint32_t blk, uint32_t n, uint32_t icap, TreeHdr *h, const double4 *__restrict__ body4,
-    const uint32_t *__restrict__ sidx, const int32_t *__restrict__ ref,
-    const uint32_t *__restrict__ off, const uint8_t *__restrict__ int_depth,
-    const uint8_t *__restrict__ int_local, const uint32_t *__restrict__ int_first, uint32_t *lvl,
+    const uint32_t *__restrict__ sidx, const uint32_t *__restrict__ body_node,
+    const int32_t *__restrict__ ref, const uint32_t *__restrict__ off,
+    const uint8_t *__restrict__ int_depth, const uint8_t *__restrict__ int_local,
+    const uint32_t *__restrict__ int_first, const uint32_t *__restrict__ int_node, uint32_t *lvl,
     InternalSums *sums, uint32_t *counts, const RecOut &o) {
     constexpr uint32_t nt = kComLocalThreads;
     __shared__ uint32_t cnt[kMaxDepth + 1], cur[kMaxDepth];
-    __shared__ unsigned long long levels;  // bit d: a local cell of depth d
-    __shared__ double4 b_s[kComBlock];     // the block's bodies {x, y, z, m}, sorted order
-    __shared__ uint32_t i_s[kComBlock];    // their input indices
-    __shared__ double4 c_s[kComLdsCells];  // cell sums {x m, y m, z m, m}
-    __shared__ uint32_t n_s[kComLdsCells]; // cell body counts
-    __shared__ uint16_t code_s[8 * kComLdsCells];
-    __shared__ uint16_t first_s[kComLdsCells];  // first sorted position - block start
+    __shared__ unsigned long long levels;        // bit d: a local cell of depth d
+    __shared__ double term_s[kTermZero + 1][4];  // {x m, y m, z m, m}: bodies, cells, zero
+    __shared__ uint32_t m_s[kTermZero + 1];      // bodies of a term: 1, a cell's count, 0
+    __shared__ uint32_t i_s[kComBlock];          // input index of a body
+    __shared__ alignas(16) uint16_t at_s[8 * kComLdsCells];  // child slot: place of its term
+    __shared__ uint16_t order_s[kComLdsCells];  // local cells bucketed by depth
     __shared__ uint8_t depth_s[kComLdsCells];   // depth; kMaxDepth if not local
     const uint32_t t = threadIdx.x;
     const uint32_t s = blk * kComBlock;
     const uint32_t e = min(n, s + kComBlock);
-    {
-        // all index loads, then all body loads, in flight together
-        uint32_t bi[kComBodiesPerThread];
-        double4 b[kComBodiesPerThread];
-#pragma unroll
-        for (int q = 0; q < kComBodiesPerThread; ++q) {
-            const uint32_t i = s + t + q * nt;
-            bi[q] = i < e ? sidx[i] : 0u;
-        }
-#pragma unroll
-        for (int q = 0; q < kComBodiesPerThread; ++q)
-            if (s + t + q * nt < e) b[q] = body4[bi[q]];
-#pragma unroll
-        for (int q = 0; q < kComBodiesPerThread; ++q) {
-            const uint32_t i = s + t + q * nt;
-            if (i >= e) continue;
-            if (b[q].w == 0) raise_flag(h, kFlagZeroMass);
-            b_s[i - s] = b[q];
-            i_s[i - s] = bi[q];
-            if (o.f32) {
-                o.group_size[i] = 0;
-                o.group_slot[i] = 0;
-            }
-        }
-    }
     if (n < 2) {  // a lone body is the root leaf: no internal cell
-        __syncthreads();
         if (t == 0) {
-            put_record(o, 0, ref_of_body(i_s[0]), term_com(body_term(b_s[0])));
+            const uint32_t q = sidx[0];
+            const double4 b = body4[q];
+            if (b.w == 0) raise_flag(h, kFlagZeroMass);
+            if (o.f32) {
+                o.group_size[0] = 0;
+                o.group_slot[0] = 0;
+            }
+            put_record(o, 0, ref_of_body(q), term_com(body_term(b)));
             put_group(o, 0, 1);
         }
         return;
     }
+    // first loads: body indices and leaf nodes, the cell range
+    uint32_t bi[kComBodiesPerThread], bn[kComBodiesPerThread];
+#pragma unroll
+    for (int q = 0; q < kComBodiesPerThread; ++q) {
+        const uint32_t i = s + t + q * nt;
+        bi[q] = i < e ? sidx[i] : 0u;
+        bn[q] = i < e ? body_node[i] : 0u;
+    }
     const uint32_t I = min(h->internal_count, icap);
     const uint32_t kb = s < n - 1 ? min(off[s], I) : I;
-    const uint32_t ke = e < n - 1 ? min(off[e], I) : I;
-    const uint32_t nc = ke - kb;
-    const uint32_t nbody = e - s;
-    if (nc > kComLdsCells) {  // the same for the whole workgroup
-        com_levels(kb, ke, [&](uint32_t k) { return int_local[k] == 1; }, int_depth, lvl, cnt,
+    const uint32_t nc = (e < n - 1 ? min(off[e], I) : I) - kb;
+    const bool fits = nc <= kComLdsCells;  // the same for the whole workgroup
+    // the cells' data and the bodies
+    uint32_t cf[kComCellsPerThread], cd[kComCellsPerThread], cn_[kComCellsPerThread];
+    double4 b[kComBodiesPerThread];
+#pragma unroll
+    for (int q = 0; q < kComBodiesPerThread; ++q)
+        if (s + t + q * nt < e) b[q] = body4[bi[q]];
+#pragma unroll
+    for (int q = 0; q < kComCellsPerThread; ++q) {
+        const uint32_t c = t + q * nt;
+        cd[q] = (uint32_t)kMaxDepth;
+        if (!fits || c >= nc) continue;
+        cf[q] = int_first[kb + c];
+        cn_[q] = int_node[kb + c];
+        const uint32_t d = min((uint32_t)int_depth[kb + c], (uint32_t)kMaxDepth - 1);
+        cd[q] = int_local[kb + c] == 1 ? d : (uint32_t)kMaxDepth;
+    }
+    if (t <= (uint32_t)kMaxDepth) cnt[t] = 0;
+    if (t < 4) term_s[kTermZero][t] = 0.0;
+    if (t == 4) m_s[kTermZero] = 0;
+    if (fits) {
+        constexpr uint32_t z2 = kTermZero | kTermZero << 16;
+        for (uint32_t c = t; c < nc; c += nt)
+            *reinterpret_cast<uint4 *>(&at_s[8 * c]) = make_uint4(z2, z2, z2, z2);
+    }
+    __syncthreads();
+    // bodies and cells into the slots of their parents (slots of other blocks'
+    // cells are left out; a cell that is not local is written and not used)
+    const uint64_t slot0 = 1ull + 8ull * kb;
+#pragma unroll
+    for (int q = 0; q < kComBodiesPerThread; ++q) {
+        const uint32_t p = t + q * nt;
+        if (s + p >= e) continue;
+        if (b[q].w == 0) raise_flag(h, kFlagZeroMass);
+        *reinterpret_cast<double4 *>(term_s[p]) = body_term(b[q]);
+        m_s[p] = 1;
+        i_s[p] = bi[q];
+        const uint64_t j = (uint64_t)bn[q] - slot0;
+        if (fits && j < 8ull * nc) at_s[j] = (uint16_t)p;
+        if (o.f32) {
+            o.group_size[s + p] = 0;
+            o.group_slot[s + p] = 0;
+        }
+    }
+    if (!fits) {
+        __syncthreads();
+        com_levels(kb, kb + nc, [&](uint32_t k) { return int_local[k] == 1; }, int_depth, lvl, cnt,
                    cur, [&](uint32_t k) {
                        sum_children_out(k, int_depth[k], int_first[k], body4, ref,
                                         sums, counts, h, o);
                    });
         return;
     }
-    if (t == 0) levels = 0;
-    for (uint32_t c = t; c < nc; c += nt) {
-        const bool local = int_local[kb + c] == 1;
-        depth_s[c] = local ? (uint8_t)min((uint32_t)int_depth[kb + c], (uint32_t)kMaxDepth - 1)
-                           : (uint8_t)kMaxDepth;
-        first_s[c] = (uint16_t)(int_first[kb + c] - s);
-    }
-    {
-        int32_t r[kComRefsPerThread];
+    uint32_t place[kComCellsPerThread];  // among the cells of its depth
 #pragma unroll
-        for (int q = 0; q < kComRefsPerThread; ++q) {
-            const uint32_t j = t + q * nt;
-            r[q] = j < 8 * nc ? ref[1ull + 8ull * kb + j] : kRefEmpty;
+    for (int q = 0; q < kComCellsPerThread; ++q) {
+        const uint32_t c = t + q * nt;
+        const bool has = c < nc;
+        if (has) {
+            const uint64_t j = (uint64_t)cn_[q] - slot0;
+            if (j < 8ull * nc) at_s[j] = (uint16_t)(kTermCell + c);
+            depth_s[c] = (uint8_t)cd[q];
         }
+        // one LDS atomic per wave and depth: the lanes of one depth by ballots
+        uint64_t peers = __ballot(has && cd[q] < (uint32_t)kMaxDepth);
 #pragma unroll
-        for (int q = 0; q < kComRefsPerThread; ++q) {
-            const uint32_t j = t + q * nt;
-            if (j >= 8 * nc) continue;
-            uint16_t code = kCodeEmpty;
-            if (r[q] >= 0) {
-                const uint32_t rl = (uint32_t)r[q] - kb;
-                code = rl < nc ? (uint16_t)rl : kCodeFar;  // far: not for a local cell
-            } else if (r[q] != kRefEmpty) {
-                code = kCodeBody;
-            }
-            code_s[j] = code;
+        for (int w = 0; w < 6; ++w) {
+            const bool bit = (cd[q] >> w) & 1u;
+            const uint64_t bal = __ballot(bit);
+            peers &= bit ? bal : ~bal;
         }
+        const uint32_t lane = t & 63u;
+        const uint32_t rank = (uint32_t)__popcll(peers & ((1ull << lane) - 1));
+        uint32_t base = 0;
+        if (((peers >> lane) & 1ull) && rank == 0)
+            base = atomicAdd(&cnt[cd[q]], (uint32_t)__popcll(peers));
+        place[q] = (uint32_t)__shfl((int)base, peers ? __ffsll((unsigned long long)peers) - 1 : 0, 64) + rank;
     }
     __syncthreads();
-    for (uint32_t c = t; c < nc; c += nt)
-        if (depth_s[c] < kMaxDepth) atomicOr(&levels, 1ull << depth_s[c]);
+    depth_starts(cnt, cur, &levels);
     __syncthreads();
-    const unsigned long long lv = levels;  // the same for every thread
-    for (int d = kMaxDepth - 1; d >= 0; --d) {
-        if (!((lv >> d) & 1ull)) continue;
-        for (uint32_t c = t; c < nc; c += nt) {
-            if (depth_s[c] != (uint32_t)d) continue;
-            double sx = 0, sy = 0, sz = 0, sm = 0;
-            uint32_t cn = 0;
-            uint32_t pos = first_s[c];
-            // digit order from 0.0, as sum_children_out
 #pragma unroll
-            for (int dd = 0; dd < 8; ++dd) {
-                const uint16_t code = code_s[8 * c + dd];
-                if (code == kCodeEmpty) continue;
-                double4 v;
-                uint32_t m = 1;
-                if (code < kComLdsCells) {
-                    v = c_s[code];
-                    m = n_s[code];
-                } else if (code == kCodeBody && pos < nbody) {
-                    v = body_term(b_s[pos]);
-                    code_s[8 * c + dd] = (uint16_t)(kCodeAt | pos);
-                } else {  // not for a local cell: the child from global memory
-                    const int32_t r = ref[1ull + 8ull * (kb + c) + dd];
-                    if (r >= 0) {
-                        const InternalSums g = sums[r];
-                        v = make_double4(g.x, g.y, g.z, g.m);
-                        m = counts[r];
-                    } else {
-                        v = body_term(body4[body_of_ref(r)]);
-                    }
-                }
-                sx += v.x;
-                sy += v.y;
-                sz += v.z;
-                sm += v.w;
-                cn += m;
-                pos += m;
-            }
-            c_s[c] = make_double4(sx, sy, sz, sm);
-            n_s[c] = cn;
-            if (sm == 0) raise_flag(h, kFlagZeroMass);
-        }
-        __syncthreads();
-    }
-    // sums, group marks and child records of the local cells
-    for (uint32_t c = t; c < nc; c += nt) {
-        if (depth_s[c] >= kMaxDepth) continue;
-        const double4 g = c_s[c];
+    for (int q = 0; q < kComCellsPerThread; ++q)
+        if (cd[q] < (uint32_t)kMaxDepth) order_s[cnt[cd[q]] + place[q]] = (uint16_t)(t + q * nt);
+    __syncthreads();
+    sum_levels<kComLocalThreads, kTermCell>(t, cnt, uniform64(levels), order_s, at_s, term_s, m_s);
+    // sums and group marks of the local cells; then bodies and cells to their
+    // record centres, in place
+#pragma unroll
+    for (int q = 0; q < kComCellsPerThread; ++q) {
+        const uint32_t c = t + q * nt;
+        if (cd[q] >= (uint32_t)kMaxDepth) continue;
+        const double4 g = *reinterpret_cast<const double4 *>(term_s[kTermCell + c]);
+        const uint32_t count = m_s[kTermCell + c];
+        if (g.w == 0) raise_flag(h, kFlagZeroMass);
         sums[kb + c] = InternalSums{g.x, g.y, g.z, g.w};
-        counts[kb + c] = n_s[c];
-        if (n_s[c] > o.rule.group_max) {
+        counts[kb + c] = count;
+        const double4 com = term_com(g);
+        if (count > o.rule.group_max) {
             uint32_t m[8];
 #pragma unroll
-            for (int dd = 0; dd < 8; ++dd) {
-                const uint16_t code = code_s[8 * c + dd];
-                m[dd] = code == kCodeEmpty ? 0u : 1u;
-                if (code < kComLdsCells) {
-                    m[dd] = n_s[code];
-                } else if (code == kCodeFar) {  // not for a local cell: global memory
-                    m[dd] = counts[ref[1ull + 8ull * (kb + c) + dd]];
-                }
-            }
-            put_child_groups(o, s + first_s[c], m);
+            for (int k = 0; k < 8; ++k) m[k] = m_s[at_s[8 * c + k]];
+            put_child_groups(o, cf[q], m);
         }
+        if (cd[q] == 0) {  // the root (the block holds every body)
+            put_record(o, 0, (int32_t)(kb + c), com);
+            if (count <= o.rule.group_max) put_group(o, cf[q], count);
+        }
+        *reinterpret_cast<double4 *>(term_s[kTermCell + c]) = com;
     }
-    for (uint32_t j = t; j < 8 * nc; j += nt) {
-        const uint32_t c = j >> 3;
-        const uint32_t dc = depth_s[c];
-        if (dc >= kMaxDepth) continue;
-        const uint64_t slot = 1ull + 8ull * kb + j;
-        const uint16_t code = code_s[j];
-        const uint32_t pc = n_s[c];
-        if (code == kCodeEmpty) {
-            put_record(o, slot, kRefEmpty, make_double4(0.0, 0.0, 0.0, 0.0));
-        } else if (code < kComLdsCells) {
-            put_record(o, slot, (int32_t)(kb + code), term_com(c_s[code]));
-        } else if ((code & kCodeAt) && code < kCodeFar) {
-            const uint32_t pos = code & ~kCodeAt;
-            put_record(o, slot, ref_of_body(i_s[pos]), term_com(body_term(b_s[pos])));
-        } else {  // not for a local cell: the child from global memory
-            const int32_t r = ref[slot];
-            if (r >= 0) {
-                const InternalSums g = sums[r];
-                put_record(o, slot, r, term_com(make_double4(g.x, g.y, g.z, g.m)));
-            } else {
-                put_record(o, slot, r, term_com(body_term(body4[body_of_ref(r)])));
-            }
+#pragma unroll
+    for (int q = 0; q < kComBodiesPerThread; ++q) {
+        double4 *v = reinterpret_cast<double4 *>(term_s[t + q * nt]);
+        if (s + t + q * nt < e) *v = term_com(*v);
+    }
+    __syncthreads();
+    // three slots per thread at a time, so that their LDS round trips overlap
+    constexpr int kAhead = 3;
+    for (uint32_t j0 = t; j0 < 8 * nc; j0 += kAhead * nt) {
+        uint32_t at[kAhead], bi2[kAhead];
+        double4 v[kAhead];
+        bool live[kAhead];
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            const uint32_t j = min(j0 + q * nt, 8 * nc - 1);
+            live[q] = j0 + q * nt < 8 * nc && depth_s[j >> 3] < kMaxDepth;
+            at[q] = at_s[j];
         }
-        if (dc == 0 && (j & 7u) == 0) {  // the root (the block holds every body)
-            put_record(o, 0, (int32_t)(kb + c), term_com(c_s[c]));
-            if (pc <= o.rule.group_max) put_group(o, s + first_s[c], pc);
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            v[q] = *reinterpret_cast<const double4 *>(term_s[at[q]]);
+            bi2[q] = i_s[min(at[q], kComBlock - 1)];
+        }
+#pragma unroll
+        for (int q = 0; q < kAhead; ++q) {
+            if (!live[q]) continue;
+            const int32_t r = at[q] < kTermCell   ? ref_of_body(bi2[q])
+                              : at[q] < kTermZero ? (int32_t)(kb + at[q] - kTermCell)
+                                                  : kRefEmpty;
+            put_record(o, slot0 + j0 + q * nt, r, v[q]);
         }
     }
 }
 
 __global__ void __launch_bounds__(kComLocalThreads) k_com_local(
     uint32_t n, uint32_t icap, TreeHdr *h, const double4 *__restrict__ body4,
-    const uint32_t *__restrict__ sidx, const int32_t *__restrict__ ref,
-    const uint32_t *__restrict__ off, const uint8_t *__restrict__ int_depth,
-    const uint8_t *__restrict__ int_local, const uint32_t *__restrict__ int_first, uint32_t *lvl,
+    const uint32_t *__restrict__ sidx, const uint32_t *__restrict__ body_node,
+    const int32_t *__restrict__ ref, const uint32_t *__restrict__ off,
+    const uint8_t *__restrict__ int_depth, const uint8_t *__restrict__ int_local,
+    const uint32_t *__restrict__ int_first, const uint32_t *__restrict__ int_node, uint32_t *lvl,
     InternalSums *sums, uint32_t *counts, RecOut o) {
-    com_local_block(blockIdx.x, n, icap, h, body4, sidx, ref, off, int_depth, int_local, int_first,
-                    lvl, sums, counts, o);
+    com_local_block(blockIdx.x, n, icap, h, body4, sidx, body_node, ref, off, int_depth, int_local,
+                    int_first, int_node, lvl, sums, counts, o);
 }
 
 // Pass 2: the cells crossing block boundaries (the table
@@ -922,26 +1017,32 @@ __global__ void __launch_bounds__(kComLocalThreads) k_com_local(
 // written then; a child summed by this workgroup is named by its LDS id
 // (cid[k], written first).  The levels, deepest first, then read LDS only.
 // More cells fall back to the same sums in global memory.
+// One wave runs the levels (sum_levels: few cells a level, no barrier) while
+// the others divide and write the records of the children it does not sum.
+// (100,003 bodies: 25.6 us a launch with one lane per cell, a branch per child
+// and a workgroup barrier per level, 13.8 now.)
 constexpr uint32_t kSpanCells = 448;
-constexpr uint32_t kChildEmpty = 0xffffffffu;
-constexpr uint32_t kChildHere = 0x80000000u;  // | LDS id of a child summed here
+constexpr uint32_t kSpanRowsAhead = 3;        // table entries per thread in flight
+constexpr int kSpanSlots = (8 * (int)kSpanCells + kComThreads - 1) / kComThreads;  // per thread
+constexpr uint32_t kSpanSum = 8 * kSpanCells;  // LDS terms: child slots, then sums
+static_assert(kSpanCells <= (uint32_t)kComThreads - 64, "a cell per thread");
+static_assert(9 * kSpanCells < 0x10000u, "16-bit places");
 // Super-block (want 0) or cross list (want 2) sb of one octree.
 __device__ __forceinline__ void com_span_block(
     uint32_t sb, uint32_t nblocks, uint32_t rows, uint32_t want, TreeHdr *h,
     const double4 *__restrict__ body4, const int32_t *__restrict__ ref,
     const uint32_t *__restrict__ spanning, const uint8_t *__restrict__ int_local,
-    const uint32_t *__restrict__ int_first, uint32_t *cid, InternalSums *sums, uint32_t *counts,
+    const uint32_t *__restrict__ int_first, const uint32_t *__restrict__ int_node, uint32_t *cid, InternalSums *sums, uint32_t *counts,
     uint32_t *cross, uint32_t cross_cap, const RecOut &o) {
     __shared__ uint32_t ncell, cnt[kMaxDepth + 1], cur[kMaxDepth];
+    __shared__ unsigned long long levels;
     __shared__ uint32_t nx, xbase, xl[kMaxDepth];  // want 0: this super-block's crossing cells
     __shared__ uint32_t list[kSpanCells];  // cell index by LDS id
-    __shared__ uint32_t fst[kSpanCells];   // first sorted position
     __shared__ uint8_t ldep[kSpanCells];
     __shared__ uint16_t order[kSpanCells];  // LDS ids bucketed by depth
-    __shared__ double4 cv[8 * kSpanCells];  // child terms
-    __shared__ uint32_t cc[8 * kSpanCells]; // child body counts, kChildEmpty, or kChildHere | id
-    __shared__ double4 sv[kSpanCells];
-    __shared__ uint32_t sn[kSpanCells];
+    __shared__ double term[9 * kSpanCells][4];  // terms of child slots (0 if empty), sums
+    __shared__ uint32_t m_s[9 * kSpanCells];    // their bodies
+    __shared__ alignas(16) uint16_t at_s[8 * kSpanCells];  // child slot: place of its term
     const uint32_t t = threadIdx.x;
     const uint32_t r0 = sb * rows;
     const uint32_t r1 = min(nblocks, r0 + rows);
@@ -956,7 +1057,6 @@ __device__ __forceinline__ void com_span_block(
         const uint32_t id = atomicAdd(&ncell, 1u);
         if (id < kSpanCells) {
             list[id] = k;
-            fst[id] = int_first[k];
             ldep[id] = (uint8_t)d;
             cid[k] = id;
             atomicAdd(&cnt[d], 1u);
@@ -969,16 +1069,23 @@ __device__ __forceinline__ void com_span_block(
     if (want == 2) {
         for (uint32_t i = t; i < ncross; i += kComThreads) take(cross[i] >> 6, cross[i] & 63u);
     } else {
-        for (uint64_t j = slot0 + t; j < slot1; j += kComThreads) {
-            const uint32_t k = spanning[j];
-            if (k == kNoCell) continue;
-            const uint8_t kind = int_local[k];
-            const uint32_t d = (uint32_t)(j % kMaxDepth);
-            if (kind == 2) {
-                const uint32_t x = atomicAdd(&nx, 1u);
-                if (x < (uint32_t)kMaxDepth) xl[x] = (k << 6) | d;
-            } else if (kind == want) {
-                take(k, d);
+        for (uint64_t j0 = slot0; j0 < slot1; j0 += (uint64_t)kSpanRowsAhead * kComThreads) {
+            uint32_t ks[kSpanRowsAhead];
+#pragma unroll
+            for (uint32_t q = 0; q < kSpanRowsAhead; ++q) {
+                const uint64_t j = j0 + q * kComThreads + t;
+                ks[q] = j < slot1 ? spanning[j] : kNoCell;
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kSpanRowsAhead; ++q) {
+                if (ks[q] == kNoCell) continue;
+                const uint32_t d = (uint32_t)((j0 + q * kComThreads + t) % kMaxDepth);
+                if (ks[q] & kSpanCross) {
+                    const uint32_t x = atomicAdd(&nx, 1u);
+                    if (x < (uint32_t)kMaxDepth) xl[x] = ((ks[q] & ~kSpanCross) << 6) | d;
+                } else {
+                    take(ks[q], d);
+                }
             }
         }
     }
@@ -1007,7 +1114,7 @@ __device__ __forceinline__ void com_span_block(
                 for (uint64_t j = slot0 + (uint32_t)d + (uint64_t)t * kMaxDepth; j < slot1;
                      j += (uint64_t)kComThreads * kMaxDepth) {
                     const uint32_t k = spanning[j];
-                    if (k != kNoCell && int_local[k] == want)
+                    if (!(k & kSpanCross))  // neither empty nor crossing
                         sum_children_out(k, (uint32_t)d, int_first[k], body4, ref,
                                          sums, counts, h, o);
                 }
@@ -1017,104 +1124,85 @@ __device__ __forceinline__ void com_span_block(
         return;
     }
     if (nk == 0) return;
-    if (t == 0) {
-        uint32_t run = 0;
-        for (int d = 0; d < kMaxDepth; ++d) {
-            const uint32_t c = cnt[d];
-            cnt[d] = run;
-            cur[d] = run;
-            run += c;
-        }
-        cnt[kMaxDepth] = run;
-    }
+    depth_starts(cnt, cur, &levels);
     __syncthreads();
-    for (uint32_t id = t; id < nk; id += kComThreads) order[atomicAdd(&cur[ldep[id]], 1u)] = (uint16_t)id;
-    for (uint32_t p = t; p < 8 * nk; p += kComThreads) {
-        const uint32_t id = p >> 3;
-        const uint32_t k = list[id];
-        const uint64_t j = 1ull + 8ull * k + (p & 7u);
-        const int32_t r = ref[j];
-        double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
-        uint32_t code = kChildEmpty;
-        if (r >= 0) {
-            if (int_local[r] == want) {
-                code = kChildHere | cid[r];  // summed by this workgroup, one level deeper
-            } else {
-                const InternalSums q = sums[r];
-                v = make_double4(q.x, q.y, q.z, q.m);
-                code = counts[r];
-                put_record(o, j, r, term_com(v));
-            }
-        } else if (r != kRefEmpty) {
-            v = body_term(body4[body_of_ref(r)]);
-            code = 1;
-            put_record(o, j, r, term_com(v));
-        } else {
-            put_record(o, j, kRefEmpty, v);
-        }
-        cv[p] = v;
-        cc[p] = code;
+    uint32_t node = 0, first = 0;  // of cell t
+    if (t < nk) {
+        order[atomicAdd(&cur[ldep[t]], 1u)] = (uint16_t)t;
+        node = int_node[list[t]];
+        first = int_first[list[t]];
     }
-    __syncthreads();
-    for (int d = kMaxDepth - 1; d >= 0; --d) {
-        const uint32_t lb = cnt[d], le = cnt[d + 1];
-        if (lb == le) continue;  // the same for every thread: LDS, read after a barrier
-        for (uint32_t j = lb + t; j < le; j += kComThreads) {
-            const uint32_t id = order[j];
-            double sx = 0, sy = 0, sz = 0, sm = 0;
-            uint32_t cn = 0;
+    // the child slots, all of a thread's loads in flight together.  A cell's
+    // sums and count mean something only if an earlier pass summed it, its id
+    // only if this workgroup does
+    int32_t r[kSpanSlots];
+    double4 v[kSpanSlots];
+    bool put[kSpanSlots];  // the record is written from here
+    uint32_t kind[kSpanSlots], here[kSpanSlots], count[kSpanSlots];
 #pragma unroll
-            for (int dd = 0; dd < 8; ++dd) {
-                const uint32_t code = cc[8 * id + dd];
-                if (code == kChildEmpty) continue;
-                double4 v;
-                uint32_t m;
-                if (code & kChildHere) {
-                    v = sv[code & ~kChildHere];
-                    m = sn[code & ~kChildHere];
-                } else {
-                    v = cv[8 * id + dd];
-                    m = code;
-                }
-                sx += v.x;
-                sy += v.y;
-                sz += v.z;
-                sm += v.w;
-                cn += m;
-            }
-            sv[id] = make_double4(sx, sy, sz, sm);
-            sn[id] = cn;
-            if (sm == 0) raise_flag(h, kFlagZeroMass);
-        }
-        __syncthreads();
+    for (int q = 0; q < kSpanSlots; ++q) {
+        const uint32_t p = t + q * kComThreads;
+        put[q] = p < 8 * nk;
+        r[q] = put[q] ? ref[1ull + 8ull * list[p >> 3] + (p & 7u)] : kRefEmpty;
     }
-    // global stores only now (a barrier also waits for them): sums, the
-    // records of the children summed here, group marks, the root
-    for (uint32_t id = t; id < nk; id += kComThreads) {
-        const double4 g = sv[id];
-        sums[list[id]] = InternalSums{g.x, g.y, g.z, g.w};
-        counts[list[id]] = sn[id];
-        if (sn[id] > o.rule.group_max) {
+#pragma unroll
+    for (int q = 0; q < kSpanSlots; ++q) {
+        v[q] = make_double4(0.0, 0.0, 0.0, 0.0);
+        kind[q] = ~want;
+        here[q] = 0;
+        count[q] = 0;
+        if (r[q] >= 0) {
+            kind[q] = int_local[r[q]];
+            here[q] = cid[r[q]];
+            count[q] = counts[r[q]];
+            v[q] = *reinterpret_cast<const double4 *>(&sums[r[q]]);
+        } else if (r[q] != kRefEmpty) {
+            v[q] = body4[body_of_ref(r[q])];
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < kSpanSlots; ++q) {
+        const uint32_t p = t + q * kComThreads;
+        if (!put[q]) continue;
+        uint32_t at = p;
+        if (kind[q] == want) {  // summed by this workgroup, one level deeper
+            at = kSpanSum + min(here[q], kSpanCells - 1);
+            put[q] = false;
+        } else {
+            if (r[q] < 0 && r[q] != kRefEmpty) {
+                v[q] = body_term(v[q]);
+                count[q] = 1;
+            }
+            *reinterpret_cast<double4 *>(term[p]) = v[q];
+            m_s[p] = count[q];
+        }
+        at_s[p] = (uint16_t)at;
+    }
+    __syncthreads();
+    if (t < 64) sum_levels<64, kSpanSum>(t, cnt, uniform64(levels), order, at_s, term, m_s);
+#pragma unroll
+    for (int q = 0; q < kSpanSlots; ++q) {
+        const uint32_t p = t + q * kComThreads;
+        if (put[q])
+            put_record(o, 1ull + 8ull * list[p >> 3] + (p & 7u), r[q],
+                       r[q] == kRefEmpty ? v[q] : term_com(v[q]));
+    }
+    __syncthreads();
+    // the cells summed here: sums, record (the root's is node 0), group marks
+    if (t < nk) {
+        const uint32_t k = list[t], bodies = m_s[kSpanSum + t];
+        const double4 g = *reinterpret_cast<const double4 *>(term[kSpanSum + t]);
+        if (g.w == 0) raise_flag(h, kFlagZeroMass);
+        sums[k] = InternalSums{g.x, g.y, g.z, g.w};
+        counts[k] = bodies;
+        put_record(o, node, (int32_t)k, term_com(g));
+        if (bodies > o.rule.group_max) {
             uint32_t m[8];
 #pragma unroll
-            for (int dd = 0; dd < 8; ++dd) {
-                const uint32_t code = cc[8 * id + dd];
-                m[dd] = code == kChildEmpty ? 0u : code & kChildHere ? sn[code & ~kChildHere] : code;
-            }
-            put_child_groups(o, fst[id], m);
-        }
-    }
-    for (uint32_t p = t; p < 8 * nk; p += kComThreads) {
-        const uint32_t id = p >> 3;
-        const uint32_t dd = p & 7u;
-        const uint32_t code = cc[p];
-        const uint32_t pc = sn[id];
-        if (code != kChildEmpty && (code & kChildHere))
-            put_record(o, 1ull + 8ull * list[id] + dd, (int32_t)list[code & ~kChildHere],
-                       term_com(sv[code & ~kChildHere]));
-        if (dd == 0 && ldep[id] == 0) {  // the root
-            put_record(o, 0, (int32_t)list[id], term_com(sv[id]));
-            if (pc <= o.rule.group_max) put_group(o, fst[id], pc);
+            for (int d = 0; d < 8; ++d) m[d] = m_s[at_s[8 * t + d]];
+            put_child_groups(o, first, m);
+        } else if (ldep[t] == 0) {
+            put_group(o, first, bodies);
         }
     }
 }
@@ -1122,10 +1210,11 @@ __device__ __forceinline__ void com_span_block(
 __global__ void __launch_bounds__(kComThreads) k_com_span(
     uint32_t nblocks, uint32_t rows, uint32_t want, TreeHdr *h, const double4 *__restrict__ body4,
     const int32_t *__restrict__ ref, const uint32_t *__restrict__ spanning,
-    const uint8_t *__restrict__ int_local, const uint32_t *__restrict__ int_first, uint32_t *cid,
-    InternalSums *sums, uint32_t *counts, uint32_t *cross, uint32_t cross_cap, RecOut o) {
+    const uint8_t *__restrict__ int_local, const uint32_t *__restrict__ int_first,
+    const uint32_t *__restrict__ int_node, uint32_t *cid, InternalSums *sums, uint32_t *counts,
+    uint32_t *cross, uint32_t cross_cap, RecOut o) {
     com_span_block(blockIdx.x, nblocks, rows, want, h, body4, ref, spanning, int_local, int_first,
-                   cid, sums, counts, cross, cross_cap, o);
+                   int_node, cid, sums, counts, cross, cross_cap, o);
 }
 
 // ---- traversal groups -------------------------------------------------------------
@@ -1451,8 +1540,8 @@ __global__ void __launch_bounds__(kThreads) k_forest_link(uint32_t slots,
     kv.w0 = w0 - fo;
     kv.w1 = w1 - fo;
     link_at(ss.li, S.n, S.icap, fb.hdr + ss.s, kv, fb.sidx + fo, fb.lcp + fo, fb.chain + fo,
-            fb.ref + S.node_off, fb.int_depth + io, fb.int_parent + io, fb.int_node + io,
-            fb.body_parent + fo, fb.int_local + io, fb.spanning + S.span_off,
+            fb.ref + S.node_off, fb.int_depth + io, fb.int_node + io,
+            fb.body_node + fo, fb.int_local + io, fb.spanning + S.span_off,
             kMaxDepth * ((S.n + kComBlock - 1) / kComBlock), fb.int_first + io, kComBlock,
             kComSuper);
 }
@@ -1485,9 +1574,9 @@ __global__ void __launch_bounds__(kComLocalThreads) k_forest_com_local(
     const ForestTree f = forest_tree(sys, e.x, fb, G, rule);
     const EnsSystem &S = f.S;
     const uint32_t fo = S.fb_off, io = S.int_off;
-    com_local_block(e.y, S.n, S.icap, f.h, fb.body4 + fo, fb.sidx + fo, fb.ref + S.node_off,
-                    fb.chain + fo, fb.int_depth + io, fb.int_local + io, fb.int_first + io,
-                    fb.int_lvl + io, fb.int_sums + io, fb.int_count + io, f.o);
+    com_local_block(e.y, S.n, S.icap, f.h, fb.body4 + fo, fb.sidx + fo, fb.body_node + fo,
+                    fb.ref + S.node_off, fb.chain + fo, fb.int_depth + io, fb.int_local + io,
+                    fb.int_first + io, fb.int_node + io, fb.int_lvl + io, fb.int_sums + io, fb.int_count + io, f.o);
 }
 
 __global__ void __launch_bounds__(kComThreads) k_forest_com_span(
@@ -1500,8 +1589,8 @@ __global__ void __launch_bounds__(kComThreads) k_forest_com_span(
     const uint32_t nblocks = (S.n + kComBlock - 1) / kComBlock;
     com_span_block(e.y, nblocks, want == 2 ? nblocks : kComSuperBlocks, want, f.h,
                    fb.body4 + fo, fb.ref + S.node_off, fb.spanning + S.span_off,
-                   fb.int_local + io, fb.int_first + io, fb.int_lvl + io, fb.int_sums + io,
-                   fb.int_count + io, fb.cross + S.cross_off,
+                   fb.int_local + io, fb.int_first + io, fb.int_node + io, fb.int_lvl + io,
+                   fb.int_sums + io, fb.int_count + io, fb.cross + S.cross_off,
                    kMaxDepth * ((S.n + kComSuper - 1) / kComSuper + 1), f.o);
 }
 
@@ -1642,8 +1731,8 @@ void launch_topology(const TreeBufs &t, const double *x, const double *y, const 
     KeyView kv{t.skey, t.klo};
     hipLaunchKernelGGL(k_link, grid, dim3(kThreads), 0, s, n, t.icap, t.hdr, kv,
                        (const uint32_t *)t.sidx, (const int32_t *)t.lcp,
-                       (const uint32_t *)t.chain, t.ref, t.int_depth, t.int_parent, t.int_node,
-                       t.body_parent, t.int_local, t.spanning, t.spanning_cap, t.int_first);
+                       (const uint32_t *)t.chain, t.ref, t.int_depth, t.int_node,
+                       t.body_node, t.int_local, t.spanning, t.spanning_cap, t.int_first);
 }
 
 void launch_max_depth(const TreeBufs &t, hipStream_t s) {
@@ -1658,22 +1747,23 @@ void launch_com(const TreeBufs &t, double G, bool f64, bool f32, GroupRule rule,
     const RecOut o{G,     (int)f64,     (int)f32,     t.cm,
                    t.rec, t.group_size, t.group_slot, rule};
     hipLaunchKernelGGL(k_com_local, dim3(nblocks), dim3(kComLocalThreads), 0, s, t.n, t.icap, t.hdr,
-                       (const double4 *)t.body4, (const uint32_t *)t.sidx, (const int32_t *)t.ref,
-                       (const uint32_t *)t.chain, (const uint8_t *)t.int_depth,
-                       (const uint8_t *)t.int_local, (const uint32_t *)t.int_first, t.int_lvl,
-                       t.int_sums, t.int_count, o);
+                       (const double4 *)t.body4, (const uint32_t *)t.sidx, (const uint32_t *)t.body_node,
+                       (const int32_t *)t.ref, (const uint32_t *)t.chain, (const uint8_t *)t.int_depth,
+                       (const uint8_t *)t.int_local, (const uint32_t *)t.int_first,
+                       (const uint32_t *)t.int_node, t.int_lvl, t.int_sums, t.int_count, o);
     if (nblocks >= 2) {
         hipLaunchKernelGGL(k_com_span, dim3(ceil_div(nblocks, kComSuperBlocks)), dim3(kComThreads),
                            0, s, nblocks, kComSuperBlocks, 0u, t.hdr, (const double4 *)t.body4,
                            (const int32_t *)t.ref, (const uint32_t *)t.spanning,
-                           (const uint8_t *)t.int_local, (const uint32_t *)t.int_first, t.int_lvl,
-                           t.int_sums, t.int_count, t.cross, t.cross_cap, o);
+                           (const uint8_t *)t.int_local, (const uint32_t *)t.int_first,
+                           (const uint32_t *)t.int_node, t.int_lvl, t.int_sums, t.int_count,
+                           t.cross, t.cross_cap, o);
         if (nblocks > kComSuperBlocks)
             hipLaunchKernelGGL(k_com_span, dim3(1), dim3(kComThreads), 0, s, nblocks, nblocks, 2u,
                                t.hdr, (const double4 *)t.body4, (const int32_t *)t.ref,
                                (const uint32_t *)t.spanning, (const uint8_t *)t.int_local,
-                               (const uint32_t *)t.int_first, t.int_lvl, t.int_sums, t.int_count,
-                               t.cross, t.cross_cap, o);
+                               (const uint32_t *)t.int_first, (const uint32_t *)t.int_node, t.int_lvl,
+                               t.int_sums, t.int_count, t.cross, t.cross_cap, o);
     }
     if (f32) {
         // the group list: slots by an exclusive scan of the marks, then a scatter

@@ -357,6 +357,25 @@ def test_tree_parity(gpu, oracle, kind, n):
     assert_canonical_equal(can, t.canonical(), f"{kind} n={n}")
 
 
+# Edges of the build's blocks: 256 and 1024 bodies (topology, centre of mass),
+# 2048 (scan), 4096 (sort), 64 blocks of 1024 (super-blocks: one body over, and a
+# second super-block of two blocks).  Sums are the reference's, bit for bit.
+@pytest.mark.parametrize("kind,n", [("cube", 3), ("cube", 255), ("plummer", 257),
+                                    ("plummer", 1023), ("disk", 1024), ("cluster", 1025),
+                                    ("plummer", 2047), ("cube", 2049), ("disk", 4095),
+                                    ("cluster", 4096), ("plummer", 4097), ("cluster", 65536),
+                                    ("plummer", 65537), ("disk", 66561)])
+def test_tree_block_edges(gpu, oracle, kind, n):
+    d = make(gpu, kind, n, seed=n)
+    t = oracle.Tree(n)
+    t.build(d["x"], d["y"], d["z"], d["m"])
+    with ctx_for(gpu, d) as c:
+        c.bh_build()
+        assert c.tree_info()["node_count"] == t.node_count
+        np.testing.assert_array_equal(c.tree_sorted(), t.export()["sorted"])
+        assert_canonical_equal(c.tree_canonical(), t.canonical(), f"{kind} n={n}")
+
+
 def test_tree_deep_runs(gpu, oracle):
     # pairs of bodies closer than edge/2^21 force the 42-digit path
     rng = np.random.default_rng(3)
