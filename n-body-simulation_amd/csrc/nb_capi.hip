@@ -204,7 +204,7 @@ void tree_free(nb_ctx *c, TreeBufs &t) {
     void *bufs[] = {t.hdr, t.aabb_part, t.skey, t.skey_alt, t.klo, t.sidx, t.sidx_alt,
                     t.lcp, t.chain, t.body_node, t.int_depth, t.int_node,
                     t.int_lvl, t.int_count, t.int_sums, t.int_local, t.int_first, t.groups,
-                    t.group_size, t.group_slot, t.body4, t.gq, t.spanning, t.cross, t.ref,
+                    t.group_size, t.body4, t.gq, t.spanning, t.cross, t.ref,
                     t.cm, t.rec, t.radix_ctl, t.scan_part};
     for (void *b : bufs) dev_free(c, b);
     t = TreeBufs();
@@ -233,7 +233,7 @@ int alloc_tree_into(nb_ctx *c, TreeBufs &t, uint32_t storage_size_param) {
 #define NB_TREE_ALLOC(ptr, count) \
     if ((rc = dev_alloc(c, &(ptr), (count)))) return undo(rc)
     NB_TREE_ALLOC(t.hdr, 1);
-    NB_TREE_ALLOC(t.aabb_part, 6ull * nb::kAabbBlocks);
+    NB_TREE_ALLOC(t.aabb_part, 7ull * nb::kAabbBlocks);
     NB_TREE_ALLOC(t.skey, n);
     NB_TREE_ALLOC(t.skey_alt, n);
     NB_TREE_ALLOC(t.klo, n);
@@ -251,7 +251,6 @@ int alloc_tree_into(nb_ctx *c, TreeBufs &t, uint32_t storage_size_param) {
     NB_TREE_ALLOC(t.int_first, t.icap);
     NB_TREE_ALLOC(t.groups, n);
     NB_TREE_ALLOC(t.group_size, n);
-    NB_TREE_ALLOC(t.group_slot, n);
     NB_TREE_ALLOC(t.body4, n);
     NB_TREE_ALLOC(t.gq, TreeBufs::kGroupQueueWords);
     // a cell crossing a COM block boundary holds that boundary's two bodies:

@@ -20,7 +20,7 @@ namespace nb {
 
 constexpr int kKeyLevels = 21;  // octant digits held by one 63-bit key word
 constexpr int kMaxDepth = 42;   // two key words
-constexpr int kAabbBlocks = 1024;
+constexpr int kAabbBlocks = 256;
 
 // device status bits, turned into NB_E_* codes by the host
 enum : uint32_t {
@@ -145,7 +145,7 @@ struct TreeBufs {
     uint32_t icap = 0;  // internal-node capacity
     uint64_t mcap = 0;  // node capacity = 1 + 8 icap
     TreeHdr *hdr = nullptr;
-    double *aabb_part = nullptr;  // 6 * kAabbBlocks
+    double *aabb_part = nullptr;  // 7 * kAabbBlocks
     uint64_t *skey = nullptr, *skey_alt = nullptr, *klo = nullptr;
     uint32_t *sidx = nullptr, *sidx_alt = nullptr;
     int32_t *lcp = nullptr;       // n entries (pair i between sorted i and i+1)
@@ -160,7 +160,6 @@ struct TreeBufs {
     uint32_t *int_first = nullptr;  // first sorted position of the cell's bodies
     uint2 *groups = nullptr;        // traversal groups {first sorted position, body count}
     uint32_t *group_size = nullptr; // per sorted position: size of the group starting there
-    uint32_t *group_slot = nullptr; // per sorted position: 1 if a group starts there, then slots
     uint32_t *spanning = nullptr;   // [block * kMaxDepth + depth]: cell crossing the block's end
     uint32_t *cross = nullptr;      // cells crossing super-block boundaries: k << 6 | depth
     uint32_t cross_cap = 0;
@@ -238,6 +237,55 @@ struct ForestBufs {
 void scan_exclusive_u32(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t *total_dev,
                         uint32_t *scratch, uint32_t scratch_cap, hipStream_t s);
 uint32_t scan_scratch_words(uint32_t n);
+// Scans whose input comes from another pass: tile sums in `part`, then a kernel
+// of one workgroup of kScanThreads per tile, kScanItems consecutive values per
+// thread, which calls scan_place.  Every workgroup adds up the sums of the tiles
+// before its own, a launch (3 to 5 us) less than scanning them first; the limit
+// is where reading them starts to cost as much (8.4 million values: 16 KB per
+// workgroup).
+constexpr int kScanTile = 2048;
+constexpr int kScanThreads = 512;
+constexpr int kScanItems = kScanTile / kScanThreads;
+constexpr uint32_t kScanPartsInline = 4096;
+// More than kScanPartsInline sums: scans them in place (true); else false.
+bool scan_parts_if_many(uint32_t *part, uint32_t nparts, hipStream_t s);
+struct ScanPlace {
+    uint32_t first;   // sum of the tiles before this one
+    uint32_t before;  // sum of this tile's threads before this one
+    uint32_t total;   // sum of this tile
+};
+// v: the thread's own sum; sh: 2 * kScanThreads / 64 words.  part null: first = 0.
+__device__ inline ScanPlace scan_place(uint32_t v, const uint32_t *__restrict__ part,
+                                       uint32_t nparts, bool scanned, uint32_t *sh) {
+    constexpr uint32_t waves = kScanThreads / 64;
+    const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+    uint32_t head = 0;
+    if (part && scanned) {
+        head = t == 0 ? part[blockIdx.x] : 0u;
+    } else if (part) {
+        for (uint32_t k = t; k < blockIdx.x; k += kScanThreads) head += part[k];
+    }
+    uint32_t inc = v;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = __shfl_up(inc, d, 64);
+        if (lane >= (uint32_t)d) inc += o;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) head += __shfl_xor(head, d, 64);
+    if (lane == 63) sh[w] = inc;
+    if (lane == 0) sh[waves + w] = head;
+    __syncthreads();
+    ScanPlace r{0, inc - v, 0};
+#pragma unroll
+    for (uint32_t k = 0; k < waves; ++k) {
+        const uint32_t c = sh[k];
+        r.before += k < w ? c : 0u;
+        r.total += c;
+        r.first += sh[waves + k];
+    }
+    return r;
+}
 // Where a radix sort left its result.
 enum class SortEnd {
     kInPlace,   // keys/vals (an even pass count, or n <= 1)
@@ -251,7 +299,16 @@ enum class SortEnd {
 // wait raises kFlagSortWait in *flags.
 SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
                            uint32_t *vals_alt, uint32_t n, int bits, uint32_t *ctl,
-                           uint32_t *flags, hipStream_t s);
+                           uint32_t *flags, bool counted, hipStream_t s);
+// counted: the caller's kernel has done the sort's first step.  It adds the
+// number of keys of each lowest digit (key & (kRadixBins - 1)) to total[digit]
+// and clears plane0[0, plane_words); total is null if there is nothing to sort.
+constexpr uint32_t kRadixBins = 512;
+struct RadixCount {
+    uint32_t *total, *plane0;
+    uint64_t plane_words;
+};
+RadixCount radix_count_args(uint32_t n, uint32_t *ctl);
 uint32_t radix_blocks_for(uint32_t n);
 uint32_t radix_ctl_words(uint32_t n);
 

@@ -50,69 +50,80 @@ __device__ inline double sycl_max(double a, double b) { return a < b ? b : a; }
 __device__ inline void raise_flag(TreeHdr *h, uint32_t f) { atomicOr(&h->status, f); }
 
 // ---- 1. AABB ---------------------------------------------------------------
-__global__ void __launch_bounds__(kThreads) k_build_begin(TreeHdr *h) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        h->internal_count = 0;
-        h->max_depth = 0;
-        h->status = 0;
-        h->deep_runs = 0;
-        h->stack_peak = 0;
-        h->group_count = 0;
-        h->group_next = 0;
-        h->cross_count = 0;
-    }
-}
-
 // Block partial extrema.  Like the reference's partials (BarnesHutOctree.cpp:
-// 58-72, value-initialised to 0.0) every partial starts at the origin.
-__global__ void __launch_bounds__(kThreads) k_aabb_partial(const double *__restrict__ x,
-                                                           const double *__restrict__ y,
-                                                           const double *__restrict__ z,
-                                                           uint32_t n, double *part,
-                                                           TreeHdr *h) {
+// 58-72, value-initialised to 0.0) every partial starts at the origin.  A
+// seventh value says whether the block met a position that is not finite.
+constexpr int kAabbThreads = 1024;
+constexpr int kAabbVals = 7;
+static_assert(kAabbBlocks <= kAabbThreads, "the final reduction reads one partial per thread");
+struct Extents {
     double mn[3] = {0.0, 0.0, 0.0}, mx[3] = {0.0, 0.0, 0.0};
     bool bad = false;
-    for (uint64_t i = (uint64_t)blockIdx.x * kThreads + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * kThreads) {
-        const double p[3] = {x[i], y[i], z[i]};
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            bad |= !isfinite(p[c]);
-            mn[c] = sycl_min(mn[c], p[c]);
-            mx[c] = sycl_max(mx[c], p[c]);
-        }
-    }
-    if (bad) raise_flag(h, kFlagAabb);
-    // min/max are exact, so any reduction order gives the reference's result
+};
+// min/max are exact, so any reduction order gives the reference's result
+__device__ inline void wave_extents(Extents &e) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            mn[c] = sycl_min(mn[c], __shfl_xor(mn[c], off, 64));
-            mx[c] = sycl_max(mx[c], __shfl_xor(mx[c], off, 64));
+            e.mn[c] = sycl_min(e.mn[c], __shfl_xor(e.mn[c], off, 64));
+            e.mx[c] = sycl_max(e.mx[c], __shfl_xor(e.mx[c], off, 64));
         }
     }
-    __shared__ double sh[kThreads / 64][6];
-    const int w = threadIdx.x >> 6;
+    e.bad = __any(e.bad);
+}
+
+// The workgroup's extents, from every thread's, into out[0..7) (LDS or global,
+// `stride` apart): min x y z, max x y z, bad.
+__device__ inline void block_extents(Extents e, double (*sh)[kAabbVals], double *out,
+                                     uint32_t stride) {
+    wave_extents(e);
+    const uint32_t w = threadIdx.x >> 6, waves = blockDim.x >> 6;
     if ((threadIdx.x & 63) == 0) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            sh[w][c] = mn[c];
-            sh[w][3 + c] = mx[c];
+            sh[w][c] = e.mn[c];
+            sh[w][3 + c] = e.mx[c];
         }
+        sh[w][6] = e.bad ? 1.0 : 0.0;
     }
     __syncthreads();
-    if (threadIdx.x < 6) {
+    if (threadIdx.x < kAabbVals) {
         double v = sh[0][threadIdx.x];
-        for (int k = 1; k < kThreads / 64; ++k)
+        for (uint32_t k = 1; k < waves; ++k)
             v = threadIdx.x < 3 ? sycl_min(v, sh[k][threadIdx.x]) : sycl_max(v, sh[k][threadIdx.x]);
-        part[(uint64_t)threadIdx.x * gridDim.x + blockIdx.x] = v;
+        out[(uint64_t)threadIdx.x * stride] = v;
     }
 }
 
+__global__ void __launch_bounds__(kAabbThreads) k_aabb_partial(const double *__restrict__ x,
+                                                               const double *__restrict__ y,
+                                                               const double *__restrict__ z,
+                                                               uint32_t n, double *part) {
+    __shared__ double sh[kAabbThreads / 64][kAabbVals];
+    Extents e;
+#pragma unroll 4
+    for (uint64_t i = (uint64_t)blockIdx.x * kAabbThreads + threadIdx.x; i < n;
+         i += (uint64_t)gridDim.x * kAabbThreads) {
+        const double p[3] = {x[i], y[i], z[i]};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            e.bad |= !isfinite(p[c]);
+            e.mn[c] = sycl_min(e.mn[c], p[c]);
+            e.mx[c] = sycl_max(e.mx[c], p[c]);
+        }
+    }
+    block_extents(e, sh, part + blockIdx.x, gridDim.x);
+}
+
 // Cubify the extents ext = {min_x, min_y, min_z, max_x, max_y, max_z}
-// (BarnesHutOctree.cpp:161-190) and store the root cube.
-__device__ inline void cubify(const double ext[6], TreeHdr *h) {
+// (BarnesHutOctree.cpp:161-190) to the root cube.
+struct RootCube {
+    double mn[3], mx[3], edge;
+    bool ok;
+};
+__device__ inline RootCube cubify(const double ext[6]) {
+    bool ok = true;
     double min_x = ext[0], min_y = ext[1], min_z = ext[2];
     double max_x = ext[3], max_y = ext[4], max_z = ext[5];
     const double x_length = fabs(max_x - min_x);
@@ -137,52 +148,18 @@ __device__ inline void cubify(const double ext[6], TreeHdr *h) {
         max_x = max_x + ((maxEdgeLength - x_length) / 2);
         max_y = max_y + ((maxEdgeLength - y_length) / 2);
     } else {
-        raise_flag(h, kFlagAabb);
+        ok = false;
     }
-    h->minx = min_x;
-    h->miny = min_y;
-    h->minz = min_z;
-    h->maxx = max_x;
-    h->maxy = max_y;
-    h->maxz = max_z;
-    h->edge = maxEdgeLength;
+    return RootCube{{min_x, min_y, min_z}, {max_x, max_y, max_z}, maxEdgeLength, ok};
 }
-
-// Final reduction on one thread per component, then one thread cubifies.
-__global__ void __launch_bounds__(kThreads) k_aabb_final(const double *part, uint32_t np,
-                                                         TreeHdr *h) {
-    __shared__ double sh[kThreads / 64][6];
-    __shared__ double ext[6];
-    // every partial already includes the origin, so 0.0 is a neutral start
-    double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    for (uint32_t k = threadIdx.x; k < np; k += kThreads) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v[c] = sycl_min(v[c], part[(uint64_t)c * np + k]);
-            v[3 + c] = sycl_max(v[3 + c], part[(uint64_t)(3 + c) * np + k]);
-        }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            v[c] = sycl_min(v[c], __shfl_xor(v[c], off, 64));
-            v[3 + c] = sycl_max(v[3 + c], __shfl_xor(v[3 + c], off, 64));
-        }
-    }
-    if ((threadIdx.x & 63) == 0)
-        for (int c = 0; c < 6; ++c) sh[threadIdx.x >> 6][c] = v[c];
-    __syncthreads();
-    if (threadIdx.x < 6) {
-        double r = sh[0][threadIdx.x];
-        for (int w = 1; w < kThreads / 64; ++w)
-            r = threadIdx.x < 3 ? sycl_min(r, sh[w][threadIdx.x]) : sycl_max(r, sh[w][threadIdx.x]);
-        ext[threadIdx.x] = r;
-    }
-    __syncthreads();
-    if (threadIdx.x != 0) return;
-    const double e6[6] = {ext[0], ext[1], ext[2], ext[3], ext[4], ext[5]};
-    cubify(e6, h);
+__device__ inline void store_cube(TreeHdr *h, const RootCube &r) {
+    h->minx = r.mn[0];
+    h->miny = r.mn[1];
+    h->minz = r.mn[2];
+    h->maxx = r.mx[0];
+    h->maxy = r.mx[1];
+    h->maxz = r.mx[2];
+    h->edge = r.edge;
 }
 
 // ---- 2. keys ---------------------------------------------------------------
@@ -194,21 +171,67 @@ __device__ inline uint64_t key_from(Cell &c, double px, double py, double pz) {
 }
 
 // Keys, identity permutation, and the packed body record {x, y, z, m} that
-// the centre-of-mass and node-record passes gather (one 32-byte load).
-__global__ void __launch_bounds__(kThreads) k_keys(const double *__restrict__ x,
-                                                   const double *__restrict__ y,
-                                                   const double *__restrict__ z,
-                                                   const double *__restrict__ m, uint32_t n,
-                                                   const TreeHdr *__restrict__ h,
-                                                   uint64_t *skey, uint32_t *sidx,
-                                                   double4 *body4) {
-    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    Cell c{h->minx, h->miny, h->minz, h->edge};
-    const double px = x[i], py = y[i], pz = z[i];
-    skey[i] = key_from(c, px, py, pz);
-    sidx[i] = i;
-    body4[i] = make_double4(px, py, pz, m[i]);
+// the centre-of-mass and node-record passes gather (one 32-byte load).  Small
+// jobs ride along, each of which took a launch of its own (3 to 5 us): every
+// workgroup finds the root cube from the partial extents (at most kAabbBlocks
+// of each, one per thread), the first one resets the header, and the sort's
+// first digit is counted.  So there are at most 256 workgroups, which take
+// their bodies in strides.
+constexpr int kKeyThreads = 1024;
+constexpr uint32_t kKeyBlocks = 256;
+__global__ void __launch_bounds__(kKeyThreads) k_keys(
+    const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
+    const double *__restrict__ m, uint32_t n, const double *__restrict__ part, uint32_t np,
+    TreeHdr *h, uint64_t *skey, uint32_t *sidx, double4 *body4, uint32_t *scan_part,
+    uint32_t scan_parts, RadixCount rc) {
+    __shared__ double sh[kKeyThreads / 64][kAabbVals];
+    __shared__ double ext[kAabbVals];
+    __shared__ RootCube root;
+    __shared__ uint32_t hist[kRadixBins];
+    const uint32_t t = threadIdx.x;
+    Extents e;
+    if (t < np) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            e.mn[c] = part[(uint64_t)c * np + t];
+            e.mx[c] = part[(uint64_t)(3 + c) * np + t];
+        }
+        e.bad = part[6ull * np + t] != 0.0;
+    }
+    if (t < kRadixBins) hist[t] = 0;
+    block_extents(e, sh, ext, 1);
+    __syncthreads();
+    if (t == 0) {
+        root = cubify(ext);
+        if (blockIdx.x == 0) {
+            store_cube(h, root);
+            h->internal_count = 0;
+            h->max_depth = 0;
+            h->status = ext[6] != 0.0 || !root.ok ? kFlagAabb : 0u;
+            h->deep_runs = 0;
+            h->stack_peak = 0;
+            h->group_count = 0;
+            h->group_next = 0;
+            h->cross_count = 0;
+        }
+    }
+    __syncthreads();
+    const uint64_t stride = (uint64_t)gridDim.x * kKeyThreads;
+    const uint64_t i0 = (uint64_t)blockIdx.x * kKeyThreads + t;
+    for (uint64_t i = i0; i < rc.plane_words; i += stride) rc.plane0[i] = 0;
+    for (uint64_t i = i0; i < scan_parts; i += stride) scan_part[i] = 0;
+    for (uint64_t i = i0; i < n; i += stride) {
+        Cell c{root.mn[0], root.mn[1], root.mn[2], root.edge};
+        const double px = x[i], py = y[i], pz = z[i];
+        const uint64_t key = key_from(c, px, py, pz);
+        skey[i] = key;
+        sidx[i] = (uint32_t)i;
+        body4[i] = make_double4(px, py, pz, m[i]);
+        atomicAdd(&hist[(uint32_t)key & (kRadixBins - 1)], 1u);
+    }
+    if (!rc.total) return;  // nothing to sort
+    __syncthreads();
+    if (t < kRadixBins && hist[t]) atomicAdd(&rc.total[t], hist[t]);
 }
 
 // ---- 4./5. LCP and deep runs --------------------------------------------------
@@ -270,17 +293,6 @@ __device__ inline void lcp_at(uint32_t i, const double *__restrict__ x,
     }
 }
 
-__global__ void __launch_bounds__(kThreads) k_lcp(const double *__restrict__ x,
-                                                  const double *__restrict__ y,
-                                                  const double *__restrict__ z, uint32_t n,
-                                                  TreeHdr *h, uint64_t *skey, uint32_t *sidx,
-                                                  uint64_t *klo, int32_t *lcp) {
-    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i + 1 >= n) return;
-    const Cell root{h->minx, h->miny, h->minz, h->edge};
-    lcp_at(i, x, y, z, n, root, h, skey, sidx, klo, lcp);
-}
-
 // chain[i] = number of internal cells owned by pair i = max(0, lcp[i] - lcp[i-1])
 __device__ inline void chain_at(uint32_t i, const int32_t *__restrict__ lcp, uint32_t *chain) {
     const int cp = i > 0 ? lcp[i - 1] : -1;
@@ -288,11 +300,85 @@ __device__ inline void chain_at(uint32_t i, const int32_t *__restrict__ lcp, uin
     chain[i] = cn > cp ? (uint32_t)(cn - cp) : 0u;
 }
 
-__global__ void __launch_bounds__(kThreads) k_chain(const int32_t *__restrict__ lcp, uint32_t n,
-                                                    uint32_t *chain) {
+// lcp of every pair, and the chain lengths of each scan tile's pairs added into
+// part[tile] (zeroed before).  A pair's chain needs the lcp of the pair before
+// it: from the keys, or at least kKeyLevels if these are equal, which leaves a
+// chain of 0.  The chains inside a run of equal keys are added by the thread
+// that sorts the run.
+__global__ void __launch_bounds__(kThreads) k_lcp(const double *__restrict__ x,
+                                                  const double *__restrict__ y,
+                                                  const double *__restrict__ z, uint32_t n,
+                                                  TreeHdr *h, uint64_t *skey, uint32_t *sidx,
+                                                  uint64_t *klo, int32_t *lcp, uint32_t *part) {
+    static_assert(kScanTile % kThreads == 0, "a workgroup's pairs lie in one tile");
+    __shared__ uint32_t ws[kThreads / 64];
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i + 1 >= n) return;
-    chain_at(i, lcp, chain);
+    uint32_t own = 0;
+    if (i + 1 < n) {
+        const Cell root{h->minx, h->miny, h->minz, h->edge};
+        lcp_at(i, x, y, z, n, root, h, skey, sidx, klo, lcp);
+        const uint64_t k0 = skey[i], k1 = skey[i + 1];
+        const uint64_t kp = i > 0 ? skey[i - 1] : 0;
+        const int cp = i == 0 ? -1 : kp == k0 ? kKeyLevels : lcp_depth(kp, k0);
+        if (k0 != k1) {
+            const int cn = lcp_depth(k0, k1);
+            own = cn > cp ? (uint32_t)(cn - cp) : 0u;
+        } else if (i == 0 || kp != k0) {  // a run's first pair: the chains of the run
+            int before = cp;
+            for (uint32_t p = i; p + 1 < n && skey[p + 1] == k0; ++p) {
+                const int d = lcp[p];
+                if (d > before) atomicAdd(&part[p / kScanTile], (uint32_t)(d - before));
+                before = d;
+            }
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) own += __shfl_xor(own, off, 64);
+    if ((threadIdx.x & 63u) == 0) ws[threadIdx.x >> 6] = own;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t sum = 0;
+        for (int w = 0; w < kThreads / 64; ++w) sum += ws[w];
+        if (sum) atomicAdd(&part[i / kScanTile], sum);
+    }
+}
+
+// Numbers the internal cells: off[i] = the chain lengths of the pairs before i
+// (tile sums in `part`), h->internal_count their total; and empties what the
+// topology pass fills in: the child slots of the tile's own cells, and the
+// table of block-crossing cells.
+__global__ void __launch_bounds__(kScanThreads) k_number(const int32_t *__restrict__ lcp,
+                                                         uint32_t pairs, uint32_t *off,
+                                                         const uint32_t *__restrict__ part,
+                                                         uint32_t nparts, bool scanned, TreeHdr *h,
+                                                         uint32_t icap, int32_t *ref,
+                                                         uint32_t *spanning, uint32_t spanning_cap) {
+    __shared__ uint32_t sh[2 * kScanThreads / 64];
+    const uint32_t t = threadIdx.x;
+    const uint64_t stride = (uint64_t)gridDim.x * kScanThreads;
+    for (uint64_t j = (uint64_t)blockIdx.x * kScanThreads + t; j < spanning_cap; j += stride)
+        spanning[j] = kNoCell;
+    const uint64_t i0 = (uint64_t)blockIdx.x * kScanTile + (uint64_t)t * kScanItems;
+    uint32_t v[kScanItems], sum = 0;
+    int before = i0 > 0 && i0 <= pairs ? lcp[i0 - 1] : -1;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        const int d = i0 + k < pairs ? lcp[i0 + k] : -1;
+        v[k] = d > before ? (uint32_t)(d - before) : 0u;
+        sum += v[k];
+        before = d;
+    }
+    const ScanPlace pl = scan_place(sum, part, nparts, scanned, sh);
+    uint32_t o = pl.first + pl.before;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        if (i0 + k < pairs) off[i0 + k] = o;
+        o += v[k];
+    }
+    if (blockIdx.x + 1 == gridDim.x && t == 0) h->internal_count = pl.first + pl.total;
+    const uint64_t ob = 1ull + 8ull * min(pl.first, icap);
+    const uint64_t oe = 1ull + 8ull * min(pl.first + pl.total, icap);
+    for (uint64_t j = ob + t; j < oe; j += kScanThreads) ref[j] = kRefEmpty;
 }
 
 // h->max_depth = depth of the deepest leaf = 1 + the deepest cell that two
@@ -366,17 +452,6 @@ struct KeyView {
         return (uint32_t)in;
     }
 };
-
-__global__ void __launch_bounds__(kThreads) k_fill(TreeHdr *h, uint32_t icap, int32_t *ref,
-                                                   uint32_t *spanning, uint32_t spanning_cap) {
-    const uint32_t I = min(h->internal_count, icap);
-    const uint64_t nodes = 1 + 8ull * I;
-    const uint64_t stride = (uint64_t)gridDim.x * kThreads;
-    for (uint64_t j = (uint64_t)blockIdx.x * kThreads + threadIdx.x; j < nodes; j += stride)
-        ref[j] = kRefEmpty;
-    for (uint64_t j = (uint64_t)blockIdx.x * kThreads + threadIdx.x; j < spanning_cap; j += stride)
-        spanning[j] = kNoCell;
-}
 
 // Internal cells owned by pair i and the leaf of sorted body i.  A cell is
 // "local" (int_local 1) when its bodies stay inside one com_block-body block
@@ -522,7 +597,8 @@ struct RecOut {
     int f64, f32;  // FP64 records (cm); FP32 records and traversal groups
     double4 *cm;
     NodeF32 *rec;
-    uint32_t *group_size, *group_slot;
+    uint32_t *group_size;
+    uint32_t *group_slot;  // 1 where a group starts, for a later scan; null: not kept
     GroupRule rule;  // group size and packing limit
 };
 
@@ -553,7 +629,7 @@ __device__ inline void put_record(const RecOut &o, uint64_t j, int32_t r, const 
 __device__ inline void put_group(const RecOut &o, uint32_t p, uint32_t size) {
     if (o.f32) {
         o.group_size[p] = size;
-        o.group_slot[p] = 1u;
+        if (o.group_slot) o.group_slot[p] = 1u;
     }
 }
 
@@ -833,7 +909,7 @@ __device__ __forceinline__ void com_local_block(
             if (b.w == 0) raise_flag(h, kFlagZeroMass);
             if (o.f32) {
                 o.group_size[0] = 0;
-                o.group_slot[0] = 0;
+                if (o.group_slot) o.group_slot[0] = 0;
             }
             put_record(o, 0, ref_of_body(q), term_com(body_term(b)));
             put_group(o, 0, 1);
@@ -892,7 +968,7 @@ __device__ __forceinline__ void com_local_block(
         if (fits && j < 8ull * nc) at_s[j] = (uint16_t)p;
         if (o.f32) {
             o.group_size[s + p] = 0;
-            o.group_slot[s + p] = 0;
+            if (o.group_slot) o.group_slot[s + p] = 0;
         }
     }
     if (!fits) {
@@ -1221,16 +1297,40 @@ __global__ void __launch_bounds__(kComThreads) k_com_span(
 // A group is a cell with at most group_max bodies whose parent holds more, or
 // a lone body whose parent holds more.  Groups partition the bodies into
 // spatially compact runs of the octree order.  Every sorted position starts
-// at most one group: mark the starts, scan, scatter -- the group list comes
-// out in octree order, so neighbouring groups share most of their walk.
-__global__ void __launch_bounds__(kThreads) k_group_scatter(uint32_t n,
-                                                            const uint32_t *__restrict__ group_size,
-                                                            const uint32_t *__restrict__ group_slot,
-                                                            uint2 *groups) {
-    const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i >= n) return;
-    const uint32_t s = group_size[i];
-    if (s) groups[group_slot[i]] = make_uint2(i, s);
+// at most one group: the starts of each scan tile are counted, and a second
+// launch writes them to their places -- the group list comes out in octree
+// order, so neighbouring groups share most of their walk.
+__global__ void __launch_bounds__(kScanThreads) k_group_count(
+    const uint32_t *__restrict__ group_size, uint32_t n, uint32_t *part) {
+    __shared__ uint32_t sh[2 * kScanThreads / 64];
+    const uint64_t i0 = (uint64_t)blockIdx.x * kScanTile + threadIdx.x;
+    uint32_t c = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        const uint64_t i = i0 + (uint64_t)k * kScanThreads;
+        if (i < n) c += group_size[i] != 0;
+    }
+    const ScanPlace pl = scan_place(c, nullptr, 0, true, sh);
+    if (threadIdx.x == 0) part[blockIdx.x] = pl.total;
+}
+
+__global__ void __launch_bounds__(kScanThreads) k_group_list(
+    const uint32_t *__restrict__ group_size, uint32_t n, const uint32_t *__restrict__ part,
+    uint32_t nparts, bool scanned, TreeHdr *h, uint2 *groups) {
+    __shared__ uint32_t sh[2 * kScanThreads / 64];
+    const uint64_t i0 = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
+    uint32_t v[kScanItems], c = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+        v[k] = i0 + k < n ? group_size[i0 + k] : 0u;
+        c += v[k] != 0;
+    }
+    const ScanPlace pl = scan_place(c, part, nparts, scanned, sh);
+    uint32_t g = pl.first + pl.before;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k)
+        if (v[k]) groups[g++] = make_uint2((uint32_t)i0 + k, v[k]);
+    if (blockIdx.x + 1 == gridDim.x && threadIdx.x == 0) h->group_count = pl.first + pl.total;
 }
 
 // ---- ensemble: the octrees of many systems ------------------------------------------
@@ -1340,7 +1440,9 @@ __global__ void __launch_bounds__(kForestThreads) k_forest_aabb(
                 v[c] = sycl_min(v[c], red[w][c]);
                 v[3 + c] = sycl_max(v[3 + c], red[w][3 + c]);
             }
-        cubify(v, h);
+        const RootCube r = cubify(v);
+        store_cube(h, r);
+        if (!r.ok) raise_flag(h, kFlagAabb);
     }
 }
 
@@ -1644,7 +1746,8 @@ void launch_forest_build(const EnsSystem *sys, const uint32_t *order, uint32_t n
     uint32_t *v = fb.sidx, *va = fb.sidx_alt;
     hipLaunchKernelGGL(k_forest_keys, dim3(blocks), dim3(kThreads), 0, s, slots,
                        (const uint16_t *)fb.fb_sys, sys, x, y, z, m, fb, k, v);
-    SortEnd end = radix_sort_u64_u32(k, v, ka, va, slots, kForestLowBits, fb.radix_ctl, status, s);
+    SortEnd end = radix_sort_u64_u32(k, v, ka, va, slots, kForestLowBits, fb.radix_ctl, status,
+                                     false, s);
     if (end == SortEnd::kRejected) return;  // reported in *status
     if (end == SortEnd::kInAlt) {
         std::swap(k, ka);
@@ -1657,7 +1760,7 @@ void launch_forest_build(const EnsSystem *sys, const uint32_t *order, uint32_t n
     while (sys_bits < 16 && (1u << sys_bits) < nsys) ++sys_bits;
     // its own control words: a control buffer must always see the same pass count
     end = radix_sort_u64_u32(k, v, ka, va, slots, 3 * kKeyLevels - kForestLowBits + sys_bits,
-                             fb.radix_ctl_sys, status, s);
+                             fb.radix_ctl_sys, status, false, s);
     if (end == SortEnd::kRejected) return;
     if (end == SortEnd::kInAlt) {
         std::swap(k, ka);
@@ -1687,27 +1790,30 @@ void launch_forest_build(const EnsSystem *sys, const uint32_t *order, uint32_t n
                        (const uint32_t *)total, items, status);
 }
 
+// workgroups of the AABB pass: 4096 bodies each, at most kAabbBlocks
+uint32_t aabb_blocks(uint32_t n) {
+    return std::min<uint32_t>(kAabbBlocks, ceil_div(n, 4 * kAabbThreads));
+}
+
 void launch_aabb(const TreeBufs &t, const double *x, const double *y, const double *z,
                  hipStream_t s) {
-    hipLaunchKernelGGL(k_build_begin, dim3(1), dim3(kThreads), 0, s, t.hdr);
-    const uint32_t nb = std::min<uint32_t>(kAabbBlocks, ceil_div(t.n, 4 * kThreads));
-    hipLaunchKernelGGL(k_aabb_partial, dim3(nb), dim3(kThreads), 0, s, x, y, z, t.n, t.aabb_part,
-                       t.hdr);
-    hipLaunchKernelGGL(k_aabb_final, dim3(1), dim3(kThreads), 0, s, (const double *)t.aabb_part, nb,
-                       t.hdr);
+    hipLaunchKernelGGL(k_aabb_partial, dim3(aabb_blocks(t.n)), dim3(kAabbThreads), 0, s, x, y, z,
+                       t.n, t.aabb_part);
 }
 
 void launch_keys(TreeBufs &t, const double *x, const double *y, const double *z,
                  const double *m, hipStream_t s) {
-    hipLaunchKernelGGL(k_keys, dim3(ceil_div(t.n, kThreads)), dim3(kThreads), 0, s, x, y, z, m,
-                       t.n, (const TreeHdr *)t.hdr, t.skey, t.sidx, t.body4);
+    hipLaunchKernelGGL(k_keys, dim3(std::min(kKeyBlocks, ceil_div(t.n, kKeyThreads))),
+                       dim3(kKeyThreads), 0, s, x, y, z, m, t.n, (const double *)t.aabb_part,
+                       aabb_blocks(t.n), t.hdr, t.skey, t.sidx, t.body4, t.scan_part,
+                       ceil_div(t.n, kScanTile), radix_count_args(t.n, t.radix_ctl));
 }
 
 void launch_key_sort(TreeBufs &t, hipStream_t s) {
     // a rejected sort (2^30 bodies or more, which the context's capacity
     // check already excludes) raises kFlagSortSize; the build reports it
     if (radix_sort_u64_u32(t.skey, t.sidx, t.skey_alt, t.sidx_alt, t.n, 3 * kKeyLevels,
-                           t.radix_ctl, &t.hdr->status, s) == SortEnd::kInAlt) {
+                           t.radix_ctl, &t.hdr->status, true, s) == SortEnd::kInAlt) {
         std::swap(t.skey, t.skey_alt);
         std::swap(t.sidx, t.sidx_alt);
     }
@@ -1719,15 +1825,13 @@ void launch_topology(const TreeBufs &t, const double *x, const double *y, const 
     const dim3 grid(ceil_div(n, kThreads));
     if (n > 1) {
         hipLaunchKernelGGL(k_lcp, grid, dim3(kThreads), 0, s, x, y, z, n, t.hdr, t.skey, t.sidx,
-                           t.klo, t.lcp);
-        hipLaunchKernelGGL(k_chain, grid, dim3(kThreads), 0, s, (const int32_t *)t.lcp, n,
-                           t.chain);
-        scan_exclusive_u32(t.chain, t.chain, n - 1, &t.hdr->internal_count, t.scan_part,
-                           t.scan_part_cap, s);
+                           t.klo, t.lcp, t.scan_part);
+        const uint32_t nparts = ceil_div(n - 1, kScanTile);
+        const bool scanned = scan_parts_if_many(t.scan_part, nparts, s);
+        hipLaunchKernelGGL(k_number, dim3(nparts), dim3(kScanThreads), 0, s,
+                           (const int32_t *)t.lcp, n - 1, t.chain, (const uint32_t *)t.scan_part,
+                           nparts, scanned, t.hdr, t.icap, t.ref, t.spanning, t.spanning_cap);
     }
-    const uint32_t fill_blocks = std::max<uint32_t>(1, std::min<uint32_t>(4096, ceil_div(8ull * n, kThreads)));
-    hipLaunchKernelGGL(k_fill, dim3(fill_blocks), dim3(kThreads), 0, s, t.hdr, t.icap, t.ref,
-                       t.spanning, t.spanning_cap);
     KeyView kv{t.skey, t.klo};
     hipLaunchKernelGGL(k_link, grid, dim3(kThreads), 0, s, n, t.icap, t.hdr, kv,
                        (const uint32_t *)t.sidx, (const int32_t *)t.lcp,
@@ -1745,7 +1849,7 @@ void launch_max_depth(const TreeBufs &t, hipStream_t s) {
 void launch_com(const TreeBufs &t, double G, bool f64, bool f32, GroupRule rule, hipStream_t s) {
     const uint32_t nblocks = ceil_div(t.n, kComBlock);
     const RecOut o{G,     (int)f64,     (int)f32,     t.cm,
-                   t.rec, t.group_size, t.group_slot, rule};
+                   t.rec, t.group_size, nullptr,     rule};
     hipLaunchKernelGGL(k_com_local, dim3(nblocks), dim3(kComLocalThreads), 0, s, t.n, t.icap, t.hdr,
                        (const double4 *)t.body4, (const uint32_t *)t.sidx, (const uint32_t *)t.body_node,
                        (const int32_t *)t.ref, (const uint32_t *)t.chain, (const uint8_t *)t.int_depth,
@@ -1766,12 +1870,13 @@ void launch_com(const TreeBufs &t, double G, bool f64, bool f32, GroupRule rule,
                                t.int_sums, t.int_count, t.cross, t.cross_cap, o);
     }
     if (f32) {
-        // the group list: slots by an exclusive scan of the marks, then a scatter
-        scan_exclusive_u32(t.group_slot, t.group_slot, t.n, &t.hdr->group_count, t.scan_part,
-                           t.scan_part_cap, s);
-        hipLaunchKernelGGL(k_group_scatter, dim3(ceil_div(t.n, kThreads)), dim3(kThreads), 0, s,
-                           t.n, (const uint32_t *)t.group_size, (const uint32_t *)t.group_slot,
-                           t.groups);
+        const uint32_t nparts = ceil_div(t.n, kScanTile);
+        hipLaunchKernelGGL(k_group_count, dim3(nparts), dim3(kScanThreads), 0, s,
+                           (const uint32_t *)t.group_size, t.n, t.scan_part);
+        const bool scanned = scan_parts_if_many(t.scan_part, nparts, s);
+        hipLaunchKernelGGL(k_group_list, dim3(nparts), dim3(kScanThreads), 0, s,
+                           (const uint32_t *)t.group_size, t.n, (const uint32_t *)t.scan_part,
+                           nparts, scanned, t.hdr, t.groups);
     }
 }
 

@@ -13,8 +13,7 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kThreads * kScanItems;
+constexpr int kItems = kScanTile / kThreads;
 constexpr int kRadixTile = 4096;       // keys per radix tile
 constexpr int kRadixTileBig = 8192;    // keys per tile from kRadixBigMin keys on
 constexpr uint32_t kRadixBigMin = 1u << 21;
@@ -57,7 +56,7 @@ __global__ void __launch_bounds__(kThreads) k_scan_reduce(const uint32_t *__rest
     const uint64_t base = (uint64_t)blockIdx.x * kScanTile;
     uint32_t s = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < kItems; ++k) {
         const uint64_t i = base + (uint64_t)k * kThreads + threadIdx.x;
         if (i < n) s += in[i];
     }
@@ -87,15 +86,15 @@ __global__ void __launch_bounds__(kThreads) k_scan_parts(uint32_t *part, uint32_
     if (threadIdx.x == 0 && total) *total = tot;
 }
 
-// Each thread scans kScanItems consecutive values; out may alias in.
+// Each thread scans kItems consecutive values; out may alias in.
 __global__ void __launch_bounds__(kThreads) k_scan_down(const uint32_t *in, uint32_t *out,
                                                         uint32_t n, const uint32_t *part) {
     __shared__ uint32_t sh[kWaves];
-    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kScanItems;
-    uint32_t v[kScanItems];
+    const uint64_t base = (uint64_t)blockIdx.x * kScanTile + (uint64_t)threadIdx.x * kItems;
+    uint32_t v[kItems];
     uint32_t s = 0;
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < kItems; ++k) {
         const uint64_t i = base + k;
         v[k] = i < n ? in[i] : 0u;
         s += v[k];
@@ -103,7 +102,7 @@ __global__ void __launch_bounds__(kThreads) k_scan_down(const uint32_t *in, uint
     uint32_t tot;
     uint32_t off = block_exclusive_scan(s, sh, &tot) + part[blockIdx.x];
 #pragma unroll
-    for (int k = 0; k < kScanItems; ++k) {
+    for (int k = 0; k < kItems; ++k) {
         const uint64_t i = base + k;
         if (i < n) out[i] = off;
         off += v[k];
@@ -120,7 +119,8 @@ __global__ void __launch_bounds__(kThreads) k_scan_down(const uint32_t *in, uint
 // ids are handed out in the order blocks start, so every tile a block waits on
 // belongs to a block that is running and that publishes its counts before it
 // waits on anything: every wait ends.  The digit totals (which do not depend
-// on the order) come from k_radix_count for pass 0 and from pass p - 1 for
+// on the order) come from
+// k_radix_count (or the caller's own kernel, see RadixCount) for pass 0 and from pass p - 1 for
 // pass p, which counts the next digit of the keys it has loaded anyway.
 //
 // Digits are 9 bits wide: 7 passes cover the 63-bit octree keys (an odd
@@ -142,7 +142,8 @@ __global__ void __launch_bounds__(kThreads) k_scan_down(const uint32_t *in, uint
 // below 2^30: octree contexts hold fewer than 2^29 bodies.
 
 constexpr int kDigitBits = 9;
-constexpr uint32_t kBins = 1u << kDigitBits;
+constexpr uint32_t kBins = kRadixBins;
+static_assert(kBins == 1u << kDigitBits, "digit width");
 constexpr int kMaxPasses = 7;
 static_assert(kMaxPasses * kDigitBits >= 63, "the passes cover the keys");
 static_assert(kBins == (uint32_t)kPassThreads, "thread tid owns digit tid");
@@ -394,14 +395,31 @@ void scan_exclusive_u32(const uint32_t *in, uint32_t *out, uint32_t n, uint32_t 
                        (const uint32_t *)scratch);
 }
 
+bool scan_parts_if_many(uint32_t *part, uint32_t nparts, hipStream_t s) {
+    if (nparts <= kScanPartsInline) return false;
+    hipLaunchKernelGGL(k_scan_parts, dim3(1), dim3(kThreads), 0, s, part, nparts,
+                       (uint32_t *)nullptr);
+    return true;
+}
+
 // tiles of a sort of n keys at the smaller tile size (the most control words)
 uint32_t radix_blocks_for(uint32_t n) { return ceil_div(n ? n : 1, kRadixTile); }
 
 uint32_t radix_ctl_words(uint32_t n) { return kCtlStatus + 2u * kBins * radix_blocks_for(n); }
 
+// tiles of a sort of n keys
+static uint32_t radix_tiles(uint32_t n) {
+    return ceil_div(n, n >= kRadixBigMin ? kRadixTileBig : kRadixTile);
+}
+
+RadixCount radix_count_args(uint32_t n, uint32_t *ctl) {
+    if (n <= 1 || n >= kStatAgg) return RadixCount{nullptr, nullptr, 0};
+    return RadixCount{ctl, ctl + kCtlStatus, (uint64_t)kBins * radix_tiles(n)};
+}
+
 SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
                            uint32_t *vals_alt, uint32_t n, int bits, uint32_t *ctl,
-                           uint32_t *flags, hipStream_t s) {
+                           uint32_t *flags, bool counted, hipStream_t s) {
     if (n >= kStatAgg || bits <= 0 || bits > kDigitBits * kMaxPasses) {
         // counts of 2^30 keys and more do not fit the status words: nothing
         // is sorted, and the caller's status word says so
@@ -412,10 +430,12 @@ SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
     // larger tiles for large sorts: half the look-back chain and longer digit
     // runs in the scatter, once there are enough tiles to fill the device
     const bool big = n >= kRadixBigMin;
-    const uint32_t nb = ceil_div(n, big ? kRadixTileBig : kRadixTile);
+    const uint32_t nb = radix_tiles(n);
     const int passes = std::max((bits + kDigitBits - 1) / kDigitBits, kMinPasses);
-    hipLaunchKernelGGL(k_radix_count, dim3(std::min(nb, kCountBlocks)), dim3(kCountThreads), 0, s,
-                       (const uint64_t *)keys, n, ctl, ctl + kCtlStatus, (uint64_t)kBins * nb);
+    if (!counted)
+        hipLaunchKernelGGL(k_radix_count, dim3(std::min(nb, kCountBlocks)), dim3(kCountThreads), 0,
+                           s, (const uint64_t *)keys, n, ctl, ctl + kCtlStatus,
+                           (uint64_t)kBins * nb);
     uint64_t *ka = keys, *kb = keys_alt;
     uint32_t *va = vals, *vb = vals_alt;
     for (int p = 0; p < passes; ++p) {
