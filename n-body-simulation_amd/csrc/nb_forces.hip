@@ -219,11 +219,18 @@ __device__ __forceinline__ float rsq_f32(float v) {
     return y;
 }
 
+// Four independent ones, one pair of wait states around them all.
+__device__ __forceinline__ void rsq4_f32(float (&v)[4]) {
+    asm("s_nop 0\n\tv_rsq_f32 %0, %0\n\tv_rsq_f32 %1, %1\n\tv_rsq_f32 %2, %2\n\t"
+        "v_rsq_f32 %3, %3\n\ts_nop 0"
+        : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+}
+
 __device__ inline void pair_f32(const float4 s, float px, float py, float pz, float eps2,
                                 float &fx, float &fy, float &fz) {
     const float dx = s.x - px, dy = s.y - py, dz = s.z - pz;
     const float r2 = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2)));
-    const float inv = rsq_f32(r2);
+    const float inv = __builtin_amdgcn_rsqf(r2);
     const float f = (s.w * inv) * (inv * inv);
     fx = fmaf(f, dx, fx);
     fy = fmaf(f, dy, fy);
@@ -959,6 +966,32 @@ struct GroupTree {
     const float4 *gquad;  // G*Q per internal cell (quadrupole walks)
 };
 
+// Four entries on NB points, in entry order, their v_rsq_f32 together.
+template <int NB>
+__device__ __forceinline__ void pairs4_f32(const float4 (&e)[4], const float (&rx)[NB],
+                                           const float (&ry)[NB], const float (&rz)[NB], float eps2,
+                                           float (&fx)[NB], float (&fy)[NB], float (&fz)[NB]) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        float dx[4], dy[4], dz[4], inv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            dx[u] = e[u].x - rx[b];
+            dy[u] = e[u].y - ry[b];
+            dz[u] = e[u].z - rz[b];
+            inv[u] = fmaf(dx[u], dx[u], fmaf(dy[u], dy[u], fmaf(dz[u], dz[u], eps2)));
+        }
+        rsq4_f32(inv);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const float f = (e[u].w * inv[u]) * (inv[u] * inv[u]);
+            fx[b] = fmaf(f, dx[u], fx[b]);
+            fy[b] = fmaf(f, dy[u], fy[b]);
+            fz[b] = fmaf(f, dz[u], fz[b]);
+        }
+    }
+}
+
 // The same for a stride known only at run time (lanes per body not a power
 // of two).
 __device__ __forceinline__ void flush_share_rt(const float4 *p, uint32_t stride, uint32_t t,
@@ -968,8 +1001,12 @@ __device__ __forceinline__ void flush_share_rt(const float4 *p, uint32_t stride,
     for (; k + 4 <= t; k += 4) {
         const float4 e[4] = {p[(k + 0) * stride], p[(k + 1) * stride], p[(k + 2) * stride],
                              p[(k + 3) * stride]};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) pair_f32(e[u], rx, ry, rz, eps2, fx, fy, fz);
+        const float px[1] = {rx}, py[1] = {ry}, pz[1] = {rz};
+        float gx[1] = {fx}, gy[1] = {fy}, gz[1] = {fz};
+        pairs4_f32<1>(e, px, py, pz, eps2, gx, gy, gz);
+        fx = gx[0];
+        fy = gy[0];
+        fz = gz[0];
     }
     for (; k < t; ++k) pair_f32(p[k * stride], rx, ry, rz, eps2, fx, fy, fz);
 }
@@ -987,10 +1024,7 @@ __device__ __forceinline__ void flush_share(const float4 *p, uint32_t t, const f
     for (; k + 4 <= t; k += 4) {
         const float4 e[4] = {p[(k + 0) * LPB], p[(k + 1) * LPB], p[(k + 2) * LPB],
                              p[(k + 3) * LPB]};
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int b = 0; b < NB; ++b) pair_f32(e[u], rx[b], ry[b], rz[b], eps2, fx[b], fy[b], fz[b]);
+        pairs4_f32<NB>(e, rx, ry, rz, eps2, fx, fy, fz);
     }
     for (; k < t; ++k) {
         const float4 e = p[k * LPB];
