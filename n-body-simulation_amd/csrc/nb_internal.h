@@ -288,8 +288,8 @@ __device__ inline ScanPlace scan_place(uint32_t v, const uint32_t *__restrict__ 
 }
 // Where a radix sort left its result.
 enum class SortEnd {
-    kInPlace,   // keys/vals (an even pass count, or n <= 1)
-    kInAlt,     // keys_alt/vals_alt (an odd pass count)
+    kInPlace,   // keys/vals
+    kInAlt,     // keys_alt/vals_alt
     kRejected,  // n >= 2^30 or bits outside [1, 63]: nothing sorted, kFlagSortSize raised
 };
 // Stable LSD radix sort of (key, val) pairs on key bits [0, bits), bits <= 63,
@@ -302,7 +302,7 @@ SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
                            uint32_t *flags, bool counted, hipStream_t s);
 // counted: the caller's kernel has done the sort's first step.  It adds the
 // number of keys of each lowest digit (key & (kRadixBins - 1)) to total[digit]
-// and clears plane0[0, plane_words); total is null if there is nothing to sort.
+// and clears plane0[0, plane_words); total is null if the sort needs no counts.
 constexpr uint32_t kRadixBins = 512;
 struct RadixCount {
     uint32_t *total, *plane0;

@@ -3,8 +3,8 @@
 // Both are written for 64-lane wavefronts: prefix sums use __shfl_up inside a
 // wave and LDS across the 4 waves of a 256-thread block; the radix sort ranks
 // keys stably with a 9-ballot "match any" on the 9-bit digit, so no
-// per-thread histogram is needed, and takes one launch per digit (plus one
-// counting launch per sort).  The octree build uses the scan for node
+// per-thread histogram is needed, and takes one launch per digit (small
+// and middling sorts: a launch of tiles sorted in LDS, then merges).  The octree build uses the scan for node
 // numbering and the sort for the octant keys (rocPRIM/hipCUB are not used).
 #include "nb_internal.h"
 
@@ -17,6 +17,7 @@ constexpr int kItems = kScanTile / kThreads;
 constexpr int kRadixTile = 4096;       // keys per radix tile
 constexpr int kRadixTileBig = 8192;    // keys per tile from kRadixBigMin keys on
 constexpr uint32_t kRadixBigMin = 1u << 21;
+constexpr uint32_t kSortMergeMax = 1u << 18;  // k_sort_tiles and k_merge_runs; above, passes
 constexpr int kPassThreads = 512;
 constexpr int kPassWaves = kPassThreads / 64;
 
@@ -244,6 +245,23 @@ __device__ inline bool look_back(const uint32_t *stat, uint32_t t, uint32_t d, u
     }
 }
 
+// Lanes of the wave whose digit equals the lane's own (valid lanes only): one
+// ballot per digit bit.
+__device__ __forceinline__ uint64_t digit_peers(uint32_t d, bool valid) {
+    uint64_t peers = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < kDigitBits; ++b) {
+        const bool bit = (d >> b) & 1u;
+        const uint64_t bal = __ballot(bit);
+        peers &= bit ? bal : ~bal;
+    }
+    return peers;
+}
+__device__ __forceinline__ uint64_t lanes_below() {
+    const uint32_t lane = lane_id();
+    return lane == 0 ? 0ull : (~0ull >> (64u - lane));
+}
+
 // One stable pass over digit (key >> 9 pass) & 511 of a tile of kTile
 // keys.  Wave w holds the tile's keys [w * kTile / 8, (w + 1) * kTile / 8) and
 // ranks them 64 at a time against its own digit counters, with no barrier between
@@ -303,19 +321,13 @@ __global__ void __launch_bounds__(kPassThreads) k_radix_pass(
         kk[r] = j < tn ? keys[tile + j] : ~0ull;
         vv[r] = j < tn ? vals[tile + j] : 0u;
     }
-    const uint64_t lt_mask = lane == 0 ? 0ull : (~0ull >> (64u - lane));
+    const uint64_t lt_mask = lanes_below();
 #pragma unroll
     for (int r = 0; r < kPassItems; ++r) {
         const bool valid = wbase + (uint32_t)r * 64u + lane < tn;
         const uint32_t d = (uint32_t)(kk[r] >> shift) & (kBins - 1);
         dg[r] = d;
-        uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < kDigitBits; ++b) {
-            const bool bit = (d >> b) & 1u;
-            const uint64_t bal = __ballot(bit);
-            peers &= bit ? bal : ~bal;
-        }
+        const uint64_t peers = digit_peers(d, valid);
         const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
         // a wave's LDS accesses complete in order: the next round reads this write
         const uint32_t before = wcnt[w][d];
@@ -380,6 +392,252 @@ __global__ void __launch_bounds__(kPassThreads) k_radix_pass(
     }
 }
 
+// ---- small and middling sorts ---------------------------------------------------
+// A pass over a few tiles is all latency: of 9.2 us in the kernel (100,003 keys,
+// 25 tiles of 4096) ranking takes 2.6 us, the look-back 1.9, two scans behind a
+// load 2.1, a tile id 0.7, and a launch comes on top, seven times.  So up to
+// kSortMergeMax keys are sorted otherwise: one launch in which every workgroup
+// sorts a tile of up to 2048 keys in LDS, all passes (k_sort_tiles), then one
+// launch per factor of eight that merges eight runs into one (k_merge_runs).
+//
+// A merged key's place is its own index plus, for each of the other seven runs,
+// the number of keys there that come before it.  Equal keys keep the order of
+// their runs, so the sort is stable.
+//
+// Whole sorts: 1024 keys 51 us in passes, 13.4 here; 100,003: 84 and 50; 262,144:
+// 27 us less here; 400,000 and 524,288: within 3 us of each other; 1,048,576: 80 us
+// more (a merge reads every key eight times over), hence the limit.
+template <int kItems_>
+__global__ void __launch_bounds__(1024) k_sort_tiles(
+    const uint64_t *__restrict__ keys, const uint32_t *__restrict__ vals,
+    uint64_t *__restrict__ okeys, uint32_t *__restrict__ ovals, uint32_t total, int passes) {
+    constexpr uint32_t waves = 16;
+    __shared__ uint32_t wcnt[waves][kBins];  // digit-d keys of wave w, then those of earlier waves
+    __shared__ uint32_t dbase[kBins];
+    __shared__ uint32_t ws[kBins / 64];
+    __shared__ uint64_t lk[1024 * kItems_];
+    __shared__ uint32_t lv[1024 * kItems_];
+    const uint32_t tid = threadIdx.x, w = tid >> 6;
+    const uint32_t j0 = w * (64u * kItems_) + lane_id();
+    const uint32_t tile = blockIdx.x * (1024u * kItems_);
+    const uint32_t n = min(total - tile, 1024u * kItems_);  // keys of this tile
+    keys += tile;
+    vals += tile;
+    okeys += tile;
+    ovals += tile;
+    uint64_t kk[kItems_];
+    uint32_t vv[kItems_], dg[kItems_], rk[kItems_];
+#pragma unroll
+    for (int r = 0; r < kItems_; ++r) {
+        const uint32_t j = j0 + 64u * r;
+        kk[r] = j < n ? keys[j] : ~0ull;
+        vv[r] = j < n ? vals[j] : 0u;
+    }
+    const uint64_t lt_mask = lanes_below();
+    for (int pass = 0; pass < passes; ++pass) {
+        const int shift = kDigitBits * pass;
+        for (uint32_t i = tid; i < waves * kBins; i += 1024) (&wcnt[0][0])[i] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kItems_; ++r) {
+            const bool valid = j0 + 64u * r < n;
+            const uint32_t d = (uint32_t)(kk[r] >> shift) & (kBins - 1);
+            const uint64_t peers = digit_peers(d, valid);
+            const uint32_t rank = (uint32_t)__popcll(peers & lt_mask);
+            // a wave's LDS accesses complete in order: the next round reads this write
+            const uint32_t before = wcnt[w][d];
+            dg[r] = d;
+            rk[r] = before + rank;
+            if (valid && rank == 0) wcnt[w][d] = before + (uint32_t)__popcll(peers);
+        }
+        __syncthreads();
+        uint32_t c = 0, inc = 0;
+        if (tid < kBins) {
+            uint32_t cnt[waves];
+#pragma unroll
+            for (uint32_t k = 0; k < waves; ++k) cnt[k] = wcnt[k][tid];
+#pragma unroll
+            for (uint32_t k = 0; k < waves; ++k) {
+                wcnt[k][tid] = c;
+                c += cnt[k];
+            }
+            inc = wave_inclusive_scan(c);
+            if (lane_id() == 63) ws[w] = inc;
+        }
+        __syncthreads();
+        if (tid < kBins) {
+            uint32_t ex = inc - c;
+#pragma unroll
+            for (uint32_t k = 0; k < kBins / 64; ++k) ex += k < w ? ws[k] : 0u;
+            dbase[tid] = ex;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kItems_; ++r) {
+            if (j0 + 64u * r < n) {
+                const uint32_t p = dbase[dg[r]] + wcnt[w][dg[r]] + rk[r];
+                lk[p] = kk[r];
+                lv[p] = vv[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kItems_; ++r) {
+            const uint32_t j = j0 + 64u * r;
+            if (j < n) {
+                kk[r] = lk[j];
+                vv[r] = lv[j];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kItems_; ++r) {
+        const uint32_t j = j0 + 64u * r;
+        if (j < n) {
+            okeys[j] = kk[r];
+            ovals[j] = vv[r];
+        }
+    }
+}
+
+constexpr int kMergeThreads = 256;
+constexpr uint32_t kMergeRuns = 8;
+constexpr uint32_t kMergeLds = 4096;  // keys of the other runs held in LDS
+// Does a key of run q come before key (of run own)?  Equal keys keep the order
+// of their runs.
+__device__ __forceinline__ bool merge_before(uint64_t other, uint32_t q, uint64_t key, uint32_t own) {
+    return q < own ? other <= key : other < key;
+}
+
+// A workgroup places kMergeThreads consecutive keys of one run.  Its first and
+// last key bound the places of all of them in each other run: a wave finds the
+// bounds with 64 probes at a time (two or three dependent loads instead of a
+// dozen).  The keys between the bounds, about kMergeThreads per run, then go to
+// LDS, where every thread bisects.  If they are more than kMergeLds (a short last
+// run, or runs of unlike ranges), every 2nd, 4th, ... goes there instead, and the
+// last steps of the bisection read global memory.
+// run: keys per sorted run (a power of two, a multiple of kMergeThreads); mask: the
+// key bits that the runs are sorted by.
+__global__ void __launch_bounds__(kMergeThreads) k_merge_runs(
+    const uint64_t *__restrict__ keys, const uint32_t *__restrict__ vals,
+    uint64_t *__restrict__ okeys, uint32_t *__restrict__ ovals, uint32_t n, uint32_t run,
+    uint64_t mask) {
+    constexpr uint32_t waves = kMergeThreads / 64, per = kMergeRuns / waves;
+    __shared__ uint64_t win[kMergeLds];
+    __shared__ uint32_t bound[2][kMergeRuns];
+    const uint32_t t = threadIdx.x, lane = lane_id(), w = t >> 6;
+    const uint32_t i0 = blockIdx.x * kMergeThreads;
+    const uint32_t i1 = min(n, i0 + kMergeThreads) - 1;    // last key
+    const uint32_t own = i0 / run;                          // this workgroup's run
+    const uint32_t first = own / kMergeRuns * kMergeRuns;   // first run of its eight
+    const uint32_t i = min(i0 + t, i1);
+    const uint64_t full = keys[i], key = full & mask;
+    const uint32_t val = vals[i];
+    const uint64_t end_key[2] = {keys[i0] & mask, keys[i1] & mask};
+    // the wave's runs, both ends: lo keys are known to come before, the next rem
+    // are open
+    uint32_t lo[2 * per], rem[2 * per];
+#pragma unroll
+    for (uint32_t k = 0; k < 2 * per; ++k) {
+        const uint32_t q = first + w * per + (k >> 1);
+        const uint64_t begin = (uint64_t)q * run;
+        lo[k] = 0;
+        rem[k] = q == own || begin >= n ? 0u : (uint32_t)min((uint64_t)run, n - begin);
+    }
+    for (;;) {
+        bool open = false;
+        uint64_t probe[2 * per];
+        uint32_t stride[2 * per];
+#pragma unroll
+        for (uint32_t k = 0; k < 2 * per; ++k) {
+            const uint64_t begin = (uint64_t)(first + w * per + (k >> 1)) * run;
+            stride[k] = (rem[k] + 63) / 64;
+            open |= rem[k] != 0;
+            const uint32_t p = (lane + 1) * stride[k] - 1;  // unused if rem is 0
+            probe[k] = rem[k] && p < rem[k] ? keys[begin + lo[k] + p] & mask : ~0ull;
+        }
+        if (!open) break;  // the same for the whole wave
+#pragma unroll
+        for (uint32_t k = 0; k < 2 * per; ++k) {
+            const uint32_t q = first + w * per + (k >> 1);
+            const bool in = rem[k] && (lane + 1) * stride[k] - 1 < rem[k];
+            const uint32_t c =
+                (uint32_t)__popcll(__ballot(in && merge_before(probe[k], q, end_key[k & 1], own)));
+            const uint32_t done = c * stride[k];
+            lo[k] += done;
+            rem[k] = rem[k] ? min(stride[k] - 1, rem[k] - done) : 0u;
+        }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < 2 * per; ++k)
+        if (lane == 0) bound[k & 1][w * per + (k >> 1)] = lo[k];
+    __syncthreads();
+    uint32_t lower[kMergeRuns], cnt[kMergeRuns], at[kMergeRuns + 1], most = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < kMergeRuns; ++q) {
+        lower[q] = bound[0][q];
+        cnt[q] = bound[1][q] - lower[q];
+        most = max(most, cnt[q]);
+    }
+    uint32_t thin = 0;  // LDS holds the last of every 2^thin keys
+    for (;; ++thin) {
+        at[0] = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < kMergeRuns; ++q) at[q + 1] = at[q] + (cnt[q] >> thin);
+        if (at[kMergeRuns] <= kMergeLds) break;
+    }
+    // key p (from 0) between run q's bounds
+    const auto key_at = [&](uint32_t q, uint32_t p) {
+        const uint64_t src = (uint64_t)(first + q) * run + lower[q] + p;
+        return src < n ? keys[src] & mask : ~0ull;
+    };
+    constexpr int kAhead = 8;  // loads in flight per thread
+    for (uint32_t j0 = t; j0 < at[kMergeRuns]; j0 += kAhead * kMergeThreads) {
+        uint64_t v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t j = min(j0 + u * kMergeThreads, at[kMergeRuns] - 1);
+            uint64_t src = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < kMergeRuns; ++q)
+                if (j >= at[q])
+                    src = (uint64_t)(first + q) * run + lower[q] + ((j - at[q] + 1) << thin) - 1;
+            v[u] = keys[src] & mask;
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (j0 + u * kMergeThreads < at[kMergeRuns]) win[j0 + u * kMergeThreads] = v[u];
+    }
+    __syncthreads();
+    uint32_t before[kMergeRuns];
+#pragma unroll
+    for (uint32_t q = 0; q < kMergeRuns; ++q) before[q] = 0;
+    const auto bisect = [&](uint32_t step, uint32_t stop, auto load) {
+        for (; step >= stop; step >>= 1) {
+            uint64_t v[kMergeRuns];
+#pragma unroll
+            for (uint32_t q = 0; q < kMergeRuns; ++q) v[q] = load(q, before[q] + step - 1);
+#pragma unroll
+            for (uint32_t q = 0; q < kMergeRuns; ++q)
+                if (before[q] + step <= cnt[q] && merge_before(v[q], first + q, key, own))
+                    before[q] += step;
+        }
+        return step;
+    };
+    uint32_t step = most ? 1u << (31 - __clz((int)most)) : 0u;
+    if (step >> thin)
+        step = bisect(step, 1u << thin, [&](uint32_t q, uint32_t p) {
+            return win[min(at[q] + (p >> thin), kMergeLds - 1)];
+        });
+    if (thin) bisect(step, 1u, key_at);
+    if (i0 + t > i1) return;
+    uint32_t pos = first * run + (i - own * run);
+#pragma unroll
+    for (uint32_t q = 0; q < kMergeRuns; ++q) pos += lower[q] + before[q];
+    okeys[pos] = full;
+    ovals[pos] = val;
+}
+
 }  // namespace
 
 uint32_t scan_scratch_words(uint32_t n) { return ceil_div(n ? n : 1, kScanTile) + 1; }
@@ -413,7 +671,7 @@ static uint32_t radix_tiles(uint32_t n) {
 }
 
 RadixCount radix_count_args(uint32_t n, uint32_t *ctl) {
-    if (n <= 1 || n >= kStatAgg) return RadixCount{nullptr, nullptr, 0};
+    if (n <= kSortMergeMax || n >= kStatAgg) return RadixCount{nullptr, nullptr, 0};
     return RadixCount{ctl, ctl + kCtlStatus, (uint64_t)kBins * radix_tiles(n)};
 }
 
@@ -427,17 +685,33 @@ SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
         return SortEnd::kRejected;
     }
     if (n <= 1) return SortEnd::kInPlace;
+    const int passes = std::max((bits + kDigitBits - 1) / kDigitBits, kMinPasses);
+    uint64_t *ka = keys, *kb = keys_alt;
+    uint32_t *va = vals, *vb = vals_alt;
+    if (n <= kSortMergeMax) {
+        const uint32_t tile = n <= 1024 ? 1024 : 2048;
+        hipLaunchKernelGGL(n <= 1024 ? k_sort_tiles<1> : k_sort_tiles<2>, dim3(ceil_div(n, tile)),
+                           dim3(1024), 0, s, (const uint64_t *)ka, (const uint32_t *)va, kb, vb, n,
+                           passes);
+        std::swap(ka, kb);
+        std::swap(va, vb);
+        const uint64_t mask = ~0ull >> (64 - std::min(64, kDigitBits * passes));
+        for (uint32_t run = tile; run < n; run *= kMergeRuns) {
+            hipLaunchKernelGGL(k_merge_runs, dim3(ceil_div(n, kMergeThreads)), dim3(kMergeThreads),
+                               0, s, (const uint64_t *)ka, (const uint32_t *)va, kb, vb, n, run, mask);
+            std::swap(ka, kb);
+            std::swap(va, vb);
+        }
+        return ka == keys ? SortEnd::kInPlace : SortEnd::kInAlt;
+    }
     // larger tiles for large sorts: half the look-back chain and longer digit
     // runs in the scatter, once there are enough tiles to fill the device
     const bool big = n >= kRadixBigMin;
     const uint32_t nb = radix_tiles(n);
-    const int passes = std::max((bits + kDigitBits - 1) / kDigitBits, kMinPasses);
     if (!counted)
         hipLaunchKernelGGL(k_radix_count, dim3(std::min(nb, kCountBlocks)), dim3(kCountThreads), 0,
                            s, (const uint64_t *)keys, n, ctl, ctl + kCtlStatus,
                            (uint64_t)kBins * nb);
-    uint64_t *ka = keys, *kb = keys_alt;
-    uint32_t *va = vals, *vb = vals_alt;
     for (int p = 0; p < passes; ++p) {
         if (big)
             hipLaunchKernelGGL(k_radix_pass<kRadixTileBig>, dim3(nb), dim3(kPassThreads), 0, s,
@@ -447,8 +721,8 @@ SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
             hipLaunchKernelGGL(k_radix_pass<kRadixTile>, dim3(nb), dim3(kPassThreads), 0, s,
                                (const uint64_t *)ka, (const uint32_t *)va, kb, vb, n, p, passes,
                                ctl, nb, flags);
-        uint64_t *tk = ka; ka = kb; kb = tk;
-        uint32_t *tv = va; va = vb; vb = tv;
+        std::swap(ka, kb);
+        std::swap(va, vb);
     }
     // an odd count ends in the scratch buffers
     return (passes & 1) ? SortEnd::kInAlt : SortEnd::kInPlace;

@@ -376,6 +376,39 @@ def test_tree_block_edges(gpu, oracle, kind, n):
         assert_canonical_equal(c.tree_canonical(), t.canonical(), f"{kind} n={n}")
 
 
+# Sorts by merging (runs of 2048 keys, then 16,384 and 131,072): a short last
+# run, one key over, the largest such sort and the first by passes.  Bodies
+# already in key order, and in its reverse, leave runs that do not overlap;
+# "blocks" repeats a few positions' neighbourhoods so that one run's keys bound
+# whole other runs (more keys between the bounds than fit the LDS).
+@pytest.mark.parametrize("kind,n,order", [("plummer", 16384, "input"), ("cube", 16385, "input"),
+                                          ("plummer", 20480, "sorted"), ("cube", 34000, "reversed"),
+                                          ("plummer", 50001, "blocks"),
+                                          ("plummer", 131329, "blocks"),
+                                          ("disk", 262144, "input"), ("cube", 262145, "reversed")])
+def test_tree_merge_sort_edges(gpu, oracle, kind, n, order):
+    d = make(gpu, kind, n, seed=n)
+    t = oracle.Tree(n)
+    t.build(d["x"], d["y"], d["z"], d["m"])
+    perm = np.arange(n)
+    if order != "input":
+        perm = np.asarray(t.export()["sorted"]).astype(np.int64)
+        if order == "reversed":
+            perm = perm[::-1]
+        elif order == "blocks":  # every third run thinly spread, the others dense
+            thin = perm[::3]
+            rest = np.setdiff1d(perm, thin, assume_unique=True)
+            perm = np.concatenate([rest[:n // 2], thin, rest[n // 2:]])
+        d = {k: np.ascontiguousarray(v[perm]) for k, v in d.items()}
+        t = oracle.Tree(n)
+        t.build(d["x"], d["y"], d["z"], d["m"])
+    with ctx_for(gpu, d) as c:
+        for _ in range(2):
+            c.bh_build()
+            np.testing.assert_array_equal(c.tree_sorted(), t.export()["sorted"])
+        assert_canonical_equal(c.tree_canonical(), t.canonical(), f"{kind} n={n} {order}")
+
+
 def test_tree_deep_runs(gpu, oracle):
     # pairs of bodies closer than edge/2^21 force the 42-digit path
     rng = np.random.default_rng(3)
