@@ -20,7 +20,7 @@ namespace nb {
 
 constexpr int kKeyLevels = 21;  // octant digits held by one 63-bit key word
 constexpr int kMaxDepth = 42;   // two key words
-constexpr int kAabbBlocks = 256;
+constexpr int kAabbBlocks = 512;
 
 // device status bits, turned into NB_E_* codes by the host
 enum : uint32_t {

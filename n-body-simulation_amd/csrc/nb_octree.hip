@@ -53,9 +53,8 @@ __device__ inline void raise_flag(TreeHdr *h, uint32_t f) { atomicOr(&h->status,
 // Block partial extrema.  Like the reference's partials (BarnesHutOctree.cpp:
 // 58-72, value-initialised to 0.0) every partial starts at the origin.  A
 // seventh value says whether the block met a position that is not finite.
-constexpr int kAabbThreads = 1024;
+constexpr int kAabbThreads = 256;
 constexpr int kAabbVals = 7;
-static_assert(kAabbBlocks <= kAabbThreads, "the final reduction reads one partial per thread");
 struct Extents {
     double mn[3] = {0.0, 0.0, 0.0}, mx[3] = {0.0, 0.0, 0.0};
     bool bad = false;
@@ -73,36 +72,13 @@ __device__ inline void wave_extents(Extents &e) {
     e.bad = __any(e.bad);
 }
 
-// The workgroup's extents, from every thread's, into out[0..7) (LDS or global,
-// `stride` apart): min x y z, max x y z, bad.
-__device__ inline void block_extents(Extents e, double (*sh)[kAabbVals], double *out,
-                                     uint32_t stride) {
-    wave_extents(e);
-    const uint32_t w = threadIdx.x >> 6, waves = blockDim.x >> 6;
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            sh[w][c] = e.mn[c];
-            sh[w][3 + c] = e.mx[c];
-        }
-        sh[w][6] = e.bad ? 1.0 : 0.0;
-    }
-    __syncthreads();
-    if (threadIdx.x < kAabbVals) {
-        double v = sh[0][threadIdx.x];
-        for (uint32_t k = 1; k < waves; ++k)
-            v = threadIdx.x < 3 ? sycl_min(v, sh[k][threadIdx.x]) : sycl_max(v, sh[k][threadIdx.x]);
-        out[(uint64_t)threadIdx.x * stride] = v;
-    }
-}
-
 __global__ void __launch_bounds__(kAabbThreads) k_aabb_partial(const double *__restrict__ x,
                                                                const double *__restrict__ y,
                                                                const double *__restrict__ z,
                                                                uint32_t n, double *part) {
     __shared__ double sh[kAabbThreads / 64][kAabbVals];
     Extents e;
-#pragma unroll 4
+#pragma unroll 8
     for (uint64_t i = (uint64_t)blockIdx.x * kAabbThreads + threadIdx.x; i < n;
          i += (uint64_t)gridDim.x * kAabbThreads) {
         const double p[3] = {x[i], y[i], z[i]};
@@ -113,7 +89,24 @@ __global__ void __launch_bounds__(kAabbThreads) k_aabb_partial(const double *__r
             e.mx[c] = sycl_max(e.mx[c], p[c]);
         }
     }
-    block_extents(e, sh, part + blockIdx.x, gridDim.x);
+    wave_extents(e);
+    const int w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            sh[w][c] = e.mn[c];
+            sh[w][3 + c] = e.mx[c];
+        }
+        sh[w][6] = e.bad ? 1.0 : 0.0;
+    }
+    __syncthreads();
+    const uint32_t c = threadIdx.x;
+    if (c < kAabbVals) {
+        double v = sh[0][c];
+        for (int k = 1; k < kAabbThreads / 64; ++k)
+            v = c < 3 ? sycl_min(v, sh[k][c]) : sycl_max(v, sh[k][c]);
+        part[(uint64_t)c * gridDim.x + blockIdx.x] = v;
+    }
 }
 
 // Cubify the extents ext = {min_x, min_y, min_z, max_x, max_y, max_z}
@@ -173,8 +166,8 @@ __device__ inline uint64_t key_from(Cell &c, double px, double py, double pz) {
 // Keys, identity permutation, and the packed body record {x, y, z, m} that
 // the centre-of-mass and node-record passes gather (one 32-byte load).  Small
 // jobs ride along, each of which took a launch of its own (3 to 5 us): every
-// workgroup finds the root cube from the partial extents (at most kAabbBlocks
-// of each, one per thread), the first one resets the header, and the sort's
+// workgroup's first wave finds the root cube from the partial extents (at most
+// kAabbBlocks of each), the first workgroup resets the header, and the sort's
 // first digit is counted.  So there are at most 256 workgroups, which take
 // their bodies in strides.
 constexpr int kKeyThreads = 1024;
@@ -184,37 +177,41 @@ __global__ void __launch_bounds__(kKeyThreads) k_keys(
     const double *__restrict__ m, uint32_t n, const double *__restrict__ part, uint32_t np,
     TreeHdr *h, uint64_t *skey, uint32_t *sidx, double4 *body4, uint32_t *scan_part,
     uint32_t scan_parts, RadixCount rc) {
-    __shared__ double sh[kKeyThreads / 64][kAabbVals];
-    __shared__ double ext[kAabbVals];
     __shared__ RootCube root;
     __shared__ uint32_t hist[kRadixBins];
     const uint32_t t = threadIdx.x;
-    Extents e;
-    if (t < np) {
+    if (t < 64) {
+        Extents e;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            e.mn[c] = part[(uint64_t)c * np + t];
-            e.mx[c] = part[(uint64_t)(3 + c) * np + t];
+        for (int k = 0; k < kAabbBlocks / 64; ++k) {
+            const uint32_t p = t + 64u * k;
+            if (p >= np) break;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                e.mn[c] = sycl_min(e.mn[c], part[(uint64_t)c * np + p]);
+                e.mx[c] = sycl_max(e.mx[c], part[(uint64_t)(3 + c) * np + p]);
+            }
+            e.bad |= part[6ull * np + p] != 0.0;
         }
-        e.bad = part[6ull * np + t] != 0.0;
+        wave_extents(e);
+        const double ext[6] = {e.mn[0], e.mn[1], e.mn[2], e.mx[0], e.mx[1], e.mx[2]};
+        const RootCube r = cubify(ext);
+        if (t == 0) {
+            root = r;
+            if (blockIdx.x == 0) {
+                store_cube(h, r);
+                h->internal_count = 0;
+                h->max_depth = 0;
+                h->status = e.bad || !r.ok ? kFlagAabb : 0u;
+                h->deep_runs = 0;
+                h->stack_peak = 0;
+                h->group_count = 0;
+                h->group_next = 0;
+                h->cross_count = 0;
+            }
+        }
     }
     if (t < kRadixBins) hist[t] = 0;
-    block_extents(e, sh, ext, 1);
-    __syncthreads();
-    if (t == 0) {
-        root = cubify(ext);
-        if (blockIdx.x == 0) {
-            store_cube(h, root);
-            h->internal_count = 0;
-            h->max_depth = 0;
-            h->status = ext[6] != 0.0 || !root.ok ? kFlagAabb : 0u;
-            h->deep_runs = 0;
-            h->stack_peak = 0;
-            h->group_count = 0;
-            h->group_next = 0;
-            h->cross_count = 0;
-        }
-    }
     __syncthreads();
     const uint64_t stride = (uint64_t)gridDim.x * kKeyThreads;
     const uint64_t i0 = (uint64_t)blockIdx.x * kKeyThreads + t;
@@ -408,13 +405,24 @@ __global__ void __launch_bounds__(kThreads) k_max_depth(const int32_t *__restric
 }
 
 // ---- 6. topology --------------------------------------------------------------
-// The sorted keys as the topology pass reads them.  `win` (optional) holds
-// skey[w0, w1) in LDS: the searches of one block stay mostly inside it.
+// The sorted keys, pairs' lcp and cell numbers as the topology pass reads them.
+// A window [w0, w1) of each sits in LDS: the searches of one block stay mostly
+// inside it, and the memory latencies of keys, lcp and numbers overlap.
 struct KeyView {
     const uint64_t *skey;
     const uint64_t *klo;
-    const uint64_t *win = nullptr;
-    uint32_t w0 = 0, w1 = 0;
+    const int32_t *lcp;
+    const uint32_t *off;
+    const uint64_t *win;
+    const int32_t *wlcp;
+    const uint32_t *woff;
+    uint32_t w0, w1;
+    __device__ inline int lcp_of(uint32_t p) const {
+        return p - w0 < w1 - w0 ? wlcp[p - w0] : lcp[p];
+    }
+    __device__ inline uint32_t off_of(uint32_t p) const {
+        return p - w0 < w1 - w0 ? woff[p - w0] : off[p];
+    }
     __device__ inline uint64_t key(uint32_t p) const {
         return p - w0 < w1 - w0 ? win[p - w0] : skey[p];
     }
@@ -428,6 +436,13 @@ struct KeyView {
         const uint64_t kp = key(p), kq = key(q);
         if (v <= kKeyLevels) return ((kp ^ kq) >> (63 - 3 * v)) == 0;
         return kp == kq && ((klo[p] ^ klo[q]) >> (63 - 3 * (v - kKeyLevels))) == 0;
+    }
+    // does the key kn of sorted body p share its first v digits with body q's?
+    __device__ inline bool same_key(uint64_t kn, uint32_t p, uint32_t q, int v) const {
+        if (v <= 0) return true;
+        const uint64_t kq = key(q);
+        if (v <= kKeyLevels) return ((kn ^ kq) >> (63 - 3 * v)) == 0;
+        return kn == kq && ((klo[p] ^ klo[q]) >> (63 - 3 * (v - kKeyLevels))) == 0;
     }
     // first sorted position of the depth-v cell that holds sorted body i
     __device__ inline uint32_t cell_start(uint32_t i, int v) const {
@@ -461,8 +476,7 @@ struct KeyView {
 // and 0 if not.
 // No atomics: every cell, node slot and table entry has exactly one writer.
 __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h, KeyView kv,
-                               const uint32_t *__restrict__ sidx, const int32_t *__restrict__ lcp,
-                               const uint32_t *__restrict__ off, int32_t *ref, uint8_t *int_depth,
+                               const uint32_t *__restrict__ sidx, int32_t *ref, uint8_t *int_depth,
                                uint32_t *int_node, uint32_t *body_node,
                                uint8_t *int_local, uint32_t *spanning, uint32_t spanning_cap,
                                uint32_t *int_first, uint32_t com_block, uint32_t com_super) {
@@ -471,15 +485,26 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
         body_node[0] = 0;
         return;
     }
-    const int cp = i > 0 ? lcp[i - 1] : -1;
-    const int cn = i + 1 < n ? lcp[i] : -1;
-    auto owner_index = [&](uint32_t a, int v) -> uint32_t {
-        const int ca = a > 0 ? lcp[a - 1] : -1;
-        return off[a] + (uint32_t)(v - ca - 1);
-    };
+    // the next block's and super-block's first keys, read before they are needed
+    const uint32_t next_block = (i / com_block + 1) * com_block;
+    const uint32_t next_super = (i / com_super + 1) * com_super;
+    const uint64_t key_block = kv.skey[min(next_block, n - 1)];
+    const uint64_t key_super = kv.skey[min(next_super, n - 1)];
+    const uint32_t body = sidx[i];
+    const int cp = i > 0 ? kv.lcp_of(i - 1) : -1;
+    const int cn = i + 1 < n ? kv.lcp_of(i) : -1;
+    // One search serves every body: the depth-cp cell that holds it holds the top
+    // of pair i's chain, or, without a chain, the body's leaf.
+    uint32_t up = 0;  // that cell's number
+    if (cp >= 0) {
+        const uint32_t a = kv.cell_start(i, cp);
+        const int ca = a > 0 ? kv.lcp_of(a - 1) : -1;
+        up = kv.off_of(a) + (uint32_t)(cp - ca - 1);
+    }
+    const uint32_t own = cn > cp ? kv.off_of(i) : 0u;  // the chain's first cell
     // internal cells owned by pair i: depths cp+1 .. cn
     for (int l = cp + 1; l <= cn; ++l) {
-        const uint32_t k = off[i] + (uint32_t)(l - cp - 1);
+        const uint32_t k = own + (uint32_t)(l - cp - 1);
         if (k >= icap) {
             raise_flag(h, kFlagNodeOverflow);
             break;
@@ -488,14 +513,12 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
         int_first[k] = i;
         // The cell's bodies start at i; it crosses into the next COM block iff
         // that block's first body shares its l-digit prefix with body i.
-        const uint32_t next_block = (i / com_block + 1) * com_block;
-        const bool local = !(next_block < n && kv.same(next_block, i, l));
+        const bool local = !(next_block < n && kv.same_key(key_block, next_block, i, l));
         if (local) {
             int_local[k] = 1;
         } else {
             // the same test at the next super-block boundary
-            const uint32_t next_super = (i / com_super + 1) * com_super;
-            const bool cross = next_super < n && kv.same(next_super, i, l);
+            const bool cross = next_super < n && kv.same_key(key_super, next_super, i, l);
             int_local[k] = cross ? 2 : 0;
             // the block of body i owns at most one crossing cell per depth:
             // the depth-l cell holding the block's last and the next block's
@@ -509,7 +532,7 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
             ref[0] = (int32_t)k;
             continue;
         }
-        const uint32_t pk = l > cp + 1 ? k - 1 : owner_index(kv.cell_start(i, cp), cp);
+        const uint32_t pk = l > cp + 1 ? k - 1 : up;
         if (pk >= icap) {
             raise_flag(h, kFlagNodeOverflow);
             break;
@@ -520,41 +543,71 @@ __device__ inline void link_at(uint32_t i, uint32_t n, uint32_t icap, TreeHdr *h
     }
     // the body's leaf: one level below the deepest cell it shares with a neighbour
     const int D = cp > cn ? cp : cn;
-    const uint32_t pk = owner_index(kv.cell_start(i, D), D);
+    const uint32_t pk = cn > cp ? own + (uint32_t)(cn - cp - 1) : up;
     if (pk >= icap) {
         raise_flag(h, kFlagNodeOverflow);
         body_node[i] = 0xffffffffu;
         return;
     }
     const uint32_t leaf = 1u + 8u * pk + kv.digit(i, D);
-    ref[leaf] = ref_of_body(sidx[i]);
+    ref[leaf] = ref_of_body(body);
     body_node[i] = leaf;
     // the deepest leaf, 1 + max lcp, is taken from the lcp array (max_depth_of)
 }
 
-constexpr uint32_t kLinkBack = 768;  // keys before a link block's own kept in LDS
+constexpr uint32_t kLinkBack = 768;  // entries before a link block's own kept in LDS
+// Loads the window of the block at b0: its kThreads entries and kLinkBack before
+// them, all loads in flight together.  kv's arrays and window are absolute here.
+// (The last pair's lcp and number, and those of one body, are never written:
+// what is loaded for them is not used.)
+__device__ __forceinline__ void link_window(KeyView &kv, uint32_t b0, uint32_t n) {
+    constexpr int rounds = (kLinkBack + kThreads) / kThreads;
+    static_assert(kLinkBack % kThreads == 0, "whole rounds");
+    __shared__ uint64_t win[kLinkBack + kThreads];
+    __shared__ int32_t wlcp[kLinkBack + kThreads];
+    __shared__ uint32_t woff[kLinkBack + kThreads];
+    const uint32_t w0 = b0 > kLinkBack ? b0 - kLinkBack : 0u;
+    const uint32_t w1 = min(n, b0 + (uint32_t)kThreads);
+    uint64_t k[rounds];
+    int32_t l[rounds];
+    uint32_t o[rounds];
+#pragma unroll
+    for (int r = 0; r < rounds; ++r) {
+        const uint32_t p = min(w0 + threadIdx.x + (uint32_t)r * kThreads, w1 - 1);
+        k[r] = kv.skey[p];
+        l[r] = kv.lcp[p];
+        o[r] = kv.off[p];
+    }
+#pragma unroll
+    for (int r = 0; r < rounds; ++r) {
+        const uint32_t j = threadIdx.x + (uint32_t)r * kThreads;
+        win[j] = k[r];
+        wlcp[j] = l[r];
+        woff[j] = o[r];
+    }
+    __syncthreads();
+    kv.win = win;
+    kv.wlcp = wlcp;
+    kv.woff = woff;
+    kv.w0 = w0;
+    kv.w1 = w1;
+}
+
+// Latency again: memory round trips and the search.  1024 bodies 10.7 us with two
+// searches per body and keys alone in LDS, 7.7 now; 100,003: 18.8 and 12.9;
+// 4,194,304: 149 and 117; the ensemble's 96 and 70.
 __global__ void __launch_bounds__(kThreads) k_link(uint32_t n, uint32_t icap, TreeHdr *h,
                                                    KeyView kv, const uint32_t *__restrict__ sidx,
-                                                   const int32_t *__restrict__ lcp,
-                                                   const uint32_t *__restrict__ off,
                                                    int32_t *ref, uint8_t *int_depth,
                                                    uint32_t *int_node, uint32_t *body_node,
                                                    uint8_t *int_local,
                                                    uint32_t *spanning, uint32_t spanning_cap,
                                                    uint32_t *int_first) {
-    // the block's keys and kLinkBack before them in LDS
-    __shared__ uint64_t win[kLinkBack + kThreads];
     const uint32_t b0 = blockIdx.x * kThreads;
-    const uint32_t w0 = b0 > kLinkBack ? b0 - kLinkBack : 0u;
-    const uint32_t w1 = min(n, b0 + (uint32_t)kThreads);
-    for (uint32_t p = w0 + threadIdx.x; p < w1; p += kThreads) win[p - w0] = kv.skey[p];
-    __syncthreads();
-    kv.win = win;
-    kv.w0 = w0;
-    kv.w1 = w1;
+    link_window(kv, b0, n);
     const uint32_t i = b0 + threadIdx.x;
     if (i >= n) return;
-    link_at(i, n, icap, h, kv, sidx, lcp, off, ref, int_depth, int_node, body_node,
+    link_at(i, n, icap, h, kv, sidx, ref, int_depth, int_node, body_node,
             int_local, spanning, spanning_cap, int_first, kComBlock, kComSuper);
 }
 
@@ -1622,26 +1675,25 @@ __global__ void __launch_bounds__(kThreads) k_forest_link(uint32_t slots,
                                                           const uint16_t *__restrict__ fb_sys,
                                                           const EnsSystem *__restrict__ sys,
                                                           ForestBufs fb) {
-    __shared__ uint64_t win[kLinkBack + kThreads];
     const uint32_t b0 = blockIdx.x * kThreads;
-    const uint32_t w0 = b0 > kLinkBack ? b0 - kLinkBack : 0u;
-    const uint32_t w1 = min(slots, b0 + (uint32_t)kThreads);
-    for (uint32_t p = w0 + threadIdx.x; p < w1; p += kThreads) win[p - w0] = fb.skey[p];
-    __syncthreads();
+    KeyView kv{fb.skey, fb.klo, fb.lcp, fb.chain};
+    link_window(kv, b0, slots);
     const uint32_t j = b0 + threadIdx.x;
     if (j >= slots) return;
     const SlotSys ss = slot_sys(j, fb_sys, sys);
     const EnsSystem &S = ss.S;
     if (!S.bh || ss.li >= S.n) return;
     const uint32_t fo = S.fb_off, io = S.int_off;
-    KeyView kv{fb.skey + fo, fb.klo + fo};
-    // window bounds relative to the system's first slot; the unsigned
-    // differences in KeyView::key place a position in or out of the window
-    // correctly also when the window starts before the system
-    kv.win = win;
-    kv.w0 = w0 - fo;
-    kv.w1 = w1 - fo;
-    link_at(ss.li, S.n, S.icap, fb.hdr + ss.s, kv, fb.sidx + fo, fb.lcp + fo, fb.chain + fo,
+    // arrays and window bounds relative to the system's first slot; the unsigned
+    // differences in KeyView place a position in or out of the window correctly
+    // also when the window starts before the system
+    kv.skey += fo;
+    kv.klo += fo;
+    kv.lcp += fo;
+    kv.off += fo;
+    kv.w0 -= fo;
+    kv.w1 -= fo;
+    link_at(ss.li, S.n, S.icap, fb.hdr + ss.s, kv, fb.sidx + fo,
             fb.ref + S.node_off, fb.int_depth + io, fb.int_node + io,
             fb.body_node + fo, fb.int_local + io, fb.spanning + S.span_off,
             kMaxDepth * ((S.n + kComBlock - 1) / kComBlock), fb.int_first + io, kComBlock,
@@ -1790,7 +1842,7 @@ void launch_forest_build(const EnsSystem *sys, const uint32_t *order, uint32_t n
                        (const uint32_t *)total, items, status);
 }
 
-// workgroups of the AABB pass: 4096 bodies each, at most kAabbBlocks
+// workgroups of the AABB pass: 1024 bodies each, at most kAabbBlocks
 uint32_t aabb_blocks(uint32_t n) {
     return std::min<uint32_t>(kAabbBlocks, ceil_div(n, 4 * kAabbThreads));
 }
@@ -1832,10 +1884,9 @@ void launch_topology(const TreeBufs &t, const double *x, const double *y, const 
                            (const int32_t *)t.lcp, n - 1, t.chain, (const uint32_t *)t.scan_part,
                            nparts, scanned, t.hdr, t.icap, t.ref, t.spanning, t.spanning_cap);
     }
-    KeyView kv{t.skey, t.klo};
+    KeyView kv{t.skey, t.klo, t.lcp, t.chain};
     hipLaunchKernelGGL(k_link, grid, dim3(kThreads), 0, s, n, t.icap, t.hdr, kv,
-                       (const uint32_t *)t.sidx, (const int32_t *)t.lcp,
-                       (const uint32_t *)t.chain, t.ref, t.int_depth, t.int_node,
+                       (const uint32_t *)t.sidx, t.ref, t.int_depth, t.int_node,
                        t.body_node, t.int_local, t.spanning, t.spanning_cap, t.int_first);
 }
 
