@@ -165,7 +165,7 @@ struct TreeBufs {
     uint32_t cross_cap = 0;
     double4 *body4 = nullptr;       // {x, y, z, m} per body, input order: one load per body
     uint32_t *gq = nullptr;         // traversal queue counters, one per XCD, 128 bytes apart
-    static constexpr uint32_t kGroupQueueWords = 8 * 32;
+    static constexpr uint32_t kGroupQueueWords = 8 * 32;  // the ensemble's queue as well
     uint32_t spanning_cap = 0;
     int32_t *ref = nullptr;
     double4 *cm = nullptr;          // FP64 records (reference-semantics traversal)
@@ -417,13 +417,13 @@ struct EnsForceArgs {
     ForestBufs fb;
     double G, theta;
     float eps2;
-    uint32_t *cursor;  // work-queue cursor (reset by launch_ens_items)
+    uint32_t *cursor;  // work-queue counters, one per XCD (reset by launch_ens_items)
     uint32_t *status;  // kFlag* bits
     uint32_t *inter;   // per body: accepted interactions (Barnes-Hut) or sources (direct)
     uint32_t direct_tpl;  // direct-sum targets per lane: 1 or 2 (items of 64 or 128 targets)
 };
 constexpr uint32_t kEnsTile = 64;  // targets per direct-sum item and lane
-// item_off = exclusive prefix of items[qorder[q]]; resets the cursor and status
+// item_off = exclusive prefix of items[qorder[q]]; resets the queue counters
 void launch_ens_items(uint32_t nq, const uint32_t *qorder, const uint32_t *items,
                       uint32_t *item_off, uint32_t *cursor, uint32_t *status, hipStream_t s);
 void launch_ens_forces(const EnsForceArgs &a, uint32_t waves, hipStream_t s);
