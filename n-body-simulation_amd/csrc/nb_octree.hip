@@ -1406,6 +1406,7 @@ __device__ inline uint32_t wg_scan_array(uint32_t *a, uint32_t m, uint32_t *wsum
     uint32_t b, e;
     wave_range(m, &b, &e);
     uint32_t s = 0;
+#pragma unroll 8
     for (uint32_t i = b + lane; i < e; i += 64) s += a[i];
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) s += __shfl_xor(s, off, 64);
@@ -1423,17 +1424,29 @@ __device__ inline uint32_t wg_scan_array(uint32_t *a, uint32_t m, uint32_t *wsum
     __syncthreads();
     uint32_t carry = wsum[w];
     const uint32_t total = wsum[kForestWaves];
-    for (uint32_t g = b; g < e; g += 64) {
-        const uint32_t i = g + lane;
-        const uint32_t v = i < e ? a[i] : 0u;
-        uint32_t inc = v;
+    constexpr uint32_t kAhead = 8;  // loads and wave scans in flight
+    for (uint32_t g = b; g < e; g += 64 * kAhead) {
+        uint32_t v[kAhead], inc[kAhead];
+#pragma unroll
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            const uint32_t i = g + 64 * u + lane;
+            v[u] = i < e ? a[i] : 0u;
+            inc[u] = v[u];
+        }
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t o = __shfl_up(inc, off, 64);
-            if (lane >= (uint32_t)off) inc += o;
+#pragma unroll
+            for (uint32_t u = 0; u < kAhead; ++u) {
+                const uint32_t o = __shfl_up(inc[u], off, 64);
+                if (lane >= (uint32_t)off) inc[u] += o;
+            }
         }
-        if (i < e) a[i] = carry + inc - v;
-        carry += __shfl(inc, 63, 64);
+#pragma unroll
+        for (uint32_t u = 0; u < kAhead; ++u) {
+            const uint32_t i = g + 64 * u + lane;
+            if (i < e) a[i] = carry + inc[u] - v[u];
+            carry += __shfl(inc[u], 63, 64);
+        }
     }
     __syncthreads();
     return total;
@@ -1445,7 +1458,7 @@ __global__ void __launch_bounds__(kForestThreads) k_forest_aabb(
     const EnsSystem *__restrict__ sys, const uint32_t *__restrict__ order,
     const double *__restrict__ gx, const double *__restrict__ gy, const double *__restrict__ gz,
     ForestBufs fb) {
-    __shared__ double red[kForestWaves][6];
+    __shared__ double red[kForestWaves][6], ext[6];
     const uint32_t s = order[blockIdx.x];
     const EnsSystem S = sys[s];
     const uint32_t n = S.n, t = threadIdx.x;
@@ -1463,37 +1476,36 @@ __global__ void __launch_bounds__(kForestThreads) k_forest_aabb(
         h->corr_pairs = 0;
     }
     __syncthreads();  // the reset precedes every flag raised below
-    double mn[3] = {0.0, 0.0, 0.0}, mx[3] = {0.0, 0.0, 0.0};
-    bool bad = false;
+    Extents e;
+#pragma unroll 8
     for (uint32_t i = t; i < n; i += kForestThreads) {
         const double p[3] = {x[i], y[i], z[i]};
+#pragma unroll
         for (int c = 0; c < 3; ++c) {
-            bad |= !isfinite(p[c]);
-            mn[c] = sycl_min(mn[c], p[c]);
-            mx[c] = sycl_max(mx[c], p[c]);
+            e.bad |= !isfinite(p[c]);
+            e.mn[c] = sycl_min(e.mn[c], p[c]);
+            e.mx[c] = sycl_max(e.mx[c], p[c]);
         }
     }
-    if (bad) raise_flag(h, kFlagAabb);
-    for (int off = 32; off >= 1; off >>= 1)
-        for (int c = 0; c < 3; ++c) {
-            mn[c] = sycl_min(mn[c], __shfl_xor(mn[c], off, 64));
-            mx[c] = sycl_max(mx[c], __shfl_xor(mx[c], off, 64));
-        }
+    if (e.bad) raise_flag(h, kFlagAabb);
+    wave_extents(e);
     if ((t & 63) == 0)
+#pragma unroll
         for (int c = 0; c < 3; ++c) {
-            red[t >> 6][c] = mn[c];
-            red[t >> 6][3 + c] = mx[c];
+            red[t >> 6][c] = e.mn[c];
+            red[t >> 6][3 + c] = e.mx[c];
         }
     __syncthreads();
-    if (t == 0) {
-        double v[6];
-        for (int c = 0; c < 6; ++c) v[c] = red[0][c];
+    if (t < 6) {
+        double v = red[0][t];
+#pragma unroll
         for (int w = 1; w < kForestWaves; ++w)
-            for (int c = 0; c < 3; ++c) {
-                v[c] = sycl_min(v[c], red[w][c]);
-                v[3 + c] = sycl_max(v[3 + c], red[w][3 + c]);
-            }
-        const RootCube r = cubify(v);
+            v = t < 3 ? sycl_min(v, red[w][t]) : sycl_max(v, red[w][t]);
+        ext[t] = v;
+    }
+    __syncthreads();
+    if (t == 0) {
+        const RootCube r = cubify(ext);
         store_cube(h, r);
         if (!r.ok) raise_flag(h, kFlagAabb);
     }

@@ -16,7 +16,9 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kItems = kScanTile / kThreads;
 constexpr int kRadixTile = 4096;       // keys per radix tile
 constexpr int kRadixTileBig = 8192;    // keys per tile from kRadixBigMin keys on
+constexpr int kRadixTileWide = 10240;  // or, where fewer rounds of tiles result
 constexpr uint32_t kRadixBigMin = 1u << 21;
+constexpr uint32_t kCus = 256;
 constexpr uint32_t kSortMergeMax = 1u << 18;  // k_sort_tiles and k_merge_runs; above, passes
 constexpr int kPassThreads = 512;
 constexpr int kPassWaves = kPassThreads / 64;
@@ -665,14 +667,23 @@ uint32_t radix_blocks_for(uint32_t n) { return ceil_div(n ? n : 1, kRadixTile); 
 
 uint32_t radix_ctl_words(uint32_t n) { return kCtlStatus + 2u * kBins * radix_blocks_for(n); }
 
-// tiles of a sort of n keys
-static uint32_t radix_tiles(uint32_t n) {
-    return ceil_div(n, n >= kRadixBigMin ? kRadixTileBig : kRadixTile);
+// Keys per tile of a sort of n keys.  Larger tiles for large sorts: half the
+// look-back chain and longer digit runs in the scatter, once there are enough
+// tiles to fill the device.  A CU holds one tile of either larger size, so time
+// goes with (rounds of tiles) x (keys per tile): 2,110,000 keys are 258 tiles of
+// 8192, a second round for two of them (41 us a pass), and 207 of 10,240 (29 us);
+// 4,194,304 are two rounds of either, and 8192 is the smaller.
+static uint32_t radix_tile(uint32_t n) {
+    if (n < kRadixBigMin) return kRadixTile;
+    const auto cost = [&](uint32_t tile) {
+        return (uint64_t)ceil_div(ceil_div(n, tile), kCus) * tile;
+    };
+    return cost(kRadixTileWide) < cost(kRadixTileBig) ? kRadixTileWide : kRadixTileBig;
 }
 
 RadixCount radix_count_args(uint32_t n, uint32_t *ctl) {
     if (n <= kSortMergeMax || n >= kStatAgg) return RadixCount{nullptr, nullptr, 0};
-    return RadixCount{ctl, ctl + kCtlStatus, (uint64_t)kBins * radix_tiles(n)};
+    return RadixCount{ctl, ctl + kCtlStatus, (uint64_t)kBins * ceil_div(n, radix_tile(n))};
 }
 
 SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
@@ -704,23 +715,17 @@ SortEnd radix_sort_u64_u32(uint64_t *keys, uint32_t *vals, uint64_t *keys_alt,
         }
         return ka == keys ? SortEnd::kInPlace : SortEnd::kInAlt;
     }
-    // larger tiles for large sorts: half the look-back chain and longer digit
-    // runs in the scatter, once there are enough tiles to fill the device
-    const bool big = n >= kRadixBigMin;
-    const uint32_t nb = radix_tiles(n);
+    const uint32_t tile = radix_tile(n), nb = ceil_div(n, tile);
+    const auto pass = tile == (uint32_t)kRadixTile      ? k_radix_pass<kRadixTile>
+                      : tile == (uint32_t)kRadixTileBig ? k_radix_pass<kRadixTileBig>
+                                                        : k_radix_pass<kRadixTileWide>;
     if (!counted)
         hipLaunchKernelGGL(k_radix_count, dim3(std::min(nb, kCountBlocks)), dim3(kCountThreads), 0,
                            s, (const uint64_t *)keys, n, ctl, ctl + kCtlStatus,
                            (uint64_t)kBins * nb);
     for (int p = 0; p < passes; ++p) {
-        if (big)
-            hipLaunchKernelGGL(k_radix_pass<kRadixTileBig>, dim3(nb), dim3(kPassThreads), 0, s,
-                               (const uint64_t *)ka, (const uint32_t *)va, kb, vb, n, p, passes,
-                               ctl, nb, flags);
-        else
-            hipLaunchKernelGGL(k_radix_pass<kRadixTile>, dim3(nb), dim3(kPassThreads), 0, s,
-                               (const uint64_t *)ka, (const uint32_t *)va, kb, vb, n, p, passes,
-                               ctl, nb, flags);
+        hipLaunchKernelGGL(pass, dim3(nb), dim3(kPassThreads), 0, s, (const uint64_t *)ka,
+                           (const uint32_t *)va, kb, vb, n, p, passes, ctl, nb, flags);
         std::swap(ka, kb);
         std::swap(va, vb);
     }

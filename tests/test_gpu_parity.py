@@ -314,6 +314,20 @@ def test_tree_sort_more_tiles_than_resident(gpu, oracle):
                 assert_canonical_equal(c.tree_canonical(), t.canonical(), "3M plummer")
 
 
+def test_tree_sort_wide_tiles(gpu, oracle):
+    # 207 sort tiles of 10,240 keys, the last one ragged: the size at which tiles
+    # of 8192 keys would need a second round
+    n = 2110001
+    d = plummer(gpu, n)
+    t = oracle.Tree(n)
+    t.build(d["x"], d["y"], d["z"], d["m"])
+    with ctx_for(gpu, d, precision=gpu.PREC_FP32C) as c:
+        for _ in range(2):
+            c.bh_build()
+            np.testing.assert_array_equal(c.tree_sorted(), t.export()["sorted"])
+        assert c.tree_info()["node_count"] == t.node_count
+
+
 def test_tree_parity_deep_clusters(gpu, oracle):
     # 40 clumps of 3000 bodies, 1e-9 across (about 31 levels below the root):
     # every clump holds a block boundary, so each brings a chain of about 31
