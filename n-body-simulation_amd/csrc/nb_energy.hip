@@ -29,8 +29,8 @@ namespace {
 //
 // One row per lane and one term at a time, as before: 10,000 bodies 1.53 ms
 // (bound by the latency of a single term on a few CUs), 131,071 19.6 ms, 300,001
-// 59 ms.  Now 0.37, 11.1 and 49 ms (rows at 131,071: 12.5; workgroups at
-// 200,001 and 300,001: 25.9 and 57 against 25.0 and 49).
+// 59 ms, 1,048,576 560 ms.  Now 0.37, 11.1, 46 and 560 ms (rows at 131,071: 12.5;
+// workgroups at 200,001 and 300,001: 25.9 and 57 against 25.0 and 49).
 constexpr uint32_t kRowsFrom = 192 * 1024;  // bodies from which the rows are faster
 constexpr uint32_t kCus = 256;              // CUs of an MI355X
 constexpr int kWaves = 16;
@@ -147,6 +147,15 @@ k_energy_terms(
 }
 
 
+// A squared distance v lies in [2^-600, 2^600) if distance_off(v) < kDistanceOff:
+// v is a sum of squares, so no sign needs masking, and the largest value of
+// several terms tests them all (1,048,576 bodies 572 ms with a test per term, 560
+// so; 400,000 89 and 83; the workgroup kernel was 3 % slower with it).
+constexpr uint32_t kDistanceOff = 1200u << 20;
+__device__ inline uint32_t distance_off(double v) {
+    return (uint32_t)__double2hiint(v) - ((1023u - 600u) << 20);
+}
+
 constexpr int kRowThreads = 256;  // bodies j per block, and sources i per LDS stage
 constexpr int kRowPer = 8;        // terms interleaved
 
@@ -187,16 +196,16 @@ __global__ void __launch_bounds__(kRowThreads) k_energy_rows(
             uint32_t ii = 0;
             for (; ii + kRowPer <= cnt; ii += kRowPer) {
                 double a[kRowPer], v[kRowPer];
-                bool core = tile_ok && mj_ok;
+                uint32_t worst = 0;
 #pragma unroll
                 for (int u = 0; u < kRowPer; ++u) {
                     const double4 si = src[ii + u];
                     const double r_x = pxj - si.x, r_y = pyj - si.y, r_z = pzj - si.z;
                     a[u] = si.w * mj;
                     v[u] = r_x * r_x + r_y * r_y + r_z * r_z;
-                    core = core && exponent_within(v[u], 600);
+                    worst = max(worst, distance_off(v[u]));
                 }
-                if (core) {
+                if (tile_ok && mj_ok && worst < kDistanceOff) {
 #pragma unroll
                     for (int u = 0; u < kRowPer; ++u) a[u] = div_core(a[u], sqrt_core(v[u]));
                 } else {
