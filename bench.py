@@ -73,12 +73,12 @@ CPU_SAMPLE_S = 10.0
 #    (profiles/bh_plummer_4m_hbm_counters.md);
 #  - 1M disk, theta 0.5: 932,786 KiB x 2 read + 133,202 KiB written
 #    (profiles/bh_disk_1m_hbm_counters.md);
-#  - 1M disk, FP64 per-body traversal (k_bh_exact): 1,106,567 KiB x 2 read +
-#    172,409 KiB written (profiles/bh_disk_1m_exact_kernel_stats.md).
+#  - 1M disk, FP64 per-body traversal (k_bh_exact_wave): 750,375 KiB x 2 read +
+#    2,231,234 KiB written (profiles/bh_disk_1m_exact_kernel_stats.md).
 TRAFFIC_BYTES = {
     ("bh_plummer_4m", 0.37375): 12.370e9,
     ("bh_disk_1m", 0.5): 2.047e9,
-    ("bh_disk_1m_exact", 0.5): 2.443e9,
+    ("bh_disk_1m_exact", 0.5): 3.822e9,
 }
 
 WORKLOADS = {
@@ -404,7 +404,7 @@ def main():
         if prec == nb.PREC_FP32C:
             peak, bound, kernel = FP32_PEAK_TFLOPS, "valu", "k_bh_group"
         else:  # the FP64 per-body traversal in the reference's order
-            peak, bound, kernel = FP64_PEAK_TFLOPS, "valu", "k_bh_exact"
+            peak, bound, kernel = FP64_PEAK_TFLOPS, "valu", "k_bh_exact_wave"
     else:
         flops = FLOP_PER_INTERACTION * float(n) * float(n)
         peak = FP32_PEAK_TFLOPS if prec == nb.PREC_FP32C else FP64_PEAK_TFLOPS

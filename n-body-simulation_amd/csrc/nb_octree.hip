@@ -13,7 +13,7 @@
 //     2[x>mid_x] + [z<mid_z], child min moved to mid on the x/y bits and on a
 //     cleared z bit.  Digits are packed most significant first into a 63-bit
 //     key, so key order is the reference's in-order body order.
-//  3. Stable radix sort of (key, body).
+//  3. Stable sort of (key, body).
 //  4. Runs of bodies sharing all 21 digits get digits 21..41 and are sorted
 //     inside the run (rare: bodies closer than edge/2^21).
 //  5. lcp[i] = depth of the deepest cell holding sorted bodies i and i+1.
@@ -23,14 +23,13 @@
 //     internal cells k in depth-first pre-order; internal cell k stores its 8
 //     children at node ids 1 + 8k + digit.
 //  6. Parents come from a galloping search for the first body of the parent
-//     cell; children count themselves into their parent.
-//  7. Centre of mass bottom-up: the last child to arrive at a cell sums the 8
-//     children in digit order 0..7 from 0.0 -- the reference's summation
+//     cell; every cell and body learns the child slot (node) it fills.
+//  7. Centre of mass level by level from the deepest cells up: a cell sums its
+//     8 children in digit order 0..7 from 0.0 -- the reference's summation
 //     (BarnesHutOctree.cpp:299-311), so every sum is bit-identical.  Cells
-//     inside a block of 4096 sorted bodies are finished by that block's
-//     workgroup (workgroup-scope atomics: agent-scope ones would write back
-//     and invalidate the L2 of an XCD at every arrival); the few cells that
-//     cross block boundaries are finished level by level by one workgroup.
+//     inside a block of 1024 sorted bodies are finished by that block's
+//     workgroup in LDS; the few cells that cross block boundaries by one
+//     workgroup per 64 blocks and one more.
 //  8. Node records for traversal (COM = numerator / mass as the reference
 //     divides per visit; an FP32 hi/lo record for the group traversal).  A
 //     cell's edge is rootEdge * 2^-depth wherever it is needed.
@@ -925,7 +924,7 @@ __device__ __forceinline__ void sum_levels(uint32_t t, const uint32_t *cnt,
 // table, so no child needs a branch.  An empty slot adds +0.0, which changes no
 // running sum that starts at +0.0.
 // (1024 bodies: 40 us with one lane per cell and a scan of all cells per level,
-// 13.5 now; 100,003: 43 and 17; 1,048,576, disk: 107 and 58.)
+// 13.5 now; 100,003: 43 and 17; 1,048,576, disk: 107 and 58; 4,194,304: 366 and 243.)
 constexpr uint32_t kComLdsCells = 576;   // about 490 per block; 537 the most seen (disk, Plummer)
 constexpr int kComLocalThreads = 512;
 constexpr int kComBodiesPerThread = kComBlock / kComLocalThreads;
