@@ -96,7 +96,7 @@ k_energy_terms(
         }
     };
     // The numerator G m_i m_j is (G m_i) m_j.  When G m_i and m_j both lie in
-    // [2^-150, 2^150), it lies in div_core's range and only the squared
+    // [2^-150, 2^150), it lies in div_sqrt_core's range and only the squared
     // distance needs checking.
     const bool mj_ok = exponent_within(mj, 150);
     const uint32_t last = min(n, (tile + 1) * kTile);  // bodies i < j of this block
@@ -120,13 +120,14 @@ k_energy_terms(
             const double gm = G * sm[u];
             a[u] = gm * mj;
             v[u] = r_x * r_x + r_y * r_y + r_z * r_z;
-            const bool ok = exponent_within(gm, 150) && exponent_within(v[u], 600);
+            const bool ok = exponent_within(gm, 150) && exponent_within(v[u], 600) &&
+                            (uint32_t)__double2loint(v[u]) < kRootOfOnes;
             core = core && (ok || (!all && c + w * kPer + u >= j));
         }
         load(c + kChunk);  // back before the barrier waits for it
         if (core) {
 #pragma unroll
-            for (int u = 0; u < kPer; ++u) a[u] = div_core(a[u], sqrt_core(v[u]));
+            for (int u = 0; u < kPer; ++u) a[u] = div_sqrt_core(a[u], v[u]);
         } else {
             for (int u = 0; u < kPer; ++u) a[u] = a[u] / sqrt(v[u]);
         }
@@ -196,7 +197,7 @@ __global__ void __launch_bounds__(kRowThreads) k_energy_rows(
             uint32_t ii = 0;
             for (; ii + kRowPer <= cnt; ii += kRowPer) {
                 double a[kRowPer], v[kRowPer];
-                uint32_t worst = 0;
+                uint32_t worst = 0, low = 0;
 #pragma unroll
                 for (int u = 0; u < kRowPer; ++u) {
                     const double4 si = src[ii + u];
@@ -204,10 +205,11 @@ __global__ void __launch_bounds__(kRowThreads) k_energy_rows(
                     a[u] = si.w * mj;
                     v[u] = r_x * r_x + r_y * r_y + r_z * r_z;
                     worst = max(worst, distance_off(v[u]));
+                    low = max(low, (uint32_t)__double2loint(v[u]));
                 }
-                if (tile_ok && mj_ok && worst < kDistanceOff) {
+                if (tile_ok && mj_ok && worst < kDistanceOff && low < kRootOfOnes) {
 #pragma unroll
-                    for (int u = 0; u < kRowPer; ++u) a[u] = div_core(a[u], sqrt_core(v[u]));
+                    for (int u = 0; u < kRowPer; ++u) a[u] = div_sqrt_core(a[u], v[u]);
                 } else {
                     for (int u = 0; u < kRowPer; ++u) a[u] = a[u] / sqrt(v[u]);
                 }

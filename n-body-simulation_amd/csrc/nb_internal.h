@@ -429,22 +429,30 @@ void launch_ens_items(uint32_t nq, const uint32_t *qorder, const uint32_t *items
 void launch_ens_forces(const EnsForceArgs &a, uint32_t waves, hipStream_t s);
 
 // ---------------------------------------------------------------------------
-// Correctly rounded FP64 square root and division for the reference-order
-// kernels, within ranges where the compiler's IEEE sequences need none of
-// their range handling.  The compiler's square root takes a v_rsq_f64
-// estimate, one Goldschmidt step for the root and its half-reciprocal and two
-// residual corrections, scaling inputs below 2^-767 and passing zero and
-// infinity through; its division takes v_rcp_f64 of the divisor, two Newton
-// steps and one residual correction of the quotient, with operand scaling
-// (v_div_scale_f64) and a special-value fix-up (v_div_fixup_f64) that change
-// nothing while dividend, divisor and quotient are normal and their exponents
-// differ by less than 768.  The cores below run the same operations without
-// that handling, so inside the guarded ranges they give the same bits; the
-// GPU tests compare every pair of the direct sum, the traversal and the
-// energy with the oracle's IEEE operations.  Outside: the plain operators.
-__device__ inline double sqrt_core(double v) {  // v in [2^-767, 2^1023)
+// Correctly rounded FP64 1 / sqrt(v) and a / sqrt(v), two IEEE operations each, for
+// the reference-order kernels, within ranges that need no handling of scales and
+// special values.
+//
+// The root: a v_rsq_f64 estimate, one Goldschmidt step for the root s and its
+// half-reciprocal h, and two residual corrections, the second from a value
+// within an ulp.  The reciprocal of s: 2 h is within a few ulps of it, two Newton
+// steps follow; the first leaves it within an ulp, and by P. Markstein
+// (Computation of elementary functions on the IBM RISC System/6000 processor,
+// IBM J. Res. Dev. 34, 1990) the second, whose residual is exact, then rounds it
+// correctly unless every bit of s's significand is 1.  The quotient a / s: a
+// times that reciprocal and one exact residual, correctly rounded by the same
+// paper.  A significand of ones is the root of exactly two values per factor of
+// four, whose low words are 0xfffffffe and 0xffffffff: low words from
+// kRootOfOnes on take the plain operators (one value in 2^31).
+//
+// Starting from 2 h instead of a v_rcp_f64 of s (a quarter-rate instruction, and
+// one more step from its 2^-26) saves 20 of about 100 cycles per 64 inverse roots.
+// 1.7e11 random values, and the neighbours of 16 million squares, give the bits of
+// the compiler's operators; so does every pair of the GPU tests.
+constexpr uint32_t kRootOfOnes = 0xfffffffeu;
+__device__ inline void root_parts(double v, double &s, double &y) {
     const double g = __builtin_amdgcn_rsq(v);
-    double s = v * g;
+    s = v * g;
     double h = g * 0.5;
     const double r = fma(-h, s, 0.5);
     s = fma(s, r, s);
@@ -452,32 +460,32 @@ __device__ inline double sqrt_core(double v) {  // v in [2^-767, 2^1023)
     double d = fma(-s, s, v);
     s = fma(d, h, s);
     d = fma(-s, s, v);
-    return fma(d, h, s);
-}
-__device__ inline double div_core(double a, double b) {  // |a|, |b| in [2^-300, 2^300]
-    double y = __builtin_amdgcn_rcp(b);
-    double e = fma(-b, y, 1.0);
-    y = fma(y, e, y);
-    e = fma(-b, y, 1.0);
-    y = fma(y, e, y);
-    const double q = a * y;
-    e = fma(-b, q, a);
-    return fma(e, y, q);
-}
-// 1.0 / sqrt(v), both operations correctly rounded (the reference's
-// inverse square root); the core for v in [2^-512, 2^512)
-__device__ inline bool inv_sqrt_in_range(double v) {  // on the sign and exponent: one compare
-    return (uint32_t)__double2hiint(v) - 0x1ff00000u < 0x40000000u;
-}
-__device__ inline double inv_sqrt_core(double v) {
-    const double s = sqrt_core(v);
-    double y = __builtin_amdgcn_rcp(s);
+    s = fma(d, h, s);
+    y = h + h;
     double e = fma(-s, y, 1.0);
     y = fma(y, e, y);
     e = fma(-s, y, 1.0);
     y = fma(y, e, y);
-    e = fma(-s, y, 1.0);  // the quotient 1.0 * y is y
-    return fma(e, y, y);
+}
+// a / sqrt(v); v in [2^-600, 2^600), low word below kRootOfOnes, |a| and the
+// quotient in [2^-600, 2^600]
+__device__ inline double div_sqrt_core(double a, double v) {
+    double s, y;
+    root_parts(v, s, y);
+    const double q = a * y;
+    const double e = fma(-s, q, a);
+    return fma(e, y, q);
+}
+// 1.0 / sqrt(v) (the reference's inverse square root); the core for v in
+// [2^-512, 2^512) with a low word below kRootOfOnes
+__device__ inline bool inv_sqrt_in_range(double v) {  // sign and exponent in one compare
+    return (uint32_t)__double2hiint(v) - 0x1ff00000u < 0x40000000u &&
+           (uint32_t)__double2loint(v) < kRootOfOnes;
+}
+__device__ inline double inv_sqrt_core(double v) {
+    double s, y;
+    root_parts(v, s, y);
+    return y;
 }
 __device__ inline double inv_sqrt_ieee(double v) {
     return inv_sqrt_in_range(v) ? inv_sqrt_core(v) : 1.0 / sqrt(v);

@@ -4,6 +4,8 @@ Bars: FP64 paths bit-exact (forces, integrator, octree sums); topology and
 body order bit-exact; FP32 paths within stated relative tolerances against
 the FP64 direct sum.
 """
+import math
+
 import numpy as np
 import pytest
 
@@ -830,6 +832,57 @@ def test_ieee_sequences_both_sides_of_their_range(gpu, oracle, sep, m1):
     r = oracle.energy(d["x"], d["y"], d["z"], d["vx"], d["vy"], d["vz"], d["m"])
     for k in ("kinetic", "potential", "total"):
         assert np.float64(e[k]).view(np.int64) == np.float64(r[k]).view(np.int64), k
+
+
+def _offset_of(d2):
+    """dx, dy with dx^2 + dy^2 == d2 in FP64 (dx^2 exact)."""
+    for m in range(1, 400):
+        dx = math.floor(math.sqrt(d2) * 2.0**20) / 2.0**20 - m * 2.0**-20
+        dy0 = math.sqrt(d2 - dx * dx)
+        for w in range(-3, 4):
+            dy = dy0 + w * math.ulp(dy0)
+            if dx * dx + dy * dy == d2:
+                return dx, dy
+    return None
+
+
+def test_inverse_root_of_ones(gpu, oracle):
+    # roots whose significand is all ones, where the reciprocal's last step would
+    # round the wrong way: 4 - 2^-50 and 4 - 2^-51 (times powers of four) as the
+    # cubed squared distance of the force, and as the squared distance of the energy
+    forces = energies = 0
+    for k in range(-6, 7):
+        for j in (1, 2):
+            target = math.ldexp(4 - j * 2.0**-51, 2 * k)
+            assert np.float64(math.sqrt(target)).view(np.int64) & (2**52 - 1) == 2**52 - 1
+            c = target ** (1 / 3)
+            roots = [c + t * math.ulp(c) for t in range(-60, 61)]
+            cubes = [d for d in roots if (d * d) * d == target]
+            for d2, energy in [(d, False) for d in cubes[:1]] + [(target, True)]:
+                off = _offset_of(d2)
+                if off is None:
+                    continue
+                d = dict(x=np.array([0.0, off[0]]), y=np.array([0.0, off[1]]), z=np.zeros(2),
+                         vx=np.zeros(2), vy=np.zeros(2), vz=np.zeros(2), m=np.array([1.0, 2.0]))
+                with ctx_for(gpu, d, theta=0.5) as ctx:
+                    if energy:
+                        e = ctx.energy()
+                        r = oracle.energy(*(d[q] for q in ("x", "y", "z", "vx", "vy", "vz", "m")))
+                        assert (np.float64(e["potential"]).view(np.int64)
+                                == np.float64(r["potential"]).view(np.int64)), (k, j)
+                        energies += 1
+                        continue
+                    direct = ctx.forces_direct()
+                    ctx.bh_build()
+                    walk = ctx.bh_forces()
+                t = oracle.Tree(2)
+                t.build(d["x"], d["y"], d["z"], d["m"])
+                for got, want in ((direct, oracle.naive_accel(d["x"], d["y"], d["z"], d["m"])),
+                                  (walk, t.bh_accel(0.5)[:3])):
+                    for a, r in zip(got, want):
+                        np.testing.assert_array_equal(bits(a), bits(r), err_msg=f"{k} {j}")
+                forces += 1
+    assert forces >= 4 and energies >= 20, (forces, energies)
 
 
 def test_bh_forces_repeatable(gpu):
