@@ -29,7 +29,7 @@ namespace {
 //
 // One row per lane and one term at a time, as before: 10,000 bodies 1.53 ms
 // (bound by the latency of a single term on a few CUs), 131,071 19.6 ms, 300,001
-// 59 ms, 1,048,576 560 ms.  Now 0.37, 11.1, 46 and 560 ms (rows at 131,071: 12.5;
+// 59 ms, 1,048,576 560 ms.  Now 0.37, 10.8, 46 and 552 ms (rows at 131,071: 12.5;
 // workgroups at 200,001 and 300,001: 25.9 and 57 against 25.0 and 49).
 constexpr uint32_t kRowsFrom = 192 * 1024;  // bodies from which the rows are faster
 constexpr uint32_t kCus = 256;              // CUs of an MI355X
@@ -112,6 +112,7 @@ k_energy_terms(
         }
         double a[kPer], v[kPer];
         bool core = mj_ok;
+        uint32_t low = 0;
 #pragma unroll
         for (int u = 0; u < kPer; ++u) {
             const double r_x = pxj - sx[u];
@@ -120,12 +121,12 @@ k_energy_terms(
             const double gm = G * sm[u];
             a[u] = gm * mj;
             v[u] = r_x * r_x + r_y * r_y + r_z * r_z;
-            const bool ok = exponent_within(gm, 150) && exponent_within(v[u], 600) &&
-                            (uint32_t)__double2loint(v[u]) < kRootOfOnes;
+            const bool ok = exponent_within(gm, 150) && exponent_within(v[u], 600);
+            low = max(low, (uint32_t)__double2loint(v[u]));
             core = core && (ok || (!all && c + w * kPer + u >= j));
         }
         load(c + kChunk);  // back before the barrier waits for it
-        if (core) {
+        if (core && low < kRootOfOnes) {
 #pragma unroll
             for (int u = 0; u < kPer; ++u) a[u] = div_sqrt_core(a[u], v[u]);
         } else {

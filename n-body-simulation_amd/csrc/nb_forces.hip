@@ -50,10 +50,11 @@ __device__ inline uint32_t wave_uniform(uint32_t v) { return __builtin_amdgcn_re
 // their SIMDs (s_setprio); a wave's terms are interleaved, with one test for
 // all that the IEEE sequences need no range handling.  16,384 bodies: 0.52 ms
 // with the additions last, sources staged in LDS and one term at a time; 0.45
-// now, 262 cycles at 2.4 GHz per 64 pairs where the 32 FP64 operations, two
-// quarter-rate estimates and three additions of a pair issue in about 208.
-// 700 bodies 0.026 -> 0.011, 5001 0.162 -> 0.086, 8192 0.262 -> 0.139, 20,001
-// 1.26 -> 0.79 ms.  T = 32 (two sources at a time) was slower than the better
+// without; 0.42 now that the reciprocal needs no v_rcp_f64, 244 cycles at 2.4 GHz
+// per 64 pairs where the 31 FP64 operations, the quarter-rate estimate and three
+// additions of a pair issue in about 188.
+// 700 bodies 0.026 -> 0.011, 5001 0.162 -> 0.082, 8192 0.262 -> 0.133, 20,001
+// 1.26 -> 0.76 ms.  T = 32 (two sources at a time) was slower than the better
 // of the two at every size.
 constexpr int kF64Waves = 16;
 constexpr int kF64Threads = 64 * kF64Waves;
@@ -132,6 +133,7 @@ __device__ __forceinline__ double direct_f64_body(uint32_t n, const double *__re
         if (computes) {
             double r_x[P], r_y[P], r_z[P], den[P], m_j[P];
             bool in_range = true;
+            uint32_t low = 0;  // one test of the low words: a test each took 0.05 ms more
 #pragma unroll
             for (int u = 0; u < P; ++u) {
                 r_x[u] = sx[u] - px;
@@ -140,10 +142,11 @@ __device__ __forceinline__ double direct_f64_body(uint32_t n, const double *__re
                 m_j[u] = sm[u];
                 den[u] = (r_x[u] * r_x[u]) + (r_y[u] * r_y[u]) + (r_z[u] * r_z[u]) + eps2;
                 den[u] = den[u] * den[u] * den[u];
-                in_range = in_range && inv_sqrt_in_range(den[u]);
+                in_range = in_range && inv_sqrt_exponent_ok(den[u]);
+                low = max(low, (uint32_t)__double2loint(den[u]));
             }
             load(c + C);  // back before the barrier waits for it
-            if (in_range) {
+            if (in_range && low < kRootOfOnes) {
 #pragma unroll
                 for (int u = 0; u < P; ++u) den[u] = inv_sqrt_core(den[u]);
             } else {

@@ -478,9 +478,11 @@ __device__ inline double div_sqrt_core(double a, double v) {
 }
 // 1.0 / sqrt(v) (the reference's inverse square root); the core for v in
 // [2^-512, 2^512) with a low word below kRootOfOnes
-__device__ inline bool inv_sqrt_in_range(double v) {  // sign and exponent in one compare
-    return (uint32_t)__double2hiint(v) - 0x1ff00000u < 0x40000000u &&
-           (uint32_t)__double2loint(v) < kRootOfOnes;
+__device__ inline bool inv_sqrt_exponent_ok(double v) {  // and the sign, in one compare
+    return (uint32_t)__double2hiint(v) - 0x1ff00000u < 0x40000000u;
+}
+__device__ inline bool inv_sqrt_in_range(double v) {
+    return inv_sqrt_exponent_ok(v) && (uint32_t)__double2loint(v) < kRootOfOnes;
 }
 __device__ inline double inv_sqrt_core(double v) {
     double s, y;
