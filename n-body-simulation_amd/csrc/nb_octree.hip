@@ -1933,8 +1933,9 @@ void launch_com(const TreeBufs &t, double G, bool f64, bool f32, GroupRule rule,
     }
     if (f32) {
         const uint32_t nparts = ceil_div(t.n, kScanTile);
-        hipLaunchKernelGGL(k_group_count, dim3(nparts), dim3(kScanThreads), 0, s,
-                           (const uint32_t *)t.group_size, t.n, t.scan_part);
+        if (nparts > 1)  // one tile has none before it (a launch of 3.6 us)
+            hipLaunchKernelGGL(k_group_count, dim3(nparts), dim3(kScanThreads), 0, s,
+                               (const uint32_t *)t.group_size, t.n, t.scan_part);
         const bool scanned = scan_parts_if_many(t.scan_part, nparts, s);
         hipLaunchKernelGGL(k_group_list, dim3(nparts), dim3(kScanThreads), 0, s,
                            (const uint32_t *)t.group_size, t.n, (const uint32_t *)t.scan_part,

@@ -1,11 +1,12 @@
-// nb_scan.hip -- device-wide exclusive scan and stable LSD radix sort.
+// nb_scan.hip -- device-wide exclusive scan and stable key sorts.
 //
-// Both are written for 64-lane wavefronts: prefix sums use __shfl_up inside a
-// wave and LDS across the 4 waves of a 256-thread block; the radix sort ranks
-// keys stably with a 9-ballot "match any" on the 9-bit digit, so no
-// per-thread histogram is needed, and takes one launch per digit (small
-// and middling sorts: a launch of tiles sorted in LDS, then merges).  The octree build uses the scan for node
-// numbering and the sort for the octant keys (rocPRIM/hipCUB are not used).
+// All are written for 64-lane wavefronts: prefix sums use __shfl_up inside a
+// wave and LDS across the 4 waves of a 256-thread block; the sorts rank keys
+// stably with a 9-ballot "match any" on the 9-bit digit, so no per-thread
+// histogram is needed.  Small and middling sorts take one launch of tiles sorted
+// in LDS, then merges; large ones one launch per digit.  The ensemble uses the
+// scan for its group lists, the octree builds the sorts for the octant keys
+// (rocPRIM/hipCUB are not used).
 #include "nb_internal.h"
 
 namespace nb {

@@ -834,6 +834,20 @@ def test_ieee_sequences_both_sides_of_their_range(gpu, oracle, sep, m1):
         assert np.float64(e[k]).view(np.int64) == np.float64(r[k]).view(np.int64), k
 
 
+@pytest.mark.parametrize("n", [1, 2, 65, 2047, 2048, 2049, 4097])
+def test_bh_group_list_edges(gpu, n):
+    # the group list at the edges of its scan tiles (2048 positions): with
+    # theta = 0 every body's list is every body, so a group missing or listed
+    # twice at another place would leave a body out or count it differently
+    d = make(gpu, "plummer", n, seed=n)
+    with ctx_for(gpu, d, theta=0.0, precision=gpu.PREC_FP32C) as c:
+        for _ in range(2):
+            c.bh_build()
+            ax = c.bh_forces()[0]
+            np.testing.assert_array_equal(c.interactions(), np.full(n, n))
+        assert np.all(np.isfinite(ax))
+
+
 def _offset_of(d2):
     """dx, dy with dx^2 + dy^2 == d2 in FP64 (dx^2 exact)."""
     for m in range(1, 400):
