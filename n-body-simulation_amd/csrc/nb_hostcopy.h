@@ -23,9 +23,16 @@
 #include <thread>
 #include <vector>
 
-#include "nb_internal.h"
-
 namespace nb {
+
+// arrays of doubles stored into pinned host memory (dst is a host address that
+// the device can write)
+struct CopyOut {
+    const double *src[6];
+    double *dst[6];
+    size_t n[6];
+};
+void launch_copy_out(const CopyOut &c, int count, hipStream_t s);
 
 class HostCopier {
   public:
@@ -47,13 +54,14 @@ class HostCopier {
     }
 
     ~HostCopier() {
-        for (hipEvent_t e : events_) (void)hipEventDestroy(e);
+        for (uint32_t k = 0; k < nevents_; ++k) (void)hipEventDestroy(events_[k]);
         if (ring_) (void)hipHostFree(ring_);
     }
 
     // Copies the arrays behind the work already issued on `stream`; returns when
-    // they have arrived.
-    hipError_t copy(hipStream_t stream, const Array *a, int count) {
+    // they have arrived.  Its callers are C entry points: nothing here throws (the
+    // threads are the only host memory asked for, and copying goes on without them).
+    hipError_t copy(hipStream_t stream, const Array *a, int count) noexcept {
         size_t total = 0;
         for (int k = 0; k < count; ++k) total += a[k].n * sizeof(double);
         if (total == 0) return hipStreamSynchronize(stream);
@@ -76,7 +84,8 @@ class HostCopier {
 
     uint8_t *ring_ = nullptr;
     size_t ring_bytes_ = 0;
-    std::vector<hipEvent_t> events_;
+    hipEvent_t events_[kSlots] = {};
+    uint32_t nevents_ = 0;
 
     hipError_t reserve(size_t bytes) {
         if (ring_bytes_ >= bytes) return hipSuccess;
@@ -116,10 +125,9 @@ class HostCopier {
     hipError_t large(hipStream_t stream, const Array *a, int count, size_t total) {
         const size_t chunk = total < 16 * kChunk ? kChunk / 4 : kChunk;
         hipError_t e = reserve(kSlots * chunk);
-        while (e == hipSuccess && events_.size() < kSlots) {
-            hipEvent_t ev;
-            e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-            if (e == hipSuccess) events_.push_back(ev);
+        while (e == hipSuccess && nevents_ < kSlots) {
+            e = hipEventCreateWithFlags(&events_[nevents_], hipEventDisableTiming);
+            if (e == hipSuccess) ++nevents_;
         }
         if (e != hipSuccess) return e;
         struct Chunk {
@@ -127,12 +135,18 @@ class HostCopier {
             const uint8_t *src;
             size_t bytes;
         };
-        std::vector<Chunk> chunks;
+        // array k has the chunks [first[k], first[k + 1])
+        uint32_t first[kArrays + 1] = {};
         for (int k = 0; k < count; ++k)
-            for (size_t o = 0, all = a[k].n * sizeof(double); o < all; o += chunk)
-                chunks.push_back({(uint8_t *)a[k].dst + o, (const uint8_t *)a[k].src + o,
-                                  std::min(chunk, all - o)});
-        const uint32_t n = (uint32_t)chunks.size();
+            first[k + 1] = first[k] + (uint32_t)((a[k].n * sizeof(double) + chunk - 1) / chunk);
+        const uint32_t n = first[count];
+        const auto chunk_at = [&](uint32_t i) {
+            int k = 0;
+            while (i >= first[k + 1]) ++k;
+            const size_t o = (size_t)(i - first[k]) * chunk;
+            return Chunk{(uint8_t *)a[k].dst + o, (const uint8_t *)a[k].src + o,
+                         std::min(chunk, a[k].n * sizeof(double) - o)};
+        };
         // Chunk i goes through slot i mod kSlots.  This thread issues the DMAs and
         // waits for them in order; arrived: chunks that lie in their slots;
         // filled[s]: chunks that have left slot s.  With threads they fill the
@@ -142,7 +156,8 @@ class HostCopier {
         for (auto &f : filled) f.store(0);
         std::atomic<bool> failed{false};
         auto fill = [&](uint32_t i) {
-            std::memcpy(chunks[i].dst, ring_ + (i % kSlots) * chunk, chunks[i].bytes);
+            const Chunk c = chunk_at(i);
+            std::memcpy(c.dst, ring_ + (i % kSlots) * chunk, c.bytes);
             filled[i % kSlots].store(i / kSlots + 1, std::memory_order_release);
         };
         auto worker = [&] {
@@ -167,8 +182,9 @@ class HostCopier {
         for (uint32_t issued = 0, got = 0; got < n && e == hipSuccess;) {
             if (issued < n && issued - got < kSlots &&
                 filled[issued % kSlots].load(std::memory_order_acquire) >= issued / kSlots) {
-                e = hipMemcpyAsync(ring_ + (issued % kSlots) * chunk, chunks[issued].src,
-                                   chunks[issued].bytes, hipMemcpyDeviceToHost, stream);
+                const Chunk c = chunk_at(issued);
+                e = hipMemcpyAsync(ring_ + (issued % kSlots) * chunk, c.src, c.bytes,
+                                   hipMemcpyDeviceToHost, stream);
                 if (e == hipSuccess) e = hipEventRecord(events_[issued % kSlots], stream);
                 ++issued;
             } else if (got < issued) {

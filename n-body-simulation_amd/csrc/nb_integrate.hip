@@ -11,6 +11,7 @@
 // roundings in the same order.
 #include <algorithm>
 
+#include "nb_hostcopy.h"
 #include "nb_internal.h"
 
 namespace nb {

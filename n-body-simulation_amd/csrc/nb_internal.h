@@ -378,14 +378,6 @@ void launch_kick_drift(uint32_t n, double dt, const double *ax, const double *ay
 void launch_kick(uint32_t n, double dt, const double *ax, const double *ay, const double *az,
                  const double *vhx, const double *vhy, const double *vhz, double *vx,
                  double *vy, double *vz, hipStream_t s);
-// arrays of doubles stored into pinned host memory (dst is a host address that
-// the device can write)
-struct CopyOut {
-    const double *src[6];
-    double *dst[6];
-    size_t n[6];
-};
-void launch_copy_out(const CopyOut &c, int count, hipStream_t s);
 // kick of step k and kick-drift of step k+1 in one pass; bit-identical to
 // launch_kick followed by launch_kick_drift, without storing v
 void launch_kick_kick_drift(uint32_t n, double dt, const double *ax, const double *ay,

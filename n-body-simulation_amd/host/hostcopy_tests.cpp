@@ -1,0 +1,118 @@
+// hostcopy_tests.cpp -- the read-back of csrc/nb_hostcopy.h on the CPU.
+//
+// The few HIP calls that it makes are stand-ins here (copies are memcpy, pinned
+// memory is malloc), so no GPU is needed and a failing call can be asked for.
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+#include <vector>
+
+#include "../csrc/nb_hostcopy.h"
+
+namespace {
+
+bool no_heap = false;  // operator new fails
+
+int failures = 0;
+void check(bool ok, const char *name, size_t n) {
+    if (!ok) ++failures;
+    std::printf("%s %s n=%zu\n", ok ? "PASS" : "FAIL", name, n);
+}
+
+}  // namespace
+
+void *operator new(size_t bytes) {
+    void *p = no_heap ? nullptr : std::malloc(bytes ? bytes : 1);
+    if (!p) throw std::bad_alloc();
+    return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
+extern "C" {
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+    *p = std::malloc(bytes);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p) {
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    *e = (hipEvent_t)std::malloc(1);
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t e) {
+    std::free((void *)e);
+    return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t) {
+    std::memcpy(dst, src, bytes);
+    return hipSuccess;
+}
+}
+
+namespace nb {
+void launch_copy_out(const CopyOut &c, int count, hipStream_t) {
+    for (int k = 0; k < count; ++k) std::memcpy(c.dst[k], c.src[k], c.n[k] * sizeof(double));
+}
+}  // namespace nb
+
+namespace {
+
+// Copies `count` arrays of n doubles; true if every one arrived and nothing past its end.
+bool copied(nb::HostCopier &copier, size_t n, int count) {
+    std::vector<std::vector<double>> src(count), dst(count);
+    std::vector<nb::HostCopier::Array> a;
+    for (int k = 0; k < count; ++k) {
+        src[k].resize(n);
+        for (size_t i = 0; i < n; ++i) src[k][i] = 1.0 + (double)i + 1e7 * k;
+        dst[k].assign(n + 1, -1.0);
+        a.push_back({dst[k].data(), src[k].data(), n});
+    }
+    bool ok = copier.copy(nullptr, a.data(), count) == hipSuccess;
+    for (int k = 0; k < count; ++k) {
+        ok = ok && std::memcmp(dst[k].data(), src[k].data(), n * sizeof(double)) == 0;
+        ok = ok && dst[k][n] == -1.0;
+    }
+    return ok;
+}
+
+// A host that refuses memory: the copy goes on with this thread alone, and no
+// exception leaves it (its callers are C entry points).
+void without_heap(size_t n) {
+    std::vector<double> src(6 * n), dst(6 * n, -1.0);
+    for (size_t i = 0; i < src.size(); ++i) src[i] = (double)i;
+    nb::HostCopier::Array a[6];
+    for (int k = 0; k < 6; ++k) a[k] = {dst.data() + k * n, src.data() + k * n, n};
+    bool ok = false;
+    {
+        nb::HostCopier copier;
+        no_heap = true;
+        try {
+            ok = copier.copy(nullptr, a, 6) == hipSuccess;
+        } catch (...) {
+        }
+        no_heap = false;
+    }
+    check(ok && dst == src, "HostCopier.withoutHeap", n);
+}
+
+}  // namespace
+
+int main() {
+    // edges of the small copies (1 MiB in all), the chunked ones (6 MiB), their
+    // chunk sizes (16 MiB in all) and a chunk's end (six arrays, or one)
+    for (size_t n : {1, 21845, 21846, 131071, 131072, 131073, 163840, 349525, 349526, 400001}) {
+        nb::HostCopier copier;
+        check(copied(copier, n, 6) && copied(copier, n, 3) && copied(copier, n, 1),
+              "HostCopier.everyArray", n);
+    }
+    for (size_t n : {21845, 131072, 400001}) without_heap(n);
+    return failures ? 1 : 0;
+}

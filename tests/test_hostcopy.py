@@ -1,0 +1,23 @@
+"""The read-back of device arrays (n-body-simulation_amd/csrc/nb_hostcopy.h) with
+stand-in HIP calls on the CPU: every array arrives whole at the edges of the copy
+paths, and failing host calls end in a status, not in an exception."""
+import os
+import subprocess
+
+from conftest import PKG
+
+HOSTCOPY_TESTS = os.path.join(PKG, "hostcopy_tests")
+
+
+def lines(name):
+    r = subprocess.run([HOSTCOPY_TESTS], capture_output=True, text=True, timeout=120)
+    assert r.returncode in (0, 1), (r.returncode, r.stdout, r.stderr)
+    return [l.split()[0] for l in r.stdout.splitlines() if l.split()[1] == "HostCopier." + name]
+
+
+def test_every_array_arrives():
+    assert lines("everyArray") == ["PASS"] * 10
+
+
+def test_no_exception_without_heap():
+    assert lines("withoutHeap") == ["PASS"] * 3
