@@ -45,12 +45,10 @@ class HostCopier {
 
     // Pinned memory for small copies of `doubles` in all, made with its owner: a
     // first copy would pay for the allocation and for a fault per page (1.6 us).
-    hipError_t reserve_small(size_t doubles) {
+    void reserve_small(size_t doubles) noexcept {
         const size_t bytes = doubles * sizeof(double);
-        if (bytes > kSmall) return hipSuccess;
-        const hipError_t e = reserve(bytes);
-        for (size_t o = 0; e == hipSuccess && o < bytes; o += 4096) ring_[o] = 0;
-        return e;
+        if (bytes > kSmall || !reserve(bytes)) return;
+        for (size_t o = 0; o < bytes; o += 4096) ring_[o] = 0;
     }
 
     ~HostCopier() {
@@ -65,8 +63,10 @@ class HostCopier {
         size_t total = 0;
         for (int k = 0; k < count; ++k) total += a[k].n * sizeof(double);
         if (total == 0) return hipStreamSynchronize(stream);
-        if (total <= kSmall) return small(stream, a, count, total);
-        if (total >= kLarge) return large(stream, a, count, total);
+        if (total <= kSmall && reserve(total)) return small(stream, a, count);
+        if (total >= kLarge && reserve(kSlots * chunk_bytes(total)) && make_events())
+            return large(stream, a, count, total);
+        // between the two, and where the runtime gives no pinned memory or events
         hipError_t e = hipSuccess;
         for (int k = 0; k < count && e == hipSuccess; ++k)
             e = hipMemcpyAsync(a[k].dst, a[k].src, a[k].n * sizeof(double), hipMemcpyDeviceToHost,
@@ -87,23 +87,34 @@ class HostCopier {
     hipEvent_t events_[kSlots] = {};
     uint32_t nevents_ = 0;
 
-    hipError_t reserve(size_t bytes) {
-        if (ring_bytes_ >= bytes) return hipSuccess;
+    static size_t chunk_bytes(size_t total) { return total < 16 * kChunk ? kChunk / 4 : kChunk; }
+
+    // false: refused, with the runtime's last error cleared (the caller has another way)
+    bool reserve(size_t bytes) {
+        if (ring_bytes_ >= bytes) return true;
         if (ring_) (void)hipHostFree(ring_);
         ring_ = nullptr;
         ring_bytes_ = 0;
-        const hipError_t e = hipHostMalloc((void **)&ring_, bytes, hipHostMallocDefault);
-        if (e != hipSuccess) {
+        if (hipHostMalloc((void **)&ring_, bytes, hipHostMallocDefault) != hipSuccess) {
             ring_ = nullptr;
-            return e;
+            (void)hipGetLastError();
+            return false;
         }
         ring_bytes_ = bytes;
-        return hipSuccess;
+        return true;
     }
 
-    hipError_t small(hipStream_t stream, const Array *a, int count, size_t total) {
-        hipError_t e = reserve(total);
-        if (e != hipSuccess) return e;
+    bool make_events() {
+        for (; nevents_ < kSlots; ++nevents_)
+            if (hipEventCreateWithFlags(&events_[nevents_], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                return false;
+            }
+        return true;
+    }
+
+    // ring_ holds the arrays
+    hipError_t small(hipStream_t stream, const Array *a, int count) {
         CopyOut arg{};
         size_t at = 0;
         for (int k = 0; k < count; ++k) {
@@ -113,7 +124,7 @@ class HostCopier {
             at += a[k].n;
         }
         launch_copy_out(arg, count, stream);
-        e = hipGetLastError();
+        const hipError_t e = hipGetLastError();
         const hipError_t s = hipStreamSynchronize(stream);
         if (e != hipSuccess) return e;
         if (s != hipSuccess) return s;
@@ -122,14 +133,10 @@ class HostCopier {
         return hipSuccess;
     }
 
+    // ring_ holds kSlots chunks and the events are there
     hipError_t large(hipStream_t stream, const Array *a, int count, size_t total) {
-        const size_t chunk = total < 16 * kChunk ? kChunk / 4 : kChunk;
-        hipError_t e = reserve(kSlots * chunk);
-        while (e == hipSuccess && nevents_ < kSlots) {
-            e = hipEventCreateWithFlags(&events_[nevents_], hipEventDisableTiming);
-            if (e == hipSuccess) ++nevents_;
-        }
-        if (e != hipSuccess) return e;
+        const size_t chunk = chunk_bytes(total);
+        hipError_t e = hipSuccess;
         struct Chunk {
             uint8_t *dst;
             const uint8_t *src;

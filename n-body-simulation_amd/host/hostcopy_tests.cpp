@@ -12,7 +12,10 @@
 
 namespace {
 
-bool no_heap = false;  // operator new fails
+bool no_heap = false;    // operator new fails
+bool no_pinned = false;  // hipHostMalloc fails
+bool no_events = false;  // hipEventCreateWithFlags fails
+hipError_t last_error = hipSuccess;
 
 int failures = 0;
 void check(bool ok, const char *name, size_t n) {
@@ -32,6 +35,7 @@ void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+    if (no_pinned) return last_error = hipErrorOutOfMemory;
     *p = std::malloc(bytes);
     return hipSuccess;
 }
@@ -40,6 +44,7 @@ hipError_t hipHostFree(void *p) {
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    if (no_events) return last_error = hipErrorOutOfMemory;
     *e = (hipEvent_t)std::malloc(1);
     return hipSuccess;
 }
@@ -50,7 +55,11 @@ hipError_t hipEventDestroy(hipEvent_t e) {
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t) {
     std::memcpy(dst, src, bytes);
     return hipSuccess;
@@ -114,5 +123,17 @@ int main() {
               "HostCopier.everyArray", n);
     }
     for (size_t n : {21845, 131072, 400001}) without_heap(n);
+    // without pinned memory, or without events: the runtime's own copies, and no
+    // error left behind for a later call
+    for (size_t n : {1, 21845, 131072, 400001}) {
+        for (bool *refused : {&no_pinned, &no_events}) {
+            nb::HostCopier copier;
+            *refused = true;
+            copier.reserve_small(6 * n);
+            const bool ok = copied(copier, n, 6) && copied(copier, n, 3) && last_error == hipSuccess;
+            *refused = false;
+            check(ok && copied(copier, n, 6), "HostCopier.refused", n);
+        }
+    }
     return failures ? 1 : 0;
 }

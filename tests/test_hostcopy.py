@@ -21,3 +21,7 @@ def test_every_array_arrives():
 
 def test_no_exception_without_heap():
     assert lines("withoutHeap") == ["PASS"] * 3
+
+
+def test_refused_pinned_memory_and_events():
+    assert lines("refused") == ["PASS"] * 8
