@@ -32,7 +32,7 @@ struct CopyOut {
     double *dst[6];
     size_t n[6];
 };
-void launch_copy_out(const CopyOut &c, int count, hipStream_t s);
+hipError_t launch_copy_out(const CopyOut &c, int count, hipStream_t s);
 
 class HostCopier {
   public:
@@ -123,8 +123,7 @@ class HostCopier {
             arg.n[k] = a[k].n;
             at += a[k].n;
         }
-        launch_copy_out(arg, count, stream);
-        const hipError_t e = hipGetLastError();
+        const hipError_t e = launch_copy_out(arg, count, stream);
         const hipError_t s = hipStreamSynchronize(stream);
         if (e != hipSuccess) return e;
         if (s != hipSuccess) return s;

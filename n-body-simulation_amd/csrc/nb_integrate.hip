@@ -95,12 +95,15 @@ __global__ void __launch_bounds__(kThreads) k_copy_out(CopyOut c) {
 
 }  // namespace
 
-void launch_copy_out(const CopyOut &c, int count, hipStream_t s) {
+// The launch's own status: the runtime's last error may be an older call's.
+hipError_t launch_copy_out(const CopyOut &c, int count, hipStream_t s) {
     size_t most = 0;
     for (int k = 0; k < count; ++k) most = std::max(most, c.n[k]);
-    if (most == 0) return;
+    if (most == 0) return hipSuccess;
     const uint32_t blocks = std::min<uint32_t>(64, ceil_div(most, kThreads));
-    hipLaunchKernelGGL(k_copy_out, dim3(blocks, count), dim3(kThreads), 0, s, c);
+    CopyOut arg = c;
+    void *args[] = {&arg};
+    return hipLaunchKernel((const void *)k_copy_out, dim3(blocks, count), dim3(kThreads), args, 0, s);
 }
 
 void launch_kick_kick_drift(uint32_t n, double dt, const double *ax, const double *ay,

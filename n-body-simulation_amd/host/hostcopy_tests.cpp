@@ -67,8 +67,9 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
 }
 
 namespace nb {
-void launch_copy_out(const CopyOut &c, int count, hipStream_t) {
+hipError_t launch_copy_out(const CopyOut &c, int count, hipStream_t) {
     for (int k = 0; k < count; ++k) std::memcpy(c.dst[k], c.src[k], c.n[k] * sizeof(double));
+    return hipSuccess;
 }
 }  // namespace nb
 
@@ -134,6 +135,14 @@ int main() {
             *refused = false;
             check(ok && copied(copier, n, 6), "HostCopier.refused", n);
         }
+    }
+    // an error that an older call left in the runtime is not this copy's, and stays
+    for (size_t n : {1, 21845, 131072, 400001}) {
+        nb::HostCopier copier;
+        last_error = hipErrorInvalidValue;
+        const bool ok = copied(copier, n, 6);
+        check(ok && last_error == hipErrorInvalidValue, "HostCopier.olderError", n);
+        last_error = hipSuccess;
     }
     return failures ? 1 : 0;
 }

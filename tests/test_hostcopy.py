@@ -25,3 +25,7 @@ def test_no_exception_without_heap():
 
 def test_refused_pinned_memory_and_events():
     assert lines("refused") == ["PASS"] * 8
+
+
+def test_older_error_is_not_reported():
+    assert lines("olderError") == ["PASS"] * 4
