@@ -63,6 +63,7 @@ class HostCopier {
         size_t total = 0;
         for (int k = 0; k < count; ++k) total += a[k].n * sizeof(double);
         if (total == 0) return hipStreamSynchronize(stream);
+        const OnDevice device(stream);
         if (total <= kSmall && reserve(total)) return small(stream, a, count);
         if (total >= kLarge && reserve(kSlots * chunk_bytes(total)) && make_events())
             return large(stream, a, count, total);
@@ -76,6 +77,21 @@ class HostCopier {
     }
 
   private:
+    // The stream's device is current while this lives, whatever the caller's is: an
+    // event is recorded, and a kernel launched, on the stream of its own device.
+    struct OnDevice {
+        int before = -1;
+        explicit OnDevice(hipStream_t stream) {
+            int own = 0, now = 0;
+            if (hipStreamGetDevice(stream, &own) == hipSuccess && hipGetDevice(&now) == hipSuccess &&
+                own != now && hipSetDevice(own) == hipSuccess)
+                before = now;
+        }
+        ~OnDevice() {
+            if (before >= 0) (void)hipSetDevice(before);
+        }
+    };
+
     static constexpr size_t kSmall = size_t(1) << 20;
     static constexpr size_t kLarge = size_t(6) << 20;
     static constexpr size_t kChunk = size_t(1) << 20;

@@ -16,6 +16,9 @@ bool no_heap = false;    // operator new fails
 bool no_pinned = false;  // hipHostMalloc fails
 bool no_events = false;  // hipEventCreateWithFlags fails
 hipError_t last_error = hipSuccess;
+int device = 0;        // the current one
+int stream_device = 0;  // the stream's
+bool wrong_device = false;  // an event or a launch of another device than the stream's
 
 int failures = 0;
 void check(bool ok, const char *name, size_t n) {
@@ -45,6 +48,7 @@ hipError_t hipHostFree(void *p) {
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
     if (no_events) return last_error = hipErrorOutOfMemory;
+    wrong_device |= device != stream_device;
     *e = (hipEvent_t)std::malloc(1);
     return hipSuccess;
 }
@@ -55,6 +59,18 @@ hipError_t hipEventDestroy(hipEvent_t e) {
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipGetDevice(int *d) {
+    *d = device;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int d) {
+    device = d;
+    return hipSuccess;
+}
+hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d) {
+    *d = stream_device;
+    return hipSuccess;
+}
 hipError_t hipGetLastError() {
     const hipError_t e = last_error;
     last_error = hipSuccess;
@@ -68,6 +84,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
 
 namespace nb {
 hipError_t launch_copy_out(const CopyOut &c, int count, hipStream_t) {
+    wrong_device |= device != stream_device;
     for (int k = 0; k < count; ++k) std::memcpy(c.dst[k], c.src[k], c.n[k] * sizeof(double));
     return hipSuccess;
 }
@@ -143,6 +160,14 @@ int main() {
         const bool ok = copied(copier, n, 6);
         check(ok && last_error == hipErrorInvalidValue, "HostCopier.olderError", n);
         last_error = hipSuccess;
+    }
+    // another device than the stream's is current: it is again afterwards
+    for (size_t n : {1, 131072, 400001}) {
+        nb::HostCopier copier;
+        stream_device = 1;
+        const bool ok = copied(copier, n, 6);
+        check(ok && !wrong_device && device == 0, "HostCopier.otherDevice", n);
+        stream_device = 0;
     }
     return failures ? 1 : 0;
 }

@@ -29,3 +29,7 @@ def test_refused_pinned_memory_and_events():
 
 def test_older_error_is_not_reported():
     assert lines("olderError") == ["PASS"] * 4
+
+
+def test_other_device_current():
+    assert lines("otherDevice") == ["PASS"] * 3
