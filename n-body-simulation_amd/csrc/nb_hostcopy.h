@@ -8,8 +8,9 @@
 //  - large ones (from kLarge) are cut into chunks that pass through a ring of
 //    pinned slots by DMA (56 GB/s), and several threads fill the caller's pages
 //    while later chunks are on their way.
-// In between, the runtime's copies into pageable memory are as fast (23,000
-// bodies 0.11 ms, 100,003 0.76; through the ring 0.57 and 0.65).
+// In between, the runtime's copies into pageable memory are the fastest: six arrays
+// of 131,073 bodies 0.40 ms, of 349,525 (16 MiB) 0.93, through the ring in chunks
+// of 256 KiB 0.59 and 1.38; of 360,000 0.94 and, in chunks of 1 MiB, 0.75.
 // Six arrays of 1024 bodies: 25 us instead of 105; of 1,048,576 bodies (50 MB)
 // 2.5 ms instead of 6.4; of 4,194,304 7.9 ms instead of 21.
 #pragma once
@@ -65,8 +66,8 @@ class HostCopier {
         if (total == 0) return hipStreamSynchronize(stream);
         const OnDevice device(stream);
         if (total <= kSmall && reserve(total)) return small(stream, a, count);
-        if (total >= kLarge && reserve(kSlots * chunk_bytes(total)) && make_events())
-            return large(stream, a, count, total);
+        if (total >= kLarge && reserve(kSlots * kChunk) && make_events())
+            return large(stream, a, count);
         // between the two, and where the runtime gives no pinned memory or events
         hipError_t e = hipSuccess;
         for (int k = 0; k < count && e == hipSuccess; ++k)
@@ -93,7 +94,7 @@ class HostCopier {
     };
 
     static constexpr size_t kSmall = size_t(1) << 20;
-    static constexpr size_t kLarge = size_t(6) << 20;
+    static constexpr size_t kLarge = size_t(16) << 20;
     static constexpr size_t kChunk = size_t(1) << 20;
     static constexpr uint32_t kSlots = 8;
     static constexpr unsigned kThreads = 8;
@@ -102,8 +103,6 @@ class HostCopier {
     size_t ring_bytes_ = 0;
     hipEvent_t events_[kSlots] = {};
     uint32_t nevents_ = 0;
-
-    static size_t chunk_bytes(size_t total) { return total < 16 * kChunk ? kChunk / 4 : kChunk; }
 
     // false: refused, with the runtime's last error cleared (the caller has another way)
     bool reserve(size_t bytes) {
@@ -149,8 +148,7 @@ class HostCopier {
     }
 
     // ring_ holds kSlots chunks and the events are there
-    hipError_t large(hipStream_t stream, const Array *a, int count, size_t total) {
-        const size_t chunk = chunk_bytes(total);
+    hipError_t large(hipStream_t stream, const Array *a, int count) {
         hipError_t e = hipSuccess;
         struct Chunk {
             uint8_t *dst;
@@ -160,14 +158,14 @@ class HostCopier {
         // array k has the chunks [first[k], first[k + 1])
         uint32_t first[kArrays + 1] = {};
         for (int k = 0; k < count; ++k)
-            first[k + 1] = first[k] + (uint32_t)((a[k].n * sizeof(double) + chunk - 1) / chunk);
+            first[k + 1] = first[k] + (uint32_t)((a[k].n * sizeof(double) + kChunk - 1) / kChunk);
         const uint32_t n = first[count];
         const auto chunk_at = [&](uint32_t i) {
             int k = 0;
             while (i >= first[k + 1]) ++k;
-            const size_t o = (size_t)(i - first[k]) * chunk;
+            const size_t o = (size_t)(i - first[k]) * kChunk;
             return Chunk{(uint8_t *)a[k].dst + o, (const uint8_t *)a[k].src + o,
-                         std::min(chunk, a[k].n * sizeof(double) - o)};
+                         std::min(kChunk, a[k].n * sizeof(double) - o)};
         };
         // Chunk i goes through slot i mod kSlots.  This thread issues the DMAs and
         // waits for them in order; arrived: chunks that lie in their slots;
@@ -179,7 +177,7 @@ class HostCopier {
         std::atomic<bool> failed{false};
         auto fill = [&](uint32_t i) {
             const Chunk c = chunk_at(i);
-            std::memcpy(c.dst, ring_ + (i % kSlots) * chunk, c.bytes);
+            std::memcpy(c.dst, ring_ + (i % kSlots) * kChunk, c.bytes);
             filled[i % kSlots].store(i / kSlots + 1, std::memory_order_release);
         };
         auto worker = [&] {
@@ -197,7 +195,7 @@ class HostCopier {
         const unsigned cores = std::max(1u, std::thread::hardware_concurrency());
         try {
             threads.reserve(kThreads);
-            for (unsigned t = 0; t < std::min(cores, total < 16 * kChunk ? 4u : kThreads); ++t)
+            for (unsigned t = 0; t < std::min(cores, kThreads); ++t)
                 threads.emplace_back(worker);
         } catch (...) {  // fewer threads, or none
         }
@@ -205,7 +203,7 @@ class HostCopier {
             if (issued < n && issued - got < kSlots &&
                 filled[issued % kSlots].load(std::memory_order_acquire) >= issued / kSlots) {
                 const Chunk c = chunk_at(issued);
-                e = hipMemcpyAsync(ring_ + (issued % kSlots) * chunk, c.src, c.bytes,
+                e = hipMemcpyAsync(ring_ + (issued % kSlots) * kChunk, c.src, c.bytes,
                                    hipMemcpyDeviceToHost, stream);
                 if (e == hipSuccess) e = hipEventRecord(events_[issued % kSlots], stream);
                 ++issued;

@@ -16,6 +16,7 @@ bool no_heap = false;    // operator new fails
 bool no_pinned = false;  // hipHostMalloc fails
 bool no_events = false;  // hipEventCreateWithFlags fails
 hipError_t last_error = hipSuccess;
+int copies = 0;  // runtime copies since it was reset
 int device = 0;        // the current one
 int stream_device = 0;  // the stream's
 bool wrong_device = false;  // an event or a launch of another device than the stream's
@@ -77,6 +78,7 @@ hipError_t hipGetLastError() {
     return e;
 }
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t) {
+    ++copies;
     std::memcpy(dst, src, bytes);
     return hipSuccess;
 }
@@ -133,14 +135,22 @@ void without_heap(size_t n) {
 }  // namespace
 
 int main() {
-    // edges of the small copies (1 MiB in all), the chunked ones (6 MiB), their
-    // chunk sizes (16 MiB in all) and a chunk's end (six arrays, or one)
+    // edges of the small copies (1 MiB in all), the chunked ones (16 MiB) and a
+    // chunk's end (six arrays, or one)
     for (size_t n : {1, 21845, 21846, 131071, 131072, 131073, 163840, 349525, 349526, 400001}) {
         nb::HostCopier copier;
         check(copied(copier, n, 6) && copied(copier, n, 3) && copied(copier, n, 1),
               "HostCopier.everyArray", n);
     }
     for (size_t n : {21845, 131072, 400001}) without_heap(n);
+    // from 1 to 16 MiB in all: one runtime copy per array; from there on, one per MiB
+    for (size_t n : {22000, 131072, 131073, 349525, 349526, 400001}) {
+        nb::HostCopier copier;
+        const int chunks = (int)((n * sizeof(double) + (1 << 20) - 1) >> 20);
+        copies = 0;
+        const bool ok = copied(copier, n, 6);
+        check(ok && copies == 6 * (n < 349526 ? 1 : chunks), "HostCopier.copiesPerArray", n);
+    }
     // without pinned memory, or without events: the runtime's own copies, and no
     // error left behind for a later call
     for (size_t n : {1, 21845, 131072, 400001}) {

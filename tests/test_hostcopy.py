@@ -33,3 +33,7 @@ def test_older_error_is_not_reported():
 
 def test_other_device_current():
     assert lines("otherDevice") == ["PASS"] * 3
+
+
+def test_copies_per_array():
+    assert lines("copiesPerArray") == ["PASS"] * 6
