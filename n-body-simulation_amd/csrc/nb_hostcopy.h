@@ -66,15 +66,27 @@ class HostCopier {
         if (total == 0) return hipStreamSynchronize(stream);
         const OnDevice device(stream);
         if (total <= kSmall && reserve(total)) return small(stream, a, count);
-        if (total >= kLarge && reserve(kSlots * kChunk) && make_events())
-            return large(stream, a, count);
-        // between the two, and where the runtime gives no pinned memory or events
-        hipError_t e = hipSuccess;
-        for (int k = 0; k < count && e == hipSuccess; ++k)
-            e = hipMemcpyAsync(a[k].dst, a[k].src, a[k].n * sizeof(double), hipMemcpyDeviceToHost,
-                               stream);
-        const hipError_t s = hipStreamSynchronize(stream);
-        return e != hipSuccess ? e : s;
+        if (total < kLarge) return runtime(stream, a, count);
+        // Pinned memory of the caller's takes a DMA itself: six arrays of 360,000
+        // bodies 0.36 ms, through the ring 0.75; of 1,048,576 0.94 and 1.77.
+        Array paged[kArrays], pinned[kArrays];
+        int npaged = 0, npinned = 0;
+        size_t bytes = 0;
+        for (int k = 0; k < count; ++k) {
+            if (is_pinned(a[k].dst)) {
+                pinned[npinned++] = a[k];
+            } else {
+                paged[npaged++] = a[k];
+                bytes += a[k].n * sizeof(double);
+            }
+        }
+        if (npinned) {
+            const hipError_t e = runtime(stream, pinned, npinned);
+            if (e != hipSuccess) return e;
+        }
+        if (bytes >= kLarge && reserve(kSlots * kChunk) && make_events())
+            return large(stream, paged, npaged);
+        return runtime(stream, paged, npaged);  // a few, or no ring to be had
     }
 
   private:
@@ -126,6 +138,24 @@ class HostCopier {
                 return false;
             }
         return true;
+    }
+
+    static bool is_pinned(const void *p) {
+        hipPointerAttribute_t at;
+        if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        return at.type == hipMemoryTypeHost;
+    }
+
+    hipError_t runtime(hipStream_t stream, const Array *a, int count) {
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < count && e == hipSuccess; ++k)
+            e = hipMemcpyAsync(a[k].dst, a[k].src, a[k].n * sizeof(double), hipMemcpyDeviceToHost,
+                               stream);
+        const hipError_t s = hipStreamSynchronize(stream);
+        return e != hipSuccess ? e : s;
     }
 
     // ring_ holds the arrays

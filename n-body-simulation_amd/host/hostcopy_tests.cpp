@@ -16,6 +16,7 @@ bool no_heap = false;    // operator new fails
 bool no_pinned = false;  // hipHostMalloc fails
 bool no_events = false;  // hipEventCreateWithFlags fails
 hipError_t last_error = hipSuccess;
+const void *pinned_from = nullptr, *pinned_to = nullptr;  // the caller's pinned memory
 int copies = 0;  // runtime copies since it was reset
 int device = 0;        // the current one
 int stream_device = 0;  // the stream's
@@ -70,6 +71,11 @@ hipError_t hipSetDevice(int d) {
 }
 hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d) {
     *d = stream_device;
+    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *at, const void *p) {
+    *at = hipPointerAttribute_t{};
+    at->type = p >= pinned_from && p < pinned_to ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
     return hipSuccess;
 }
 hipError_t hipGetLastError() {
@@ -132,6 +138,23 @@ void without_heap(size_t n) {
     check(ok && dst == src, "HostCopier.withoutHeap", n);
 }
 
+// The first `own` of six arrays lie in pinned memory of the caller's.
+void pinned_destinations(size_t n, int own) {
+    std::vector<double> src(6 * n), dst(6 * n, -1.0);
+    for (size_t i = 0; i < src.size(); ++i) src[i] = (double)i;
+    nb::HostCopier::Array a[6];
+    for (int k = 0; k < 6; ++k) a[k] = {dst.data() + k * n, src.data() + k * n, n};
+    pinned_from = dst.data();
+    pinned_to = dst.data() + own * n;
+    nb::HostCopier copier;
+    copies = 0;
+    const bool ok = copier.copy(nullptr, a, 6) == hipSuccess && dst == src;
+    const int chunks = (int)((n * sizeof(double) + (1 << 20) - 1) >> 20);
+    const bool ring = (6 - own) * n * sizeof(double) >= 16u << 20;
+    check(ok && copies == own + (6 - own) * (ring ? chunks : 1), "HostCopier.pinned", n);
+    pinned_from = pinned_to = nullptr;
+}
+
 }  // namespace
 
 int main() {
@@ -171,6 +194,7 @@ int main() {
         check(ok && last_error == hipErrorInvalidValue, "HostCopier.olderError", n);
         last_error = hipSuccess;
     }
+    for (int own : {1, 3, 6}) pinned_destinations(400001, own);
     // another device than the stream's is current: it is again afterwards
     for (size_t n : {1, 131072, 400001}) {
         nb::HostCopier copier;

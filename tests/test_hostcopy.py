@@ -37,3 +37,7 @@ def test_other_device_current():
 
 def test_copies_per_array():
     assert lines("copiesPerArray") == ["PASS"] * 6
+
+
+def test_pinned_destinations_take_the_dma():
+    assert lines("pinned") == ["PASS"] * 3
