@@ -65,7 +65,7 @@ class HostCopier {
         for (int k = 0; k < count; ++k) total += a[k].n * sizeof(double);
         if (total == 0) return hipStreamSynchronize(stream);
         const OnDevice device(stream);
-        if (total <= kSmall && reserve(total)) return small(stream, a, count);
+        if (total <= (count == 1 ? kOne : kSmall) && reserve(total)) return small(stream, a, count);
         if (total < kLarge) return runtime(stream, a, count);
         // Pinned memory of the caller's takes a DMA itself: six arrays of 360,000
         // bodies 0.36 ms, through the ring 0.75; of 1,048,576 0.94 and 1.77.
@@ -106,6 +106,9 @@ class HostCopier {
     };
 
     static constexpr size_t kSmall = size_t(1) << 20;
+    // One array alone: the runtime takes 21 us up to 16 KiB and 9.1 us just above (64
+    // KiB 11.4, 1 MiB 64), the kernel 13.4 and as much (14.5, 66).
+    static constexpr size_t kOne = size_t(16) << 10;
     static constexpr size_t kLarge = size_t(16) << 20;
     static constexpr size_t kChunk = size_t(1) << 20;
     static constexpr uint32_t kSlots = 8;

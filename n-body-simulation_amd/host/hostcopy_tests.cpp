@@ -194,6 +194,13 @@ int main() {
         check(ok && last_error == hipErrorInvalidValue, "HostCopier.olderError", n);
         last_error = hipSuccess;
     }
+    // one array alone: without a runtime copy up to 16 KiB
+    for (size_t n : {1, 2048, 2049, 131072, 131073}) {
+        nb::HostCopier copier;
+        copies = 0;
+        const bool ok = copied(copier, n, 1);
+        check(ok && copies == (n <= 2048 ? 0 : 1), "HostCopier.oneArray", n);
+    }
     for (int own : {1, 3, 6}) pinned_destinations(400001, own);
     // another device than the stream's is current: it is again afterwards
     for (size_t n : {1, 131072, 400001}) {

@@ -41,3 +41,7 @@ def test_copies_per_array():
 
 def test_pinned_destinations_take_the_dma():
     assert lines("pinned") == ["PASS"] * 3
+
+
+def test_one_array():
+    assert lines("oneArray") == ["PASS"] * 5
