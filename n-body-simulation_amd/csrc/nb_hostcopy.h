@@ -8,8 +8,10 @@
 //  - large ones (from kLarge) are cut into chunks that pass through a ring of
 //    pinned slots by DMA (56 GB/s), and several threads fill the caller's pages
 //    while later chunks are on their way.
-// In between, the runtime's copies into pageable memory are the fastest: six arrays
-// of 131,073 bodies 0.40 ms, of 349,525 (16 MiB) 0.93, through the ring in chunks
+// In between, the runtime's copies into pageable memory are as fast or the fastest:
+// six arrays of 21,846 bodies (1 MiB) 0.100 ms and by the kernel 0.061, of 43,690
+// (2 MiB) 0.146 and 0.107, but into the caller's pinned memory 0.095 and 0.098; of
+// 131,073 bodies 0.40 ms, of 349,525 (16 MiB) 0.93, through the ring in chunks
 // of 256 KiB 0.59 and 1.38; of 360,000 0.94 and, in chunks of 1 MiB, 0.75.
 // Six arrays of 1024 bodies: 25 us instead of 105; of 1,048,576 bodies (50 MB)
 // 2.5 ms instead of 6.4; of 4,194,304 7.9 ms instead of 21.
@@ -105,7 +107,7 @@ class HostCopier {
         }
     };
 
-    static constexpr size_t kSmall = size_t(1) << 20;
+    static constexpr size_t kSmall = size_t(7) << 18;
     // One array alone: the runtime takes 21 us up to 16 KiB and 9.1 us just above (64
     // KiB 11.4, 1 MiB 64), the kernel 13.4 and as much (14.5, 66).
     static constexpr size_t kOne = size_t(16) << 10;

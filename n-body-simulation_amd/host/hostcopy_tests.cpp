@@ -158,21 +158,22 @@ void pinned_destinations(size_t n, int own) {
 }  // namespace
 
 int main() {
-    // edges of the small copies (1 MiB in all), the chunked ones (16 MiB) and a
+    // edges of the small copies (1.75 MiB in all), the chunked ones (16 MiB) and a
     // chunk's end (six arrays, or one)
-    for (size_t n : {1, 21845, 21846, 131071, 131072, 131073, 163840, 349525, 349526, 400001}) {
+    for (size_t n : {1, 38229, 38230, 131071, 131072, 131073, 163840, 349525, 349526, 400001}) {
         nb::HostCopier copier;
         check(copied(copier, n, 6) && copied(copier, n, 3) && copied(copier, n, 1),
               "HostCopier.everyArray", n);
     }
     for (size_t n : {21845, 131072, 400001}) without_heap(n);
-    // from 1 to 16 MiB in all: one runtime copy per array; from there on, one per MiB
-    for (size_t n : {22000, 131072, 131073, 349525, 349526, 400001}) {
+    // up to 1.75 MiB in all: no runtime copy; to 16 MiB one per array; from there on,
+    // one per MiB
+    for (size_t n : {21846, 38229, 38230, 131072, 131073, 349525, 349526, 400001}) {
         nb::HostCopier copier;
         const int chunks = (int)((n * sizeof(double) + (1 << 20) - 1) >> 20);
         copies = 0;
         const bool ok = copied(copier, n, 6);
-        check(ok && copies == 6 * (n < 349526 ? 1 : chunks), "HostCopier.copiesPerArray", n);
+        check(ok && copies == 6 * (n < 38230 ? 0 : n < 349526 ? 1 : chunks), "HostCopier.copiesPerArray", n);
     }
     // without pinned memory, or without events: the runtime's own copies, and no
     // error left behind for a later call

@@ -36,7 +36,7 @@ def test_other_device_current():
 
 
 def test_copies_per_array():
-    assert lines("copiesPerArray") == ["PASS"] * 6
+    assert lines("copiesPerArray") == ["PASS"] * 8
 
 
 def test_pinned_destinations_take_the_dma():
