@@ -471,7 +471,7 @@ int nb_create(nb_ctx **out, uint32_t n, const nb_params *p) {
     if (hipHostMalloc((void **)&c->hdr_host, sizeof(TreeHdr), hipHostMallocDefault) != hipSuccess)
         return bail(NB_E_HIP);
     std::memset(c->hdr_host, 0, sizeof(TreeHdr));
-    c->copier.reserve_small(6ull * n);
+    c->copier.reserve_for(n);
     if ((rc = alloc_tree(c))) return bail(rc);
     if (p->quadrupole && (rc = ensure_quad_buffers(c))) return bail(rc);
     if (hipMemsetAsync(c->x, 0, 13 * c->stride * sizeof(double), c->stream) != hipSuccess)

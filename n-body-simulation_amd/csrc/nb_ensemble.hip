@@ -347,7 +347,7 @@ int nb_ensemble_create(nb_ensemble **out, uint32_t nsys, const uint32_t *sizes,
         return bail(rc);
     f.slots = (uint32_t)fo;
     f.scan_cap = nb::scan_scratch_words((uint32_t)fo) + 1;
-    e->copier.reserve_small(6 * total);
+    e->copier.reserve_for(total);
     if (hipHostMalloc((void **)&e->status_host, sizeof(uint32_t), hipHostMallocDefault) != hipSuccess)
         return bail(NB_E_HIP);
     *e->status_host = 0;

@@ -17,6 +17,7 @@ bool no_pinned = false;  // hipHostMalloc fails
 bool no_events = false;  // hipEventCreateWithFlags fails
 hipError_t last_error = hipSuccess;
 const void *pinned_from = nullptr, *pinned_to = nullptr;  // the caller's pinned memory
+int allocations = 0;  // of pinned memory and events, since it was reset
 int copies = 0;  // runtime copies since it was reset
 int device = 0;        // the current one
 int stream_device = 0;  // the stream's
@@ -40,6 +41,7 @@ void operator delete(void *p, size_t) noexcept { std::free(p); }
 
 extern "C" {
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+    ++allocations;
     if (no_pinned) return last_error = hipErrorOutOfMemory;
     *p = std::malloc(bytes);
     return hipSuccess;
@@ -49,6 +51,7 @@ hipError_t hipHostFree(void *p) {
     return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) {
+    ++allocations;
     if (no_events) return last_error = hipErrorOutOfMemory;
     wrong_device |= device != stream_device;
     *e = (hipEvent_t)std::malloc(1);
@@ -181,7 +184,7 @@ int main() {
         for (bool *refused : {&no_pinned, &no_events}) {
             nb::HostCopier copier;
             *refused = true;
-            copier.reserve_small(6 * n);
+            copier.reserve_for(n);
             const bool ok = copied(copier, n, 6) && copied(copier, n, 3) && last_error == hipSuccess;
             *refused = false;
             check(ok && copied(copier, n, 6), "HostCopier.refused", n);
@@ -201,6 +204,14 @@ int main() {
         copies = 0;
         const bool ok = copied(copier, n, 1);
         check(ok && copies == (n <= 2048 ? 0 : 1), "HostCopier.oneArray", n);
+    }
+    // what the copies of a state and of accelerations need is made with the owner
+    for (size_t n : {1, 21846, 38229, 38230, 76458, 76459, 349525, 349526, 700000}) {
+        nb::HostCopier copier;
+        copier.reserve_for(n);
+        allocations = 0;
+        const bool ok = copied(copier, n, 6) && copied(copier, n, 3);
+        check(ok && allocations == 0, "HostCopier.madeWithOwner", n);
     }
     for (int own : {1, 3, 6}) pinned_destinations(400001, own);
     // another device than the stream's is current: it is again afterwards

@@ -45,3 +45,7 @@ def test_pinned_destinations_take_the_dma():
 
 def test_one_array():
     assert lines("oneArray") == ["PASS"] * 5
+
+
+def test_made_with_owner():
+    assert lines("madeWithOwner") == ["PASS"] * 9
