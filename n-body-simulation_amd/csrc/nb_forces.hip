@@ -370,10 +370,10 @@ __global__ void __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per
 k_direct_f32c(uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
               const double *__restrict__ z, const double *__restrict__ m, double G, float eps2,
               uint32_t chunk, double *partial, double *ax_out, double *ay_out, double *az_out) {
-    __shared__ double comb[kSplitWaves * 3 * 64 * PL];
-    static_assert(sizeof(float4) * kSplitTile * kSplitWaves <= sizeof(comb), "stages fit");
+    __shared__ double4 lds[kSplitWaves * 3 * 16 * PL];  // the stages, then the waves' sums
+    static_assert(sizeof(float4) * kSplitTile * kSplitWaves <= sizeof(lds), "stages fit");
     const uint32_t lane = threadIdx.x & 63u;
-    float4 *stage = reinterpret_cast<float4 *>(comb) + (threadIdx.x >> 6) * kSplitTile;
+    float4 *stage = table_as<float4>(lds) + (threadIdx.x >> 6) * kSplitTile;
     asm("" : "+v"(eps2));  // a scalar operand would end the double issue
     float px[PL], py[PL], pz[PL], fx[PL], fy[PL], fz[PL];
     double ax[PL], ay[PL], az[PL];
@@ -439,7 +439,7 @@ k_direct_f32c(uint32_t n, const double *__restrict__ x, const double *__restrict
                 fx[q] = fy[q] = fz[q] = 0.f;
             }
         });
-    split_finish<PL>(n, 1.0, ax, ay, az, comb, partial, ax_out, ay_out, az_out);
+    split_finish<PL>(n, 1.0, ax, ay, az, table_as<double>(lds), partial, ax_out, ay_out, az_out);
 }
 
 // FP64 pairs (the reference's formula, NaiveAlgorithm.cpp:318-351, with
@@ -451,10 +451,10 @@ __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
     uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, double G, double eps2,
     uint32_t chunk, double *partial, double *ax_out, double *ay_out, double *az_out) {
-    __shared__ double comb[kSplitWaves * 3 * 64 * kF64fPerLane];
-    static_assert(sizeof(double4) * kSplitTile * kSplitWaves <= sizeof(comb), "stages fit");
+    __shared__ double4 lds[kSplitWaves * 3 * 16 * kF64fPerLane];  // the stages, then the waves' sums
+    static_assert(sizeof(double4) * kSplitTile * kSplitWaves <= sizeof(lds), "stages fit");
     const uint32_t lane = threadIdx.x & 63u;
-    double4 *stage = reinterpret_cast<double4 *>(comb) + (threadIdx.x >> 6) * kSplitTile;
+    double4 *stage = lds + (threadIdx.x >> 6) * kSplitTile;
     double px[kF64fPerLane], py[kF64fPerLane], pz[kF64fPerLane];
     double ax[kF64fPerLane], ay[kF64fPerLane], az[kF64fPerLane];
 #pragma unroll
@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
             }
         },
         [] {});
-    split_finish<kF64fPerLane>(n, G, ax, ay, az, comb, partial, ax_out, ay_out, az_out);
+    split_finish<kF64fPerLane>(n, G, ax, ay, az, table_as<double>(lds), partial, ax_out, ay_out, az_out);
 }
 
 // ---------------------------------------------------------------------------

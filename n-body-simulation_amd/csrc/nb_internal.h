@@ -89,7 +89,7 @@ struct GroupRule {
     uint32_t pack_max;   // sibling groups are packed in cells of at most this many bodies
 };
 
-struct InternalSums {
+struct alignas(double4) InternalSums {  // read as one double4
     double x, y, z, m;  // centre-of-mass numerators and mass
 };
 
@@ -137,6 +137,15 @@ constexpr uint32_t kComSuper = kComBlock * kComSuperBlocks;
 __device__ inline void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// A table seen as an array of another type.  A vector access needs the alignment of
+// its type, which the table's declared element must have: an LDS array of doubles is
+// only promised 8 bytes, wherever the compiler happens to put it.
+template <typename T, typename U>
+__device__ inline T *table_as(U *table) {
+    static_assert(alignof(U) % alignof(T) == 0, "the table's elements are aligned for T");
+    return reinterpret_cast<T *>(table);
 }
 
 // Device buffers of one octree.

@@ -841,9 +841,10 @@ __device__ inline void com_levels(uint32_t kb, uint32_t ke, Keep keep,
 template <uint32_t kThreads_, uint32_t kCell>
 __device__ __forceinline__ void sum_levels(uint32_t t, const uint32_t *cnt,
                                            unsigned long long lv, const uint16_t *order,
-                                           const uint16_t *at_s, double (*term)[4], uint32_t *m_s) {
+                                           const uint16_t *at_s, double4 *term4, uint32_t *m_s) {
     constexpr uint32_t step = kThreads_ / 4;
     const uint32_t comp = t & 3u;
+    double *term = table_as<double>(term4) + comp;  // place p at term[4 p]
     const int starts = (int)cnt[min(t & 63u, (uint32_t)kMaxDepth)];
     uint32_t base = 0, end = 0;  // the next step's cells [base, min(base + step, end)): uniform
     bool fresh = false;          // the next step opens a level
@@ -883,7 +884,7 @@ __device__ __forceinline__ void sum_levels(uint32_t t, const uint32_t *cnt,
             double v[8];
             uint32_t m[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) v[k] = term[at[k]][comp];
+            for (int k = 0; k < 8; ++k) v[k] = term[4 * at[k]];
 #pragma unroll
             for (int k = 0; k < 8; ++k) m[k] = m_s[at[k]];
             double sum = 0;
@@ -893,7 +894,7 @@ __device__ __forceinline__ void sum_levels(uint32_t t, const uint32_t *cnt,
                 sum += v[k];
                 count += m[k];
             }
-            term[kCell + c][comp] = sum;
+            term[4 * (kCell + c)] = sum;
             m_s[kCell + c] = count;  // the same from all four lanes
         }
         if (kThreads_ == 64)
@@ -945,7 +946,7 @@ __device__ __forceinline__ void com_local_block(
     constexpr uint32_t nt = kComLocalThreads;
     __shared__ uint32_t cnt[kMaxDepth + 1], cur[kMaxDepth];
     __shared__ unsigned long long levels;        // bit d: a local cell of depth d
-    __shared__ double term_s[kTermZero + 1][4];  // {x m, y m, z m, m}: bodies, cells, zero
+    __shared__ double4 term_s[kTermZero + 1];    // {x m, y m, z m, m}: bodies, cells, zero
     __shared__ uint32_t m_s[kTermZero + 1];      // bodies of a term: 1, a cell's count, 0
     __shared__ uint32_t i_s[kComBlock];          // input index of a body
     __shared__ alignas(16) uint16_t at_s[8 * kComLdsCells];  // child slot: place of its term
@@ -997,7 +998,7 @@ __device__ __forceinline__ void com_local_block(
         cd[q] = int_local[kb + c] == 1 ? d : (uint32_t)kMaxDepth;
     }
     if (t <= (uint32_t)kMaxDepth) cnt[t] = 0;
-    if (t < 4) term_s[kTermZero][t] = 0.0;
+    if (t < 4) table_as<double>(&term_s[kTermZero])[t] = 0.0;
     if (t == 4) m_s[kTermZero] = 0;
     if (fits) {
         constexpr uint32_t z2 = kTermZero | kTermZero << 16;
@@ -1013,7 +1014,7 @@ __device__ __forceinline__ void com_local_block(
         const uint32_t p = t + q * nt;
         if (s + p >= e) continue;
         if (b[q].w == 0) raise_flag(h, kFlagZeroMass);
-        *reinterpret_cast<double4 *>(term_s[p]) = body_term(b[q]);
+        term_s[p] = body_term(b[q]);
         m_s[p] = 1;
         i_s[p] = bi[q];
         const uint64_t j = (uint64_t)bn[q] - slot0;
@@ -1071,7 +1072,7 @@ __device__ __forceinline__ void com_local_block(
     for (int q = 0; q < kComCellsPerThread; ++q) {
         const uint32_t c = t + q * nt;
         if (cd[q] >= (uint32_t)kMaxDepth) continue;
-        const double4 g = *reinterpret_cast<const double4 *>(term_s[kTermCell + c]);
+        const double4 g = term_s[kTermCell + c];
         const uint32_t count = m_s[kTermCell + c];
         if (g.w == 0) raise_flag(h, kFlagZeroMass);
         sums[kb + c] = InternalSums{g.x, g.y, g.z, g.w};
@@ -1087,11 +1088,11 @@ __device__ __forceinline__ void com_local_block(
             put_record(o, 0, (int32_t)(kb + c), com);
             if (count <= o.rule.group_max) put_group(o, cf[q], count);
         }
-        *reinterpret_cast<double4 *>(term_s[kTermCell + c]) = com;
+        term_s[kTermCell + c] = com;
     }
 #pragma unroll
     for (int q = 0; q < kComBodiesPerThread; ++q) {
-        double4 *v = reinterpret_cast<double4 *>(term_s[t + q * nt]);
+        double4 *v = &term_s[t + q * nt];
         if (s + t + q * nt < e) *v = term_com(*v);
     }
     __syncthreads();
@@ -1109,7 +1110,7 @@ __device__ __forceinline__ void com_local_block(
         }
 #pragma unroll
         for (int q = 0; q < kAhead; ++q) {
-            v[q] = *reinterpret_cast<const double4 *>(term_s[at[q]]);
+            v[q] = term_s[at[q]];
             bi2[q] = i_s[min(at[q], kComBlock - 1)];
         }
 #pragma unroll
@@ -1168,7 +1169,7 @@ __device__ __forceinline__ void com_span_block(
     __shared__ uint32_t list[kSpanCells];  // cell index by LDS id
     __shared__ uint8_t ldep[kSpanCells];
     __shared__ uint16_t order[kSpanCells];  // LDS ids bucketed by depth
-    __shared__ double term[9 * kSpanCells][4];  // terms of child slots (0 if empty), sums
+    __shared__ double4 term[9 * kSpanCells];  // terms of child slots (0 if empty), sums
     __shared__ uint32_t m_s[9 * kSpanCells];    // their bodies
     __shared__ alignas(16) uint16_t at_s[8 * kSpanCells];  // child slot: place of its term
     const uint32_t t = threadIdx.x;
@@ -1283,7 +1284,7 @@ __device__ __forceinline__ void com_span_block(
             kind[q] = int_local[r[q]];
             here[q] = cid[r[q]];
             count[q] = counts[r[q]];
-            v[q] = *reinterpret_cast<const double4 *>(&sums[r[q]]);
+            v[q] = *table_as<const double4>(&sums[r[q]]);
         } else if (r[q] != kRefEmpty) {
             v[q] = body4[body_of_ref(r[q])];
         }
@@ -1301,7 +1302,7 @@ __device__ __forceinline__ void com_span_block(
                 v[q] = body_term(v[q]);
                 count[q] = 1;
             }
-            *reinterpret_cast<double4 *>(term[p]) = v[q];
+            term[p] = v[q];
             m_s[p] = count[q];
         }
         at_s[p] = (uint16_t)at;
@@ -1319,7 +1320,7 @@ __device__ __forceinline__ void com_span_block(
     // the cells summed here: sums, record (the root's is node 0), group marks
     if (t < nk) {
         const uint32_t k = list[t], bodies = m_s[kSpanSum + t];
-        const double4 g = *reinterpret_cast<const double4 *>(term[kSpanSum + t]);
+        const double4 g = term[kSpanSum + t];
         if (g.w == 0) raise_flag(h, kFlagZeroMass);
         sums[k] = InternalSums{g.x, g.y, g.z, g.w};
         counts[k] = bodies;
