@@ -326,7 +326,8 @@ __device__ __forceinline__ void split_stages(uint32_t j0, uint32_t j1,
                                              const double *__restrict__ z,
                                              const double *__restrict__ m, T4 *stage, T4 pad,
                                              Pack pack, Use use, EndRun end_run) {
-    const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+    // uniform: the lanes of a wave hand each other their stage in these loops
+    const uint32_t lane = threadIdx.x & 63u, w = wave_uniform(threadIdx.x >> 6);
     constexpr uint32_t run = kRun * kSplitTile;
     double sx = 0, sy = 0, sz = 0, sm = 0;
     auto load = [&](uint32_t j) {
