@@ -341,8 +341,15 @@ __device__ __forceinline__ void split_stages(uint32_t j0, uint32_t j1,
     uint32_t k = j0 + w * run, end = k + run;
     load(k + lane);
     while (k < j1) {
+        // by component: a select between two structures goes through scratch memory
         const T4 p = pack(sx, sy, sz, sm);
-        stage[lane] = k + lane < j1 ? p : pad;
+        const bool real = k + lane < j1;
+        T4 s;
+        s.x = real ? p.x : pad.x;
+        s.y = real ? p.y : pad.y;
+        s.z = real ? p.z : pad.z;
+        s.w = real ? p.w : pad.w;
+        stage[lane] = s;
         const uint32_t cnt = min(kSplitTile, j1 - k);
         k += kSplitTile;
         const bool last = k == end || k >= j1;
