@@ -822,7 +822,12 @@ k_bh_exact_wave(uint32_t n, const uint32_t *__restrict__ order, const double *__
         const uint32_t k = (uint32_t)level % kFrames;
         wave_lds_sync();
         if (lane < 8) {
-            L.cm[k][lane] = c;
+            // by component: the compiler passes a whole structure through scratch memory
+            double *to = table_as<double>(&L.cm[k][lane]);
+            to[0] = c.x;
+            to[1] = c.y;
+            to[2] = c.z;
+            to[3] = c.w;
             L.ref[k][lane] = r;
         }
         wave_lds_sync();

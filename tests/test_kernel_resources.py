@@ -41,7 +41,8 @@ def scratch(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("kernel,count", [("k_direct_f32c", 2), ("k_direct_f64f", 1)])
+@pytest.mark.parametrize("kernel,count", [("k_direct_f32c", 2), ("k_direct_f64f", 1),
+                                          ("k_bh_exact_wave", 1)])
 def test_no_scratch(scratch, kernel, count):
     sizes = {k: v for k, v in scratch.items() if kernel in k}
     assert len(sizes) == count, sizes
