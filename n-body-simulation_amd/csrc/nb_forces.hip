@@ -2144,24 +2144,35 @@ void launch_bh_exact(const TreeBufs &t, const double *x, const double *y, const 
                      double G, double eps2, double theta, double *ax, double *ay, double *az,
                      uint32_t *interactions, hipStream_t s) {
     // Waves of 64 bodies from 100,000 bodies at theta 0.5 and below, up to
-    // 210,000 at theta 1.05 and above: they need fewer instructions per node but
+    // 170,000 at theta 0.85 and above: they need fewer instructions per node but
     // leave one wave per 64 bodies, whose visits follow one another, and short
     // walks share less.  Traversal, ms (teams, waves, a stack per lane):
-    //   80,001 disk, 0.5      0.79   1.27   1.42
-    //   100,003 Plummer, 0.7  1.03   1.05   1.24
-    //   100,003 Plummer, 1.05 0.49   0.56   0.57
-    //   131,072 Plummer, 0.5  2.68   2.40   2.86
-    //   150,001 disk, 1.05    0.34   0.44   0.37
-    //   200,001 disk, 0.7     0.96   0.91   0.97
-    //   262,144 Plummer, 0.7  2.48   1.48   1.87
-    //   205,001 disk, 1.05    0.47   0.49   0.42
-    //   230,001 Plummer, 1.05 1.14   0.77   0.84
-    //   300,001 disk, 0.85    -      0.85   0.79
-    //   600,000 Plummer, 1.05 2.60   1.46   1.62
-    //   1,048,576 disk, 1.05  2.36   1.49   1.49
-    // (a stack per lane still did a little better on short walks of 0.2 to 0.5 M
-    // bodies of a disk, whose neighbours share little of them)
-    const double from = 100e3 + 200e3 * std::min(std::max(theta - 0.5, 0.0), 0.55);
+    //   80,001 disk, 0.5      0.80   1.19   1.43
+    //   100,003 Plummer, 0.7  1.00   1.02   1.21
+    //   100,003 Plummer, 1.05 0.48   0.54   0.55
+    //   120,001 Plummer, 0.5  2.41   2.18   2.74
+    //   150,001 disk, 1.05    0.35   0.44   0.37
+    //   150,001 Plummer, 1.05 0.66   0.63   0.66
+    //   180,001 disk, 0.85    0.61   0.64   0.57
+    //   180,001 disk, 1.05    0.41   0.45   0.40
+    //   180,001 Plummer, 1.05 0.78   0.64   0.68
+    //   205,001 disk, 0.7     0.99   0.86   1.01
+    //   205,001 disk, 1.05    0.46   0.48   0.43
+    //   205,001 Plummer, 1.05 0.89   0.69   0.77
+    //   262,144 disk, 0.85    0.86   0.75   0.68
+    //   262,144 Plummer, 0.7  2.40   1.42   1.80
+    //   300,001 disk, 0.85    0.98   0.82   0.80
+    //   300,001 disk, 1.05    0.66   0.59   0.51
+    //   400,001 disk, 1.05    0.87   0.68   0.64
+    //   500,001 disk, 1.05    1.08   0.81   0.84
+    //   600,001 Plummer, 1.05 2.49   1.35   1.54
+    //   1,048,576 disk, 1.05  2.27   1.39   1.40
+    // The line lies where the two lose as much on a disk as they gain on a Plummer
+    // sphere (the sizes alone do not tell these apart).  A stack per lane, 1.2 KB of
+    // memory per body, did better on short walks of 170,000 to 500,000 bodies of a disk,
+    // whose neighbours share little of them: up to 16 % (300,001, 1.05), and worse
+    // on the spheres of that range, by 2 to 17 %.
+    const double from = 100e3 + 200e3 * std::min(std::max(theta - 0.5, 0.0), 0.35);
     if (t.n >= from)
         hipLaunchKernelGGL(k_bh_exact_wave, dim3(ceil_div(t.n, 64 * kExactWaves)),
                            dim3(kExactThreads), 0, s, t.n, (const uint32_t *)t.sidx, x, y, z,

@@ -496,6 +496,24 @@ def test_bh_exact_kernels_bitexact(gpu, oracle, kind, n, theta):
             np.testing.assert_array_equal(bits(a), bits(r))
 
 
+# Both sides of the rule between the two kernels at larger opening angles: 170,000
+# bodies from theta 0.85 on.
+@pytest.mark.parametrize("kind,n,theta", [("plummer", 169999, 0.85), ("disk", 170017, 0.85),
+                                          ("disk", 169991, 1.05), ("plummer", 170033, 1.4)])
+def test_bh_exact_kernel_rule_bitexact(gpu, oracle, kind, n, theta):
+    d = make(gpu, kind, n, seed=23)
+    t = oracle.Tree(n)
+    t.build(d["x"], d["y"], d["z"], d["m"])
+    rx, ry, rz, rint = t.bh_accel(theta)
+    with ctx_for(gpu, d, theta=theta) as c:
+        c.bh_build()
+        ax, ay, az = c.bh_forces()
+        inter = c.interactions()
+    np.testing.assert_array_equal(inter, rint)
+    for a, r in ((ax, rx), (ay, ry), (az, rz)):
+        np.testing.assert_array_equal(bits(a), bits(r))
+
+
 def test_bh_exact_deep_runs(gpu, oracle):
     # pairs closer than edge/2^21: each pair hangs under ~25 single-child
     # cells, so the walk opens long chains whose pushed batches are all empty
