@@ -316,6 +316,29 @@ def test_tree_sort_more_tiles_than_resident(gpu, oracle):
                 assert_canonical_equal(c.tree_canonical(), t.canonical(), "3M plummer")
 
 
+def test_tree_more_scan_tiles_than_read_inline(gpu, oracle):
+    # 4,097 scan tiles of pairs and 4,098 of bodies: above 4,096 the tile sums are
+    # scanned by a launch of their own, for the cells' numbers and the groups' places.
+    # Every body must be in one group: its interactions are counted and its force
+    # is near the direct sum's (opening angle 0.7: about 1e-3 in the median).
+    n = 8390657
+    d = plummer(gpu, n)
+    t = oracle.Tree(n)
+    t.build(d["x"], d["y"], d["z"], d["m"])
+    with ctx_for(gpu, d, precision=gpu.PREC_FP32C, theta=0.7) as c:
+        c.bh_build()
+        np.testing.assert_array_equal(c.tree_sorted(), t.export()["sorted"])
+        assert c.tree_info()["node_count"] == t.node_count
+        a = c.bh_forces()
+        assert np.all(c.interactions() > 0)
+        sample = np.linspace(0, n - 1, 512).astype(np.uint32)
+        ref = c.forces_direct_targets(sample)
+    norm = np.sqrt(sum(r ** 2 for r in ref))
+    err = np.sqrt(sum((g[sample] - r) ** 2 for g, r in zip(a, ref))) / norm
+    assert np.median(err) < 3e-3, np.median(err)
+    assert np.percentile(err, 99) < 0.05, np.percentile(err, 99)
+
+
 def test_tree_sort_wide_tiles(gpu, oracle):
     # 207 sort tiles of 10,240 keys, the last one ragged: the size at which tiles
     # of 8192 keys would need a second round
