@@ -699,6 +699,29 @@ def test_state_read_back(gpu, n):
         assert all(np.all(a == 0) for a in c.accel())
 
 
+# Accelerations read back at the edges of the copy paths (three arrays: one kernel up
+# to 1.75 MiB, the runtime's copies up to 16 MiB, then chunks of 1 MiB), into memory
+# that holds something else, against the snapshot, which takes another way.
+@pytest.mark.parametrize("n", [2, 33, 21846, 30001, 76458, 76459, 349527, 699050, 699051, 800001])
+def test_accel_read_back(gpu, n):
+    d = plummer(gpu, n)
+    with ctx_for(gpu, d, precision=gpu.PREC_FP32C, theta=1.0) as c:
+        c.bh_build()
+        assert c.lib.nb_bh_forces(c.h) == 0
+        c.snapshot_begin()
+        snap = c.snapshot_wait()
+        for _ in range(2):
+            got = [np.full(n, np.nan) for _ in range(3)]
+            assert c.lib.nb_get_accel(c.h, *[g.ctypes.data_as(gpu._dp) for g in got]) == 0
+            for g, k in zip(got, ("ax", "ay", "az")):
+                np.testing.assert_array_equal(bits(g), bits(snap[k]))
+                assert np.all(np.isfinite(g)) and np.any(g != 0)
+        assert not np.array_equal(got[0], got[1]) and not np.array_equal(got[1], got[2])
+        only = np.full(n, np.nan)
+        assert c.lib.nb_get_accel(c.h, None, None, only.ctypes.data_as(gpu._dp)) == 0
+        np.testing.assert_array_equal(bits(only), bits(snap["az"]))
+
+
 def test_coincident_bodies_reported(gpu):
     d = uniform_cube(100, 2)
     d["x"][5], d["y"][5], d["z"][5] = d["x"][9], d["y"][9], d["z"][9]
