@@ -78,7 +78,7 @@ CPU_SAMPLE_S = 10.0
 TRAFFIC_BYTES = {
     ("bh_plummer_4m", 0.37375): 12.370e9,
     ("bh_disk_1m", 0.5): 2.047e9,
-    ("bh_disk_1m_exact", 0.5): 3.822e9,
+    ("bh_disk_1m_exact", 0.5): 1.291e9,
 }
 
 WORKLOADS = {

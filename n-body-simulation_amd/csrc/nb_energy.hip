@@ -18,8 +18,8 @@ namespace {
 // lane).  For each chunk of 48 sources the waves compute the terms (three
 // sources per wave, read through the scalar cache, interleaved) into one of two
 // LDS tiles, and wave 0 adds the previous tile in source order first.  Two
-// workgroups per CU (64 VGPRs; with one, 131,071 bodies take 14.4 ms instead of
-// 11.1).
+// workgroups per CU (64 VGPRs, 2 more of them spilled; with one workgroup, 131,071
+// bodies take 14.4 ms instead of 11.1).
 //
 // k_energy_rows: a lane computes and adds its body's terms by itself, eight
 // interleaved, without the workgroup's barriers and LDS tiles (about 165 cycles
@@ -161,9 +161,11 @@ __device__ inline uint32_t distance_off(double v) {
 constexpr int kRowThreads = 256;  // bodies j per block, and sources i per LDS stage
 constexpr int kRowPer = 8;        // terms interleaved
 
-// All blocks are resident from the start, dealt round the CUs, so every second
-// round of kCus blocks counts its tiles the other way: long and short rows sum
-// up alike on each CU (300,001 bodies: 58.7 ms without).
+// Up to 458,752 bodies all blocks are resident from the start (7 per CU with 68
+// VGPRs), dealt round the CUs, so every second round of kCus blocks counts its
+// tiles the other way: long and short rows sum up alike on each CU (300,001 bodies:
+// 58.7 ms without).  Beyond, the rounds still go from the longest rows to the
+// shortest, and blocks that start later fill in behind those that end.
 __global__ void __launch_bounds__(kRowThreads) k_energy_rows(
     uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ vx, const double *__restrict__ vy,

@@ -316,7 +316,7 @@ int nb_ensemble_create(nb_ensemble **out, uint32_t nsys, const uint32_t *sizes,
     if (io >= (1ull << 32) || fo >= (1ull << 30) || span >= (1ull << 32) || xo >= (1ull << 32))
         return bail(NB_E_INVALID_ARG);
     int rc;
-    // one allocation, so that the arrays of a small ensemble leave in one DMA
+    // one allocation, the arrays at equal strides of whole 256-byte lines
     double **st[] = {&e->x, &e->y, &e->z, &e->vx, &e->vy, &e->vz, &e->ax,
                      &e->ay, &e->az, &e->vhx, &e->vhy, &e->vhz, &e->m};
     const uint64_t stride = (total + 31) / 32 * 32;  // 256-byte lines

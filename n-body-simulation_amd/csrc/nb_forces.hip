@@ -369,9 +369,9 @@ __device__ __forceinline__ void split_stages(uint32_t j0, uint32_t j1,
 
 // FP32 pairs on absolute FP32 positions with G*m as the source weight; the
 // FP32 sums of every 256 sources (kF32cRun stages, from a multiple of 256) are
-// folded into FP64.  Bound by vector issue: 50,021 bodies in 0.703 ms (0.773
+// folded into FP64.  Bound by vector issue: 50,021 bodies in 0.656 ms (0.773
 // with 256-source stages shared by a block and no wait states around the
-// v_rsq_f32), 43 cycles at 2.4 GHz per 64 pairs, where a loop of such pairs alone takes 36-38.
+// v_rsq_f32), 41 cycles at 2.4 GHz per 64 pairs, where a loop of such pairs alone takes 36-38.
 // PL: targets per lane, 1 for small sums (twice the waves).
 template <int PL>
 __global__ void __launch_bounds__(kSplitThreads) __attribute__((amdgpu_waves_per_eu(8)))
@@ -453,8 +453,10 @@ k_direct_f32c(uint32_t n, const double *__restrict__ x, const double *__restrict
 // FP64 pairs (the reference's formula, NaiveAlgorithm.cpp:318-351, with
 // m r^-3 from rsqrt3_f64 and fused multiply-adds); G is applied to the sum, as
 // in the reference (:348-351).  Bound by vector issue: 16 full-rate FP64
-// instructions and the quarter-rate estimate, 80 cycles per 64 pairs; 16,384
-// bodies in 0.169-0.173 ms (0.172-0.176 before), 3001 in 0.019 ms (0.052).
+// instructions, the quarter-rate estimate and two moves (the compiler puts the
+// addend 1.5 where its fused multiply-add leaves the result), about 88 of the 96
+// cycles per 64 pairs that 16,384 bodies take; those in 0.165 ms (0.172-0.176
+// before), 3001 in 0.0145 ms (0.052).
 __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
     uint32_t n, const double *__restrict__ x, const double *__restrict__ y,
     const double *__restrict__ z, const double *__restrict__ m, double G, double eps2,
@@ -525,7 +527,7 @@ __global__ void __launch_bounds__(kSplitThreads) k_direct_f64f(
 // Two kernels walk it in that order, one for small systems and one for large
 // ones (launch_bh_exact chooses).  A stack per lane, one body per lane, loaded
 // each node's record from 64 places and ran the branch of the term for the few
-// lanes that needed it: 1M-body disk at theta 0.5 10.4 ms, now 6.0 (waves); 1024
+// lanes that needed it: 1M-body disk at theta 0.5 10.4 ms, now 5.5 (waves); 1024
 // bodies 0.52 ms, now 0.107; 30,001 (Plummer, theta 1.05) 0.47, now 0.174
 // (teams).
 //
@@ -776,7 +778,7 @@ k_bh_exact_team(uint32_t n, const uint32_t *__restrict__ order, const double *__
 // same for the whole wave: its record is an LDS broadcast (through v_readlane or
 // the scalar cache: 7.2 and 8.2 ms on the 1M-body disk), empty slots cost a bit
 // of a mask.  Bound by FP64 issue: on that disk a wave visits 2826 nodes, of
-// which a body accepts 1130, at about 320 cycles each.
+// which a body accepts 1130, at about 290 cycles each.
 constexpr uint32_t kFrames = 8;  // levels of a wave's path whose children are kept in LDS
 struct WaveLds {
     double4 cm[kFrames][8];           // by visit position
@@ -1983,9 +1985,11 @@ __device__ inline void direct_tile(const double *__restrict__ x, const double *_
 // Persistent: every wave takes items from the queue until it is empty.  As in
 // k_bh_group the queue is cut into one contiguous chunk per XCD (the items of a
 // system follow each other, so its tree stays in one L2) and a wave goes on with
-// the next chunk when its own is empty, and 96 VGPRs leave five waves per SIMD.
-// 128 systems, 2.1 million bodies: 1.97 ms with one queue and four waves, 1.89 now
-// (1.91 with one queue); 24 systems 0.600 and 0.555; 512 systems 6.25 and 6.14.
+// the next chunk when its own is empty, and 96 VGPRs leave five waves per
+// SIMD (the walk's constants of a system do not all fit: 6 VGPRs and 28 SGPRs are spilled,
+// 28 bytes of scratch).  One queue, four waves per SIMD and no VGPR spilled before; forces
+// of a step, ms, before and now: 24 systems (0.4 million bodies) 0.634 and 0.555, 128 (1.9
+// million) 1.72 and 1.69, 512 (8.0 million) 6.75 and 6.66.
 __global__ void __launch_bounds__(kGroup) __attribute__((amdgpu_waves_per_eu(5)))
 k_ens_forces(EnsForceArgs a) {
     __shared__ uint32_t stk[kStackCap];
@@ -2096,10 +2100,11 @@ struct SplitPlan {
 };
 // Small sums are cut as finely as the kernels allow (one run or stage per wave
 // and, FP32, one target per lane), to have as many waves as they can: FP32
-// 0.0147 ms for 1024 bodies, 0.0177 for 3001 and 0.0545 for 12,001 (two targets
-// per lane 0.024, 0.027 and 0.059; blocks of 512 targets and 256 sources 0.027,
-// 0.050 and 0.081); at 16,384 both take 0.086, beyond, two targets per lane are
-// faster (50,021: 0.703 against 0.725).
+// 0.013 ms for 1024 bodies, 0.0175 for 3001 and 0.051 for 12,001 with the reduction
+// (two targets per lane 0.024, 0.027 and 0.059; blocks of 512 targets and 256
+// sources 0.027, 0.050 and 0.081); at 16,384 both were alike, beyond, two targets per lane
+// faster (50,021: 0.703 against 0.725).  Figures of the alternatives are those of
+// stages that went through scratch memory, 3 to 7 % slower than now.
 SplitPlan split_plan(bool fp64, uint32_t n) {
     SplitPlan p;
     p.per_lane = fp64 ? (uint32_t)kF64fPerLane : (n < 16384 ? 1u : 2u);

@@ -1,7 +1,7 @@
 // nb_hostcopy.h -- device arrays into a caller's pageable host memory.
 //
-// hipMemcpyAsync into pageable memory takes about 17 us per call and runs at
-// 8 GB/s, bound by one thread that faults in and fills the caller's pages.  Here
+// hipMemcpyAsync into pageable memory takes 9 to 21 us per call and runs at 8 to
+// 18 GB/s, bound by one thread that faults in and fills the caller's pages.  Here
 // the arrays go through pinned memory owned by the context or ensemble:
 //  - small copies (up to kSmall) by one kernel that stores them there, one wait,
 //    and a memcpy per array;
@@ -49,7 +49,7 @@ class HostCopier {
     // Pinned memory for the copies of six arrays (a state) or three (accelerations) of
     // n doubles, made with its owner: a first copy would pay for the allocation and
     // for a fault per page (1.6 us).  The first accelerations of 30,001 bodies took
-    // 83 us that way, 45 now; the first state of 360,000 1.4 ms.
+    // 83 us that way, 52 now; the first state of 360,000 1.4 ms, 0.9 now.
     void reserve_for(size_t n) noexcept {
         if (6 * n * sizeof(double) >= kLarge) {
             if (reserve(kSlots * kChunk)) (void)make_events();

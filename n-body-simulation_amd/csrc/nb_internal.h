@@ -1,10 +1,10 @@
 // nb_internal.h -- shared declarations of libnbody_hip.so (not installed).
 //
 // Data layout in HBM (all arrays structure-of-arrays, 256-byte aligned):
-//   state     x y z vx vy vz vhx vhy vhz ax ay az m        13 x N doubles
+//   state     x y z vx vy vz ax ay az vhx vhy vhz m        13 x N doubles, one allocation
 //   octree    per sorted position:  skey (u64), sidx (u32), klo (u64), lcp (i32)
-//             per internal node k:  depth, parent, node id, child count,
-//                                   arrival counter, sums {x*m, y*m, z*m, m}, count
+//             per internal node k:  depth, node id, first sorted position, body count,
+//                                   sums {x*m, y*m, z*m, m}, blocks crossed (int_local)
 //             per node id:          ref (i32), cm {com_x, com_y, com_z, m} (double4)
 //                                   or an FP32 record (NodeF32)
 // A node id is 0 for the root and 1 + 8*k + digit for the child with octant
